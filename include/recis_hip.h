@@ -286,6 +286,36 @@ int recis_idmap_clear(recis_idmap* m, void* stream);
 /* IdMap::Reserve (not implemented for the reference GPU map, gpu_id_map.cu:105-108). */
 int recis_idmap_reserve(recis_idmap* m, int64_t n_keys, void* stream);
 
+/* mode of recis_lookup_pool_readonly beside RECIS_SUM and RECIS_MEAN: the sum over the segment divided by the sum of
+ * its weights (the sparse-mode mean, csrc/ops/segment_ops_kernel.cu:92-108) */
+#define RECIS_LOOKUP_WEIGHT_MEAN 4
+
+/* One feature of recis_lookup_pool_readonly. */
+typedef struct recis_lookup_job {
+  const int64_t* ids;   /* [n_ids] */
+  int64_t n_ids;
+  const void* offsets;  /* [n_seg + 1] int32 / int64; NULL: n_seg segments of `width` ids each */
+  int off_is64;
+  int64_t n_seg;
+  int64_t width;
+  const void* weight;   /* [n_ids] or NULL = 1; rounded to the row type first */
+  int weight_dtype;
+  int64_t table_id;     /* with `tagged`: ids are looked up as (id & (2^52 - 1)) | table_id << 52 (ids_encode) */
+} recis_lookup_job;
+
+/*
+ * The evaluation forward of an embedding in one pass, for n_jobs features of one table: every id is
+ * looked up in the map (nothing is inserted; an unknown key reads as a row of zeros), the rows are
+ * read where the blocks keep them and pooled per segment. `out` [sum of n_seg, D] of the row type,
+ * feature after feature; float32 accumulation. Stands in for ids_encode + ids_partition +
+ * IdMap::Lookup(readonly) + block_gather + segment_reduce_forward
+ * (csrc/embedding/hashtable.cc:153-165, recis/nn/modules/embedding_engine.py:607-675). mode:
+ * RECIS_SUM, RECIS_MEAN or RECIS_LOOKUP_WEIGHT_MEAN.
+ */
+int recis_lookup_pool_readonly(recis_idmap* map, const recis_lookup_job* jobs, int64_t n_jobs, int tagged,
+                               const void* const* emb_blocks_dev, int64_t n_blocks, int64_t block_rows,
+                               int64_t row_pitch_bytes, int row_dtype, void* out, int64_t D, int mode, void* stream);
+
 /*
  * Stand-alone allocator ops over a caller-held free list kept in blocks
  * (device array of block pointers).

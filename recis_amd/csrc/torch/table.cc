@@ -833,6 +833,74 @@ c10::optional<std::tuple<BatchPlanPtr, at::Tensor, at::Tensor>> Hashtable::Dense
   return std::make_tuple(plan, index, out);
 }
 
+std::vector<at::Tensor> Hashtable::LookupPoolReadonly(const std::vector<at::Tensor>& values,
+                                                      const std::vector<c10::optional<at::Tensor>>& offsets,
+                                                      const std::vector<c10::optional<at::Tensor>>& weights,
+                                                      const c10::optional<std::vector<int64_t>>& tags, bool mean) {
+  const size_t n = values.size();
+  TORCH_CHECK(n > 0 && offsets.size() == n && weights.size() == n && (!tags.has_value() || tags->size() == n),
+              "lookup_pool_readonly: one entry per feature in every list");
+  c10::DeviceGuard guard(device_);
+  MakeRoom(0);
+  auto emb = slot_group_->EmbSlot();
+  const auto& chunks = emb->Chunks();
+  const int64_t D = emb->FlatSize();
+  const int code = dtype_code(dtype_);
+  std::vector<recis_lookup_job> jobs(n);
+  std::vector<at::Tensor> keep;  // converted inputs, alive until the launch is queued
+  keep.reserve(3 * n);
+  auto here = [&](const at::Tensor& t, at::ScalarType type) -> const at::Tensor& {
+    if (t.device() == device_ && t.scalar_type() == type && t.is_contiguous()) return t;
+    keep.push_back(t.to(at::TensorOptions().device(device_).dtype(type)).contiguous());
+    return keep.back();
+  };
+  int64_t total = 0, n_ids = 0;
+  std::vector<int64_t> split(n);
+  for (size_t k = 0; k < n; ++k) {
+    recis_lookup_job& j = jobs[k];
+    const at::Tensor& v = here(values[k], at::kLong);
+    j.ids = v.data_ptr<int64_t>();
+    j.n_ids = v.numel();
+    if (offsets[k].has_value() && offsets[k]->defined()) {
+      const at::Tensor& o = here(*offsets[k], offsets[k]->scalar_type() == at::kLong ? at::kLong : at::kInt);
+      TORCH_CHECK(o.numel() >= 1, "offsets must hold at least one entry");
+      j.offsets = o.data_ptr();
+      j.off_is64 = index_kind(o, "offsets");
+      j.n_seg = o.numel() - 1;
+      j.width = 0;
+    } else {
+      j.offsets = nullptr;
+      j.off_is64 = 0;
+      j.width = values[k].dim() <= 1 ? 1 : values[k].size(-1);
+      j.n_seg = j.width > 0 ? j.n_ids / j.width : 0;
+    }
+    j.weight = nullptr;
+    j.weight_dtype = 0;
+    if (weights[k].has_value() && weights[k]->defined()) {
+      const auto type = weights[k]->scalar_type();
+      const bool taken = type == at::kFloat || type == at::kBFloat16 || type == at::kHalf;
+      const at::Tensor& w = here(*weights[k], taken ? type : dtype_);
+      TORCH_CHECK(w.numel() == j.n_ids, "weight holds ", w.numel(), " values for ", j.n_ids, " ids");
+      j.weight = w.data_ptr();
+      j.weight_dtype = dtype_code(w.scalar_type());
+    }
+    j.table_id = tags.has_value() ? (*tags)[k] : 0;
+    split[k] = j.n_seg;
+    total += j.n_seg;
+    n_ids += j.n_ids;
+  }
+  const int mode = !mean ? RECIS_SUM : n_ids > 5 * (total + 1) ? RECIS_MEAN : RECIS_LOOKUP_WEIGHT_MEAN;
+  at::Tensor out = at::empty({total, D}, at::TensorOptions().device(device_).dtype(dtype_));
+  at::Tensor table = block_ptr_table(chunks);
+  check(recis_lookup_pool_readonly(map_->map, jobs.data(), static_cast<int64_t>(n), tags.has_value() ? 1 : 0,
+                                   reinterpret_cast<const void* const*>(table.data_ptr()),
+                                   static_cast<int64_t>(chunks.size()), emb->ChunkRows(),
+                                   recis::hipabi::row_pitch_bytes(chunks[0]), code, out.data_ptr(), D, mode,
+                                   stream_of(device_)));
+  if (n == 1) return {out};
+  return at::split_with_sizes(out, split, 0);
+}
+
 void Hashtable::AcceptSplitGrad(const at::Tensor& index_in, const BatchPlanPtr& plan,
                                 const std::vector<c10::optional<at::Tensor>>& grads, const std::vector<int64_t>& split,
                                 const c10::optional<at::Tensor>& src, const c10::optional<at::Tensor>& coef, int64_t key,

@@ -307,6 +307,15 @@ class Hashtable : public torch::CustomClassHolder {
   c10::optional<std::tuple<recis::BatchPlanPtr, at::Tensor, at::Tensor>> DenseLookupExpand(
       const std::vector<at::Tensor>& cols, const c10::optional<std::vector<int64_t>>& tags,
       const c10::optional<std::string>& stamp_slot, const c10::optional<at::Tensor>& stamp_value);
+  // The evaluation forward of several features in one pass (recis_lookup_pool_readonly): ids straight to
+  // pooled rows, no batch plan, nothing inserted. offsets[k] undefined = the rows of a dense tensor
+  // ([B] or [..., width]). One [segments, D] output per feature, views of one buffer. `mean`: over
+  // more than five ids per segment on average the sum is divided by the length of the segment, else by
+  // the sum of its weights (recis/nn/functional/embedding_ops.py:332-420).
+  std::vector<at::Tensor> LookupPoolReadonly(const std::vector<at::Tensor>& values,
+                                             const std::vector<c10::optional<at::Tensor>>& offsets,
+                                             const std::vector<c10::optional<at::Tensor>>& weights,
+                                             const c10::optional<std::vector<int64_t>>& tags, bool mean);
   // The backward of an output that was handed out in parts (`split` rows each): `grads` are the parts'
   // gradients as autograd delivers them (None = zeros). Consecutive slices of one buffer are used in
   // place, anything else is concatenated; then the count of `plan` is settled (`settle`) and the

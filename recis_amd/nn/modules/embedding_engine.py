@@ -14,6 +14,7 @@ which is the reference's group_exchange_ids / group_exchange_embs / group_reduce
 pipeline with the all-to-alls removed (one GPU owns the whole table).
 """
 import hashlib
+import math
 from collections import OrderedDict
 from typing import Dict, Union
 
@@ -113,6 +114,33 @@ class EmbeddingEngine(torch.nn.Module):
             values = values.long()
         return values, weight, offsets.to(torch.int32), shape, unit, dense
 
+    def _evaluate(self, table, info, tag_of, names, opt0, inputs, outputs):
+        """The features of one runtime group in evaluation mode: ids straight to pooled rows in one native call
+        (``HashtableImpl.lookup_pool_readonly``), without the plan a training lookup makes for its backward."""
+        vals, offs, weights, prefixes = [], [], [], []
+        for name in names:
+            data = inputs[name]
+            if type(data) is torch.Tensor:
+                vals.append(data)
+                offs.append(None)
+                weights.append(None)
+                prefixes.append(None if data.dim() <= 2 else data.shape[:-1])
+            elif isinstance(data, RaggedTensor):
+                offsets = data.offsets()[-1]
+                shape = data.real_shape(0, -1)
+                if math.prod(shape) != offsets.numel() - 1:
+                    raise RuntimeError("RaggedTensor must pad before lookup, got: %s (%s)" % (data, name))
+                vals.append(data.values())
+                offs.append(offsets)
+                weights.append(data.weight() if opt0.use_weight else None)
+                prefixes.append(None if len(shape) == 1 else shape)
+            else:
+                raise TypeError("feature %s: expected RaggedTensor or Tensor, got %s" % (name, type(data)))
+        parts = table._hashtable_impl.lookup_pool_readonly(
+            vals, offs, weights, [tag_of[n] for n in names] if info.is_coalesce() else None, opt0.combiner == "mean")
+        for name, part, prefix in zip(names, parts, prefixes):
+            outputs[name] = part if prefix is None else part.reshape(tuple(prefix) + (part.shape[1],))
+
     def forward(self, inputs: Dict[str, Union[torch.Tensor, RaggedTensor]]):
         outputs = {}
         # the same input objects under two combiners (a sequence pooled AND kept row by row) are
@@ -144,6 +172,10 @@ class EmbeddingEngine(torch.nn.Module):
                             for name, part in zip(names, res[1:]):
                                 outputs[name] = part
                             continue
+                if (not table.training and opt0.combiner in ("sum", "mean")
+                        and table._dtype in (torch.float32, torch.bfloat16, torch.float16)):
+                    self._evaluate(table, info, tag_of, names, opt0, inputs, outputs)
+                    continue
                 vals, weights, offs, shapes, dense = [], [], [], [], []
                 all_unit = True
                 any_weight = opt0.use_weight and any(

@@ -343,6 +343,11 @@ class HashTable(torch.nn.Module):
             if hooked:
                 self._filter_hook_impl(emb_idx)
             return embedding.view(shape + tuple(embedding.shape[1:])) if len(shape) != 1 else embedding
+        if not self.training and len(self._embedding_shape) == 1 and self._dtype in (torch.float32, torch.bfloat16,
+                                                                                    torch.float16):
+            # nothing is inserted and nothing flows back: ids straight to rows, no dedup
+            embedding = self._hashtable_impl.lookup_pool_readonly([ids], [None], [None], None, False)[0]
+            return embedding.view(shape + tuple(embedding.shape[1:])) if len(shape) != 1 else embedding
         uids, index, plan = self._unique(ids)
         if self.training and self._dtype not in (torch.int8, torch.int32, torch.int64):
             emb_idx, embedding = HashTableLookupHelpFunction.apply(uids, self._hashtable_impl,
