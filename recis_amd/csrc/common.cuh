@@ -240,7 +240,14 @@ struct KernelTimer {
 int get_workspace(hipStream_t stream, size_t bytes, void** out);
 
 // Per-(device, stream) pinned host words and an event, for handing a device-side count to the
-// host while later kernels of the same call are still running.
+// host while later kernels of the same call are still running. Every call takes the next of
+// kCountRing slots (a ticket); a slot is handed out again kCountRing calls later.
+constexpr int kCountRing = 16;
 int get_count_staging(hipStream_t stream, int64_t** host, hipEvent_t* event);
+int64_t last_count_ticket(hipStream_t stream);  // this thread's last one on the stream, else the stream's; -1: none yet
+// The slot of `ticket`; false when it was never issued or has been handed out again.
+bool find_count_staging(hipStream_t stream, int64_t ticket, int64_t** host, hipEvent_t* event);
+// One more pinned word of the stream, for a call that waits for the stream before it reads it.
+int get_flag_word(hipStream_t stream, int64_t** host);
 
 }  // namespace recis_hip

@@ -318,10 +318,8 @@ extern "C" int recis_partition_order(const int64_t* ids, int64_t n, int64_t* sor
   if (int rc = get_workspace(stream, std::max(sort_off + sort_bytes, bins_bytes) + 256, &ws)) return rc;
 
   if (nb_log2 >= 0) {
-    int64_t* staged = nullptr;
-    hipEvent_t staged_event = nullptr;
-    if (int rc = get_count_staging(stream, &staged, &staged_event)) return rc;
-    int64_t* too_big = staged + 2;  // (words 0 and 1 are the batch plan's)
+    int64_t* too_big = nullptr;
+    if (int rc = get_flag_word(stream, &too_big)) return rc;
     int32_t* bin_total = static_cast<int32_t*>(ws);
     int32_t* bin_cursor = bin_total + nb;
     int32_t* bin_start = bin_cursor + nb;

@@ -87,24 +87,68 @@ int get_workspace(hipStream_t stream, size_t bytes, void** out) {
   return RECIS_OK;
 }
 
+// A ring of pinned words per (device, stream), so that the counts of several plans can be under way
+// at once: a caller that does not wait for a count can still fetch it after it has queued later plans.
 struct CountStaging {
-  int64_t* host = nullptr;  // pinned
-  hipEvent_t event = nullptr;
+  int64_t* host = nullptr;  // pinned, kCountRing slots of 8 words and one more for get_flag_word
+  hipEvent_t event[kCountRing] = {};
+  int64_t issued = 0;       // the next ticket; ticket t uses slot t % kCountRing
 };
 static std::map<std::pair<int, hipStream_t>, CountStaging> g_staging;
 
+// the last ticket this thread took: two threads may queue plans on one stream
+struct LastTicket {
+  int dev = -1;
+  hipStream_t stream = nullptr;
+  int64_t ticket = -1;
+};
+static thread_local LastTicket t_last;
+
+static int staging_of(int dev, hipStream_t stream, CountStaging** out) {  // g_mu is held
+  CountStaging& c = g_staging[std::make_pair(dev, stream)];
+  if (c.host == nullptr) {
+    RECIS_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&c.host), 64 * (kCountRing + 1), hipHostMallocDefault));
+    for (int w = 0; w < 8 * (kCountRing + 1); ++w) c.host[w] = 0;
+    for (int k = 0; k < kCountRing; ++k) RECIS_CHECK_HIP(hipEventCreateWithFlags(&c.event[k], hipEventDisableTiming));
+  }
+  *out = &c;
+  return RECIS_OK;
+}
+
 int get_count_staging(hipStream_t stream, int64_t** host, hipEvent_t* event) {
+  const int dev = current_device();
+  std::lock_guard<std::mutex> l(g_mu);
+  CountStaging* c = nullptr;
+  if (int rc = staging_of(dev, stream, &c)) return rc;
+  t_last = LastTicket{dev, stream, c->issued++};
+  *host = c->host + 8 * (t_last.ticket % kCountRing);
+  *event = c->event[t_last.ticket % kCountRing];
+  return RECIS_OK;
+}
+
+int get_flag_word(hipStream_t stream, int64_t** host) {
+  std::lock_guard<std::mutex> l(g_mu);
+  CountStaging* c = nullptr;
+  if (int rc = staging_of(current_device(), stream, &c)) return rc;
+  *host = c->host + 8 * kCountRing;
+  return RECIS_OK;
+}
+
+int64_t last_count_ticket(hipStream_t stream) {
+  const int dev = current_device();
+  if (t_last.dev == dev && t_last.stream == stream) return t_last.ticket;
+  std::lock_guard<std::mutex> l(g_mu);
+  return g_staging[std::make_pair(dev, stream)].issued - 1;
+}
+
+bool find_count_staging(hipStream_t stream, int64_t ticket, int64_t** host, hipEvent_t* event) {
   int dev = current_device();
   std::lock_guard<std::mutex> l(g_mu);
   CountStaging& c = g_staging[std::make_pair(dev, stream)];
-  if (c.host == nullptr) {
-    RECIS_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&c.host), 64, hipHostMallocDefault));
-    for (int w = 0; w < 8; ++w) c.host[w] = 0;
-    RECIS_CHECK_HIP(hipEventCreateWithFlags(&c.event, hipEventDisableTiming));
-  }
-  *host = c.host;
-  *event = c.event;
-  return RECIS_OK;
+  if (ticket < 0 || ticket >= c.issued || c.issued - ticket > kCountRing) return false;
+  *host = c.host + 8 * (ticket % kCountRing);
+  *event = c.event[ticket % kCountRing];
+  return true;
 }
 
 bool g_profile_on = false;

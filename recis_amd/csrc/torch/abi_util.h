@@ -114,6 +114,8 @@ inline std::vector<int64_t> numels(const std::vector<at::Tensor>& ts) {
 // A 1-D integer tensor on any device as host values.
 std::vector<int64_t> host_values(const at::Tensor& t);
 
+using TensorOrNone = c10::optional<at::Tensor>;
+
 inline const void* opt_ptr(const c10::optional<at::Tensor>& t) {
   return t.has_value() && t->defined() ? t->data_ptr() : nullptr;
 }

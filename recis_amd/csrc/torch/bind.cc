@@ -199,6 +199,8 @@ TORCH_LIBRARY(recis, m) {
       .def("settle_lookup", &Hashtable::SettleLookup)
       .def("expand_rows", &Hashtable::ExpandRows)
       .def("dense_lookup_expand", &Hashtable::DenseLookupExpand)
+      .def("dense_lookup_train", &Hashtable::DenseLookupTrain)
+      .def("lookup_train", &Hashtable::LookupTrain)
       .def("lookup_pool_readonly", &Hashtable::LookupPoolReadonly)
       .def("accept_split_grad", &Hashtable::AcceptSplitGrad)
       .def("accept_grad_ex", &Hashtable::AcceptGradEx)

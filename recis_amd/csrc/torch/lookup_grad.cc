@@ -1,0 +1,288 @@
+// The training lookups of the module layer with their autograd nodes: what EmbeddingEngine and
+// HashTable call once per table and step (recis/nn/modules/embedding_engine.py:607-675,
+// recis/nn/modules/hashtable.py:425-586). The forward queues dedup + lookup + pooling, the node's
+// backward hands the gradients to the table unsummed; neither waits for the device, and nothing per
+// feature is left to Python (a node written in Python costs 2 us per output each way: with 39
+// features that was most of a small step).
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/function.h>
+#include <torch/csrc/autograd/functions/utils.h>
+
+#include <algorithm>
+
+#include "abi_util.h"
+#include "ops.h"
+#include "table.h"
+
+using recis::BatchPlanPtr;
+using recis::hipabi::block_ptr_table;
+using recis::hipabi::check;
+using recis::hipabi::dtype_code;
+using recis::hipabi::index_kind;
+using recis::hipabi::stream_of;
+using recis::hipabi::TensorOrNone;
+
+namespace {
+
+// Rows [first, first + rows) of a contiguous [n, D] buffer as a tensor of its own (not a view in
+// autograd's sense: the parts do not overlap and each is an output of the node).
+at::Tensor rows_of(const at::Tensor& whole, int64_t first, at::IntArrayRef shape) {
+  auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(whole.storage()), whole.key_set(), whole.dtype());
+  impl->set_storage_offset(whole.storage_offset() + first * whole.size(1));
+  impl->set_sizes_contiguous(shape);
+  return at::Tensor(std::move(impl));
+}
+
+// The backward of one lookup of a table: the parts' gradients go to the table as they come.
+struct LookupBackward : public torch::autograd::Node {
+  c10::intrusive_ptr<Hashtable> table;
+  BatchPlanPtr plan;
+  at::Tensor index;
+  std::vector<int64_t> split;        // rows per output
+  at::Tensor offsets, weight;        // pooled segments; both undefined: one id per segment
+  bool mean = false;
+  std::vector<int64_t> batch, seq;   // padded outputs (tile): samples and rows per sample of each
+  bool tile = false;
+
+  torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+    TORCH_CHECK(plan.defined(), torch::autograd::ERR_BACKWARD_TWICE);
+    at::NoGradGuard no_grad;
+    if (tile) {
+      table->AcceptTileGrad(index, plan, offsets, batch, seq, grads);
+      return {};
+    }
+    std::vector<TensorOrNone> parts;
+    parts.reserve(grads.size());
+    for (auto& g : grads) parts.push_back(g.defined() ? TensorOrNone(std::move(g)) : c10::nullopt);
+    TensorOrNone src, coef;
+    if (offsets.defined()) {
+      auto lists = plan->SrcCoefForPool(offsets, weight.defined() ? TensorOrNone(weight) : c10::nullopt, mean);
+      src = std::get<0>(lists);
+      coef = std::get<1>(lists);
+    }
+    table->AcceptSplitGrad(index, plan, parts, split, src, coef, plan->serial(), /*may_miss=*/false, /*settle=*/false);
+    return {};
+  }
+  void release_variables() override {
+    plan.reset();
+    index.reset();
+    offsets.reset();
+    weight.reset();
+  }
+  std::string name() const override { return "RecisLookupBackward"; }
+};
+
+// The outputs of a lookup, with the node behind them when gradients are recorded.
+std::vector<at::Tensor> outputs_of(const at::Tensor& whole, const std::vector<std::vector<int64_t>>& shapes,
+                                   const std::vector<int64_t>& split, const std::shared_ptr<LookupBackward>& node) {
+  std::vector<at::Tensor> out;
+  out.reserve(split.size());
+  int64_t first = 0;
+  for (size_t k = 0; k < split.size(); ++k) {
+    out.push_back(rows_of(whole, first, shapes[k]));
+    first += split[k];
+  }
+  if (at::GradMode::is_enabled()) {
+    for (auto& o : out) torch::autograd::set_history(o, node);
+  }
+  return out;
+}
+
+}  // namespace
+
+c10::optional<std::vector<at::Tensor>> Hashtable::DenseLookupTrain(const std::vector<at::Tensor>& cols,
+                                                                   const c10::optional<std::vector<int64_t>>& tags,
+                                                                   const c10::optional<std::string>& stamp_slot,
+                                                                   const c10::optional<at::Tensor>& stamp_value) {
+  auto found = DenseLookupExpand(cols, tags, stamp_slot, stamp_value);
+  if (!found.has_value()) return c10::nullopt;
+  auto node = std::make_shared<LookupBackward>();
+  node->table = c10::intrusive_ptr<Hashtable>::reclaim_copy(this);
+  node->plan = std::get<0>(*found);
+  node->index = std::get<1>(*found);
+  const at::Tensor& out = std::get<2>(*found);
+  std::vector<std::vector<int64_t>> shapes;
+  for (const auto& c : cols) {
+    node->split.push_back(c.size(0));
+    shapes.push_back({c.size(0), out.size(1)});
+  }
+  NoteUnsettled(node->plan);
+  return outputs_of(out, shapes, node->split, node);
+}
+
+// Segments of several features as one list: the given offsets, and 0, width, 2 * width, ... for the dense
+// tensors (undefined entries). int32.
+at::Tensor Hashtable::GroupOffsets(const std::vector<TensorOrNone>& offsets, const std::vector<int64_t>& segments,
+                                   const std::vector<int64_t>& widths, const std::vector<int64_t>& n_ids) const {
+  auto i32 = at::TensorOptions().device(device_).dtype(at::kInt);
+  std::vector<at::Tensor> offs;
+  for (size_t k = 0; k < offsets.size(); ++k) {
+    if (offsets[k].has_value() && offsets[k]->defined()) {
+      offs.push_back(offsets[k]->to(i32).contiguous());
+    } else {
+      offs.push_back(at::arange(segments[k] + 1, i32).mul_(widths[k]));
+    }
+  }
+  if (offs.size() == 1) return offs[0];
+  auto ptrs = recis::hipabi::host_ptrs<void>(offs);
+  auto sizes = recis::hipabi::numels(offs);
+  int64_t total = 1;
+  for (int64_t s : segments) total += s;
+  at::Tensor out = at::empty({total}, i32);
+  check(recis_merge_offsets(ptrs.data(), sizes.data(), n_ids.data(), static_cast<int64_t>(offs.size()), 0, out.data_ptr(),
+                            stream_of(device_)));
+  return out;
+}
+
+c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor>> Hashtable::LookupTrain(
+    const std::vector<at::Tensor>& values, const std::vector<TensorOrNone>& offsets,
+    const std::vector<TensorOrNone>& weights, const c10::optional<std::vector<int64_t>>& tags,
+    const std::string& combiner, const std::vector<int64_t>& tile_len, bool lean,
+    const c10::optional<BatchPlanPtr>& shared_plan, const c10::optional<at::Tensor>& shared_offsets) {
+  const size_t n = values.size();
+  TORCH_CHECK(n > 0 && offsets.size() == n && weights.size() == n, "lookup_train: one entry per feature in every list");
+  TORCH_CHECK(combiner == "sum" || combiner == "mean" || combiner == "tile", "lookup_train: combiner ", combiner);
+  const bool tile = combiner == "tile", mean = combiner == "mean";
+  TORCH_CHECK(!tile || tile_len.size() == n, "lookup_train: one tile_len per feature");
+  c10::DeviceGuard guard(device_);
+  std::vector<at::Tensor> ids;
+  std::vector<int64_t> segments(n), widths(n), n_ids(n);
+  ids.reserve(n);
+  bool unit = true, any_weight = false;
+  int64_t total_ids = 0, total_segments = 0;
+  for (size_t k = 0; k < n; ++k) {
+    const at::Tensor& v = values[k];
+    const bool as_is = v.device() == device_ && v.scalar_type() == at::kLong && v.is_contiguous();
+    ids.push_back((as_is ? v : v.to(at::TensorOptions().device(device_).dtype(at::kLong)).contiguous()).view({-1}));
+    n_ids[k] = ids[k].numel();
+    if (offsets[k].has_value() && offsets[k]->defined()) {
+      segments[k] = offsets[k]->numel() - 1;
+      unit = false;
+    } else {
+      widths[k] = v.dim() <= 1 ? 1 : v.size(-1);
+      segments[k] = widths[k] > 0 ? n_ids[k] / widths[k] : 0;
+      unit = unit && widths[k] == 1;
+    }
+    any_weight = any_weight || (weights[k].has_value() && weights[k]->defined());
+    total_ids += n_ids[k];
+    total_segments += segments[k];
+  }
+  // few ids per segment: "mean" divides by the sum of the weights (embedding_ops.py:332-420), another path
+  if (mean && !(static_cast<double>(total_ids) / static_cast<double>(total_segments + 1) > 5)) return c10::nullopt;
+  const bool unit_path = unit && !tile;
+
+  BatchPlanPtr plan;
+  at::Tensor merged;
+  if (shared_plan.has_value() && shared_plan->defined()) {
+    plan = *shared_plan;
+    merged = shared_offsets.has_value() ? *shared_offsets : at::Tensor();
+  } else {
+    plan = PlanLookup(ids, tags, /*wait=*/false, /*need_inverse=*/!(unit_path && lean), /*need_pos=*/false);
+  }
+  if (!merged.defined() && !unit_path) merged = GroupOffsets(offsets, segments, widths, n_ids);
+  c10::optional<at::Tensor> found = PlanIndex(plan);
+  at::Tensor index = found.has_value() ? *found : LookupIndexCounted(plan, true);
+
+  auto node = std::make_shared<LookupBackward>();
+  node->table = c10::intrusive_ptr<Hashtable>::reclaim_copy(this);
+  node->plan = plan;
+  node->index = index;
+  node->offsets = merged;
+  node->mean = mean;
+  auto emb = slot_group_->EmbSlot();
+  const auto& chunks = emb->Chunks();
+  const int64_t D = emb->FlatSize();
+  std::vector<std::vector<int64_t>> shapes(n);
+  at::Tensor out;
+  if (tile) {
+    const int64_t U = plan->U();  // the padded gather reads a dense copy of the rows: this forward needs the count
+    at::Tensor rows = recis::functional::block_gather(SettleLookup(index, U, plan), chunks, emb->ChunkRows(), kNullIndex,
+                                                      false);
+    out = recis::functional::ragged_tile(segments, tile_len, plan->inverse(), merged, rows)[0];
+    node->tile = true;
+    node->batch = segments;
+    node->seq = tile_len;
+    for (size_t k = 0; k < n; ++k) {
+      node->split.push_back(segments[k] * tile_len[k]);
+      shapes[k] = {segments[k], tile_len[k] * D};
+    }
+  } else {
+    at::Tensor weight;
+    if (any_weight) {
+      std::vector<at::Tensor> parts;
+      auto opt = at::TensorOptions().device(device_).dtype(dtype_);
+      for (size_t k = 0; k < n; ++k) {
+        const bool has = weights[k].has_value() && weights[k]->defined();
+        TORCH_CHECK(!has || weights[k]->numel() == n_ids[k], "weight holds ", has ? weights[k]->numel() : 0,
+                    " values for ", n_ids[k], " ids");
+        parts.push_back(has ? weights[k]->reshape({-1}).to(opt) : at::ones({n_ids[k]}, opt));
+      }
+      weight = n == 1 ? parts[0].contiguous() : at::cat(parts);
+      node->weight = weight;
+      // (the backward of one weighted id per segment walks the segments like any other)
+      if (unit_path) node->offsets = GroupOffsets(offsets, segments, widths, n_ids);
+    }
+    if (unit_path) {
+      out = ExpandRows(plan, index, weight.defined() ? c10::optional<at::Tensor>(weight) : c10::nullopt, c10::nullopt,
+                       c10::nullopt);
+    } else {
+      at::Tensor rev = plan->inverse(), table = block_ptr_table(chunks);
+      out = at::empty({total_segments, D}, chunks[0].options());
+      check(recis_segment_reduce_forward_blocks(
+          reinterpret_cast<const void* const*>(table.data_ptr()), static_cast<int64_t>(chunks.size()), emb->ChunkRows(),
+          recis::hipabi::row_pitch_bytes(chunks[0]), index.data_ptr<int64_t>(), dtype_code(dtype_),
+          weight.defined() ? weight.data_ptr() : nullptr, weight.defined() ? dtype_code(weight.scalar_type()) : 0,
+          rev.data_ptr(), 0, merged.data_ptr(), index_kind(merged, "offsets"), out.data_ptr(), dtype_code(dtype_), plan->n(),
+          index.numel(), total_segments, D, mean ? RECIS_MEAN : RECIS_SUM, stream_of(device_)));
+    }
+    node->split = segments;
+    for (size_t k = 0; k < n; ++k) shapes[k] = {segments[k], D};
+  }
+  NoteUnsettled(plan);
+  return std::make_tuple(outputs_of(out, shapes, node->split, node), plan, merged);
+}
+
+void Hashtable::NoteUnsettled(const BatchPlanPtr& plan) {
+  if (unsettled_.empty() || unsettled_.back().get() != plan.get()) unsettled_.push_back(plan);
+}
+
+void Hashtable::SettleArrived(size_t most_left) {
+  size_t done = 0;
+  while (done < unsettled_.size()) {
+    const BatchPlanPtr plan = unsettled_[done];
+    const bool wait = unsettled_.size() - done > most_left;
+    if (!wait && !plan->TryU()) break;
+    ++done;
+    const int64_t U = [&] {
+      try {
+        return plan->U();
+      } catch (...) {  // a device-side error: reported once
+        unsettled_.erase(unsettled_.begin(), unsettled_.begin() + done);
+        throw;
+      }
+    }();
+    SettleCount(U, plan);
+  }
+  unsettled_.erase(unsettled_.begin(), unsettled_.begin() + done);
+}
+
+void Hashtable::AcceptTileGrad(const at::Tensor& index, const BatchPlanPtr& plan, const at::Tensor& offsets,
+                               const std::vector<int64_t>& batch, const std::vector<int64_t>& seq,
+                               const std::vector<at::Tensor>& grads) {
+  const int64_t D = slot_group_->EmbSlot()->FlatSize();
+  at::Tensor like;
+  for (const auto& g : grads)
+    if (g.defined() && !like.defined()) like = g;
+  if (!like.defined()) return;  // no gradient reached any part
+  at::Tensor src = plan->SrcForTile(batch, seq, offsets);
+  std::vector<at::Tensor> parts;
+  bool one_type = true;
+  for (size_t k = 0; k < grads.size(); ++k) {
+    const int64_t rows = batch[k] * seq[k];
+    parts.push_back(grads[k].defined() ? grads[k].reshape({rows, D}) : at::zeros({rows, D}, like.options()));
+    one_type = one_type && parts[k].scalar_type() == parts[0].scalar_type();
+  }
+  const bool apart = parts.size() <= 8 && one_type;
+  AcceptPlannedGrad(index, plan, apart ? parts : std::vector<at::Tensor>{at::cat(parts)}, apart, src, c10::nullopt,
+                    c10::nullopt, plan->serial(), false);
+}

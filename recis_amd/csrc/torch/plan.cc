@@ -1,8 +1,6 @@
 #include "plan.h"
 
 #include <atomic>
-#include <mutex>
-#include <unordered_map>
 
 #include "abi_util.h"
 #include "ops.h"
@@ -15,9 +13,6 @@ namespace {
 
 constexpr int64_t kPlanJobs = 64;  // arrays one recis_unique_plan_jobs call takes
 
-std::mutex g_staged_mu;
-// stream -> serial of the plan whose count is on its way to that stream's staging word
-std::unordered_map<void*, int64_t> g_staged;
 std::atomic<int64_t> g_serial{1};
 
 std::string describe_device_errors(int bits) {
@@ -41,17 +36,16 @@ at::Tensor flat_ids(const at::Tensor& t) {
   return t.to(at::kLong).contiguous().view({-1});
 }
 
-}  // namespace
-
-void raise_staged_device_errors(void* stream) {
-  int bits = 0;
-  check(recis_hip_staged_device_errors(&bits, stream));
-  if (bits) {
-    int polled = 0;
-    check(recis_hip_poll_device_errors(&polled));  // waits for the device and clears the word
-    TORCH_CHECK(false, "librecis_hip: device-side errors in earlier kernels: ", describe_device_errors(bits | polled));
-  }
+// The bits that travelled to the host with a staged count, as an exception.
+void raise_device_errors(int bits) {
+  if (bits == 0) return;
+  int polled = 0;
+  check(recis_hip_poll_device_errors(&polled));  // waits for the device and clears the word
+  // (two counts that were under way together carry one error's bits twice: it is raised once)
+  TORCH_CHECK(polled == 0, "librecis_hip: device-side errors in earlier kernels: ", describe_device_errors(bits | polled));
 }
+
+}  // namespace
 
 BatchPlanPtr BatchPlan::Make(const std::vector<at::Tensor>& ids_in, const c10::optional<std::vector<int64_t>>& tags,
                              recis_idmap* map, bool wait, bool need_inverse, bool need_pos) {
@@ -92,12 +86,6 @@ BatchPlanPtr BatchPlan::Make(const std::vector<at::Tensor>& ids_in, const c10::o
   if (map != nullptr) p->index_buf_ = at::empty({n}, i64);
   p->stream_ = stream_of(dev);
   int64_t count = 0;
-  {
-    // every launch overwrites the stream's staging word: an earlier plan whose count is still
-    // outstanding there must read its own device word from now on
-    std::lock_guard<std::mutex> lock(g_staged_mu);
-    g_staged.erase(p->stream_);
-  }
   auto ptrs = host_ptrs<int64_t>(jobs);
   auto sizes = numels(jobs);
   auto i32p = [](const at::Tensor& t) { return t.defined() ? t.data_ptr<int32_t>() : nullptr; };
@@ -107,39 +95,32 @@ BatchPlanPtr BatchPlan::Make(const std::vector<at::Tensor>& ids_in, const c10::o
                                p->counts_.data_ptr<int64_t>(),
                                p->index_buf_.defined() ? p->index_buf_.data_ptr<int64_t>() : nullptr,
                                wait ? &count : nullptr, wait ? 0 : RECIS_PLAN_STAGE_COUNT, p->stream_));
-  if (wait) {
-    p->U_ = count;
-    raise_staged_device_errors(p->stream_);
-  } else {
-    std::lock_guard<std::mutex> lock(g_staged_mu);
-    g_staged[p->stream_] = p->serial_;
-  }
+  check(recis_unique_plan_ticket(&p->ticket_, p->stream_));
+  if (wait) p->U();
   return p;
 }
 
-int64_t BatchPlan::U() {
-  if (U_ < 0) {
-    bool staged = false;
-    {
-      std::lock_guard<std::mutex> lock(g_staged_mu);
-      auto it = g_staged.find(stream_);
-      if (it != g_staged.end() && it->second == serial_) {
-        staged = true;
-        g_staged.erase(it);
-      }
-    }
-    if (staged) {
-      c10::DeviceGuard guard(device());
-      int64_t count = 0;
-      check(recis_unique_plan_count(&count, stream_));
-      U_ = count;
-      raise_staged_device_errors(stream_);
-    } else {  // a later plan took the stream's staging word: read this plan's own device word
-      U_ = counts_[0].item<int64_t>();
-    }
+bool BatchPlan::FetchU(bool wait) {
+  if (U_ >= 0) return true;
+  c10::DeviceGuard guard(device());
+  int64_t count = -1;
+  int bits = 0;
+  check(recis_unique_plan_count_of(ticket_, wait ? 1 : 0, &count, &bits, stream_));
+  if (count < 0) {
+    if (!wait) return false;
+    count = counts_[0].item<int64_t>();  // many later plans of the stream have taken over the staging words
   }
+  U_ = count;
+  raise_device_errors(bits);
+  return true;
+}
+
+int64_t BatchPlan::U() {
+  FetchU(true);
   return U_;
 }
+
+bool BatchPlan::TryU() { return FetchU(false); }
 
 at::Tensor BatchPlan::unique() {
   if (!unique_.defined()) unique_ = unique_buf_.narrow(0, 0, U());

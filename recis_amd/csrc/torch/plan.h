@@ -22,7 +22,7 @@ class BatchPlan : public torch::CustomClassHolder {
   // ids: the batch as one or more id tensors laid end to end; tags (one per tensor) tag every id
   // with its table as ids_encode does. map != nullptr: the unique ids are found or inserted in that
   // id map in the same pass and index_buf holds their rows. wait == false returns without the host
-  // copy of the unique count (at most one such plan per stream has its count on the way).
+  // copy of the unique count.
   static c10::intrusive_ptr<BatchPlan> Make(const std::vector<at::Tensor>& ids,
                                             const c10::optional<std::vector<int64_t>>& tags, recis_idmap* map,
                                             bool wait, bool need_inverse, bool need_pos);
@@ -32,6 +32,8 @@ class BatchPlan : public torch::CustomClassHolder {
   int64_t hot_cap() const { return hot_cap_; }
   // The number of unique ids on the host; a plan made with wait == false fetches it here.
   int64_t U();
+  // The same without waiting: whether the host has the count now.
+  bool TryU();
   // The count if the host has it already, else the number of ids: for kernels that take the count
   // from device memory and only need a bound to size their grid.
   int64_t U_bound() const { return U_ < 0 ? n_ : U_; }
@@ -73,7 +75,8 @@ class BatchPlan : public torch::CustomClassHolder {
                                                            bool mean, bool want_pool,
                                                            const std::vector<int64_t>* batch,
                                                            const std::vector<int64_t>* seq);
-  int64_t n_ = 0, serial_ = 0, hot_cap_ = 0, U_ = -1;
+  bool FetchU(bool wait);
+  int64_t n_ = 0, serial_ = 0, hot_cap_ = 0, U_ = -1, ticket_ = -1;
   void* stream_ = nullptr;
   at::Tensor unique_buf_, inverse_, row_start_, occ_, pos_, hot_items_, counts_, index_buf_, unique_;
   std::vector<std::pair<const void*, int64_t>> lookup_calls_;
@@ -90,9 +93,5 @@ using BatchPlanPtr = c10::intrusive_ptr<BatchPlan>;
 // of a recis_idmap, for callers that hold one through the C ABI) with the find-or-insert in it.
 BatchPlanPtr unique_plan(std::vector<at::Tensor> ids, c10::optional<std::vector<int64_t>> tags, int64_t idmap_handle,
                          bool wait, bool need_inverse, bool need_pos);
-
-// Soft errors of the device (bad row index, full id map, ...) that travelled to host memory with
-// the last staged unique count of `stream`, as an exception.
-void raise_staged_device_errors(void* stream);
 
 }  // namespace recis

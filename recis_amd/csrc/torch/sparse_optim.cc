@@ -86,6 +86,7 @@ void SparseOptimizer::step() {
       std::vector<PlannedGrad> planned = p.second->TakePlannedGrad();
       if (!planned.empty()) {
         UpdatePlanned(p.second, planned);
+        p.second->SettleArrived(2);
         continue;
       }
     }

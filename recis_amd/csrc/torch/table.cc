@@ -738,6 +738,7 @@ std::tuple<at::Tensor, at::Tensor> Hashtable::EvictOlder(const std::string& stam
 BatchPlanPtr Hashtable::PlanLookup(const std::vector<at::Tensor>& ids, const c10::optional<std::vector<int64_t>>& tags,
                                    bool wait, bool need_inverse, bool need_pos) {
   c10::DeviceGuard guard(device_);
+  SettleArrived(1);
   BatchPlanPtr plan = recis::BatchPlan::Make(ids, tags, map_->map, wait, need_inverse, need_pos);
   int64_t call = 0;
   check(recis_idmap_last_call(map_->map, &call));

@@ -307,6 +307,33 @@ class Hashtable : public torch::CustomClassHolder {
   c10::optional<std::tuple<recis::BatchPlanPtr, at::Tensor, at::Tensor>> DenseLookupExpand(
       const std::vector<at::Tensor>& cols, const c10::optional<std::vector<int64_t>>& tags,
       const c10::optional<std::string>& stamp_slot, const c10::optional<at::Tensor>& stamp_value);
+  // DenseLookupExpand as a differentiable lookup: one [B, D] output per column, whose backward hands the
+  // columns' gradients to the table (AcceptSplitGrad). See lookup_grad.cc.
+  c10::optional<std::vector<at::Tensor>> DenseLookupTrain(const std::vector<at::Tensor>& cols,
+                                                          const c10::optional<std::vector<int64_t>>& tags,
+                                                          const c10::optional<std::string>& stamp_slot,
+                                                          const c10::optional<at::Tensor>& stamp_value);
+  // The differentiable training lookup of a group of features that share a combiner ("sum", "mean" out of
+  // the table; "tile": padded, tile_len[k] rows per sample): plan + find-or-insert + pooling, one
+  // output per feature. offsets[k] undefined = the rows of a dense tensor. A plan that another group of the
+  // same inputs made is taken over (shared_plan, shared_offsets); `lean`: no other group can come to
+  // share this one's plan. Returns (outputs, plan, merged offsets | undefined), or None when "mean" has
+  // few ids per segment (then it divides by the sum of the weights: another path).
+  c10::optional<std::tuple<std::vector<at::Tensor>, recis::BatchPlanPtr, at::Tensor>> LookupTrain(
+      const std::vector<at::Tensor>& values, const std::vector<c10::optional<at::Tensor>>& offsets,
+      const std::vector<c10::optional<at::Tensor>>& weights, const c10::optional<std::vector<int64_t>>& tags,
+      const std::string& combiner, const std::vector<int64_t>& tile_len, bool lean,
+      const c10::optional<recis::BatchPlanPtr>& shared_plan, const c10::optional<at::Tensor>& shared_offsets);
+  // Lookups whose unique count the host has not read yet (LookupTrain and DenseLookupTrain do not wait
+  // for it). SettleArrived tells the id map the counts that have arrived, which keeps its bounds
+  // tight, and raises what their kernels reported; it waits for the oldest ones until `most_left` are
+  // left, so that a program that never waits for the device is told within two steps.
+  void NoteUnsettled(const recis::BatchPlanPtr& plan);
+  void SettleArrived(size_t most_left);
+  // The gradients of the padded outputs of one lookup, kept as separate arrays.
+  void AcceptTileGrad(const at::Tensor& index, const recis::BatchPlanPtr& plan, const at::Tensor& offsets,
+                      const std::vector<int64_t>& batch, const std::vector<int64_t>& seq,
+                      const std::vector<at::Tensor>& grads);
   // The evaluation forward of several features in one pass (recis_lookup_pool_readonly): ids straight to
   // pooled rows, no batch plan, nothing inserted. offsets[k] undefined = the rows of a dense tensor
   // ([B] or [..., width]). One [segments, D] output per feature, views of one buffer. `mean`: over
@@ -351,6 +378,8 @@ class Hashtable : public torch::CustomClassHolder {
 
  private:
   void MakeRoom(int64_t incoming);
+  at::Tensor GroupOffsets(const std::vector<c10::optional<at::Tensor>>& offsets, const std::vector<int64_t>& segments,
+                          const std::vector<int64_t>& widths, const std::vector<int64_t>& n_ids) const;
   at::Tensor OnDevice(const at::Tensor& ids) const;
   bool OneLaunchSums(const PlannedGrad& a, const PlannedGrad& b) const;
   at::Tensor SumOf(const PlannedGrad& g) const;
@@ -368,6 +397,7 @@ class Hashtable : public torch::CustomClassHolder {
   std::vector<bool> grad_unique_;
   std::vector<std::pair<int64_t, size_t>> grad_keys_;
   std::vector<PlannedGrad> planned_;
+  std::vector<recis::BatchPlanPtr> unsettled_;
   // the index tensor the last embedding_lookup returned, and whether the ids it was given are
   // known to hold no duplicates (they came out of ids_partition): accept_grad of exactly that tensor
   // needs no dedup

@@ -15,8 +15,7 @@ from ...ragged.tensor import RaggedTensor
 from ..functional.embedding_ops import ragged_embedding_segment_reduce
 from ..hashtable_hook import AdmitHook, FilterHook
 from ..initializers import ConstantInitializer, Initializer
-from .hashtable import (GradIDMeanFunction, HashTable, HashTableLookupHelpFunction, accept_planned_grad, gen_slice,
-                        plan_lookup)
+from .hashtable import GradIDMeanFunction, HashTable, HashTableLookupHelpFunction, accept_planned_grad, gen_slice
 
 
 class _Done:
@@ -126,68 +125,49 @@ def lookup_unique_rows(hashtable: HashTable, unique_ids, admit_hook=None, traina
 
 
 class LookupPoolFunction(torch.autograd.Function):
-    """Lookup of a plan's unique ids and sum / mean pooling straight out of the table: the
-    ``[U, D]`` copy of the looked-up rows (lookup function + ``ragged_embedding_segment_reduce``,
-    recis/nn/modules/embedding.py:592-624) is never made. Backward reduces the pooled
-    gradients per unique row over the plan and hands (row index, gradient) to the table."""
+    """Read-only lookup (an admit hook keeps new keys out) of a plan's unique ids in training and sum / mean pooling
+    straight out of the table: the ``[U, D]`` copy of the looked-up rows (lookup function +
+    ``ragged_embedding_segment_reduce``, recis/nn/modules/embedding.py:592-624) is never made. Backward hands the
+    pooled gradients to the table unsummed; keys the table does not hold carry a negative index and take none. (The
+    lookup that admits keys is ``HashtableImpl.lookup_train``.)"""
 
     @staticmethod
-    def forward(ctx, backward_holder, impl, plan, weight, offsets, combiner, readonly, unit_segments=False,
-                split=None):
-        """``split``: row counts to cut the pooled output into (one part per feature of a group that is pooled
+    def forward(ctx, backward_holder, impl, plan, weight, offsets, combiner, unit_segments=False, split=None):
+        """``unit_segments``: one id per segment (sum == mean == the row itself), so every unique row is read once and
+        written to its occurrences. ``split``: row counts to cut the pooled output into (one part per feature of a group that is pooled
         in one go); the parts are returned as separate outputs, views of the one buffer, and backward takes
         their gradients as they come: slices of one buffer are used in place, anything else is concatenated."""
-        late_count = not readonly
-        if readonly:
-            index = impl.lookup_index(plan.unique, True)
-        else:
-            # Nothing in this forward waits for the unique count: the lookup and the expansion take
-            # it from device memory, the pooling kernel only follows the plan's inverse (which names
-            # rows below the count), and the host reads it in backward, long after it has arrived.
-            # `index` is the full-length buffer; its first plan.U entries are the rows. A plan made by
-            # make_plan for this table brings them along (dedup and lookup were one pass).
-            index = impl.plan_index(plan)
-            if index is None:
-                index = impl.lookup_index_counted(plan, True)
+        index = impl.lookup_index(plan.unique, True)
         if unit_segments:
-            # one id per segment (sum == mean == the row itself): every unique row is read once and
-            # written to its occurrences, instead of one index chase per output row
             out = impl.expand_rows(plan, index, weight, None, None)
         else:
             chunks, chunk_rows = impl.emb_blocks()
-            out = ops.segment_reduce_forward_blocks(chunks, chunk_rows, index, weight, plan.inverse, offsets,
-                                                    combiner)
-        ctx.impl, ctx.plan, ctx.combiner, ctx.readonly, ctx.late_count = impl, plan, combiner, readonly, late_count
+            out = ops.segment_reduce_forward_blocks(chunks, chunk_rows, index, weight, plan.inverse, offsets, combiner)
+        ctx.impl, ctx.plan, ctx.combiner = impl, plan, combiner
         ctx.split, ctx.out_shape = split, tuple(out.shape)
         ctx.save_for_backward(index, weight, offsets)
+        ctx.set_materialize_grads(False)
         ctx.mark_non_differentiable(index)
-        if split is None:
-            return index, out
-        return (index,) + tuple(torch.split(out, split))
+        return (index,) + (tuple(torch.split(out, split)) if split is not None else (out,))
 
     @staticmethod
     def backward(ctx, _grad_index, *grads):
         index, weight, offsets = ctx.saved_tensors
-        if ctx.late_count:
-            ctx.impl.settle_count(ctx.plan.U, ctx.plan)
-            index = index[: ctx.plan.U]
+        if all(g is None for g in grads):
+            return (None,) * 8
         grad = grads[0] if ctx.split is None else _joined(grads, ctx.split, ctx.out_shape)
         # sum / mean: the gradient of a unique row is a gather-reduce over its occurrence list; it is handed
-        # over unsummed, so that the optimizer step can sum and update the row in one launch (keys the table
-        # does not hold carry a negative index and take no gradient)
+        # over unsummed, so that the optimizer step can sum and update the row in one launch
         src, coef = ctx.plan.src_coef_for_pool(offsets.contiguous(), weight, ctx.combiner == "mean")
-        accept_planned_grad(ctx.impl, index, ctx.plan, grad.contiguous(), src, coef,
-                            key=None if ctx.readonly else ctx.plan.serial, may_miss=ctx.readonly)
-        return (None,) * 9
+        accept_planned_grad(ctx.impl, index, ctx.plan, grad.contiguous(), src, coef, may_miss=True)
+        return (None,) * 8
 
 
 def _joined(grads, split, shape):
     """The gradients of the parts of one pooled output as one ``shape`` tensor: in place when they are
     consecutive slices of one buffer (what a caller that keeps its gradients in one array hands over),
     concatenated otherwise (a missing gradient counts as zeros)."""
-    like = next((g for g in grads if g is not None), None)
-    if like is None:
-        return torch.zeros(shape, device="cuda")
+    like = next(g for g in grads if g is not None)
     first = grads[0]
     if first is not None and first.is_contiguous():
         at = first.data_ptr()
@@ -202,83 +182,6 @@ def _joined(grads, split, shape):
     return torch.cat([g if g is not None else like.new_zeros((rows, shape[1])) for g, rows in zip(grads, split)])
 
 
-class DenseLookupFunction(torch.autograd.Function):
-    """Dedup, lookup and pooling of a group of dense id columns (``[B]`` / ``[B, 1]`` int64: one id per
-    sample, so sum == mean == the row itself) as ONE native call each way
-    (``HashtableImpl.dense_lookup_expand`` forward, ``accept_split_grad`` backward): what the per-feature
-    loop of ``EmbeddingEngine.forward`` + ``LookupPoolFunction`` do for such a group, without the Python
-    work per feature. One output per column, views of the one ``[N, D]`` buffer; nothing waits for the
-    unique count. ``forward`` returns None instead when a column is something else."""
-
-    @staticmethod
-    def forward(ctx, backward_holder, impl, cols, tags, stamp):
-        res = impl.dense_lookup_expand(cols, tags, None if stamp is None else stamp[0],
-                                       None if stamp is None else stamp[1])
-        if res is None:
-            ctx.mark_non_differentiable()
-            return None
-        plan, index, out = res
-        split = [c.shape[0] for c in cols]
-        ctx.impl, ctx.plan, ctx.split = impl, plan, split
-        ctx.save_for_backward(index)
-        ctx.mark_non_differentiable(index)
-        return (index,) + tuple(torch.split(out, split))
-
-    @staticmethod
-    def backward(ctx, _grad_index, *grads):
-        (index,) = ctx.saved_tensors
-        # the gradients of the columns, as they come (slices of one buffer are used in place); the sum per
-        # unique row is left to the optimizer step, which then updates the row in the same launch
-        ctx.impl.accept_split_grad(index, ctx.plan, list(grads), ctx.split, None, None, ctx.plan.serial, False, True)
-        return None, None, None, None, None
-
-
-class LookupTileFunction(torch.autograd.Function):
-    """Lookup of a plan's unique ids and the padded gather of several features at once, ONE output
-    per feature (``[bs[f], tile_len[f] * D]``, views of one buffer: the list form of the tile
-    combiner, recis/nn/modules/embedding_engine.py:383-411). Backward hands the features' gradients
-    to the table unsummed, as separate arrays: no concatenation of the padded gradients, and the
-    optimizer step sums them (together with the gradient of a pooled output of the same lookup, if
-    there is one) where it updates the rows."""
-
-    @staticmethod
-    def forward(ctx, backward_holder, impl, plan, offsets, bs, tile_len, readonly):
-        bs, tile_len = [int(b) for b in bs], [int(t) for t in tile_len]
-        U = plan.U   # the padded gather reads a dense copy of the rows: this forward needs the count
-        if readonly:
-            index = impl.lookup_index(plan.unique, True)
-        else:
-            index = impl.plan_index(plan)   # a plan made for this table brings the rows along
-            if index is None:
-                index = impl.lookup_index_counted(plan, True)
-            index = impl.settle_lookup(index, U, plan)
-        chunks, chunk_rows = impl.emb_blocks()
-        rows = ops.block_gather(index, chunks, chunk_rows, -1, readonly)
-        out, _ = ops.ragged_tile(bs, tile_len, plan.inverse, offsets, rows)
-        D = rows.shape[1]
-        ctx.impl, ctx.plan, ctx.readonly, ctx.bs, ctx.tile_len, ctx.D = impl, plan, readonly, bs, tile_len, D
-        ctx.save_for_backward(index, offsets)
-        ctx.mark_non_differentiable(index)
-        n_rows = [b * t for b, t in zip(bs, tile_len)]
-        return (index,) + tuple(p.view(b, t * D) for p, b, t in zip(torch.split(out, n_rows), bs, tile_len))
-
-    @staticmethod
-    def backward(ctx, _grad_index, *grads):
-        index, offsets = ctx.saved_tensors
-        plan, D = ctx.plan, ctx.D
-        n_rows = [b * t for b, t in zip(ctx.bs, ctx.tile_len)]
-        like = next((g for g in grads if g is not None), None)
-        if like is not None:
-            src = plan.src_for_tile(ctx.bs, ctx.tile_len, offsets.contiguous())
-            parts = [(g if g is not None else like.new_zeros((n, D))).reshape(n, D) for g, n in zip(grads, n_rows)]
-            key = None if ctx.readonly else plan.serial
-            if len(parts) <= 8 and len({p.dtype for p in parts}) == 1:
-                accept_planned_grad(ctx.impl, index, plan, parts, src, key=key, may_miss=ctx.readonly)
-            else:
-                accept_planned_grad(ctx.impl, index, plan, torch.cat(parts), src, key=key, may_miss=ctx.readonly)
-        return (None,) * 7
-
-
 def _pools_out_of_the_table(hashtable, opt, n_occ, n_offsets):
     """Whether lookup_and_pool takes the path that pools straight out of the table rows."""
     float_table = hashtable._dtype in (torch.float32, torch.bfloat16, torch.float16)
@@ -287,44 +190,25 @@ def _pools_out_of_the_table(hashtable, opt, n_occ, n_offsets):
     return opt.combiner in ("sum", "mean") and float_table and not sparse_mean and not id_mean
 
 
-def make_plan(hashtable: HashTable, ids, offsets, opt, has_weight=False, unit_segments=False, tags=None):
-    """The batch plan of ``ids`` for ``lookup_and_pool``. When what follows is the training lookup
-    that admits new keys and pools out of the table, dedup and find-or-insert run as one pass
-    (``HashtableImpl.plan_lookup``) and the plan carries the rows; ``unit_segments`` plans leave
-    out the per-occurrence arrays nobody reads (the expansion and its backward walk the lists).
-    ``ids`` may be a list of id tensors with their table ``tags`` (``ops.ids_unique_plan``)."""
-    n_occ = sum(t.numel() for t in ids) if isinstance(ids, (list, tuple)) else ids.numel()
-    if (hashtable.training and opt.trainable and opt.admit_hook is None
-            and _pools_out_of_the_table(hashtable, opt, n_occ, offsets.numel())):
-        lean = bool(unit_segments)
-        return plan_lookup(hashtable._hashtable_impl, ids, need_inverse=not lean, tags=tags)
-    return ops.ids_unique_plan(ids, wait=False, need_pos=False, tags=tags)
-
-
 def lookup_and_pool(hashtable: HashTable, plan, weight, offsets, opt, unit_segments=False, combiner_kwargs=None,
                     split=None):
-    """Rows of the plan's unique ids pooled per segment. Sum / mean over a float table go
-    through ``LookupPoolFunction`` (pooling reads the table directly); everything else looks the
-    rows up first and pools the copy. ``unit_segments``: the caller built ``offsets`` as
-    0, 1, 2, ... (dense ``[B, 1]`` id tensors), so segment i holds exactly occurrence i.
-    ``split``: return the pooled rows cut into parts of these row counts (a tuple)."""
-    impl = hashtable._hashtable_impl
+    """Rows of the plan's unique ids pooled per segment, for what ``HashtableImpl.lookup_train`` and
+    ``lookup_pool_readonly`` leave over. Under an admit hook sum / mean over a float table go through
+    ``LookupPoolFunction`` (pooling reads the table directly); everything else looks the rows up first and pools the
+    copy. ``unit_segments``: ``offsets`` are 0, 1, 2, ... (dense ``[B, 1]`` id tensors). ``split``: return the pooled
+    rows cut into parts of these row counts (a tuple)."""
     id_mean = opt.grad_reduce_by == "id" and hashtable.training and opt.trainable
     if _pools_out_of_the_table(hashtable, opt, plan.n, offsets.numel()):
+        impl = hashtable._hashtable_impl
         if weight is not None and weight.dtype != hashtable._dtype:
             weight = weight.to(hashtable._dtype)
-        if hashtable.training and opt.trainable:
-            readonly = opt.admit_hook is not None
-            if readonly:
-                from .hashtable_hook_impl import HashtableHookFactory, ReadOnlyHookImpl
-                admit = HashtableHookFactory().create_admit_hook(hashtable, opt.admit_hook)
-                assert isinstance(admit, ReadOnlyHookImpl), "admit hook only support ReadOnlyHook yet, but got: %s" % admit
+        if hashtable.training and opt.trainable:  # under an admit hook, or lookup_train would have taken it
+            from .hashtable_hook_impl import HashtableHookFactory, ReadOnlyHookImpl
+            admit = HashtableHookFactory().create_admit_hook(hashtable, opt.admit_hook)
+            assert isinstance(admit, ReadOnlyHookImpl), "admit hook only support ReadOnlyHook yet, but got: %s" % admit
             index, *outs = LookupPoolFunction.apply(hashtable._backward_holder, impl, plan, weight, offsets,
-                                                    opt.combiner, readonly, unit_segments, split)
-            if not isinstance(hashtable._filter_hook_impl, torch.nn.Identity):
-                # a step filter stamps the looked-up rows: it needs the rows proper (the index may
-                # be the full-length buffer of the forward that does not wait for the count)
-                hashtable._filter_hook_impl(index[: plan.U] if not readonly else index)
+                                                    opt.combiner, unit_segments, split)
+            hashtable._filter_hook_impl(index)
             return outs[0] if split is None else tuple(outs)
         readonly = (not hashtable.training) or opt.admit_hook is not None
         index = impl.lookup_index(plan.unique.detach(), readonly)
@@ -365,7 +249,6 @@ class DynamicEmbedding(torch.nn.Module):
             reserve_rows=emb_opt.reserve_rows)
 
     def deal_with_tensor(self, input_tensor: Union[torch.Tensor, RaggedTensor]):
-        self._unit_segments = False
         if isinstance(input_tensor, RaggedTensor):
             val = input_tensor.values()
             weight = input_tensor.weight()
@@ -381,7 +264,6 @@ class DynamicEmbedding(torch.nn.Module):
             offsets = torch.arange(bs + 1, device=val.device) * fea_dim
             weight = None
             shape = tuple(input_tensor.shape[:-1])
-            self._unit_segments = fea_dim == 1
         else:
             raise TypeError("DynamicEmbedding only support RaggedTensor or dense tensor, got %s" % type(input_tensor))
         return val, offsets, weight, shape
@@ -395,11 +277,27 @@ class DynamicEmbedding(torch.nn.Module):
             weight = input_weights
         if weight is not None:
             weight = weight.to(dev) if opt.use_weight else None
-        plan = make_plan(self._hashtable, val, offsets, opt, weight is not None, self._unit_segments)
-        out = lookup_and_pool(self._hashtable, plan, weight, offsets, opt, unit_segments=self._unit_segments)
+        out = self._pooled(val, offsets, weight, input_ids.shape[1] if type(input_ids) is torch.Tensor and input_ids.dim() == 2 else None)
         if opt.combiner == "tile":
             return out.view(tuple(shape) + (opt.combiner_kwargs["tile_len"] * opt.embedding_dim,))
         return out.view(tuple(shape) + (opt.embedding_dim,))
+
+    def _pooled(self, val, offsets, weight, width):
+        """The rows of ``val`` pooled per segment: in one native call where the table, the combiner and the mode
+        allow it. ``width`` ids per segment when the ids were a dense tensor."""
+        opt, table = self._emb_opt, self._hashtable
+        if table._dtype in (torch.float32, torch.bfloat16, torch.float16) and opt.combiner in ("sum", "mean"):
+            ids, offs = (val, offsets) if width is None or weight is not None else (val.view(-1, width), None)
+            if not table.training:
+                return table._hashtable_impl.lookup_pool_readonly([ids], [offs], [weight], None, opt.combiner == "mean")[0]
+            if opt.trainable and opt.admit_hook is None and opt.grad_reduce_by != "id":
+                res = table._hashtable_impl.lookup_train([ids], [offs], [weight], None, opt.combiner, [], True, None, None)
+                if res is not None:
+                    if not isinstance(table._filter_hook_impl, torch.nn.Identity):
+                        table._filter_hook_impl(res[1].index_buf[: res[1].U])
+                    return res[0][0]
+        plan = ops.ids_unique_plan(val, wait=False, need_pos=False)
+        return lookup_and_pool(table, plan, weight, offsets, opt)
 
     # The staged form of forward (embedding.py:498-624), which EmbeddingEngine-style callers drive
     # stage by stage. With one GPU the two all-to-alls are the identity: exchange_ids is the dedup,

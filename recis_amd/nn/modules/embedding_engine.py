@@ -23,9 +23,8 @@ import torch
 from ... import ops
 from ...ragged.tensor import RaggedTensor
 from ..functional.embedding_ops import RaggedTileParts
-from .embedding import (DenseLookupFunction, EmbeddingOption, LookupTileFunction, lookup_and_pool, lookup_unique_rows,
-                        make_plan)
-from .hashtable import HashTable, gen_slice, plan_lookup
+from .embedding import EmbeddingOption, lookup_and_pool, lookup_unique_rows
+from .hashtable import HashTable, gen_slice
 
 
 def _key(text):
@@ -55,6 +54,7 @@ class EmbeddingEngine(torch.nn.Module):
             grp.features[name] = opt
         # per feature: the key of its runtime group (features of a table that are pooled together)
         self._runtime_key = {name: opt.runtime_info() for name, opt in self._emb_options.items()}
+        self._runtime_cache = {}
         self._offsets_cache = {}  # offsets of dense id tensors, which depend on their shape only
         self._tags = {}
         self._tables = torch.nn.ModuleDict()
@@ -114,9 +114,24 @@ class EmbeddingEngine(torch.nn.Module):
             values = values.long()
         return values, weight, offsets.to(torch.int32), shape, unit, dense
 
-    def _evaluate(self, table, info, tag_of, names, opt0, inputs, outputs):
-        """The features of one runtime group in evaluation mode: ids straight to pooled rows in one native call
-        (``HashtableImpl.lookup_pool_readonly``), without the plan a training lookup makes for its backward."""
+    def _runtime_groups(self, gkey, grp, inputs):
+        """The features of a table that ``inputs`` holds, those that are pooled together in one list each: a function
+        of the names alone, worked out once per set of names."""
+        key = (gkey,) + tuple(inputs)
+        hit = self._runtime_cache.get(key)
+        if hit is None:
+            if len(self._runtime_cache) >= 64:
+                self._runtime_cache.clear()
+            runtime = OrderedDict()
+            for name in grp.features:
+                if name in inputs:
+                    runtime.setdefault(self._runtime_key[name], []).append(name)
+            hit = self._runtime_cache[key] = runtime
+        return hit
+
+    def _arrays(self, names, opt, inputs):
+        """(values, offsets | None, weight | None, shape prefix | None) of every feature, as lists: what the native
+        lookups of a group take. offsets None = a dense tensor, prefix None = one row per sample."""
         vals, offs, weights, prefixes = [], [], [], []
         for name in names:
             data = inputs[name]
@@ -132,14 +147,39 @@ class EmbeddingEngine(torch.nn.Module):
                     raise RuntimeError("RaggedTensor must pad before lookup, got: %s (%s)" % (data, name))
                 vals.append(data.values())
                 offs.append(offsets)
-                weights.append(data.weight() if opt0.use_weight else None)
+                weights.append(data.weight() if opt.use_weight else None)
                 prefixes.append(None if len(shape) == 1 else shape)
             else:
                 raise TypeError("feature %s: expected RaggedTensor or Tensor, got %s" % (name, type(data)))
-        parts = table._hashtable_impl.lookup_pool_readonly(
-            vals, offs, weights, [tag_of[n] for n in names] if info.is_coalesce() else None, opt0.combiner == "mean")
+        return vals, offs, weights, prefixes
+
+    def _evaluate(self, table, tags, names, opt, inputs, outputs):
+        """The features of one runtime group in evaluation mode: ids straight to pooled rows in one native call
+        (``HashtableImpl.lookup_pool_readonly``), without the plan a training lookup makes for its backward."""
+        vals, offs, weights, prefixes = self._arrays(names, opt, inputs)
+        parts = table._hashtable_impl.lookup_pool_readonly(vals, offs, weights, tags, opt.combiner == "mean")
         for name, part, prefix in zip(names, parts, prefixes):
             outputs[name] = part if prefix is None else part.reshape(tuple(prefix) + (part.shape[1],))
+
+    def _train(self, table, tags, names, opt, inputs, outputs, plans, same, alone):
+        """The features of one runtime group in training mode: plan, find-or-insert, pooling (or the padded gather)
+        and the node of their backward in one native call (``HashtableImpl.lookup_train``). False when the group
+        needs the general path."""
+        vals, offs, weights, prefixes = self._arrays(names, opt, inputs)
+        tile_len = [int(self._emb_options[n].combiner_kwargs["tile_len"]) for n in names] if opt.combiner == "tile" else []
+        offsets, plan = plans.get(same, (None, None))
+        res = table._hashtable_impl.lookup_train(vals, offs, weights, tags, opt.combiner, tile_len, alone, plan, offsets)
+        if res is None:
+            return False
+        parts, plan, offsets = res
+        if same not in plans:
+            plans[same] = (offsets, plan)
+        if not isinstance(table._filter_hook_impl, torch.nn.Identity):
+            # a step filter stamps the looked-up rows: it needs the rows proper, hence the count
+            table._filter_hook_impl(plan.index_buf[: plan.U])
+        for name, part, prefix in zip(names, parts, prefixes):
+            outputs[name] = part if prefix is None else part.reshape(tuple(prefix) + (part.shape[1],))
+        return True
 
     def forward(self, inputs: Dict[str, Union[torch.Tensor, RaggedTensor]]):
         outputs = {}
@@ -153,29 +193,32 @@ class EmbeddingEngine(torch.nn.Module):
             tag_of = self._tags.get(gkey)
             if tag_of is None:  # the 12-bit table index of every feature's shared name, fixed after construction
                 tag_of = self._tags[gkey] = {n: info.child_index(o.shared_name) for n, o in grp.features.items()}
-            runtime = OrderedDict()
-            for name in grp.features:
-                if name in inputs:
-                    runtime.setdefault(self._runtime_key[name], []).append(name)
+            runtime = self._runtime_groups(gkey, grp, inputs)
             for names in runtime.values():
                 opt0 = grp.features[names[0]]
-                if (table.training and opt0.combiner in ("sum", "mean") and opt0.trainable and opt0.admit_hook is None
-                        and opt0.grad_reduce_by != "id" and table._dtype in (torch.float32, torch.bfloat16, torch.float16)
-                        and all(type(inputs[n]) is torch.Tensor for n in names)):
-                    # dense id columns only: tagging, dedup, lookup and the rows of every column in one native call
-                    stamp = getattr(table._filter_hook_impl, "stamp_target", lambda: None)()
-                    if stamp is not None or isinstance(table._filter_hook_impl, torch.nn.Identity):
-                        res = DenseLookupFunction.apply(table._backward_holder, table._hashtable_impl,
-                                                        [inputs[n] for n in names],
-                                                        [tag_of[n] for n in names] if info.is_coalesce() else None, stamp)
-                        if res is not None:
-                            for name, part in zip(names, res[1:]):
-                                outputs[name] = part
-                            continue
-                if (not table.training and opt0.combiner in ("sum", "mean")
-                        and table._dtype in (torch.float32, torch.bfloat16, torch.float16)):
-                    self._evaluate(table, info, tag_of, names, opt0, inputs, outputs)
+                tags = [tag_of[n] for n in names] if info.is_coalesce() else None
+                float_table = table._dtype in (torch.float32, torch.bfloat16, torch.float16)
+                if not table.training and opt0.combiner in ("sum", "mean") and float_table:
+                    self._evaluate(table, tags, names, opt0, inputs, outputs)
                     continue
+                same = (gkey,) + tuple((id(inputs[n]), tag_of[n]) for n in names)
+                if (table.training and opt0.combiner in ("sum", "mean", "tile") and opt0.trainable and opt0.admit_hook is None
+                        and opt0.grad_reduce_by != "id" and float_table):
+                    if opt0.combiner != "tile" and all(type(inputs[n]) is torch.Tensor for n in names):
+                        # dense id columns only: nothing but the columns to hand over
+                        stamp = getattr(table._filter_hook_impl, "stamp_target", lambda: None)()
+                        if stamp is not None or isinstance(table._filter_hook_impl, torch.nn.Identity):
+                            parts = table._hashtable_impl.dense_lookup_train(
+                                [inputs[n] for n in names], tags, None if stamp is None else stamp[0],
+                                None if stamp is None else stamp[1])
+                            if parts is not None:
+                                outputs.update(zip(names, parts))
+                                continue
+                    # lean (no per-occurrence arrays) only if no other option can come to share the plan
+                    alone = len(runtime) == 1 or sum(
+                        1 for k in runtime.values() if any(inputs[n] is inputs[names[0]] for n in k)) == 1
+                    if self._train(table, tags, names, opt0, inputs, outputs, plans, same, alone):
+                        continue
                 vals, weights, offs, shapes, dense = [], [], [], [], []
                 all_unit = True
                 any_weight = opt0.use_weight and any(
@@ -202,14 +245,8 @@ class EmbeddingEngine(torch.nn.Module):
                         w = torch.ones(v.numel(), device=dev)
                     weights.append(None if w is None else w.to(dev))
                     shapes.append(shape)
-                same = (gkey,) + tuple((id(inputs[n]), tag_of[n]) for n in names)
-                if same in plans:
-                    offsets, plan = plans[same]
-                else:
-                    # the id tensors go to the plan as they are: it tags (ids_encode) / concatenates them
-                    # in its own reads
-                    tags = [tag_of[n] for n in names] if info.is_coalesce() else None
-                    ids = vals if (tags is not None or len(vals) > 1) else vals[0]
+                offsets, plan = plans.get(same, (None, None))
+                if offsets is None:  # (a plan of one id per segment comes without offsets)
                     if len(offs) == 1:
                         offsets = offs[0]
                     elif all(d is not None for d in dense):  # dense id tensors only: a function of the shapes
@@ -217,16 +254,11 @@ class EmbeddingEngine(torch.nn.Module):
                             offs, [v.numel() for v in vals]))
                     else:
                         offsets = ops.merge_offsets(offs, [v.numel() for v in vals])
-                    if opt0.combiner == "tile":
-                        if (table.training and opt0.trainable and opt0.admit_hook is None
-                                and table._dtype in (torch.float32, torch.bfloat16, torch.float16)):
-                            plan = plan_lookup(table._hashtable_impl, ids, tags=tags)   # dedup + find-or-insert, one pass
-                        else:
-                            plan = ops.ids_unique_plan(ids, wait=False, need_pos=False, tags=tags)
-                    else:  # lean (no per-occurrence arrays) only if no other option can come to share it
-                        alone = sum(1 for k in runtime.values() if any(inputs[n] is inputs[names[0]] for n in k)) == 1
-                        plan = make_plan(table, ids, offsets, opt0, any_weight, unit_segments=all_unit and alone,
-                                         tags=tags)
+                if plan is None:
+                    # the id tensors go to the plan as they are: it tags (ids_encode) / concatenates them
+                    # in its own reads
+                    ids = vals if (tags is not None or len(vals) > 1) else vals[0]
+                    plan = ops.ids_unique_plan(ids, wait=False, need_pos=False, tags=tags)
                     plans[same] = (offsets, plan)
                 weight = None
                 if all(w is not None for w in weights):
@@ -242,13 +274,6 @@ class EmbeddingEngine(torch.nn.Module):
                         width = pooled.shape[1]
                         parts = [p.view(b, t * width) for p, b, t in zip(
                             torch.split(pooled, [b * t for b, t in zip(seg_counts, tile_lens)]), seg_counts, tile_lens)]
-                    elif (table.training and opt0.trainable and opt0.admit_hook is None
-                          and table._dtype in (torch.float32, torch.bfloat16, torch.float16)):
-                        # lookup and padded gather as one function: the rows the plan brought along are used
-                        # (no second lookup of the same ids) and the gradients reach the table unsummed
-                        index, *parts = LookupTileFunction.apply(table._backward_holder, table._hashtable_impl,
-                                                                 plan, offsets, seg_counts, tile_lens, False)
-                        table._filter_hook_impl(index)
                     else:
                         emb = lookup_unique_rows(table, plan.unique, opt0.admit_hook, opt0.trainable,
                                                  grad_key=plan.serial)

@@ -149,6 +149,7 @@ class HashTableLookupHelpFunction(torch.autograd.Function):
             "admit hook only support ReadOnlyHook yet, but got: %s" % admit_hook_impl
         index, embedding = hashtable.embedding_lookup(ids.detach(), admit_hook_impl is not None)
         ctx.save_for_backward(index)
+        ctx.set_materialize_grads(False)  # the index takes no gradient: no zeros are made for it
         ctx.hashtable = hashtable
         ctx.mark_non_differentiable(index)
         return index, embedding
@@ -228,6 +229,7 @@ class LookupExpandFunction(torch.autograd.Function):
             ctx.settled = True
         ctx.impl, ctx.plan, ctx.slice_num, ctx.readonly = impl, plan, slice_num, readonly
         ctx.save_for_backward(index)
+        ctx.set_materialize_grads(False)  # the index takes no gradient: no zeros are made for it
         ctx.mark_non_differentiable(index)
         return index, out
 
@@ -338,6 +340,11 @@ class HashTable(torch.nn.Module):
             stamp = getattr(self._filter_hook_impl, "stamp_target", lambda: None)()
             # a hook that cannot stamp in that pass gets the rows proper afterwards, which needs the count
             hooked = stamp is None and not isinstance(self._filter_hook_impl, torch.nn.Identity)
+            if admit_hook_impl is None and not hooked and self._worker_num == 1:
+                # dedup, lookup, one row per request and the node of their backward in one native call
+                embedding = self._hashtable_impl.dense_lookup_train(
+                    [ids.contiguous()], None, None if stamp is None else stamp[0], None if stamp is None else stamp[1])[0]
+                return embedding.view(shape + tuple(embedding.shape[1:])) if len(shape) != 1 else embedding
             emb_idx, embedding = LookupExpandFunction.apply(self._backward_holder, self._hashtable_impl, ids,
                                                             self._worker_num, admit_hook_impl is not None, stamp, hooked)
             if hooked:

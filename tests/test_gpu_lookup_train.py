@@ -1,0 +1,97 @@
+"""The training lookups that do not wait for the device (HashtableImpl.lookup_train / dense_lookup_train): counts of
+several plans under way at once, errors that arrive late, both backward passes over one node."""
+import numpy as np
+import pytest
+import torch
+
+from recis_amd import _lib, ops
+from recis_amd.nn import EmbeddingEngine, EmbeddingOption, HashTable
+from recis_amd.nn.modules.hashtable import HashtableRegister, filter_out_sparse_param
+from recis_amd.optim import SparseAdagrad
+from recis_amd.ragged import RaggedTensor
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("count", [2, 16, 17, 40])
+def test_counts_of_plans_under_way_together(rng, count):
+    """More plans than the ring of staging words holds: the oldest ones read their own device word."""
+    batches = [rng.integers(0, 50 + 37 * k, size=3000) for k in range(count)]
+    plans = [ops.ids_unique_plan(torch.from_numpy(b).cuda(), wait=False) for b in batches]
+    for k in rng.permutation(count):
+        assert plans[k].U == len(np.unique(batches[k]))
+    assert _lib.poll_device_errors() == 0
+
+
+def _trained_table():
+    HashtableRegister().clear()
+    ht = HashTable([8], block_size=64, name="late")
+    return ht, SparseAdagrad(filter_out_sparse_param(ht), lr=0.1)
+
+
+def test_device_errors_arrive_within_two_steps():
+    ht, opt = _trained_table()
+    good = torch.arange(100, device="cuda")
+    bad = good.clone()
+    bad[7] = -1  # a key the map reserves
+    with pytest.raises(RuntimeError, match="index outside"):
+        for ids in (bad, good, good):
+            ht(ids).backward(torch.ones(100, 8, device="cuda"))
+            opt.step()
+            opt.zero_grad()
+    ht(good)
+    assert _lib.poll_device_errors() == 0  # raised once, cleared
+
+
+def test_second_backward_and_no_grad():
+    ht, opt = _trained_table()
+    ids = torch.arange(50, device="cuda")
+    out = ht(ids)
+    out.sum().backward(retain_graph=True)
+    out.sum().backward()
+    with pytest.raises(RuntimeError, match="second time"):
+        out.sum().backward()
+    opt.step()
+    rows = ht._hashtable_impl.lookup_pool_readonly([ids], [None], [None], None, False)[0]
+    torch.testing.assert_close(rows, torch.full((50, 8), -0.1, device="cuda"))  # one Adagrad step of a gradient of 2
+    with torch.no_grad():
+        assert not ht(ids).requires_grad
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+def test_group_of_dense_and_ragged_features_matches_torch(rng, weighted):
+    """One group of a dense column, a wide dense tensor and a ragged feature: pooled rows and one Adagrad step against
+    index_add_ in float64."""
+    HashtableRegister().clear()
+    names, D, B = ["a", "b", "c"], 8, 77
+    eng = EmbeddingEngine({n: EmbeddingOption(embedding_dim=D, shared_name="one", combiner="sum", use_weight=True)
+                           for n in names})
+    opt = SparseAdagrad(filter_out_sparse_param(eng), lr=0.1)
+    lens = rng.integers(0, 6, size=B)
+    off = np.concatenate([[0], np.cumsum(lens)])
+    n = int(off[-1])
+    ids = {"a": rng.integers(0, 40, size=(B, 1)), "b": rng.integers(0, 40, size=(B, 3)), "c": rng.integers(0, 40, size=n)}
+    w = (rng.random(n) + 0.5).astype(np.float32) if weighted else np.ones(n, np.float32)
+    x = {k: torch.from_numpy(v).cuda() for k, v in ids.items() if k != "c"}
+    x["c"] = RaggedTensor(torch.from_numpy(ids["c"]).cuda(), torch.from_numpy(off.astype(np.int32)).cuda(),
+                          torch.from_numpy(w).cuda() if weighted else None)
+    (table,) = eng.hashtables().values()
+    start = rng.standard_normal((40, D)).astype(np.float32)
+    table.insert(torch.arange(40, device="cuda"), torch.from_numpy(start).cuda())
+    ups = {k: rng.standard_normal((B, D)).astype(np.float32) for k in names}
+    out = eng(x)
+    seg = {"a": np.arange(B), "b": np.repeat(np.arange(B), 3), "c": np.repeat(np.arange(B), lens)}
+    coef = {"a": np.ones(B), "b": np.ones(3 * B), "c": w.astype(np.float64)}
+    grad = np.zeros((40, D))
+    for k in names:
+        exp = np.zeros((B, D))
+        np.add.at(exp, seg[k], coef[k][:, None] * start[ids[k].reshape(-1)].astype(np.float64))
+        np.testing.assert_allclose(out[k].detach().cpu().numpy(), exp, rtol=1e-5, atol=1e-5)
+        np.add.at(grad, ids[k].reshape(-1), coef[k][:, None] * ups[k][seg[k]])
+    torch.autograd.backward([out[k] for k in names], [torch.from_numpy(ups[k]).cuda() for k in names])
+    opt.step()
+    rows = table._hashtable_impl.lookup_pool_readonly([torch.arange(40, device="cuda")], [None], [None], None, False)[0]
+    # the first step moves by lr * sign(g): g is far from zero against its float32 sum
+    clear = np.abs(grad) > 1e-3
+    np.testing.assert_allclose(rows.cpu().numpy()[clear], (start - 0.1 * np.sign(grad))[clear], rtol=1e-4, atol=1e-4)
+    assert _lib.poll_device_errors() == 0
