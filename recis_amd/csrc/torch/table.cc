@@ -935,12 +935,15 @@ void Hashtable::AcceptSplitGrad(const at::Tensor& index_in, const BatchPlanPtr& 
       }
     }
     if (!like.defined()) return;  // no gradient reached any part
-    std::vector<at::Tensor> parts;
-    for (size_t f = 0; f < grads.size(); ++f) {
-      parts.push_back(grads[f].has_value() && grads[f]->defined() ? grads[f]->reshape({split[f], D})
-                                                                  : at::zeros({split[f], D}, like.options()));
+    whole = CollectRows(grads, split, like);
+    if (!whole.defined()) {  // mixed types or devices: torch's rules for them
+      std::vector<at::Tensor> parts;
+      for (size_t f = 0; f < grads.size(); ++f) {
+        parts.push_back(grads[f].has_value() && grads[f]->defined() ? grads[f]->reshape({split[f], D})
+                                                                    : at::zeros({split[f], D}, like.options()));
+      }
+      whole = at::cat(parts, 0);
     }
-    whole = at::cat(parts, 0);
   }
   at::Tensor index = index_in;
   if (settle) {
@@ -950,6 +953,35 @@ void Hashtable::AcceptSplitGrad(const at::Tensor& index_in, const BatchPlanPtr& 
   }
   AcceptPlannedGrad(index, plan, {whole}, false, src.has_value() && src->defined() ? *src : plan->occ(), coef,
                     c10::nullopt, key, may_miss);
+}
+
+// The parts' rows laid end to end in one [rows, D] array. Undefined when a part is no plain tensor of like's type on the
+// table's device.
+at::Tensor Hashtable::CollectRows(const std::vector<c10::optional<at::Tensor>>& grads, const std::vector<int64_t>& split,
+                                  const at::Tensor& like) const {
+  const int64_t D = slot_group_->EmbSlot()->FlatSize();
+  if (like.device() != device_ || (like.element_size() != 4 && like.element_size() != 2)) return at::Tensor();
+  const int64_t size = like.element_size();
+  std::vector<at::Tensor> keep;
+  std::vector<const void*> base(grads.size(), nullptr);
+  std::vector<int64_t> stride(grads.size(), 0);
+  int64_t rows = 0;
+  for (size_t f = 0; f < grads.size(); ++f) {
+    rows += split[f];
+    if (!grads[f].has_value() || !grads[f]->defined()) continue;  // reads as zeros
+    at::Tensor g = *grads[f];
+    if (g.layout() != at::kStrided || g.device() != device_ || g.scalar_type() != like.scalar_type() || g.is_neg())
+      return at::Tensor();
+    if (g.dim() != 2 || g.size(0) != split[f] || g.size(1) != D) g = g.reshape({split[f], D});
+    if (D > 1 && g.stride(1) != 1) g = g.contiguous();
+    base[f] = g.data_ptr();
+    stride[f] = g.stride(0) * size;
+    keep.push_back(std::move(g));
+  }
+  at::Tensor out = at::empty({rows, D}, like.options().memory_format(at::MemoryFormat::Contiguous));
+  check(recis_collect_rows(base.data(), stride.data(), split.data(), static_cast<int64_t>(split.size()),
+                           D * size, static_cast<int>(size), out.data_ptr(), stream_of(device_)));
+  return out;
 }
 
 // ------------------------------------------------------------------------------------ gradients

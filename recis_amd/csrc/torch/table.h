@@ -352,6 +352,8 @@ class Hashtable : public torch::CustomClassHolder {
                        const std::vector<c10::optional<at::Tensor>>& grads, const std::vector<int64_t>& split,
                        const c10::optional<at::Tensor>& src, const c10::optional<at::Tensor>& coef, int64_t key,
                        bool may_miss, bool settle);
+  at::Tensor CollectRows(const std::vector<c10::optional<at::Tensor>>& grads, const std::vector<int64_t>& split,
+                         const at::Tensor& like) const;
   // accept_grad whose caller knows that grad_index has no duplicates (`unique`), and / or that two
   // calls with one `key` (!= 0) hand over gradients for the same rows in the same order (the second
   // is then added onto the first).
