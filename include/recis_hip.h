@@ -683,6 +683,15 @@ int recis_csr_gather_reduce_adagrad(const void* rows, int rows_dtype, int64_t n_
                                     void* stream);
 
 /*
+ * The rows of several arrays laid end to end in one dense array out [sum of part_counts, row_bytes]: part
+ * f holds part_counts[f] rows, part_stride_bytes[f] apart (0: one row over and over); a NULL part reads as
+ * zeros. What the backward of a lookup with several outputs does with their gradients, column
+ * slices of one wide gradient for instance.
+ */
+int recis_collect_rows(const void* const* part_rows, const int64_t* part_stride_bytes, const int64_t* part_counts,
+                       int64_t n_parts, int64_t row_bytes, int elem_bytes, void* out, void* stream);
+
+/*
  * Gather-reduce with TWO inputs over the same occurrence lists: list entry k of unique id u adds
  * a.coef[k] * a.rows[a.src[k]] + b.coef[k] * b.rows[b.src[k]] (a negative src skips that term;
  * coef NULL = 1). A lookup whose rows feed two outputs, a pooled one and an unpooled, padded one
@@ -698,15 +707,6 @@ int recis_csr_gather_reduce_adagrad(const void* rows, int rows_dtype, int64_t n_
  * The result equals recis_csr_gather_reduce(a) followed by recis_csr_gather_reduce(b, accumulate)
  * up to fp32 rounding (here both inputs go through one chain of fused multiply-adds, there the
  * first sum is rounded to the output before the second is added).
-/*
- * The rows of several arrays laid end to end in one dense array out [sum of part_counts, row_bytes]: part
- * f holds part_counts[f] rows, part_stride_bytes[f] apart (0: one row over and over); a NULL part reads as
- * zeros. What the backward of a lookup with several outputs does with their gradients, column
- * slices of one wide gradient for instance.
- */
-int recis_collect_rows(const void* const* part_rows, const int64_t* part_stride_bytes, const int64_t* part_counts,
-                       int64_t n_parts, int64_t row_bytes, int elem_bytes, void* out, void* stream);
-
  */
 typedef struct recis_csr_input {
   const void* rows;   /* [n_rows, D] */
