@@ -136,6 +136,22 @@ int recis_segment_reduce_forward_blocks(const void* const* emb_blocks_dev, int64
                                         const void* offsets, int off_is64, void* out, int out_dtype,
                                         int64_t B, int64_t U, int64_t S, int64_t D, int mode,
                                         void* stream);
+/*
+ * The same, and for every occurrence that lies in a segment 8 bytes of occ_out [B]: its segment (int32)
+ * and its coefficient in the backward (float: weight, divided by the length of the segment for MEAN).
+ * recis_csr_lists_from_occ puts them in the order of a plan's lists: what recis_csr_fill_lists finds by
+ * searching the offsets for every entry (src_pool_out and coef_out; coef_out may be NULL). SUM and MEAN.
+ */
+int recis_segment_reduce_forward_blocks_occ(const void* const* emb_blocks_dev, int64_t n_blocks,
+                                            int64_t block_rows, int64_t row_pitch_bytes,
+                                            const int64_t* row_index, int emb_dtype,
+                                            const void* weight, int weight_dtype,
+                                            const void* reverse_indices, int rev_is64,
+                                            const void* offsets, int off_is64, void* out, int out_dtype,
+                                            int64_t B, int64_t U, int64_t S, int64_t D, int mode,
+                                            void* occ_out, void* stream);
+int recis_csr_lists_from_occ(const int32_t* list, int64_t n, const void* occ, const void* offsets,
+                             int off_is64, int64_t S, int32_t* src_out, float* coef_out, void* stream);
 
 /*
  * Backward of the ragged-mode pooling: scatters the pooled gradient back to the

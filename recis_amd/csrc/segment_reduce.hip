@@ -47,7 +47,21 @@ struct SegArgs {
   const void* const* blocks;
   int64_t block_rows, n_blocks;
   int64_t pitch;  // elements from one row of a block to the next
+  int2* occ;      // [B] or NULL: (segment, coefficient as its bits) of every occurrence, for the backward
 };
+
+// What the backward asks about the occurrences [start, end) of segment s, written by the segment's team while it walks
+// them anyway: the backward takes the occurrences in the order of their ids, where finding an occurrence's segment
+// among the offsets again costs half a dozen scattered reads.
+__device__ __forceinline__ void note_occurrences(const SegArgs& a, int64_t s, int64_t start, int64_t end, int64_t seg_len,
+                                                 int lane_t, int team) {
+  if (a.occ == nullptr) return;  // uniform
+  for (int64_t r = start + lane_t; r < end; r += team) {
+    float w = a.weight ? load_weight(a.weight, a.wdt, r) : 1.0f;
+    if (a.mean) w /= static_cast<float>(seg_len);
+    a.occ[r] = make_int2(static_cast<int>(s), __float_as_int(w));
+  }
+}
 
 // Address of unique row idx (idx < U checked by the caller) in the block list, nullptr = zero row.
 template <typename TIn>
@@ -113,6 +127,7 @@ seg_pool_fwd_kernel(const TIn* __restrict__ emb, TOut* __restrict__ out, SegArgs
   const int col_stride = VEC << a.lpr_log2;
   const int D = a.D;
   const float scale = (a.mean && end > start) ? 1.0f / static_cast<float>(end - start) : 1.0f;
+  if constexpr (BLK) note_occurrences(a, s, start, end, end - start, lane_t, 1 << a.team_log2);
 
   auto fetch = [&](int64_t r, int c0, float (&v)[VEC], float& w) {
     int64_t idx;
@@ -253,6 +268,7 @@ seg_pool_fwd_fast_kernel(const TIn* __restrict__ emb, TOut* __restrict__ out, Se
   const int col_stride = VEC << a.lpr_log2;
   const int D = a.D;
   const float scale = (a.mean && seg_len > 0) ? 1.0f / static_cast<float>(seg_len) : 1.0f;
+  if constexpr (BLK) note_occurrences(a, s, start, end, seg_len, lane_t, team);
 
   const TIn* zero_row = reinterpret_cast<const TIn*>(g_zero_row);
   const int64_t zero_at = BLK ? 0 : zero_row - emb;
@@ -357,6 +373,22 @@ seg_pool_fwd_fast_kernel(const TIn* __restrict__ emb, TOut* __restrict__ out, Se
       store_pack<TOut, VEC>(out + s * D + c0, acc);
     }
   }
+}
+
+// src / coef per list entry out of what the forward noted per occurrence: one scattered 8-byte read each
+// (0.49 M entries 7.6 us, 0.5 TB/s: bound by the number of those reads; the search of the offsets took 23).
+__global__ void __launch_bounds__(kBlock)
+lists_from_occ_kernel(const int32_t* __restrict__ list, int64_t n, const int2* __restrict__ occ, const void* offsets,
+                      int off64, int64_t S, int32_t* __restrict__ src, float* __restrict__ coef) {
+  const int64_t k = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+  if (k >= n) return;
+  const int64_t i = list[k];
+  const int64_t first = load_index(offsets, off64, 0), last = load_index(offsets, off64, S);
+  if (static_cast<uint64_t>(i) >= static_cast<uint64_t>(n)) return;
+  const int2 o = occ[i];
+  const bool covered = i >= first && i < last;  // an occurrence in no segment: not noted, adds nothing
+  src[k] = covered ? o.x : -1;
+  if (coef) coef[k] = covered ? __int_as_float(o.y) : 0.f;
 }
 
 // MAX combiner: element-wise maximum and the occurrence that produced it.
@@ -985,6 +1017,7 @@ struct BlockSource {
   const void* const* blocks;
   int64_t block_rows, n_blocks;
   int64_t row_pitch_bytes;  // 0: rows lie back to back
+  int2* occ;                // see SegArgs
 };
 
 static int forward_impl(const void* unique_emb, const BlockSource* blk, int emb_dtype, const void* weight,
@@ -1039,6 +1072,7 @@ static int forward_impl(const void* unique_emb, const BlockSource* blk, int emb_
   a.blocks = blk ? blk->blocks : nullptr;
   a.block_rows = blk ? blk->block_rows : 1;
   a.n_blocks = blk ? blk->n_blocks : 0;
+  a.occ = blk ? blk->occ : nullptr;
   a.pitch = D;
   if (blk && blk->row_pitch_bytes) {
     RECIS_REQUIRE(blk->row_pitch_bytes >= D * in_sz && blk->row_pitch_bytes % in_sz == 0 &&
@@ -1149,17 +1183,43 @@ extern "C" int recis_segment_reduce_forward(
                       off_is64, out, out_dtype, argmax_out, B, U, S, D, mode, stream_);
 }
 
+extern "C" int recis_segment_reduce_forward_blocks_occ(
+    const void* const* emb_blocks_dev, int64_t n_blocks, int64_t block_rows, int64_t row_pitch_bytes,
+    const int64_t* row_index, int emb_dtype, const void* weight, int weight_dtype, const void* reverse_indices, int rev_is64,
+    const void* offsets, int off_is64, void* out, int out_dtype, int64_t B, int64_t U, int64_t S,
+    int64_t D, int mode, void* occ_out, void* stream_) {
+  RECIS_REQUIRE(mode != RECIS_MAX, "the MAX combiner takes dense rows (recis_segment_reduce_forward)");
+  RECIS_REQUIRE(n_blocks >= 0 && block_rows > 0, "bad block list");
+  RECIS_REQUIRE(U == 0 || (emb_blocks_dev != nullptr && row_index != nullptr), "NULL block list / row_index");
+  RECIS_REQUIRE(occ_out == nullptr || (mode != RECIS_TILE && S < INT32_MAX && reinterpret_cast<uintptr_t>(occ_out) % 8 == 0),
+                "occ_out: pooled segments, 8-byte aligned");
+  BlockSource blk{row_index, emb_blocks_dev, block_rows, n_blocks, row_pitch_bytes, static_cast<int2*>(occ_out)};
+  return forward_impl(nullptr, &blk, emb_dtype, weight, weight_dtype, reverse_indices, rev_is64, offsets, off_is64,
+                      out, out_dtype, nullptr, B, U, S, D, mode, stream_);
+}
+
 extern "C" int recis_segment_reduce_forward_blocks(
     const void* const* emb_blocks_dev, int64_t n_blocks, int64_t block_rows, int64_t row_pitch_bytes,
     const int64_t* row_index, int emb_dtype, const void* weight, int weight_dtype, const void* reverse_indices, int rev_is64,
     const void* offsets, int off_is64, void* out, int out_dtype, int64_t B, int64_t U, int64_t S,
     int64_t D, int mode, void* stream_) {
-  RECIS_REQUIRE(mode != RECIS_MAX, "the MAX combiner takes dense rows (recis_segment_reduce_forward)");
-  RECIS_REQUIRE(n_blocks >= 0 && block_rows > 0, "bad block list");
-  RECIS_REQUIRE(U == 0 || (emb_blocks_dev != nullptr && row_index != nullptr), "NULL block list / row_index");
-  BlockSource blk{row_index, emb_blocks_dev, block_rows, n_blocks, row_pitch_bytes};
-  return forward_impl(nullptr, &blk, emb_dtype, weight, weight_dtype, reverse_indices, rev_is64, offsets, off_is64,
-                      out, out_dtype, nullptr, B, U, S, D, mode, stream_);
+  return recis_segment_reduce_forward_blocks_occ(emb_blocks_dev, n_blocks, block_rows, row_pitch_bytes, row_index, emb_dtype,
+                                                 weight, weight_dtype, reverse_indices, rev_is64, offsets, off_is64, out,
+                                                 out_dtype, B, U, S, D, mode, nullptr, stream_);
+}
+
+extern "C" int recis_csr_lists_from_occ(const int32_t* list, int64_t n, const void* occ, const void* offsets, int off_is64,
+                                        int64_t S, int32_t* src_out, float* coef_out, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  RECIS_REQUIRE(n >= 0 && n < INT32_MAX && S >= 0, "bad size");
+  if (n == 0) return RECIS_OK;
+  RECIS_REQUIRE(list && occ && offsets && src_out, "NULL argument");
+  const dim3 grid(static_cast<uint32_t>((n + kBlock - 1) / kBlock));
+  RECIS_TIME_KERNEL("lists_from_occ_kernel", stream)
+  lists_from_occ_kernel<<<grid, dim3(kBlock), 0, stream>>>(list, n, static_cast<const int2*>(occ), offsets, off_is64, S, src_out,
+                                                          coef_out);
+  RECIS_LAUNCH_CHECK();
+  return RECIS_OK;
 }
 
 extern "C" int recis_segment_reduce_backward(
@@ -1196,6 +1256,7 @@ extern "C" int recis_segment_reduce_backward(
   const int lpr_log2 = std::min(6, ilog2_ceil((D + vec - 1) / vec));
 
   SegArgs a;
+  a.occ = nullptr;
   a.weight = weight;
   a.rev = reverse_indices;
   a.offs = offsets;

@@ -216,6 +216,18 @@ std::tuple<at::Tensor, c10::optional<at::Tensor>> BatchPlan::SrcCoefForPool(cons
   return std::make_tuple(fill_src_, fill_coef_.defined() ? c10::optional<at::Tensor>(fill_coef_) : c10::nullopt);
 }
 
+std::tuple<at::Tensor, c10::optional<at::Tensor>> BatchPlan::SrcCoefFromOcc(const at::Tensor& occ,
+                                                                             const at::Tensor& offsets, bool coef) {
+  c10::DeviceGuard guard(device());
+  auto i32 = at::TensorOptions().device(device()).dtype(at::kInt);
+  at::Tensor src = at::empty({n_}, i32), c;
+  if (coef) c = at::empty({n_}, i32.dtype(at::kFloat));
+  check(recis_csr_lists_from_occ(occ_.data_ptr<int32_t>(), n_, occ.data_ptr(), offsets.data_ptr(),
+                                 index_kind(offsets, "offsets"), offsets.numel() - 1, src.data_ptr<int32_t>(),
+                                 coef ? c.data_ptr<float>() : nullptr, stream_of(device())));
+  return std::make_tuple(src, coef ? c10::optional<at::Tensor>(c) : c10::nullopt);
+}
+
 at::Tensor BatchPlan::SrcForTile(const std::vector<int64_t>& batch, const std::vector<int64_t>& seq,
                                  const at::Tensor& offsets) {
   return std::get<2>(FillLists(offsets, at::Tensor(), false, false, &batch, &seq));

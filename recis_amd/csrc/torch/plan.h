@@ -55,6 +55,9 @@ class BatchPlan : public torch::CustomClassHolder {
   std::tuple<at::Tensor, c10::optional<at::Tensor>> SrcCoefForPool(const at::Tensor& offsets,
                                                                    const c10::optional<at::Tensor>& weight,
                                                                    bool mean);
+  // The same from what the forward noted per occurrence (recis_segment_reduce_forward_blocks_occ).
+  std::tuple<at::Tensor, c10::optional<at::Tensor>> SrcCoefFromOcc(const at::Tensor& occ, const at::Tensor& offsets,
+                                                                   bool coef);
   // src per list entry for the backward of the padded gather (ragged_tile).
   at::Tensor SrcForTile(const std::vector<int64_t>& batch, const std::vector<int64_t>& seq,
                         const at::Tensor& offsets);

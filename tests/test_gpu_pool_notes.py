@@ -1,0 +1,75 @@
+"""Pooling of table rows with weights, and what it notes per occurrence for the backward, against torch in 64 bits and
+recis_csr_fill_lists."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from recis_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _p(t):
+    return ctypes.c_void_p(None if t is None else t.data_ptr())
+
+
+def _i(x):
+    return ctypes.c_int64(x)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("weighted,mean", [(True, False), (True, True), (False, True), (False, False)])
+@pytest.mark.parametrize("segments,mean_len,dim", [(300, 1, 16), (1000, 7, 24), (257, 30, 64), (129, 8, 256), (33, 400, 128),
+                                                   (500, 9, 3)])
+def test_pool_rows_with_notes(rng, dtype, weighted, mean, segments, mean_len, dim):
+    dev = "cuda"
+    lens = rng.poisson(mean_len, segments)
+    lead = 5  # ids in front of the first segment and behind the last: in none
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32) + lead).to(dev)
+    n, rows = int(off[-1]) + lead, 200
+    emb = torch.randn(rows, dim, device=dev).to(dtype)
+    row_index = torch.from_numpy(rng.permutation(rows)).to(dev)
+    row_index[3] = -1  # a key the table does not hold reads as zeros
+    rev = torch.from_numpy(rng.integers(0, rows, n).astype(np.int32)).to(dev)
+    weight = (torch.rand(n, device=dev) + 0.5).to(dtype) if weighted else None
+    blocks = torch.tensor([emb.data_ptr()], dtype=torch.int64, device=dev)
+    out = torch.empty(segments, dim, dtype=dtype, device=dev)
+    occ = torch.empty(n, 2, dtype=torch.int32, device=dev)
+    code = _lib.dtype_code(dtype)
+    rc = _lib.lib().recis_segment_reduce_forward_blocks_occ(
+        _p(blocks), _i(1), _i(rows), _i(0), _p(row_index), code, _p(weight), code if weighted else 0, _p(rev), 0, _p(off),
+        0, _p(out), code, _i(n), _i(rows), _i(segments), _i(dim), _lib.MODES["mean" if mean else "sum"], _p(occ), _lib.stream_ptr())
+    assert rc == 0
+    table = emb.double()[row_index.clamp(min=0)] * (row_index >= 0).double()[:, None]
+    seg = torch.repeat_interleave(torch.arange(segments, device=dev), (off[1:] - off[:-1]).long())
+    coef = weight.double()[lead:n - lead] if weighted else torch.ones(n - 2 * lead, dtype=torch.float64, device=dev)
+    want = torch.zeros(segments, dim, dtype=torch.float64, device=dev)
+    terms = table[rev.long()[lead:n - lead]] * coef[:, None]
+    want.index_add_(0, seg, terms)
+    size = torch.zeros_like(want).index_add_(0, seg, terms.abs())
+    if mean:
+        length = (off[1:] - off[:-1]).clamp(min=1).double()[:, None]
+        want, size = want / length, size / length
+    # a sum of L terms in float32: (L + 1) * 2^-24 of the terms' size, and one rounding to the table's type
+    bound = (int(lens.max()) + 2) * 2.0 ** -24 * size + (2.0 ** -8 if dtype == torch.bfloat16 else 0) * want.abs() + 1e-30
+    assert bool(((out.double() - want).abs() <= bound).all())
+
+    order = torch.from_numpy(rng.permutation(n).astype(np.int32)).to(dev)
+    lists = []
+    for notes in (True, False):
+        src = torch.empty(n, dtype=torch.int32, device=dev)
+        c = torch.empty(n, dtype=torch.float32, device=dev) if weighted or mean else None
+        if notes:
+            rc = _lib.lib().recis_csr_lists_from_occ(_p(order), _i(n), _p(occ), _p(off), 0, _i(segments), _p(src), _p(c),
+                                                     _lib.stream_ptr())
+        else:
+            rc = _lib.lib().recis_csr_fill_lists(_p(order), _i(n), _p(off), 0, _i(segments), _p(weight), code if weighted else 0,
+                                                 int(mean), _p(src), _p(c), None, None, _i(0), None, _lib.stream_ptr())
+        assert rc == 0
+        lists.append((src, c))
+    assert torch.equal(lists[0][0], lists[1][0])
+    if lists[0][1] is not None:
+        assert torch.equal(lists[0][1], lists[1][1])
+    assert _lib.poll_device_errors() == 0
