@@ -1388,9 +1388,18 @@ plan_assign_new_kernel(Slot* __restrict__ table, const NewRec* __restrict__ new_
   // nb here = 1 + buckets: the new keys among the heavy ids, then those of every bucket
   extern __shared__ int32_t first_new[];  // [nb + 1], then kPartBlock words of scan scratch
   // a batch of known keys only (the steady state of a table that is not growing): nothing to scan
+  // or to hand out, and nobody to wait for: the first workgroup does the bookkeeping, the others leave before they take a
+  // ticket (256 tickets on one word are served one after the other: 8.3 -> 4.4 us for the 1024 buckets of a large batch)
   const bool any_new = __hip_atomic_load(&sync[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;  // uniform
-  if (any_new) scan_counts(new_count, nb, first_new, first_new + nb + 1);
-  const int64_t n_new = any_new ? first_new[nb] : 0;
+  if (!any_new) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+      commit_new_keys(state, 0);
+      publish(state, mirror, seq);
+    }
+    return;
+  }
+  scan_counts(new_count, nb, first_new, first_new + nb + 1);
+  const int64_t n_new = first_new[nb];
   const int64_t old_cur = state[ST_CUR], old_free = state[ST_FREE];
   for (int b = blockIdx.x; b < nb && n_new > 0; b += gridDim.x) {
     const int32_t cnt = new_count[b];
