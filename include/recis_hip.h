@@ -215,6 +215,13 @@ int recis_ragged_tile(const int64_t* batch, const int64_t* seq, int64_t n_featur
                       const void* value, int value_is64, int64_t n_values, const void* offset,
                       int off_is64, const void* table, int64_t table_rows, int dtype, void* out,
                       int64_t D, void* stream);
+/* The forward with the rows read where the table keeps them: value names unique ids below U, unique id u
+ * is row row_index[u] of the block list (negative: zeros; blocks as in recis_segment_reduce_forward_blocks). */
+int recis_ragged_tile_blocks(const int64_t* batch, const int64_t* seq, int64_t n_features,
+                             const void* value, int value_is64, int64_t n_values, const void* offset,
+                             int off_is64, const void* const* emb_blocks_dev, int64_t n_blocks,
+                             int64_t block_rows, int64_t row_pitch_bytes, const int64_t* row_index,
+                             int64_t U, int dtype, void* out, int64_t D, void* stream);
 int recis_ragged_tile_back(const int64_t* batch, const int64_t* seq, int64_t n_features,
                            const void* value, int value_is64, int64_t n_values,
                            const void* offset, int off_is64, const void* dy, int dtype,

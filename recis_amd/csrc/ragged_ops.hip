@@ -14,12 +14,23 @@
 namespace recis_hip {
 namespace {
 
+// Rows in a block list: unique row idx is row row_index[idx] (negative = zeros).
+struct TileBlocks {
+  const int64_t* row_index;
+  const void* const* blocks;
+  int64_t block_rows, n_blocks;
+  int64_t pitch;  // elements from one row of a block to the next
+};
+
 // One feature of ragged_tile: `batch` samples, `seq` output rows per sample.
 // Output row (b, t) = table[value[off[b] + t]] if t < len_b else 0.
-template <typename T, int VEC>
+// Bound by the stores (2 GB at 6.7 TB/s for 4 features of 2048 samples of 1000 rows of 256 bytes), under which the chain
+// value -> row index -> row of BLK is hidden: a dense copy of the unique rows first cost 20 us and the host's
+// wait for their number, and the gather itself takes 80 us a feature instead of 78.
+template <typename T, int VEC, bool BLK>
 __global__ void __launch_bounds__(kBlock)
 tile_fwd_kernel(const void* __restrict__ value, int val64, const void* __restrict__ offset, int off64,
-                const T* __restrict__ table, int64_t table_rows, T* __restrict__ out, int64_t batch,
+                const T* __restrict__ table, int64_t table_rows, TileBlocks blk, T* __restrict__ out, int64_t batch,
                 int64_t seq, int64_t n_values, int D, int lpr_log2, int blocks_per_sample, int* err) {
   // one sample per group of `blocks_per_sample` workgroups: no per-lane division, the sample's
   // two offsets are uniform loads; most output rows are padding, written once and not read here
@@ -34,10 +45,24 @@ tile_fwd_kernel(const void* __restrict__ value, int val64, const void* __restric
     raise_device_error(err, RECIS_DEVERR_OFFSETS);
   } else if (t < end - start) {
     const int64_t idx = load_index(value, val64, start + t);
-    if (static_cast<uint64_t>(idx) < static_cast<uint64_t>(table_rows))
-      src = table + idx * D;
-    else
+    if (static_cast<uint64_t>(idx) >= static_cast<uint64_t>(table_rows)) {
       raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
+    } else if constexpr (BLK) {
+      const int64_t ri = blk.row_index[idx];
+      if (ri >= 0) {  // else a key the table does not hold: zeros
+        int64_t k = 0, r = ri;
+        if (blk.n_blocks > 1) {
+          k = ri / blk.block_rows;
+          r = ri - k * blk.block_rows;
+        }
+        if (k >= blk.n_blocks || r >= blk.block_rows)
+          raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
+        else
+          src = static_cast<const T*>(blk.blocks[k]) + r * blk.pitch;
+      }
+    } else {
+      src = table + idx * D;
+    }
   }
   T* dst = out + (b * seq + t) * D;
   for (int c0 = cl * VEC; c0 < D; c0 += VEC << lpr_log2) {
@@ -197,10 +222,10 @@ using namespace recis_hip;
 
 extern "C" {
 
-int recis_ragged_tile(const int64_t* batch, const int64_t* seq, int64_t n_features, const void* value,
-                      int value_is64, int64_t n_values, const void* offset, int off_is64,
-                      const void* table, int64_t table_rows, int dtype, void* out, int64_t D,
-                      void* stream_) {
+static int ragged_tile_impl(const int64_t* batch, const int64_t* seq, int64_t n_features, const void* value,
+                            int value_is64, int64_t n_values, const void* offset, int off_is64, const void* table,
+                            int64_t table_rows, const TileBlocks* rows_in, int64_t row_pitch_bytes, int dtype, void* out,
+                            int64_t D, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   RECIS_REQUIRE(n_features >= 0 && n_values >= 0 && table_rows >= 0, "negative size");
   RECIS_REQUIRE(D >= 1 && D <= (1 << 20), "embedding dim %lld out of range", (long long)D);
@@ -212,6 +237,16 @@ int recis_ragged_tile(const int64_t* batch, const int64_t* seq, int64_t n_featur
   RECIS_REQUIRE(err != nullptr, "could not reach the device error word");
   const int vb = pick_vec_bytes(D * esz, reinterpret_cast<uintptr_t>(table) | reinterpret_cast<uintptr_t>(out));
   const int vec = std::max(1, vb / esz);
+  TileBlocks blk{};
+  if (rows_in) {  // blocks are 16-byte aligned by contract
+    blk = *rows_in;
+    blk.pitch = D;
+    if (row_pitch_bytes) {
+      RECIS_REQUIRE(row_pitch_bytes >= D * esz && row_pitch_bytes % esz == 0 && row_pitch_bytes % vb == 0,
+                    "row pitch of %lld bytes does not fit rows of %lld elements", (long long)row_pitch_bytes, (long long)D);
+      blk.pitch = row_pitch_bytes / esz;
+    }
+  }
   const int lpr_log2 = std::min(6, ilog2_ceil((D + vec - 1) / vec));
   const int rows_per_block = kBlock >> lpr_log2;
   int64_t obase = 0, rbase = 0;
@@ -228,11 +263,18 @@ int recis_ragged_tile(const int64_t* batch, const int64_t* seq, int64_t n_featur
       int rc = dispatch_t_vec(dtype, vec, [&](auto t, auto vtag) {
         using T = decltype(t);
         constexpr int VEC = decltype(vtag)::value;
-        RECIS_TIME_KERNEL("tile_fwd_kernel", stream)
-        tile_fwd_kernel<T, VEC><<<dim3(grid), dim3(kBlock), 0, stream>>>(
-            value, value_is64, off_f, off_is64, static_cast<const T*>(table), table_rows,
-            static_cast<T*>(out) + rbase * D, batch[f], seq[f], n_values, static_cast<int>(D), lpr_log2,
-            static_cast<int>(blocks_per_sample), err);
+        auto launch = [&](auto in_blocks) {
+          tile_fwd_kernel<T, VEC, decltype(in_blocks)::value><<<dim3(grid), dim3(kBlock), 0, stream>>>(
+              value, value_is64, off_f, off_is64, static_cast<const T*>(table), table_rows, blk,
+              static_cast<T*>(out) + rbase * D, batch[f], seq[f], n_values, static_cast<int>(D), lpr_log2,
+              static_cast<int>(blocks_per_sample), err);
+        };
+        RECIS_TIME_KERNEL("tile_fwd_kernel", stream) {
+          if (rows_in)
+            launch(std::true_type{});
+          else
+            launch(std::false_type{});
+        }
         RECIS_LAUNCH_CHECK();
         return RECIS_OK;
       });
@@ -242,6 +284,26 @@ int recis_ragged_tile(const int64_t* batch, const int64_t* seq, int64_t n_featur
     rbase += rows;
   }
   return RECIS_OK;
+}
+
+int recis_ragged_tile(const int64_t* batch, const int64_t* seq, int64_t n_features, const void* value,
+                      int value_is64, int64_t n_values, const void* offset, int off_is64,
+                      const void* table, int64_t table_rows, int dtype, void* out, int64_t D,
+                      void* stream_) {
+  return ragged_tile_impl(batch, seq, n_features, value, value_is64, n_values, offset, off_is64, table, table_rows, nullptr, 0,
+                          dtype, out, D, stream_);
+}
+
+int recis_ragged_tile_blocks(const int64_t* batch, const int64_t* seq, int64_t n_features, const void* value,
+                             int value_is64, int64_t n_values, const void* offset, int off_is64,
+                             const void* const* emb_blocks_dev, int64_t n_blocks, int64_t block_rows,
+                             int64_t row_pitch_bytes, const int64_t* row_index, int64_t U, int dtype, void* out,
+                             int64_t D, void* stream_) {
+  RECIS_REQUIRE(n_blocks >= 0 && block_rows > 0, "bad block list");
+  RECIS_REQUIRE(U == 0 || (emb_blocks_dev != nullptr && row_index != nullptr), "NULL block list / row_index");
+  const TileBlocks blk{row_index, emb_blocks_dev, block_rows, n_blocks, D};
+  return ragged_tile_impl(batch, seq, n_features, value, value_is64, n_values, offset, off_is64, nullptr, U, &blk,
+                          row_pitch_bytes, dtype, out, D, stream_);
 }
 
 int recis_ragged_tile_back(const int64_t* batch, const int64_t* seq, int64_t n_features, const void* value,

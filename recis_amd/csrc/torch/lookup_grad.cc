@@ -211,10 +211,15 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor>> Has
   std::vector<std::vector<int64_t>> shapes(n);
   at::Tensor out;
   if (tile) {
-    const int64_t U = plan->U();  // the padded gather reads a dense copy of the rows: this forward needs the count
-    at::Tensor rows = recis::functional::block_gather(SettleLookup(index, U, plan), chunks, emb->ChunkRows(), kNullIndex,
-                                                      false);
-    out = recis::functional::ragged_tile(segments, tile_len, plan->inverse(), merged, rows)[0];
+    int64_t rows = 0;
+    for (size_t k = 0; k < n; ++k) rows += segments[k] * tile_len[k];
+    out = at::empty({rows, D}, at::TensorOptions().device(device_).dtype(dtype_));
+    at::Tensor rev = plan->inverse(), table = block_ptr_table(chunks);
+    check(recis_ragged_tile_blocks(segments.data(), tile_len.data(), static_cast<int64_t>(n), rev.data_ptr(), 0, plan->n(),
+                                   merged.data_ptr(), index_kind(merged, "offsets"),
+                                   reinterpret_cast<const void* const*>(table.data_ptr()), static_cast<int64_t>(chunks.size()),
+                                   emb->ChunkRows(), chunks.empty() ? 0 : recis::hipabi::row_pitch_bytes(chunks[0]),
+                                   index.data_ptr<int64_t>(), index.numel(), dtype_code(dtype_), out.data_ptr(), D, stream_of(device_)));
     node->tile = true;
     node->batch = segments;
     node->seq = tile_len;
