@@ -251,6 +251,8 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor>> Has
       out = at::empty({total_segments, D}, chunks[0].options());
       if (at::GradMode::is_enabled() && NotesOccurrences(plan->n(), total_segments, weight.defined()))
         node->occ = at::empty({plan->n()}, index.options());
+      else if (at::GradMode::is_enabled())
+        plan->NotePool(merged, weight, mean);
       check(recis_segment_reduce_forward_blocks_occ(
           reinterpret_cast<const void* const*>(table.data_ptr()), static_cast<int64_t>(chunks.size()), emb->ChunkRows(),
           recis::hipabi::row_pitch_bytes(chunks[0]), index.data_ptr<int64_t>(), dtype_code(dtype_),

@@ -205,15 +205,27 @@ std::tuple<at::Tensor, c10::optional<at::Tensor>> BatchPlan::SrcCoefForPool(cons
     return std::make_tuple(fill_src_, fill_coef_.defined() ? c10::optional<at::Tensor>(fill_coef_) : c10::nullopt);
   }
   auto filled = FillLists(offsets, has_w ? *weight : at::Tensor(), mean, true, nullptr, nullptr);
+  KeepPoolLists(offsets, has_w ? *weight : at::Tensor(), mean, std::get<0>(filled), std::get<1>(filled));
+  return std::make_tuple(fill_src_, fill_coef_.defined() ? c10::optional<at::Tensor>(fill_coef_) : c10::nullopt);
+}
+
+void BatchPlan::KeepPoolLists(const at::Tensor& offsets, const at::Tensor& weight, bool mean, const at::Tensor& src,
+                              const at::Tensor& coef) {
   fill_offsets_ = offsets.data_ptr();
-  fill_weight_ = wp;
+  fill_weight_ = weight.defined() ? weight.data_ptr() : nullptr;
   fill_keep_offsets_ = offsets;  // alive as long as the cache entry: its address cannot be handed out again
-  fill_keep_weight_ = has_w ? *weight : at::Tensor();
+  fill_keep_weight_ = weight;
   fill_mean_ = mean;
   fill_valid_ = true;
-  fill_src_ = std::get<0>(filled);
-  fill_coef_ = std::get<1>(filled);
-  return std::make_tuple(fill_src_, fill_coef_.defined() ? c10::optional<at::Tensor>(fill_coef_) : c10::nullopt);
+  fill_src_ = src;
+  fill_coef_ = coef;
+}
+
+void BatchPlan::NotePool(const at::Tensor& offsets, const at::Tensor& weight, bool mean) {
+  if (offsets.numel() - 1 == n_ && !weight.defined()) return;  // SrcCoefForPool has nothing to fill
+  note_offsets_ = offsets;
+  note_weight_ = weight;
+  note_mean_ = mean;
 }
 
 std::tuple<at::Tensor, c10::optional<at::Tensor>> BatchPlan::SrcCoefFromOcc(const at::Tensor& occ,
@@ -230,6 +242,11 @@ std::tuple<at::Tensor, c10::optional<at::Tensor>> BatchPlan::SrcCoefFromOcc(cons
 
 at::Tensor BatchPlan::SrcForTile(const std::vector<int64_t>& batch, const std::vector<int64_t>& seq,
                                  const at::Tensor& offsets) {
+  if (note_offsets_.defined() && !fill_valid_ && note_offsets_.is_same(offsets)) {
+    auto both = FillLists(offsets, note_weight_, note_mean_, true, &batch, &seq);
+    KeepPoolLists(offsets, note_weight_, note_mean_, std::get<0>(both), std::get<1>(both));
+    return std::get<2>(both);
+  }
   return std::get<2>(FillLists(offsets, at::Tensor(), false, false, &batch, &seq));
 }
 

@@ -58,6 +58,9 @@ class BatchPlan : public torch::CustomClassHolder {
   // The same from what the forward noted per occurrence (recis_segment_reduce_forward_blocks_occ).
   std::tuple<at::Tensor, c10::optional<at::Tensor>> SrcCoefFromOcc(const at::Tensor& occ, const at::Tensor& offsets,
                                                                    bool coef);
+  // A pooled output of this plan whose backward will ask for SrcCoefForPool(offsets, weight, mean): a padded
+  // output over the same offsets that comes first then fills both lists in one launch (one search of the offsets).
+  void NotePool(const at::Tensor& offsets, const at::Tensor& weight, bool mean);
   // src per list entry for the backward of the padded gather (ragged_tile).
   at::Tensor SrcForTile(const std::vector<int64_t>& batch, const std::vector<int64_t>& seq,
                         const at::Tensor& offsets);
@@ -88,6 +91,10 @@ class BatchPlan : public torch::CustomClassHolder {
   const void* fill_weight_ = nullptr;
   bool fill_mean_ = false, fill_valid_ = false;
   at::Tensor fill_src_, fill_coef_, fill_keep_offsets_, fill_keep_weight_;
+  void KeepPoolLists(const at::Tensor& offsets, const at::Tensor& weight, bool mean, const at::Tensor& src,
+                     const at::Tensor& coef);
+  at::Tensor note_offsets_, note_weight_;  // NotePool; undefined: none
+  bool note_mean_ = false;
 };
 
 using BatchPlanPtr = c10::intrusive_ptr<BatchPlan>;
