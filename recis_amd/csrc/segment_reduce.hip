@@ -47,6 +47,7 @@ struct SegArgs {
   const void* const* blocks;
   int64_t block_rows, n_blocks;
   int64_t pitch;  // elements from one row of a block to the next
+  int in_runs;    // kernels that stream rows in order: workgroups placed in runs (see block_in_runs)
   int2* occ;      // [B] or NULL: (segment, coefficient as its bits) of every occurrence, for the backward
 };
 
@@ -83,9 +84,13 @@ __device__ __forceinline__ const TIn* block_row(const SegArgs& a, int64_t idx) {
 // The workgroup's place in a grid whose workgroups stream through memory side by side. Workgroups go round the 8 XCDs in
 // the order of their index; here runs of kXcdRun consecutive places are worked by one XCD (a part of the grid
 // that does not fill 8 runs is left as it is). Neighbouring workgroups' ends share memory pages and lines, and every
-// XCD then walks eight long streams instead of every eighth 30 KB of one. Measured, 0.52 M segments of 30 rows of 256
-// bytes (4 GB; runs of 1, 4, 16, 64, 512, an eighth of the grid): written 735, 710, 722, 725, 677, 676 us, read 687, 677, 676,
-// 666, 666, 693 us.
+// XCD then walks a stream of its own instead of every eighth 30 KB of one.
+// Measured, us for 4 GB in segments of 30 rows of 256 bytes (runs of 1, 4, 16, 64, 512, an eighth of the grid): written 735,
+// 710, 722, 725, 677, 676, read 687, 677, 676, 666, 666, 693. The shorter the segments, the less a workgroup has of its
+// stream; as is / in runs for the same 4 GB in segments of 6, 8, 12, 14, 16, 30 rows: written 903 / 963, 817 / 884, 752 / 841,
+// 737 / 714, 720 / 683, 746 / 695, read 1125 / 1131, 952 / 943, 832 / 807, 807 / 785, 745 / 723, 694 / 670. So the host asks
+// for runs where a workgroup reads 8 KB of rows or writes 16 KB.
+constexpr int64_t kRunReadBytes = 8 << 10, kRunWriteBytes = 16 << 10;
 constexpr uint32_t kXcds = 8, kXcdRun = 512;
 __device__ __forceinline__ uint32_t block_in_runs() {
   constexpr uint32_t group = kXcds * kXcdRun;
@@ -255,7 +260,7 @@ template <typename TIn, typename TOut, int VEC, int KIND, bool BLK, bool WG = fa
 __global__ void __launch_bounds__(kBlock)
 seg_pool_fwd_fast_kernel(const TIn* __restrict__ emb, TOut* __restrict__ out, SegArgs a) {
   extern __shared__ float s_wave_part[];  // WG only: [waves][D]
-  const uint32_t place = KIND == kFastPlain && !BLK && !WG ? block_in_runs() : blockIdx.x;
+  const uint32_t place = KIND == kFastPlain && !BLK && !WG && a.in_runs ? block_in_runs() : blockIdx.x;
   const int64_t s = WG ? static_cast<int64_t>(place)
                        : static_cast<int64_t>(place) * (kBlock >> a.team_log2) + (threadIdx.x >> a.team_log2);
   if (s >= a.S) return;  // whole teams leave together
@@ -486,7 +491,7 @@ template <typename TIn, typename TOut, int VEC, int KIND>
 __global__ void __launch_bounds__(kBlock)
 seg_max_fwd_fast_kernel(const TIn* __restrict__ emb, TOut* __restrict__ out, int32_t* __restrict__ argmax,
                         SegArgs a) {
-  const uint32_t place = KIND == kFastPlain ? block_in_runs() : blockIdx.x;
+  const uint32_t place = KIND == kFastPlain && a.in_runs ? block_in_runs() : blockIdx.x;
   const int64_t s = static_cast<int64_t>(place) * (kBlock >> a.team_log2) + (threadIdx.x >> a.team_log2);
   if (s >= a.S) return;  // whole teams leave together
   int64_t start = load_index(a.offs, a.off64, s);
@@ -679,7 +684,7 @@ fill_zero_rows_kernel(TOut* __restrict__ p, int64_t n_packs) {
 template <typename TG, typename TOut, int VEC, int KIND>
 __global__ void __launch_bounds__(kBlock)
 seg_pool_bwd_fast_kernel(const TG* __restrict__ grad_out, TOut* __restrict__ grad_unique, SegArgs a) {
-  const uint32_t place = KIND == kFastPlain ? block_in_runs() : blockIdx.x;
+  const uint32_t place = KIND == kFastPlain && a.in_runs ? block_in_runs() : blockIdx.x;
   const int64_t s = static_cast<int64_t>(place) * (kBlock >> a.team_log2) + (threadIdx.x >> a.team_log2);
   if (s >= a.S) return;  // whole teams leave together
   int64_t start = load_index(a.offs, a.off64, s);
@@ -869,7 +874,7 @@ template <typename TG, typename TOut, int VEC, int KIND>
 __global__ void __launch_bounds__(kBlock)
 seg_max_bwd_rows_kernel(const TG* __restrict__ grad_out, const int32_t* __restrict__ argmax,
                         TOut* __restrict__ grad_unique, SegArgs a) {
-  const uint32_t place = KIND == kFastPlain ? block_in_runs() : blockIdx.x;
+  const uint32_t place = KIND == kFastPlain && a.in_runs ? block_in_runs() : blockIdx.x;
   const int64_t s = static_cast<int64_t>(place) * (kBlock >> a.team_log2) + (threadIdx.x >> a.team_log2);
   if (s >= a.S) return;  // whole teams leave together
   int64_t start = load_index(a.offs, a.off64, s);
@@ -1091,6 +1096,7 @@ static int forward_impl(const void* unique_emb, const BlockSource* blk, int emb_
   a.block_rows = blk ? blk->block_rows : 1;
   a.n_blocks = blk ? blk->n_blocks : 0;
   a.occ = blk ? blk->occ : nullptr;
+  a.in_runs = B * D * dtype_size(emb_dtype) * (kBlock >> a.team_log2) >= kRunReadBytes * S;
   a.pitch = D;
   if (blk && blk->row_pitch_bytes) {
     RECIS_REQUIRE(blk->row_pitch_bytes >= D * in_sz && blk->row_pitch_bytes % in_sz == 0 &&
@@ -1288,6 +1294,7 @@ extern "C" int recis_segment_reduce_backward(
   a.lpr_log2 = lpr_log2;
   a.team_log2 = pick_team_log2(B, S, lpr_log2);
   a.mean = (mode == RECIS_MEAN);
+  a.in_runs = B * D * out_sz * (kBlock >> a.team_log2) >= kRunWriteBytes * S;
   // 1 GiB is far past what L2 and the 256 MB memory-side cache keep for the next kernel
   a.nt_out = U * D * out_sz >= (int64_t(1) << 30);
   a.nt_in = 0;
