@@ -150,7 +150,7 @@ at::Tensor Hashtable::GroupOffsets(const std::vector<TensorOrNone>& offsets, con
   return out;
 }
 
-c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor>> Hashtable::LookupTrain(
+c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::Tensor>> Hashtable::LookupTrain(
     const std::vector<at::Tensor>& values, const std::vector<TensorOrNone>& offsets,
     const std::vector<TensorOrNone>& weights, const c10::optional<std::vector<int64_t>>& tags,
     const std::string& combiner, const std::vector<int64_t>& tile_len, bool lean,
@@ -265,7 +265,7 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor>> Has
     for (size_t k = 0; k < n; ++k) shapes[k] = {segments[k], D};
   }
   NoteUnsettled(plan);
-  return std::make_tuple(outputs_of(out, shapes, node->split, node), plan, merged);
+  return std::make_tuple(outputs_of(out, shapes, node->split, node), plan, merged, index);
 }
 
 void Hashtable::NoteUnsettled(const BatchPlanPtr& plan) {

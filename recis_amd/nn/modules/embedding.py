@@ -294,7 +294,7 @@ class DynamicEmbedding(torch.nn.Module):
                 res = table._hashtable_impl.lookup_train([ids], [offs], [weight], None, opt.combiner, [], True, None, None)
                 if res is not None:
                     if not isinstance(table._filter_hook_impl, torch.nn.Identity):
-                        table._filter_hook_impl(res[1].index_buf[: res[1].U])
+                        table._filter_hook_impl(res[3][: res[1].U])
                     return res[0][0]
         plan = ops.ids_unique_plan(val, wait=False, need_pos=False)
         return lookup_and_pool(table, plan, weight, offsets, opt)

@@ -171,12 +171,13 @@ class EmbeddingEngine(torch.nn.Module):
         res = table._hashtable_impl.lookup_train(vals, offs, weights, tags, opt.combiner, tile_len, alone, plan, offsets)
         if res is None:
             return False
-        parts, plan, offsets = res
+        parts, plan, offsets, index = res
         if same not in plans:
             plans[same] = (offsets, plan)
         if not isinstance(table._filter_hook_impl, torch.nn.Identity):
-            # a step filter stamps the looked-up rows: it needs the rows proper, hence the count
-            table._filter_hook_impl(plan.index_buf[: plan.U])
+            # a step filter stamps the looked-up rows: it needs the rows proper, hence the count (and the rows this
+            # lookup found: a plan that another group made need not know any)
+            table._filter_hook_impl(index[: plan.U])
         for name, part, prefix in zip(names, parts, prefixes):
             outputs[name] = part if prefix is None else part.reshape(tuple(prefix) + (part.shape[1],))
         return True

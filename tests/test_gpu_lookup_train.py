@@ -6,11 +6,17 @@ import torch
 
 from recis_amd import _lib, ops
 from recis_amd.nn import EmbeddingEngine, EmbeddingOption, HashTable
+from recis_amd.nn.hashtable_hook import FilterHook
 from recis_amd.nn.modules.hashtable import HashtableRegister, filter_out_sparse_param
+from recis_amd.nn.modules.hashtable_hook_impl import HashtableHookFactory
 from recis_amd.optim import SparseAdagrad
 from recis_amd.ragged import RaggedTensor
 
 pytestmark = pytest.mark.gpu
+
+
+def _offsets(lens):
+    return torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)).cuda()
 
 
 @pytest.mark.parametrize("count", [2, 16, 17, 40])
@@ -95,3 +101,61 @@ def test_group_of_dense_and_ragged_features_matches_torch(rng, weighted):
     clear = np.abs(grad) > 1e-3
     np.testing.assert_allclose(rows.cpu().numpy()[clear], (start - 0.1 * np.sign(grad))[clear], rtol=1e-4, atol=1e-4)
     assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("second", ["tile", "sum"])
+def test_step_filter_stamps_rows_of_a_plan_made_without_the_map(rng, second):
+    """One input under "mean" with few ids per segment (the general path, whose plan knows no map) and under a combiner
+    that takes that plan over: the rows looked up by it are stamped, the gradients of both reach them."""
+    HashtableRegister().clear()
+    HashtableHookFactory().clear_filters()
+    D, B, seq = 8, 60, 4
+    common = dict(embedding_dim=D, block_size=64, shared_name="stamped", use_weight=False,
+                  filter_hook=FilterHook("GlobalStepFilter", {"filter_step": 5}))
+    kw = {"combiner_kwargs": {"tile_len": seq}} if second == "tile" else {}
+    eng = EmbeddingEngine({"m": EmbeddingOption(combiner="mean", **common),
+                           "x": EmbeddingOption(combiner=second, **kw, **common)})
+    eng.train()
+    opt = SparseAdagrad(filter_out_sparse_param(eng), lr=0.1)
+    (table,) = eng.hashtables().values()
+    impl = table._hashtable_impl
+    (step_filter,) = [f for fs in HashtableHookFactory().get_filters().values() for f in fs.values()]
+    start = rng.standard_normal((30, D)).astype(np.float32)
+    impl.insert(torch.arange(30, device="cuda"), torch.from_numpy(start).cuda())
+    step_filter.update_step(7)
+    lens = rng.integers(1, 4, B)
+    ids = rng.integers(0, 25, lens.sum())
+    rt = RaggedTensor(torch.from_numpy(ids).cuda(), _offsets(lens))
+    out = eng({"m": rt, "x": rt})
+    seg = np.repeat(np.arange(B), lens)
+    place = np.arange(len(ids)) - np.repeat(np.cumsum(lens) - lens, lens)
+    rows = start[ids].astype(np.float64)
+    mean = np.zeros((B, D))
+    np.add.at(mean, seg, rows / lens[seg][:, None])
+    np.testing.assert_allclose(out["m"].detach().cpu().numpy(), mean, rtol=1e-5, atol=1e-6)
+    up_m = rng.random((B, D)) + 0.5
+    grad = np.zeros((30, D))
+    np.add.at(grad, ids, up_m[seg] / lens[seg][:, None])
+    if second == "tile":
+        up_x = rng.random((B, seq, D)) + 0.5
+        padded = np.zeros((B, seq, D))
+        padded[seg[place < seq], place[place < seq]] = rows[place < seq]
+        np.testing.assert_allclose(out["x"].detach().cpu().numpy().reshape(B, seq, D), padded, rtol=1e-6)
+        np.add.at(grad, ids[place < seq], up_x[seg[place < seq], place[place < seq]])
+    else:
+        up_x = rng.random((B, D)) + 0.5
+        total = np.zeros((B, D))
+        np.add.at(total, seg, rows)
+        np.testing.assert_allclose(out["x"].detach().cpu().numpy(), total, rtol=1e-5, atol=1e-5)
+        np.add.at(grad, ids, up_x[seg])
+    torch.autograd.backward([out["m"], out["x"]], [torch.from_numpy(up_m.astype(np.float32)).cuda(),
+                                                   torch.from_numpy(up_x.astype(np.float32).reshape(B, -1)).cuda()])
+    opt.step()
+    keys, where = impl.ids_map()
+    stamp = torch.cat(impl.get_slot(step_filter._name).kernel_blocks()[0]).view(-1)[where].cpu().numpy()
+    accum = torch.cat(impl.get_slot("sparse_adagrad_accum").kernel_blocks()[0])[where].double().cpu().numpy()
+    used = np.isin(keys.cpu().numpy(), ids)
+    assert (stamp == np.where(used, 7, 0)).all()
+    # sums of up to about 20 terms in float32, squared
+    np.testing.assert_allclose(accum, grad[keys.cpu().numpy()] ** 2, rtol=2e-5, atol=1e-10)
+    HashtableHookFactory().clear_filters()
