@@ -1,8 +1,9 @@
 // The training lookups of the module layer with their autograd nodes: what EmbeddingEngine and
 // HashTable call once per table and step (recis/nn/modules/embedding_engine.py:607-675,
-// recis/nn/modules/hashtable.py:425-586). The forward queues dedup + lookup + pooling, the node's
-// backward hands the gradients to the table unsummed; neither waits for the device, and nothing per
-// feature is left to Python (a node written in Python costs 2 us per output each way: with 39
+// recis/nn/modules/hashtable.py:425-586). The forward queues dedup + lookup + pooling without waiting
+// for the device. The node's backward hands the gradients to the table unsummed; the batch's unique count, and what
+// the plan's kernels reported with it, is read there, behind the forward's launches: it has arrived or is about to, and
+// a plan that dropped entries raises before its gradient has reached the table. Nothing per feature is left to Python (a node written in Python costs 2 us per output each way: with 39
 // features that was most of a small step).
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/function.h>
@@ -65,7 +66,7 @@ struct LookupBackward : public torch::autograd::Node {
       src = std::get<0>(lists);
       coef = std::get<1>(lists);
     }
-    table->AcceptSplitGrad(index, plan, parts, split, src, coef, plan->serial(), /*may_miss=*/false, /*settle=*/false);
+    table->AcceptSplitGrad(index, plan, parts, split, src, coef, plan->serial(), /*may_miss=*/false, /*settle=*/true);
     return {};
   }
   void release_variables() override {
@@ -122,7 +123,6 @@ c10::optional<std::vector<at::Tensor>> Hashtable::DenseLookupTrain(const std::ve
     node->split.push_back(c.size(0));
     shapes.push_back({c.size(0), out.size(1)});
   }
-  NoteUnsettled(node->plan);
   return outputs_of(out, shapes, node->split, node);
 }
 
@@ -264,32 +264,7 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
     node->split = segments;
     for (size_t k = 0; k < n; ++k) shapes[k] = {segments[k], D};
   }
-  NoteUnsettled(plan);
   return std::make_tuple(outputs_of(out, shapes, node->split, node), plan, merged, index);
-}
-
-void Hashtable::NoteUnsettled(const BatchPlanPtr& plan) {
-  if (unsettled_.empty() || unsettled_.back().get() != plan.get()) unsettled_.push_back(plan);
-}
-
-void Hashtable::SettleArrived(size_t most_left) {
-  size_t done = 0;
-  while (done < unsettled_.size()) {
-    const BatchPlanPtr plan = unsettled_[done];
-    const bool wait = unsettled_.size() - done > most_left;
-    if (!wait && !plan->TryU()) break;
-    ++done;
-    const int64_t U = [&] {
-      try {
-        return plan->U();
-      } catch (...) {  // a device-side error: reported once
-        unsettled_.erase(unsettled_.begin(), unsettled_.begin() + done);
-        throw;
-      }
-    }();
-    SettleCount(U, plan);
-  }
-  unsettled_.erase(unsettled_.begin(), unsettled_.begin() + done);
 }
 
 void Hashtable::AcceptTileGrad(const at::Tensor& index, const BatchPlanPtr& plan, const at::Tensor& offsets,
@@ -309,6 +284,6 @@ void Hashtable::AcceptTileGrad(const at::Tensor& index, const BatchPlanPtr& plan
     one_type = one_type && parts[k].scalar_type() == parts[0].scalar_type();
   }
   const bool apart = parts.size() <= 8 && one_type;
-  AcceptPlannedGrad(index, plan, apart ? parts : std::vector<at::Tensor>{at::cat(parts)}, apart, src, c10::nullopt,
-                    c10::nullopt, plan->serial(), false);
+  std::vector<at::Tensor> rows = apart ? parts : std::vector<at::Tensor>{at::cat(parts)};
+  AcceptPlannedGrad(SettledRows(index, plan), plan, rows, apart, src, c10::nullopt, c10::nullopt, plan->serial(), false);
 }

@@ -100,27 +100,17 @@ BatchPlanPtr BatchPlan::Make(const std::vector<at::Tensor>& ids_in, const c10::o
   return p;
 }
 
-bool BatchPlan::FetchU(bool wait) {
-  if (U_ >= 0) return true;
+int64_t BatchPlan::U() {
+  if (U_ >= 0) return U_;
   c10::DeviceGuard guard(device());
   int64_t count = -1;
   int bits = 0;
-  check(recis_unique_plan_count_of(ticket_, wait ? 1 : 0, &count, &bits, stream_));
-  if (count < 0) {
-    if (!wait) return false;
-    count = counts_[0].item<int64_t>();  // many later plans of the stream have taken over the staging words
-  }
+  check(recis_unique_plan_count_of(ticket_, 1, &count, &bits, stream_));
+  if (count < 0) count = counts_[0].item<int64_t>();  // many later plans of the stream have taken over the staging words
   U_ = count;
   raise_device_errors(bits);
-  return true;
-}
-
-int64_t BatchPlan::U() {
-  FetchU(true);
   return U_;
 }
-
-bool BatchPlan::TryU() { return FetchU(false); }
 
 at::Tensor BatchPlan::unique() {
   if (!unique_.defined()) unique_ = unique_buf_.narrow(0, 0, U());

@@ -32,8 +32,6 @@ class BatchPlan : public torch::CustomClassHolder {
   int64_t hot_cap() const { return hot_cap_; }
   // The number of unique ids on the host; a plan made with wait == false fetches it here.
   int64_t U();
-  // The same without waiting: whether the host has the count now.
-  bool TryU();
   // The count if the host has it already, else the number of ids: for kernels that take the count
   // from device memory and only need a bound to size their grid.
   int64_t U_bound() const { return U_ < 0 ? n_ : U_; }
@@ -81,7 +79,6 @@ class BatchPlan : public torch::CustomClassHolder {
                                                            bool mean, bool want_pool,
                                                            const std::vector<int64_t>* batch,
                                                            const std::vector<int64_t>* seq);
-  bool FetchU(bool wait);
   int64_t n_ = 0, serial_ = 0, hot_cap_ = 0, U_ = -1, ticket_ = -1;
   void* stream_ = nullptr;
   at::Tensor unique_buf_, inverse_, row_start_, occ_, pos_, hot_items_, counts_, index_buf_, unique_;

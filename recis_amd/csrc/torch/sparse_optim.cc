@@ -86,7 +86,6 @@ void SparseOptimizer::step() {
       std::vector<PlannedGrad> planned = p.second->TakePlannedGrad();
       if (!planned.empty()) {
         UpdatePlanned(p.second, planned);
-        p.second->SettleArrived(2);
         continue;
       }
     }

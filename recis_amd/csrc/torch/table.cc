@@ -738,7 +738,6 @@ std::tuple<at::Tensor, at::Tensor> Hashtable::EvictOlder(const std::string& stam
 BatchPlanPtr Hashtable::PlanLookup(const std::vector<at::Tensor>& ids, const c10::optional<std::vector<int64_t>>& tags,
                                    bool wait, bool need_inverse, bool need_pos) {
   c10::DeviceGuard guard(device_);
-  SettleArrived(1);
   BatchPlanPtr plan = recis::BatchPlan::Make(ids, tags, map_->map, wait, need_inverse, need_pos);
   int64_t call = 0;
   check(recis_idmap_last_call(map_->map, &call));
@@ -777,6 +776,12 @@ at::Tensor Hashtable::SettleLookup(const at::Tensor& index_buf, int64_t n_true, 
   SettleCount(n_true, plan);
   MakeRoom(n_true);
   return index_buf.narrow(0, 0, n_true);
+}
+
+at::Tensor Hashtable::SettledRows(const at::Tensor& index, const BatchPlanPtr& plan) {
+  const int64_t U = plan->U();
+  SettleCount(U, plan);
+  return index.numel() > U ? index.narrow(0, 0, U) : index;
 }
 
 at::Tensor Hashtable::ExpandRows(const BatchPlanPtr& plan, const at::Tensor& row_index,
@@ -945,12 +950,7 @@ void Hashtable::AcceptSplitGrad(const at::Tensor& index_in, const BatchPlanPtr& 
       whole = at::cat(parts, 0);
     }
   }
-  at::Tensor index = index_in;
-  if (settle) {
-    const int64_t U = plan->U();
-    SettleCount(U, plan);
-    if (index.numel() > U) index = index.narrow(0, 0, U);
-  }
+  at::Tensor index = settle ? SettledRows(index_in, plan) : index_in;
   AcceptPlannedGrad(index, plan, {whole}, false, src.has_value() && src->defined() ? *src : plan->occ(), coef,
                     c10::nullopt, key, may_miss);
 }

@@ -325,12 +325,9 @@ class Hashtable : public torch::CustomClassHolder {
       const std::vector<c10::optional<at::Tensor>>& weights, const c10::optional<std::vector<int64_t>>& tags,
       const std::string& combiner, const std::vector<int64_t>& tile_len, bool lean,
       const c10::optional<recis::BatchPlanPtr>& shared_plan, const c10::optional<at::Tensor>& shared_offsets);
-  // Lookups whose unique count the host has not read yet (LookupTrain and DenseLookupTrain do not wait
-  // for it). SettleArrived tells the id map the counts that have arrived, which keeps its bounds
-  // tight, and raises what their kernels reported; it waits for the oldest ones until `most_left` are
-  // left, so that a program that never waits for the device is told within two steps.
-  void NoteUnsettled(const recis::BatchPlanPtr& plan);
-  void SettleArrived(size_t most_left);
+  // The rows of a plan's unique ids out of the full-length buffer: waits for the count if it is still on its way,
+  // raises what the plan's kernels reported, tells the id map.
+  at::Tensor SettledRows(const at::Tensor& index, const recis::BatchPlanPtr& plan);
   // The gradients of the padded outputs of one lookup, kept as separate arrays.
   void AcceptTileGrad(const at::Tensor& index, const recis::BatchPlanPtr& plan, const at::Tensor& offsets,
                       const std::vector<int64_t>& batch, const std::vector<int64_t>& seq,
@@ -400,7 +397,6 @@ class Hashtable : public torch::CustomClassHolder {
   std::vector<bool> grad_unique_;
   std::vector<std::pair<int64_t, size_t>> grad_keys_;
   std::vector<PlannedGrad> planned_;
-  std::vector<recis::BatchPlanPtr> unsettled_;
   // the index tensor the last embedding_lookup returned, and whether the ids it was given are
   // known to hold no duplicates (they came out of ids_partition): accept_grad of exactly that tensor
   // needs no dedup
