@@ -8,6 +8,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/function.h>
 #include <torch/csrc/autograd/functions/utils.h>
+#include <torch/csrc/autograd/saved_variable.h>
 
 #include <algorithm>
 
@@ -34,21 +35,27 @@ at::Tensor rows_of(const at::Tensor& whole, int64_t first, at::IntArrayRef shape
   return at::Tensor(std::move(impl));
 }
 
+using torch::autograd::SavedVariable;
+
 // The backward of one lookup of a table: the parts' gradients go to the table as they come.
 struct LookupBackward : public torch::autograd::Node {
   c10::intrusive_ptr<Hashtable> table;
   BatchPlanPtr plan;
-  at::Tensor index;
+  SavedVariable saved_index;
   std::vector<int64_t> split;        // rows per output
-  at::Tensor offsets, weight;        // pooled segments; both undefined: one id per segment
+  // Pooled segments; both undefined: one id per segment. They may be the caller's own tensors: saved as any node saves its
+  // inputs, so that a buffer refilled before the backward is refused and saved-tensor hooks see them.
+  SavedVariable saved_offsets, saved_weight;
   at::Tensor occ;                    // what the pooling noted per occurrence, or undefined
   bool mean = false;
   std::vector<int64_t> batch, seq;   // padded outputs (tile): samples and rows per sample of each
   bool tile = false;
 
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
+    std::lock_guard<std::mutex> lock(mutex_);
     TORCH_CHECK(plan.defined(), torch::autograd::ERR_BACKWARD_TWICE);
     at::NoGradGuard no_grad;
+    const at::Tensor index = saved_index.unpack(), offsets = saved_offsets.unpack(), weight = saved_weight.unpack();
     if (tile) {
       table->AcceptTileGrad(index, plan, offsets, batch, seq, grads);
       return {};
@@ -70,10 +77,11 @@ struct LookupBackward : public torch::autograd::Node {
     return {};
   }
   void release_variables() override {
+    std::lock_guard<std::mutex> lock(mutex_);
     plan.reset();
-    index.reset();
-    offsets.reset();
-    weight.reset();
+    saved_index.reset_data();
+    saved_offsets.reset_data();
+    saved_weight.reset_data();
     occ.reset();
   }
   std::string name() const override { return "RecisLookupBackward"; }
@@ -89,7 +97,7 @@ bool NotesOccurrences(int64_t n, int64_t segments, bool weighted) {
   return n <= (int64_t(1) << 19) || segments > 8192;
 }
 
-// The outputs of a lookup, with the node behind them when gradients are recorded.
+// The outputs of a lookup, with the node behind them (none when gradients are not recorded).
 std::vector<at::Tensor> outputs_of(const at::Tensor& whole, const std::vector<std::vector<int64_t>>& shapes,
                                    const std::vector<int64_t>& split, const std::shared_ptr<LookupBackward>& node) {
   std::vector<at::Tensor> out;
@@ -99,7 +107,7 @@ std::vector<at::Tensor> outputs_of(const at::Tensor& whole, const std::vector<st
     out.push_back(rows_of(whole, first, shapes[k]));
     first += split[k];
   }
-  if (at::GradMode::is_enabled()) {
+  if (node) {
     for (auto& o : out) torch::autograd::set_history(o, node);
   }
   return out;
@@ -113,17 +121,22 @@ c10::optional<std::vector<at::Tensor>> Hashtable::DenseLookupTrain(const std::ve
                                                                    const c10::optional<at::Tensor>& stamp_value) {
   auto found = DenseLookupExpand(cols, tags, stamp_slot, stamp_value);
   if (!found.has_value()) return c10::nullopt;
-  auto node = std::make_shared<LookupBackward>();
-  node->table = c10::intrusive_ptr<Hashtable>::reclaim_copy(this);
-  node->plan = std::get<0>(*found);
-  node->index = std::get<1>(*found);
   const at::Tensor& out = std::get<2>(*found);
   std::vector<std::vector<int64_t>> shapes;
+  std::vector<int64_t> split;
   for (const auto& c : cols) {
-    node->split.push_back(c.size(0));
+    split.push_back(c.size(0));
     shapes.push_back({c.size(0), out.size(1)});
   }
-  return outputs_of(out, shapes, node->split, node);
+  std::shared_ptr<LookupBackward> node;
+  if (at::GradMode::is_enabled()) {
+    node = std::make_shared<LookupBackward>();
+    node->table = c10::intrusive_ptr<Hashtable>::reclaim_copy(this);
+    node->plan = std::get<0>(*found);
+    node->saved_index = SavedVariable(std::get<1>(*found), false);
+    node->split = split;
+  }
+  return outputs_of(out, shapes, split, node);
 }
 
 // Segments of several features as one list: the given offsets, and 0, width, 2 * width, ... for the dense
@@ -199,17 +212,13 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
   c10::optional<at::Tensor> found = PlanIndex(plan);
   at::Tensor index = found.has_value() ? *found : LookupIndexCounted(plan, true);
 
-  auto node = std::make_shared<LookupBackward>();
-  node->table = c10::intrusive_ptr<Hashtable>::reclaim_copy(this);
-  node->plan = plan;
-  node->index = index;
-  node->offsets = merged;
-  node->mean = mean;
+  const bool recorded = at::GradMode::is_enabled();
   auto emb = slot_group_->EmbSlot();
   const auto& chunks = emb->Chunks();
   const int64_t D = emb->FlatSize();
   std::vector<std::vector<int64_t>> shapes(n);
-  at::Tensor out;
+  std::vector<int64_t> split = segments;
+  at::Tensor out, weight, occ, back_offsets = merged;
   if (tile) {
     int64_t rows = 0;
     for (size_t k = 0; k < n; ++k) rows += segments[k] * tile_len[k];
@@ -220,15 +229,11 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
                                    reinterpret_cast<const void* const*>(table.data_ptr()), static_cast<int64_t>(chunks.size()),
                                    emb->ChunkRows(), chunks.empty() ? 0 : recis::hipabi::row_pitch_bytes(chunks[0]),
                                    index.data_ptr<int64_t>(), index.numel(), dtype_code(dtype_), out.data_ptr(), D, stream_of(device_)));
-    node->tile = true;
-    node->batch = segments;
-    node->seq = tile_len;
     for (size_t k = 0; k < n; ++k) {
-      node->split.push_back(segments[k] * tile_len[k]);
+      split[k] = segments[k] * tile_len[k];
       shapes[k] = {segments[k], tile_len[k] * D};
     }
   } else {
-    at::Tensor weight;
     if (any_weight) {
       std::vector<at::Tensor> parts;
       auto opt = at::TensorOptions().device(device_).dtype(dtype_);
@@ -239,9 +244,8 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
         parts.push_back(has ? weights[k]->reshape({-1}).to(opt) : at::ones({n_ids[k]}, opt));
       }
       weight = n == 1 ? parts[0].contiguous() : at::cat(parts);
-      node->weight = weight;
       // (the backward of one weighted id per segment walks the segments like any other)
-      if (unit_path) node->offsets = GroupOffsets(offsets, segments, widths, n_ids);
+      if (unit_path) back_offsets = GroupOffsets(offsets, segments, widths, n_ids);
     }
     if (unit_path) {
       out = ExpandRows(plan, index, weight.defined() ? c10::optional<at::Tensor>(weight) : c10::nullopt, c10::nullopt,
@@ -249,9 +253,9 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
     } else {
       at::Tensor rev = plan->inverse(), table = block_ptr_table(chunks);
       out = at::empty({total_segments, D}, chunks[0].options());
-      if (at::GradMode::is_enabled() && NotesOccurrences(plan->n(), total_segments, weight.defined()))
-        node->occ = at::empty({plan->n()}, index.options());
-      else if (at::GradMode::is_enabled())
+      if (recorded && NotesOccurrences(plan->n(), total_segments, weight.defined()))
+        occ = at::empty({plan->n()}, index.options());
+      else if (recorded)
         plan->NotePool(merged, weight, mean);
       check(recis_segment_reduce_forward_blocks_occ(
           reinterpret_cast<const void* const*>(table.data_ptr()), static_cast<int64_t>(chunks.size()), emb->ChunkRows(),
@@ -259,12 +263,28 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
           weight.defined() ? weight.data_ptr() : nullptr, weight.defined() ? dtype_code(weight.scalar_type()) : 0,
           rev.data_ptr(), 0, merged.data_ptr(), index_kind(merged, "offsets"), out.data_ptr(), dtype_code(dtype_), plan->n(),
           index.numel(), total_segments, D, mean ? RECIS_MEAN : RECIS_SUM,
-          node->occ.defined() ? node->occ.data_ptr() : nullptr, stream_of(device_)));
+          occ.defined() ? occ.data_ptr() : nullptr, stream_of(device_)));
     }
-    node->split = segments;
     for (size_t k = 0; k < n; ++k) shapes[k] = {segments[k], D};
   }
-  return std::make_tuple(outputs_of(out, shapes, node->split, node), plan, merged, index);
+  std::shared_ptr<LookupBackward> node;
+  if (recorded) {
+    node = std::make_shared<LookupBackward>();
+    node->table = c10::intrusive_ptr<Hashtable>::reclaim_copy(this);
+    node->plan = plan;
+    node->saved_index = SavedVariable(index, false);
+    node->saved_offsets = SavedVariable(back_offsets, false);
+    node->saved_weight = SavedVariable(weight, false);
+    node->occ = occ;
+    node->mean = mean;
+    node->tile = tile;
+    node->split = split;
+    if (tile) {
+      node->batch = segments;
+      node->seq = tile_len;
+    }
+  }
+  return std::make_tuple(outputs_of(out, shapes, split, node), plan, merged, index);
 }
 
 void Hashtable::AcceptTileGrad(const at::Tensor& index, const BatchPlanPtr& plan, const at::Tensor& offsets,

@@ -201,3 +201,61 @@ def test_a_faulty_batch_does_not_reach_the_table(rng, kind):
     step(good)
     assert _lib.poll_device_errors() == 0
     assert not torch.equal(state()["embedding"], before["embedding"])
+
+
+@pytest.mark.parametrize("combiner,weighted,what", [("tile", False, "offsets"), ("sum", False, "offsets"), ("sum", True, "weight"),
+                                                    ("mean", True, "offsets")])
+def test_inputs_refilled_before_the_backward_are_refused(rng, combiner, weighted, what):
+    HashtableRegister().clear()
+    kw = {"combiner_kwargs": {"tile_len": 5}} if combiner == "tile" else {}
+    eng = EmbeddingEngine({"a": EmbeddingOption(embedding_dim=8, block_size=64, shared_name="refilled", use_weight=weighted,
+                                                combiner=combiner, **kw)})
+    eng.train()
+    lens = rng.integers(8, 12, 40)
+    off = _offsets(lens)
+    n = int(off[-1])
+    weight = torch.rand(n, device="cuda") + 0.5 if weighted else None
+    out = eng({"a": RaggedTensor(torch.from_numpy(rng.integers(0, 50, n)).cuda(), off, weight)})["a"]
+    if what == "weight":
+        weight.mul_(2)
+    else:
+        off.copy_(_offsets(rng.permutation(lens)))
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
+@pytest.mark.parametrize("combiner", ["tile", "sum", "mean"])
+def test_saved_tensor_hooks_see_the_inputs(rng, combiner):
+    """What the backward needs of the caller's tensors goes through saved-tensor hooks (offloading, checkpointing)."""
+    lens = rng.integers(8, 12, 40)
+    ids = rng.integers(0, 50, lens.sum())
+    weight = (rng.random(len(ids)) + 0.5).astype(np.float32)
+    up = rng.random((40, 8 * (5 if combiner == "tile" else 1))).astype(np.float32)
+    got = []
+    for hooked in (False, True):
+        HashtableRegister().clear()
+        kw = {"combiner_kwargs": {"tile_len": 5}} if combiner == "tile" else {}
+        eng = EmbeddingEngine({"a": EmbeddingOption(embedding_dim=8, block_size=64, shared_name="offloaded",
+                                                    use_weight=combiner != "tile", combiner=combiner, **kw)})
+        eng.train()
+        opt = SparseAdagrad(filter_out_sparse_param(eng), lr=0.1)
+        x = {"a": RaggedTensor(torch.from_numpy(ids).cuda(), _offsets(lens), torch.from_numpy(weight).cuda())}
+        packed = []
+
+        def pack(t):
+            packed.append((t.dtype, t.numel()))
+            return t.cpu()
+
+        if hooked:
+            with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+                out = eng(x)["a"]
+            assert (torch.int32, 41) in packed
+            assert combiner == "tile" or (torch.float32, len(ids)) in packed
+        else:
+            out = eng(x)["a"]
+        out.backward(torch.from_numpy(up).cuda())
+        opt.step()
+        (table,) = eng.hashtables().values()
+        table.eval()
+        got.append(table(torch.arange(50, device="cuda")))
+    assert got[0].any() and torch.equal(got[0], got[1])
