@@ -496,7 +496,7 @@ int recis_partition_order(const int64_t* ids, int64_t n, int64_t* sorted_ids, in
  *                          of unique ids is known and stores it there
  *   flags                  RECIS_PLAN_STAGE_COUNT: send the count towards the host but do not
  *                          wait; recis_unique_plan_count(stream) fetches the last one of the
- *                          stream, recis_unique_plan_count_of any of the last 16
+ *                          stream, recis_unique_plan_count_of that of a ticket
  * The unique ids are ordered as follows: first the few ids that make up a sizeable share of the
  * batch (found by sampling; at most 64), then the ids of the hash buckets (a bucket = the top bits
  * of a 64-bit mix of the id) that hold more than one and a half times the average, then those of
@@ -572,11 +572,13 @@ int recis_unique_plan_count(int64_t* unique_count_host, void* stream);
  * staged count every step notice, one step late at most, what recis_hip_poll_device_errors would
  * report after a device-wide wait. */
 int recis_hip_staged_device_errors(int* bits, void* stream);
-/* The same for a caller that does not wait before it queues later plans: every staged count of a
- * stream has a ticket (recis_unique_plan_ticket: the last one's), and the counts of the last 16
- * tickets stay readable. count = -1: not there yet (only with wait == 0), or the ticket is too old
- * (then counts_out_dev[0] still holds it). error_bits as of the moment the count was staged. */
+/* The same for a caller that does not wait before it queues later plans. recis_unique_plan_ticket takes a ticket for the
+ * count that the calling thread staged last on the stream; the count then stays readable, whatever is queued later and
+ * by whomever, until recis_unique_plan_release. ticket = -1: this thread staged none there since its last ticket, or 4096
+ * tickets are out. recis_unique_plan_count_of: count = -1: not there yet (only with wait == 0), or no such
+ * ticket (counts_out_dev[0] holds the count then). error_bits as of the moment the count was staged. */
 int recis_unique_plan_ticket(int64_t* ticket, void* stream);
+int recis_unique_plan_release(int64_t ticket);
 int recis_unique_plan_count_of(int64_t ticket, int wait, int64_t* count, int* error_bits, void* stream);
 
 /*

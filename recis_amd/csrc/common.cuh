@@ -239,14 +239,16 @@ struct KernelTimer {
 // calls on that stream. Never shrinks; released at process exit.
 int get_workspace(hipStream_t stream, size_t bytes, void** out);
 
-// Per-(device, stream) pinned host words and an event, for handing a device-side count to the
-// host while later kernels of the same call are still running. Every call takes the next of
-// kCountRing slots (a ticket); a slot is handed out again kCountRing calls later.
-constexpr int kCountRing = 16;
+// Pinned host words and an event, for handing a device-side count to the host while later kernels
+// of the same call are still running. They stay the calling thread's until it asks for the next ones, or
+// belong to a ticket until that is given back.
 int get_count_staging(hipStream_t stream, int64_t** host, hipEvent_t* event);
-int64_t last_count_ticket(hipStream_t stream);  // this thread's last one on the stream, else the stream's; -1: none yet
-// The slot of `ticket`; false when it was never issued or has been handed out again.
-bool find_count_staging(hipStream_t stream, int64_t ticket, int64_t** host, hipEvent_t* event);
+// Those of this thread's last count on the stream, else of the stream's; false: there is none.
+bool last_count_staging(hipStream_t stream, int64_t** host, hipEvent_t* event);
+// A ticket for the count this thread has just staged on the stream; -1: there is none, or too many are out.
+int64_t take_count_ticket(hipStream_t stream);
+bool find_count_ticket(int64_t ticket, int64_t** host, hipEvent_t* event);
+void give_count_ticket(int64_t ticket);
 // One more pinned word of the stream, for a call that waits for the stream before it reads it.
 int get_flag_word(hipStream_t stream, int64_t** host);
 

@@ -1839,7 +1839,7 @@ int recis_unique_plan_count(int64_t* unique_count_host, void* stream_) {
   RECIS_REQUIRE(unique_count_host != nullptr, "unique_count_host must not be NULL");
   int64_t* staged = nullptr;
   hipEvent_t staged_event = nullptr;
-  RECIS_REQUIRE(find_count_staging(stream, last_count_ticket(stream), &staged, &staged_event), "no count was staged");
+  RECIS_REQUIRE(last_count_staging(stream, &staged, &staged_event), "no count was staged");
   RECIS_CHECK_HIP(hipEventSynchronize(staged_event));
   *unique_count_host = staged[0];
   return RECIS_OK;
@@ -1850,24 +1850,29 @@ int recis_hip_staged_device_errors(int* bits, void* stream_) {
   RECIS_REQUIRE(bits != nullptr, "bits must not be NULL");
   int64_t* staged = nullptr;
   hipEvent_t staged_event = nullptr;
-  *bits = find_count_staging(stream, last_count_ticket(stream), &staged, &staged_event) ? static_cast<int>(staged[1]) : 0;
+  *bits = last_count_staging(stream, &staged, &staged_event) ? static_cast<int>(staged[1]) : 0;
   return RECIS_OK;
 }
 
 int recis_unique_plan_ticket(int64_t* ticket, void* stream_) {
   RECIS_REQUIRE(ticket != nullptr, "ticket must not be NULL");
-  *ticket = last_count_ticket(static_cast<hipStream_t>(stream_));
+  *ticket = take_count_ticket(static_cast<hipStream_t>(stream_));
+  return RECIS_OK;
+}
+
+int recis_unique_plan_release(int64_t ticket) {
+  give_count_ticket(ticket);
   return RECIS_OK;
 }
 
 int recis_unique_plan_count_of(int64_t ticket, int wait, int64_t* count, int* error_bits, void* stream_) {
-  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  (void)stream_;  // (a ticket is of one stream)
   RECIS_REQUIRE(count && error_bits, "NULL argument");
   *count = -1;
   *error_bits = 0;
   int64_t* staged = nullptr;
   hipEvent_t event = nullptr;
-  if (!find_count_staging(stream, ticket, &staged, &event)) return RECIS_OK;
+  if (!find_count_ticket(ticket, &staged, &event)) return RECIS_OK;
   if (wait) {
     RECIS_CHECK_HIP(hipEventSynchronize(event));
   } else {

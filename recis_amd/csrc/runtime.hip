@@ -87,68 +87,128 @@ int get_workspace(hipStream_t stream, size_t bytes, void** out) {
   return RECIS_OK;
 }
 
-// A ring of pinned words per (device, stream), so that the counts of several plans can be under way
-// at once: a caller that does not wait for a count can still fetch it after it has queued later plans.
-struct CountStaging {
-  int64_t* host = nullptr;  // pinned, kCountRing slots of 8 words and one more for get_flag_word
-  hipEvent_t event[kCountRing] = {};
-  int64_t issued = 0;       // the next ticket; ticket t uses slot t % kCountRing
-};
-static std::map<std::pair<int, hipStream_t>, CountStaging> g_staging;
-
-// the last ticket this thread took: two threads may queue plans on one stream
-struct LastTicket {
+// Pinned words and an event for the count of a plan. A slot belongs to one (device, stream), so that whoever takes it
+// next writes behind the kernels of whoever had it before. It is held by the thread that staged a count with it, until that
+// thread stages another; or by a ticket, until the ticket is given back: never handed out while a count in it may still be read.
+struct CountSlot {
+  int64_t* host = nullptr;
+  hipEvent_t event = nullptr;
   int dev = -1;
   hipStream_t stream = nullptr;
+  const void* holder = nullptr;  // the thread (its t_staged), NULL with a ticket or when free
   int64_t ticket = -1;
 };
-static thread_local LastTicket t_last;
+struct CountStaging {
+  std::vector<CountSlot*> free;
+  CountSlot* last = nullptr;     // the stream's last staged count
+  int64_t* flag_word = nullptr;  // pinned, see get_flag_word
+};
+constexpr int kSlotChunk = 32;      // slots of one pinned allocation
+constexpr size_t kMaxTickets = 4096;  // outstanding at once (a plan without one reads its own device word)
+// (never destroyed: threads and plans may outlive this library's static objects)
+static auto& g_staging = *new std::map<std::pair<int, hipStream_t>, CountStaging>;
+static auto& g_tickets = *new std::map<int64_t, CountSlot*>;
+static int64_t g_next_ticket = 1;
 
-static int staging_of(int dev, hipStream_t stream, CountStaging** out) {  // g_mu is held
-  CountStaging& c = g_staging[std::make_pair(dev, stream)];
-  if (c.host == nullptr) {
-    RECIS_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&c.host), 64 * (kCountRing + 1), hipHostMallocDefault));
-    for (int w = 0; w < 8 * (kCountRing + 1); ++w) c.host[w] = 0;
-    for (int k = 0; k < kCountRing; ++k) RECIS_CHECK_HIP(hipEventCreateWithFlags(&c.event[k], hipEventDisableTiming));
-  }
-  *out = &c;
-  return RECIS_OK;
+struct StagedHere {  // the last count this thread staged
+  CountSlot* slot = nullptr;
+  ~StagedHere();
+};
+static thread_local StagedHere t_staged;
+
+static void give_back_held() {  // g_mu is held
+  CountSlot* s = t_staged.slot;
+  t_staged.slot = nullptr;
+  if (s == nullptr || s->holder != &t_staged) return;
+  s->holder = nullptr;
+  g_staging[std::make_pair(s->dev, s->stream)].free.push_back(s);
+}
+StagedHere::~StagedHere() {
+  std::lock_guard<std::mutex> l(g_mu);
+  give_back_held();
 }
 
 int get_count_staging(hipStream_t stream, int64_t** host, hipEvent_t* event) {
   const int dev = current_device();
   std::lock_guard<std::mutex> l(g_mu);
-  CountStaging* c = nullptr;
-  if (int rc = staging_of(dev, stream, &c)) return rc;
-  t_last = LastTicket{dev, stream, c->issued++};
-  *host = c->host + 8 * (t_last.ticket % kCountRing);
-  *event = c->event[t_last.ticket % kCountRing];
+  give_back_held();
+  CountStaging& c = g_staging[std::make_pair(dev, stream)];
+  if (c.free.empty()) {
+    int64_t* words = nullptr;
+    RECIS_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&words), 64 * kSlotChunk, hipHostMallocDefault));
+    for (int w = 0; w < 8 * kSlotChunk; ++w) words[w] = 0;
+    for (int k = kSlotChunk - 1; k >= 0; --k) {
+      CountSlot* s = new CountSlot;
+      s->host = words + 8 * k;
+      s->dev = dev;
+      s->stream = stream;
+      c.free.push_back(s);
+    }
+  }
+  CountSlot* s = c.free.back();
+  if (s->event == nullptr) RECIS_CHECK_HIP(hipEventCreateWithFlags(&s->event, hipEventDisableTiming));
+  c.free.pop_back();
+  s->holder = &t_staged;
+  t_staged.slot = s;
+  c.last = s;
+  *host = s->host;
+  *event = s->event;
   return RECIS_OK;
 }
 
 int get_flag_word(hipStream_t stream, int64_t** host) {
+  const int dev = current_device();
   std::lock_guard<std::mutex> l(g_mu);
-  CountStaging* c = nullptr;
-  if (int rc = staging_of(current_device(), stream, &c)) return rc;
-  *host = c->host + 8 * kCountRing;
+  CountStaging& c = g_staging[std::make_pair(dev, stream)];
+  if (c.flag_word == nullptr)
+    RECIS_CHECK_HIP(hipHostMalloc(reinterpret_cast<void**>(&c.flag_word), 64, hipHostMallocDefault));
+  *host = c.flag_word;
   return RECIS_OK;
 }
 
-int64_t last_count_ticket(hipStream_t stream) {
+bool last_count_staging(hipStream_t stream, int64_t** host, hipEvent_t* event) {
   const int dev = current_device();
-  if (t_last.dev == dev && t_last.stream == stream) return t_last.ticket;
   std::lock_guard<std::mutex> l(g_mu);
-  return g_staging[std::make_pair(dev, stream)].issued - 1;
+  CountSlot* s = t_staged.slot;
+  if (s == nullptr || s->dev != dev || s->stream != stream) s = g_staging[std::make_pair(dev, stream)].last;
+  if (s == nullptr) return false;
+  *host = s->host;
+  *event = s->event;
+  return true;
 }
 
-bool find_count_staging(hipStream_t stream, int64_t ticket, int64_t** host, hipEvent_t* event) {
-  int dev = current_device();
+int64_t take_count_ticket(hipStream_t stream) {
+  const int dev = current_device();
   std::lock_guard<std::mutex> l(g_mu);
-  CountStaging& c = g_staging[std::make_pair(dev, stream)];
-  if (ticket < 0 || ticket >= c.issued || c.issued - ticket > kCountRing) return false;
-  *host = c.host + 8 * (ticket % kCountRing);
-  *event = c.event[ticket % kCountRing];
+  CountSlot* s = t_staged.slot;
+  if (s == nullptr || s->dev != dev || s->stream != stream) return -1;
+  if (s->holder == &t_staged && g_tickets.size() < kMaxTickets) {
+    s->holder = nullptr;
+    s->ticket = g_next_ticket++;
+    g_tickets[s->ticket] = s;
+    t_staged.slot = nullptr;
+    return s->ticket;
+  }
+  return -1;
+}
+
+bool find_count_ticket(int64_t ticket, int64_t** host, hipEvent_t* event) {
+  std::lock_guard<std::mutex> l(g_mu);
+  auto it = g_tickets.find(ticket);
+  if (it == g_tickets.end()) return false;
+  *host = it->second->host;
+  *event = it->second->event;
   return true;
+}
+
+void give_count_ticket(int64_t ticket) {
+  std::lock_guard<std::mutex> l(g_mu);
+  auto it = g_tickets.find(ticket);
+  if (it == g_tickets.end()) return;
+  CountSlot* s = it->second;
+  g_tickets.erase(it);
+  s->ticket = -1;
+  g_staging[std::make_pair(s->dev, s->stream)].free.push_back(s);
 }
 
 bool g_profile_on = false;

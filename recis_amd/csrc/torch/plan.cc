@@ -36,13 +36,13 @@ at::Tensor flat_ids(const at::Tensor& t) {
   return t.to(at::kLong).contiguous().view({-1});
 }
 
-// The bits that travelled to the host with a staged count, as an exception.
+// The bits that travelled to the host with a staged count (-1: not known) as an exception.
 void raise_device_errors(int bits) {
   if (bits == 0) return;
   int polled = 0;
   check(recis_hip_poll_device_errors(&polled));  // waits for the device and clears the word
   // (two counts that were under way together carry one error's bits twice: it is raised once)
-  TORCH_CHECK(polled == 0, "librecis_hip: device-side errors in earlier kernels: ", describe_device_errors(bits | polled));
+  TORCH_CHECK(polled == 0, "librecis_hip: device-side errors in earlier kernels: ", describe_device_errors(polled));
 }
 
 }  // namespace
@@ -106,10 +106,19 @@ int64_t BatchPlan::U() {
   int64_t count = -1;
   int bits = 0;
   check(recis_unique_plan_count_of(ticket_, 1, &count, &bits, stream_));
-  if (count < 0) count = counts_[0].item<int64_t>();  // many later plans of the stream have taken over the staging words
+  if (count < 0) {  // no ticket was left for this plan: its own device words
+    count = counts_[0].item<int64_t>();
+    bits = -1;
+  }
   U_ = count;
+  GiveTicket();
   raise_device_errors(bits);
   return U_;
+}
+
+void BatchPlan::GiveTicket() {
+  if (ticket_ >= 0) recis_unique_plan_release(ticket_);
+  ticket_ = -1;
 }
 
 at::Tensor BatchPlan::unique() {

@@ -19,6 +19,7 @@ namespace recis {
 
 class BatchPlan : public torch::CustomClassHolder {
  public:
+  ~BatchPlan() override { GiveTicket(); }
   // ids: the batch as one or more id tensors laid end to end; tags (one per tensor) tag every id
   // with its table as ids_encode does. map != nullptr: the unique ids are found or inserted in that
   // id map in the same pass and index_buf holds their rows. wait == false returns without the host
@@ -79,6 +80,8 @@ class BatchPlan : public torch::CustomClassHolder {
                                                            bool mean, bool want_pool,
                                                            const std::vector<int64_t>* batch,
                                                            const std::vector<int64_t>* seq);
+  void GiveTicket();
+  // ticket_: of the staged count, this plan's own until the count has been read
   int64_t n_ = 0, serial_ = 0, hot_cap_ = 0, U_ = -1, ticket_ = -1;
   void* stream_ = nullptr;
   at::Tensor unique_buf_, inverse_, row_start_, occ_, pos_, hot_items_, counts_, index_buf_, unique_;

@@ -1,5 +1,8 @@
 """The training lookups whose forward does not wait for the device (HashtableImpl.lookup_train / dense_lookup_train): counts of
 several plans under way at once, errors that come with them, both backward passes over one node."""
+import ctypes
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -259,3 +262,86 @@ def test_saved_tensor_hooks_see_the_inputs(rng, combiner):
         table.eval()
         got.append(table(torch.arange(50, device="cuda")))
     assert got[0].any() and torch.equal(got[0], got[1])
+
+
+def test_errors_of_many_tables_in_one_step(rng):
+    """Counts and error bits of more plans than a step of few tables has: each plan's own are there in its backward."""
+    HashtableRegister().clear()
+    tables = [HashTable([8], block_size=64, name="many%d" % k) for k in range(24)]
+    ids = torch.arange(50, device="cuda")
+    bad = ids.clone()
+    bad[3] = -1
+
+    def step(faulty):
+        sum((t(bad if k == faulty else ids)).sum() for k, t in enumerate(tables)).backward()
+        for t in tables:
+            t.clear_grad()
+
+    step(None)
+    with pytest.raises(RuntimeError, match="index outside"):
+        step(2)
+    step(None)
+    assert _lib.poll_device_errors() == 0
+
+
+def test_a_count_stays_until_it_is_released(rng):
+    lib = _lib.lib()
+    stream = _lib.stream_ptr()
+
+    def queue(n_distinct, n=3000):
+        ids = torch.from_numpy(np.concatenate([np.arange(n_distinct), rng.integers(0, n_distinct, n - n_distinct)])).cuda()
+        n = ids.numel()
+        cap = n
+        out = [torch.empty(n, dtype=torch.int64, device="cuda"), torch.empty(n + 1, dtype=torch.int32, device="cuda"),
+               torch.empty(n, dtype=torch.int32, device="cuda"), torch.empty(2 * cap, dtype=torch.int32, device="cuda"),
+               torch.empty(2, dtype=torch.int64, device="cuda")]
+        p = _lib.ptr
+        _lib.check(lib.recis_unique_plan(p(ids), _lib.i64(n), p(out[0]), p(None), p(out[1]), p(out[2]), p(None), p(out[3]),
+                                         _lib.i64(cap), p(out[4]), p(None), 1, stream))
+        keep.append((ids, out))
+
+    def ticket():
+        t = ctypes.c_int64(-1)
+        _lib.check(lib.recis_unique_plan_ticket(ctypes.byref(t), stream))
+        return t.value
+
+    def count_of(t, wait=1):
+        c, bits = ctypes.c_int64(0), ctypes.c_int(0)
+        _lib.check(lib.recis_unique_plan_count_of(_lib.i64(t), wait, ctypes.byref(c), ctypes.byref(bits), stream))
+        return c.value
+
+    keep = []
+    queue(77)
+    first = ticket()
+    for k in range(60):  # later plans, with a ticket and without one
+        queue(100 + k)
+        if k % 2:
+            t = ticket()
+            assert ticket() == -1  # one ticket a count
+            assert count_of(t) == 100 + k
+            _lib.check(lib.recis_unique_plan_release(_lib.i64(t)))
+            assert count_of(t) == -1
+    assert count_of(first) == 77
+    _lib.check(lib.recis_unique_plan_release(_lib.i64(first)))
+    queue(500)
+    last = ctypes.c_int64(0)
+    _lib.check(lib.recis_unique_plan_count(ctypes.byref(last), stream))
+    assert last.value == 500
+    # another thread's counts on the stream are its own
+    got = []
+
+    def other():
+        for k in range(40):
+            queue(200 + k)
+        t = ticket()
+        got.append(count_of(t))
+        _lib.check(lib.recis_unique_plan_release(_lib.i64(t)))
+
+    queue(600)
+    mine = ticket()
+    thread = threading.Thread(target=other)
+    thread.start()
+    thread.join()
+    assert got == [239] and count_of(mine) == 600
+    _lib.check(lib.recis_unique_plan_release(_lib.i64(mine)))
+    assert _lib.poll_device_errors() == 0
