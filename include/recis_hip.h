@@ -86,6 +86,10 @@ int recis_hip_probe_random_rows(void* table, int64_t rows, int64_t row_bytes, co
 /* Synchronises the current device, returns the soft-error bits raised by
  * kernels since the last poll in *bits and clears them. */
 int recis_hip_poll_device_errors(int* bits);
+/* Whether a kernel that looks (the last one of a batch plan with a staged count, recis_lookup_pool_readonly's) has found
+ * bits in the current device's error word since the last poll; read from host memory, no wait. For callers
+ * that nothing else ever brings the bits: poll when it is not 0. */
+int recis_hip_device_errors_reported(int* reported);
 
 /* ------------------------------------------------------------------------- *
  * Pooling: ragged gather + segment reduce

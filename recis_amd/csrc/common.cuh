@@ -48,6 +48,7 @@ int fail(int code, const char* fmt, ...);
 // outside the range the host promised skip the access and set a bit here
 // instead of faulting the GPU. Read with recis_hip_poll_device_errors().
 int* device_error_word(int device);
+int* error_report_word(int device);  // pinned, see report_device_errors
 int current_device();
 
 // --------------------------------------------------------------- storage types
@@ -156,6 +157,12 @@ __device__ __forceinline__ void store_index(void* p, int is64, int64_t i, int64_
 
 __device__ __forceinline__ void raise_device_error(int* err_word, int bit) {
   atomicOr(err_word, bit);
+}
+
+// Tells the host that the error word holds bits (recis_hip_device_errors_reported): a store to pinned memory, on the way of
+// an error only.
+__device__ __forceinline__ void report_device_errors(int* report_word) {
+  __hip_atomic_store(report_word, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // ---------------------------------------------------------------- row geometry

@@ -52,7 +52,13 @@ struct PoolArgs {
   int64_t id_mask;                      // of the id's own bits; ~0 = ids are taken as they are
   int D, lpr_log2, mode;                // RECIS_SUM, RECIS_MEAN or RECIS_LOOKUP_WEIGHT_MEAN
   int* err;
+  int* report;  // pinned: this call has no count for the error bits to travel with
 };
+
+__device__ __forceinline__ void raise_and_report(const PoolArgs& a, int bit) {
+  raise_device_error(a.err, bit);
+  report_device_errors(a.report);
+}
 
 // A row of zeros (D <= 8192 of at most 4 bytes): what an id without a row reads, so that the loads of
 // a round need no branch around each.
@@ -83,7 +89,7 @@ __device__ __forceinline__ uint64_t address_of_row(const PoolArgs& a, int64_t ro
     r = row - b * a.block_rows;
   }
   if (b >= a.n_blocks || r >= a.block_rows) {
-    raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
+    raise_and_report(a, RECIS_DEVERR_INDEX_RANGE);
     return 0;
   }
   return reinterpret_cast<uint64_t>(static_cast<const T*>(a.blocks[b]) + r * a.pitch);
@@ -138,7 +144,11 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
   const int n_here = min(teams << spt_log2, n_seg - seg0);
   const void* offs = job.offs;
 
-  if (tid == 0) s_bad = 0;
+  if (tid == 0) {
+    s_bad = 0;
+    // what earlier kernels of the device found
+    if (tile == 0 && __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) report_device_errors(a.report);
+  }
   if (offs == nullptr) {
     for (int i = tid; i <= n_here; i += kBlock) s_off[i] = (seg0 + i) * width;
     __syncthreads();
@@ -154,7 +164,7 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
     if (bad) s_bad = 1;
     __syncthreads();
     if (s_bad) {  // uniform; the tile's rows come out as zeros
-      if (tid == 0) raise_device_error(a.err, RECIS_DEVERR_OFFSETS);
+      if (tid == 0) raise_and_report(a, RECIS_DEVERR_OFFSETS);
       for (int i = tid; i <= n_here; i += kBlock) s_off[i] = 0;
       __syncthreads();
     }
@@ -349,8 +359,10 @@ extern "C" int recis_lookup_pool_readonly(recis_idmap* map, const recis_lookup_j
   a.id_mask = tagged ? (int64_t(1) << 52) - 1 : ~int64_t(0);
   a.D = static_cast<int>(D);
   a.mode = mode;
-  a.err = device_error_word(current_device());
-  RECIS_REQUIRE(a.err != nullptr, "could not reach the device error word");
+  const int dev = current_device();
+  a.err = device_error_word(dev);
+  a.report = error_report_word(dev);
+  RECIS_REQUIRE(a.err != nullptr && a.report != nullptr, "could not reach the device error word");
   // blocks are 16-byte aligned by contract
   const int vec_bytes = pick_vec_bytes(D * size, reinterpret_cast<uintptr_t>(out));
   a.pitch = D;

@@ -793,6 +793,7 @@ struct BucketArgs {
   int64_t hot_cap;
   volatile int64_t* staged;  // pinned host words (unique count, soft-error bits) or NULL
   int* err;
+  int* report;  // with staged
   uint32_t spin_limit;
   // fused find-or-insert in the id map
   Slot* table;
@@ -896,7 +897,9 @@ __device__ __forceinline__ void finish_ticket(const BucketArgs& a) {
   // workgroup scope waits for exactly that (one of device scope would write back the whole L2)
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   if (atomicAdd(&a.sync[1], 1) == (1 << a.g.nb_log2)) {  // the buckets and the heavy ids' workgroup
-    a.staged[1] = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int bits = __hip_atomic_load(a.err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (bits != 0) report_device_errors(a.report);  // (a count may never be asked for)
+    a.staged[1] = bits;
     a.staged[0] = __hip_atomic_load(&a.counts[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
@@ -1442,12 +1445,14 @@ plan_inverse_from_lists_kernel(const int32_t* __restrict__ row_start, const int3
 }
 
 __global__ void plan_empty_kernel(int64_t* __restrict__ counts, int32_t* __restrict__ row_start,
-                                  volatile int64_t* total_host, const int* __restrict__ err) {
+                                  volatile int64_t* total_host, const int* __restrict__ err, int* report) {
   if (threadIdx.x < 2) counts[threadIdx.x] = 0;
   if (threadIdx.x == 0) {
     row_start[0] = 0;
     if (total_host) {
-      total_host[1] = err ? __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+      const int bits = __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (bits != 0) report_device_errors(report);
+      total_host[1] = bits;
       total_host[0] = 0;
     }
   }
@@ -1639,6 +1644,8 @@ static int plan_launch(const PlanLayout& L, char* base, const int64_t* ids, cons
   a.hot_items = hot_items_out;
   a.hot_cap = hot_cap;
   a.staged = staged;
+  a.report = staged ? error_report_word(current_device()) : nullptr;
+  RECIS_REQUIRE(!staged || a.report, "could not reach the error report word");
   a.err = err;
   a.spin_limit = g_spin_limit.load(std::memory_order_relaxed);
   a.table = nullptr;
@@ -1690,7 +1697,9 @@ static int plan_entry(recis_idmap* map, const int64_t* ids, int64_t n, int64_t* 
     if (int rc = get_count_staging(stream, &staged, &staged_event)) return rc;
   }
   if (n == 0) {
-    plan_empty_kernel<<<1, 64, 0, stream>>>(counts_out_dev, row_start_out, staged, err);
+    int* report = stage ? error_report_word(current_device()) : nullptr;
+    RECIS_REQUIRE(!stage || report, "could not reach the error report word");
+    plan_empty_kernel<<<1, 64, 0, stream>>>(counts_out_dev, row_start_out, staged, err, report);
     RECIS_LAUNCH_CHECK();
     if (stage) RECIS_CHECK_HIP(hipEventRecord(staged_event, stream));
     if (unique_count_host) *unique_count_host = 0;
@@ -1815,7 +1824,7 @@ int recis_unique_plan_noalloc(const int64_t* ids, int64_t n, int64_t* unique_out
   int* err = device_error_word(dev);
   RECIS_REQUIRE(err != nullptr, "could not reach the device error word");
   if (n == 0) {
-    plan_empty_kernel<<<1, 64, 0, stream>>>(counts_out_dev, row_start_out, nullptr, err);
+    plan_empty_kernel<<<1, 64, 0, stream>>>(counts_out_dev, row_start_out, nullptr, err, nullptr);
     RECIS_LAUNCH_CHECK();
     return RECIS_OK;
   }

@@ -3,6 +3,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <atomic>
 #include <map>
 #include <mutex>
 #include <string>
@@ -57,6 +58,22 @@ int* device_error_word(int device) {
   if (rc != hipSuccess) return nullptr;
   g_err_words[device] = static_cast<int*>(p);
   return g_err_words[device];
+}
+
+// A pinned word per device: not zero once a kernel that looks has found bits in the error word. The host reads it
+// without waiting, for calls that have no count to come with the bits.
+static std::atomic<int*> g_report_words[kMaxDevices];
+
+int* error_report_word(int device) {
+  if (device < 0 || device >= kMaxDevices) return nullptr;
+  if (int* known = g_report_words[device].load(std::memory_order_acquire)) return known;
+  std::lock_guard<std::mutex> l(g_mu);
+  if (int* known = g_report_words[device].load(std::memory_order_relaxed)) return known;
+  void* p = nullptr;
+  if (hipHostMalloc(&p, 64, hipHostMallocPortable) != hipSuccess) return nullptr;
+  *static_cast<volatile int*>(p) = 0;
+  g_report_words[device].store(static_cast<int*>(p), std::memory_order_release);
+  return static_cast<int*>(p);
 }
 
 struct Workspace {
@@ -286,8 +303,18 @@ int recis_hip_poll_device_errors(int* bits) {
   int* w = device_error_word(dev);
   RECIS_REQUIRE(w != nullptr, "could not reach the device error word");
   RECIS_CHECK_HIP(hipDeviceSynchronize());
+  if (int* reported = error_report_word(dev)) *static_cast<volatile int*>(reported) = 0;
   RECIS_CHECK_HIP(hipMemcpy(bits, w, sizeof(int), hipMemcpyDeviceToHost));
   if (*bits) RECIS_CHECK_HIP(hipMemset(w, 0, sizeof(int)));
+  return RECIS_OK;
+}
+
+int recis_hip_device_errors_reported(int* reported) {
+  using namespace recis_hip;
+  RECIS_REQUIRE(reported != nullptr, "reported must not be NULL");
+  const int* w = error_report_word(current_device());
+  RECIS_REQUIRE(w != nullptr, "could not reach the error report word");
+  *reported = *static_cast<const volatile int*>(w);
   return RECIS_OK;
 }
 

@@ -47,6 +47,12 @@ void raise_device_errors(int bits) {
 
 }  // namespace
 
+void raise_reported_errors() {
+  int reported = 0;
+  check(recis_hip_device_errors_reported(&reported));
+  if (reported) raise_device_errors(-1);
+}
+
 BatchPlanPtr BatchPlan::Make(const std::vector<at::Tensor>& ids_in, const c10::optional<std::vector<int64_t>>& tags,
                              recis_idmap* map, bool wait, bool need_inverse, bool need_pos) {
   TORCH_CHECK(!tags.has_value() || tags->size() == ids_in.size(), "unique_plan: ", tags.has_value() ? tags->size() : 0,

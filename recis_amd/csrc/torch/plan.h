@@ -104,4 +104,8 @@ using BatchPlanPtr = c10::intrusive_ptr<BatchPlan>;
 BatchPlanPtr unique_plan(std::vector<at::Tensor> ids, c10::optional<std::vector<int64_t>> tags, int64_t idmap_handle,
                          bool wait, bool need_inverse, bool need_pos);
 
+// Raises what earlier kernels of the current device are known to have found (no wait unless there is something):
+// for lookups whose count nobody may ever read.
+void raise_reported_errors();
+
 }  // namespace recis

@@ -738,6 +738,7 @@ std::tuple<at::Tensor, at::Tensor> Hashtable::EvictOlder(const std::string& stam
 BatchPlanPtr Hashtable::PlanLookup(const std::vector<at::Tensor>& ids, const c10::optional<std::vector<int64_t>>& tags,
                                    bool wait, bool need_inverse, bool need_pos) {
   c10::DeviceGuard guard(device_);
+  recis::raise_reported_errors();
   BatchPlanPtr plan = recis::BatchPlan::Make(ids, tags, map_->map, wait, need_inverse, need_pos);
   int64_t call = 0;
   check(recis_idmap_last_call(map_->map, &call));
@@ -847,6 +848,7 @@ std::vector<at::Tensor> Hashtable::LookupPoolReadonly(const std::vector<at::Tens
   TORCH_CHECK(n > 0 && offsets.size() == n && weights.size() == n && (!tags.has_value() || tags->size() == n),
               "lookup_pool_readonly: one entry per feature in every list");
   c10::DeviceGuard guard(device_);
+  recis::raise_reported_errors();
   MakeRoom(0);
   auto emb = slot_group_->EmbSlot();
   const auto& chunks = emb->Chunks();

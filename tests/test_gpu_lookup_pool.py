@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from recis_amd import _lib
+from recis_amd import _lib, ops
 from recis_amd.nn import EmbeddingEngine, EmbeddingOption, HashTable
 from recis_amd.nn.modules.hashtable import HashtableRegister
 from recis_amd.ragged import RaggedTensor
@@ -119,3 +119,52 @@ def test_lookup_pool_flags_bad_offsets(rng):
     out = ht._hashtable_impl.lookup_pool_readonly([ids], [torch.tensor([0, 4, 3, 99], device="cuda")], [None], None, False)
     assert out[0].shape == (3, 8) and not out[0].any()
     assert _lib.poll_device_errors() & _lib.DEVERR_OFFSETS
+
+
+def _offsets(lens):
+    return torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)).cuda()
+
+
+@pytest.mark.parametrize("where", ["this", "earlier", "engine"])
+def test_evaluation_raises_what_kernels_reported(where):
+    """Evaluation reads no count that error bits could come with: a later call raises them, without a poll by hand."""
+    HashtableRegister().clear()
+    eng = EmbeddingEngine({"a": EmbeddingOption(embedding_dim=8, block_size=64, shared_name="served", combiner="sum")})
+    eng.eval()
+    (table,) = eng.hashtables().values()
+    table.eval()
+    ids = torch.arange(10, device="cuda")
+    good = RaggedTensor(ids, _offsets([5, 5]))
+    eng({"a": good})
+    if where == "this":
+        eng({"a": RaggedTensor(ids, torch.tensor([0, 4, 3, 10], device="cuda", dtype=torch.int32))})
+    elif where == "earlier":  # another kernel of the device
+        ops.segment_reduce_forward(torch.ones(10, 8, device="cuda"), None, None,
+                                   torch.tensor([0, 4, 3, 10], device="cuda", dtype=torch.int32), "sum")
+        eng({"a": good})
+    else:
+        for _ in range(3):
+            table(ids)
+        eng({"a": RaggedTensor(ids, torch.tensor([0, 4, 30, 10], device="cuda", dtype=torch.int32))})
+    torch.cuda.synchronize()
+    with pytest.raises(RuntimeError, match="offsets not monotone"):
+        table(ids) if where == "engine" else eng({"a": good})
+    eng({"a": good})
+    torch.cuda.synchronize()
+    eng({"a": good})
+    assert _lib.poll_device_errors() == 0
+
+
+def test_training_raises_what_evaluation_reported():
+    HashtableRegister().clear()
+    ht = HashTable([8], block_size=64, name="served")
+    ids = torch.arange(10, device="cuda")
+    ht(ids)
+    ht.eval()
+    ops.segment_reduce_forward(torch.ones(10, 8, device="cuda"), None, None,
+                               torch.tensor([0, 4, 3, 10], device="cuda", dtype=torch.int32), "sum")
+    ht(ids)
+    ht.train()
+    with pytest.raises(RuntimeError, match="offsets not monotone"):
+        ht(ids).sum().backward()
+    assert _lib.poll_device_errors() == 0
