@@ -397,17 +397,22 @@ seg_pool_fwd_fast_kernel(const TIn* __restrict__ emb, TOut* __restrict__ out, Se
 
 // src / coef per list entry out of what the forward noted per occurrence: one scattered 8-byte read each
 // (0.49 M entries 7.6 us, 0.5 TB/s: bound by the number of those reads; the search of the offsets took 23).
+// A segment with bad offsets has noted nothing, so a note counts only when the segment it names is one the pooling
+// walked and holds the occurrence: then that segment's team, or another that walked the occurrence, has written it.
 __global__ void __launch_bounds__(kBlock)
 lists_from_occ_kernel(const int32_t* __restrict__ list, int64_t n, const int2* __restrict__ occ, const void* offsets,
                       int off64, int64_t S, int32_t* __restrict__ src, float* __restrict__ coef) {
   const int64_t k = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
   if (k >= n) return;
   const int64_t i = list[k];
-  const int64_t first = load_index(offsets, off64, 0), last = load_index(offsets, off64, S);
   if (static_cast<uint64_t>(i) >= static_cast<uint64_t>(n)) return;
   const int2 o = occ[i];
-  const bool covered = i >= first && i < last;  // an occurrence in no segment: not noted, adds nothing
-  src[k] = covered ? o.x : -1;
+  bool covered = static_cast<uint64_t>(static_cast<int64_t>(o.x)) < static_cast<uint64_t>(S);
+  if (covered) {
+    const int64_t start = load_index(offsets, off64, o.x), end = load_index(offsets, off64, o.x + 1);
+    covered = start >= 0 && end <= n && start <= i && i < end;
+  }
+  src[k] = covered ? o.x : -1;  // -1: an occurrence in no segment adds nothing
   if (coef) coef[k] = covered ? __int_as_float(o.y) : 0.f;
 }
 

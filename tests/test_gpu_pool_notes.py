@@ -73,3 +73,41 @@ def test_pool_rows_with_notes(rng, dtype, weighted, mean, segments, mean_len, di
     if lists[0][1] is not None:
         assert torch.equal(lists[0][1], lists[1][1])
     assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("off64", [0, 1])
+@pytest.mark.parametrize("weighted,mean", [(False, False), (True, True)])
+@pytest.mark.parametrize("offsets", [[0, 4, 99, 8], [0, 4, 8, -3, 8], [-2, 3, 8], [0, 3, 3, 8], [2, 5, 7]])
+def test_occurrences_of_bad_segments_have_no_notes(rng, offsets, weighted, mean, off64):
+    """Segments with bad offsets note nothing: their occurrences, which added nothing to any output, take no
+    gradient, whatever the buffer of the notes held before."""
+    n, dim, rows, S = 8, 4, 5, len(offsets) - 1
+    dev = "cuda"
+    off = torch.tensor(offsets, dtype=torch.int64 if off64 else torch.int32, device=dev)
+    emb = torch.randn(rows, dim, device=dev)
+    row_index = torch.arange(rows, device=dev)
+    rev = torch.from_numpy(rng.integers(0, rows, n).astype(np.int32)).to(dev)
+    weight = torch.rand(n, device=dev) + 0.5 if weighted else None
+    blocks = torch.tensor([emb.data_ptr()], dtype=torch.int64, device=dev)
+    out = torch.empty(S, dim, device=dev)
+    order = torch.from_numpy(rng.permutation(n).astype(np.int32)).to(dev)
+    want_src, want_coef = np.full(n, -1), np.zeros(n)
+    for s, (a, b) in enumerate(zip(offsets[:-1], offsets[1:])):
+        if 0 <= a <= b <= n:
+            want_src[a:b] = s
+            want_coef[a:b] = (weight[a:b].cpu().numpy() if weighted else 1.0) / np.float32((b - a) if mean else 1)
+    for junk in (0, 1, S - 1, S, -1, 1 << 30):
+        occ = torch.empty(n, 2, dtype=torch.int32, device=dev)
+        occ[:, 0] = junk
+        occ[:, 1] = torch.tensor([7.5], device=dev).view(torch.int32)
+        assert _lib.lib().recis_segment_reduce_forward_blocks_occ(
+            _p(blocks), _i(1), _i(rows), _i(0), _p(row_index), 0, _p(weight), 0, _p(rev), 0, _p(off), off64, _p(out), 0, _i(n),
+            _i(rows), _i(S), _i(dim), _lib.MODES["mean" if mean else "sum"], _p(occ), _lib.stream_ptr()) == 0
+        src = torch.full((n,), 123, dtype=torch.int32, device=dev)
+        coef = torch.full((n,), 123.0, device=dev)
+        assert _lib.lib().recis_csr_lists_from_occ(_p(order), _i(n), _p(occ), _p(off), off64, _i(S), _p(src), _p(coef),
+                                                   _lib.stream_ptr()) == 0
+        at = order.cpu().numpy()
+        assert (src.cpu().numpy() == want_src[at]).all(), junk
+        np.testing.assert_allclose(coef.cpu().numpy(), want_coef[at], rtol=2.0 ** -23)  # one division in float32
+    _lib.poll_device_errors()
