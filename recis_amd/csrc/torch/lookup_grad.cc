@@ -88,13 +88,20 @@ struct LookupBackward : public torch::autograd::Node {
 };
 
 // Whether the pooling notes segment and coefficient of every occurrence for the backward (recis_csr_lists_from_occ), or
-// the backward searches the offsets (recis_csr_fill_lists). The notes cost one scattered 8-byte read an entry, the search
-// one per step that its table of 2048 offsets does not save. Measured, us (search, notes): 43 thousand ids in 4096
-// segments 9.9, 3.0; 0.49 M in 65536 23.2, 7.6; 1.56 M in 8192 15.8 - 20.7, 21.2 (the notes outgrow an XCD's L2 and the
-// search has two steps left). One id per segment, unweighted: the lists are the answer themselves.
+// the backward searches the offsets (recis_csr_fill_lists). The notes cost a write and one scattered 8-byte read an entry,
+// whatever the segments; up to half a million entries (4 MB of notes, an XCD's L2) that is always the cheaper. Beyond it the
+// reads miss the L2, and what the search costs depends on the offsets beyond its table of 2048 in LDS: few when segments are
+// long. Measured, us (search - notes with their writing; power-law ids), per ids of a segment on average:
+//   unweighted          8     30    100    400        weighted     8     30    100    400
+//   0.26 M            7.6    6.4    4.6    3.3                   8.4    7.1    5.4    4.0
+//   0.52 M            8.8    4.8    4.0    2.1                   9.9    6.2    4.7    3.1
+//   0.79 M            8.5    1.3   -1.7   -2.8                  11.6    4.5    1.4   -0.8
+//   1.05 M           11.2    2.6   -4.3   -5.4                  15.6    8.1    1.9   -0.9
+//   2.10 M           23.8    8.9  -13.2  -19.8                  36.3   21.4    2.7   -7.6
+// One id per segment, unweighted: the lists are the answer themselves.
 bool NotesOccurrences(int64_t n, int64_t segments, bool weighted) {
   if (n == 0 || segments == 0 || (segments == n && !weighted)) return false;
-  return n <= (int64_t(1) << 19) || segments > 8192;
+  return n <= (int64_t(1) << 19) || n <= (weighted ? 128 : 32) * segments;
 }
 
 // The outputs of a lookup, with the node behind them (none when gradients are not recorded).
