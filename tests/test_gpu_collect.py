@@ -70,3 +70,13 @@ def test_step_with_column_slices_matches_dense_gradients(rng, optim, dim):
         rows.append(torch.cat([out[n] for n in names], dim=1))
     torch.testing.assert_close(rows[0], rows[1], rtol=1e-4, atol=1e-5)
     assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("dtype,dim", [(torch.float32, 4), (torch.float32, 16), (torch.bfloat16, 10), (torch.float32, 300)])
+@pytest.mark.parametrize("n_parts,count", [(1, 8191), (2, 33333), (3, 65536), (17, 9001)])
+def test_collect_rows_of_few_large_parts(dtype, dim, n_parts, count):
+    """Few parts: a workgroup takes more rows of each, up to what its lane groups have in flight."""
+    wide = torch.randn(count, n_parts * dim, device="cuda").to(dtype)
+    parts = list(wide.split(dim, 1))
+    rc, out = _collect(parts, [count] * n_parts, dim, dtype)
+    assert rc == 0 and torch.equal(out, torch.cat(parts))
