@@ -43,6 +43,7 @@ struct LookupBackward : public torch::autograd::Node {
   BatchPlanPtr plan;
   SavedVariable saved_index;
   std::vector<int64_t> split;        // rows per output
+  std::vector<int64_t> first_shape;  // of the first output
   // Pooled segments; both undefined: one id per segment. They may be the caller's own tensors: saved as any node saves its
   // inputs, so that a buffer refilled before the backward is refused and saved-tensor hooks see them.
   SavedVariable saved_offsets, saved_weight;
@@ -56,6 +57,10 @@ struct LookupBackward : public torch::autograd::Node {
     TORCH_CHECK(plan.defined(), torch::autograd::ERR_BACKWARD_TWICE);
     at::NoGradGuard no_grad;
     const at::Tensor index = saved_index.unpack(), offsets = saved_offsets.unpack(), weight = saved_weight.unpack();
+    // Functions behind the outputs that returned no gradient: zeros, which still are one (the rows take a step of
+    // their momentum). An output that is undefined beside others that are not counts as zeros anyway.
+    if (!grads.empty() && std::none_of(grads.begin(), grads.end(), [](const at::Tensor& g) { return g.defined(); }))
+      grads[0] = at::zeros(first_shape, at::TensorOptions().device(index.device()).dtype(table->dtype()));
     if (tile) {
       table->AcceptTileGrad(index, plan, offsets, batch, seq, grads);
       return {};
@@ -142,6 +147,7 @@ c10::optional<std::vector<at::Tensor>> Hashtable::DenseLookupTrain(const std::ve
     node->plan = std::get<0>(*found);
     node->saved_index = SavedVariable(std::get<1>(*found), false);
     node->split = split;
+    node->first_shape = shapes[0];
   }
   return outputs_of(out, shapes, split, node);
 }
@@ -286,6 +292,7 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
     node->mean = mean;
     node->tile = tile;
     node->split = split;
+    node->first_shape = shapes[0];
     if (tile) {
       node->batch = segments;
       node->seq = tile_len;

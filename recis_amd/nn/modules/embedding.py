@@ -144,7 +144,7 @@ class LookupPoolFunction(torch.autograd.Function):
             chunks, chunk_rows = impl.emb_blocks()
             out = ops.segment_reduce_forward_blocks(chunks, chunk_rows, index, weight, plan.inverse, offsets, combiner)
         ctx.impl, ctx.plan, ctx.combiner = impl, plan, combiner
-        ctx.split, ctx.out_shape = split, tuple(out.shape)
+        ctx.split, ctx.out_shape, ctx.out_dtype = split, tuple(out.shape), out.dtype
         ctx.save_for_backward(index, weight, offsets)
         ctx.set_materialize_grads(False)
         ctx.mark_non_differentiable(index)
@@ -153,8 +153,9 @@ class LookupPoolFunction(torch.autograd.Function):
     @staticmethod
     def backward(ctx, _grad_index, *grads):
         index, weight, offsets = ctx.saved_tensors
-        if all(g is None for g in grads):
-            return (None,) * 8
+        if all(g is None for g in grads):  # a function behind the outputs returned none: zeros, which still are a gradient
+            grads = (torch.zeros(ctx.out_shape if ctx.split is None else (ctx.split[0], ctx.out_shape[1]), dtype=ctx.out_dtype,
+                                 device=offsets.device),) + grads[1:]
         grad = grads[0] if ctx.split is None else _joined(grads, ctx.split, ctx.out_shape)
         # sum / mean: the gradient of a unique row is a gather-reduce over its occurrence list; it is handed
         # over unsummed, so that the optimizer step can sum and update the row in one launch

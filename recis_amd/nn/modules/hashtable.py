@@ -150,13 +150,14 @@ class HashTableLookupHelpFunction(torch.autograd.Function):
         index, embedding = hashtable.embedding_lookup(ids.detach(), admit_hook_impl is not None)
         ctx.save_for_backward(index)
         ctx.set_materialize_grads(False)  # the index takes no gradient: no zeros are made for it
-        ctx.hashtable = hashtable
+        ctx.hashtable, ctx.out_like = hashtable, (embedding.shape, embedding.dtype, embedding.device)
         ctx.mark_non_differentiable(index)
         return index, embedding
 
     @staticmethod
     def backward(ctx, grad_output_index, grad_output_emb):
         (index,) = ctx.saved_tensors
+        grad_output_emb = _or_zeros(grad_output_emb, ctx.out_like)
         ctx.hashtable.accept_grad_ex(index, grad_output_emb.contiguous(), True,
                                      0 if ctx.grad_key is None else int(ctx.grad_key))
         return None, None, None, None, None
@@ -228,6 +229,7 @@ class LookupExpandFunction(torch.autograd.Function):
             index = index[: plan.U]
             ctx.settled = True
         ctx.impl, ctx.plan, ctx.slice_num, ctx.readonly = impl, plan, slice_num, readonly
+        ctx.out_like = (out.shape, out.dtype, out.device)
         ctx.save_for_backward(index)
         ctx.set_materialize_grads(False)  # the index takes no gradient: no zeros are made for it
         ctx.mark_non_differentiable(index)
@@ -237,7 +239,7 @@ class LookupExpandFunction(torch.autograd.Function):
     def backward(ctx, _grad_index, grad):
         (index,) = ctx.saved_tensors
         plan = ctx.plan
-        flat = grad.reshape(plan.n, -1).contiguous()
+        flat = _or_zeros(grad, ctx.out_like).reshape(plan.n, -1).contiguous()
         if ctx.slice_num != 1:
             flat = flat / ctx.slice_num
         if not ctx.settled:
@@ -247,6 +249,12 @@ class LookupExpandFunction(torch.autograd.Function):
         # sums and updates the row); keys the table does not hold (negative index) take no gradient
         accept_planned_grad(ctx.impl, index, plan, flat, plan.occ, may_miss=ctx.readonly)
         return None, None, None, None, None, None, None
+
+
+def _or_zeros(grad, like):
+    """The gradient of an output; zeros when a function behind it returned none. (A gradient of zeros still is one: the
+    rows take a step of their momentum.)"""
+    return grad if grad is not None else torch.zeros(like[0], dtype=like[1], device=like[2])
 
 
 def _scatter_sum(grad_rows, index, unique_size, plan=None):

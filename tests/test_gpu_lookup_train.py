@@ -9,8 +9,8 @@ import torch
 
 from recis_amd import _lib, ops
 from recis_amd.nn import EmbeddingEngine, EmbeddingOption, HashTable
-from recis_amd.nn.hashtable_hook import FilterHook
-from recis_amd.nn.modules.hashtable import HashtableRegister, filter_out_sparse_param
+from recis_amd.nn.hashtable_hook import AdmitHook, FilterHook
+from recis_amd.nn.modules.hashtable import HashTableLookupHelpFunction, HashtableRegister, filter_out_sparse_param
 from recis_amd.nn.modules.hashtable_hook_impl import HashtableHookFactory
 from recis_amd.optim import SparseAdagrad, SparseAdam
 from recis_amd.ragged import RaggedTensor
@@ -345,3 +345,57 @@ def test_a_count_stays_until_it_is_released(rng):
     assert got == [239] and count_of(mine) == 600
     _lib.check(lib.recis_unique_plan_release(_lib.i64(mine)))
     assert _lib.poll_device_errors() == 0
+
+
+class _TakesNoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x):
+        return x * 1.0
+
+    @staticmethod
+    def backward(ctx, g):
+        return None
+
+
+@pytest.mark.parametrize("kind", ["table", "admit", "helper", "engine_dense", "engine_sum", "engine_tile",
+                                  "engine_admit"])
+def test_no_gradient_for_an_output_counts_as_zeros(rng, kind):
+    """A function behind the lookup that returns no gradient for it: the rows of the batch take a gradient of zeros (with
+    Adam a step of their momentum), as when autograd hands zeros over."""
+    rows = []
+    for way in ("none", "zeros"):
+        HashtableRegister().clear()
+        ids = torch.arange(40, device="cuda")
+        if kind.startswith("engine"):
+            kw = {"combiner_kwargs": {"tile_len": 5}} if kind == "engine_tile" else {}
+            module = EmbeddingEngine({"a": EmbeddingOption(embedding_dim=8, block_size=64, shared_name="nograd", use_weight=False,
+                                                           combiner="tile" if kind == "engine_tile" else "sum",
+                                                           admit_hook=AdmitHook("ReadOnly") if kind == "engine_admit" else None, **kw)})
+            x = ids if kind == "engine_dense" else RaggedTensor(ids, _offsets([4] * 10))
+            call = lambda: module({"a": x})["a"]
+        else:
+            module = HashTable([8], block_size=64, name="nograd", grad_reduce_by="worker")
+            admit = AdmitHook("ReadOnly") if kind == "admit" else None
+            if kind == "helper":
+                call = lambda: HashTableLookupHelpFunction.apply(ids, module._hashtable_impl, module._backward_holder, None)[1]
+            else:
+                call = lambda: module(ids, admit)
+        module.train()
+        tables = filter_out_sparse_param(module)
+        (impl,) = tables.values()
+        impl.insert(ids, torch.ones(40, 8, device="cuda"))
+        opt = SparseAdam(tables, lr=0.1)
+        out = call()
+        out.backward(torch.ones_like(out))
+        opt.step()
+        opt.zero_grad()
+        moved = torch.cat(impl.slot_group().slot_by_name("embedding").kernel_blocks()[0]).clone()
+        out = call()
+        if way == "none":
+            _TakesNoGradient.apply(out).sum().backward()
+        else:
+            out.backward(torch.zeros_like(out))
+        opt.step()
+        rows.append(torch.cat(impl.slot_group().slot_by_name("embedding").kernel_blocks()[0]).clone())
+        assert not torch.equal(rows[-1], moved)
+    assert torch.equal(rows[0], rows[1])
