@@ -15,7 +15,8 @@ from ...ragged.tensor import RaggedTensor
 from ..functional.embedding_ops import ragged_embedding_segment_reduce
 from ..hashtable_hook import AdmitHook, FilterHook
 from ..initializers import ConstantInitializer, Initializer
-from .hashtable import GradIDMeanFunction, HashTable, HashTableLookupHelpFunction, accept_planned_grad, gen_slice
+from .hashtable import (GradIDMeanFunction, HashTable, HashTableLookupHelpFunction, accept_planned_grad, gen_slice,
+                        pools_readonly)
 
 
 class _Done:
@@ -289,9 +290,9 @@ class DynamicEmbedding(torch.nn.Module):
         opt, table = self._emb_opt, self._hashtable
         if table._dtype in (torch.float32, torch.bfloat16, torch.float16) and opt.combiner in ("sum", "mean"):
             ids, offs = (val, offsets) if width is None or weight is not None else (val.view(-1, width), None)
-            if not table.training:
+            if not table.training and pools_readonly(table):
                 return table._hashtable_impl.lookup_pool_readonly([ids], [offs], [weight], None, opt.combiner == "mean")[0]
-            if opt.trainable and opt.admit_hook is None and opt.grad_reduce_by != "id":
+            if table.training and opt.trainable and opt.admit_hook is None and opt.grad_reduce_by != "id":
                 res = table._hashtable_impl.lookup_train([ids], [offs], [weight], None, opt.combiner, [], True, None, None)
                 if res is not None:
                     if not isinstance(table._filter_hook_impl, torch.nn.Identity):

@@ -24,7 +24,7 @@ from ... import ops
 from ...ragged.tensor import RaggedTensor
 from ..functional.embedding_ops import RaggedTileParts
 from .embedding import EmbeddingOption, lookup_and_pool, lookup_unique_rows
-from .hashtable import HashTable, gen_slice
+from .hashtable import HashTable, gen_slice, pools_readonly
 
 
 def _key(text):
@@ -199,7 +199,7 @@ class EmbeddingEngine(torch.nn.Module):
                 opt0 = grp.features[names[0]]
                 tags = [tag_of[n] for n in names] if info.is_coalesce() else None
                 float_table = table._dtype in (torch.float32, torch.bfloat16, torch.float16)
-                if not table.training and opt0.combiner in ("sum", "mean") and float_table:
+                if not table.training and opt0.combiner in ("sum", "mean") and pools_readonly(table):
                     self._evaluate(table, tags, names, opt0, inputs, outputs)
                     continue
                 same = (gkey,) + tuple((id(inputs[n]), tag_of[n]) for n in names)

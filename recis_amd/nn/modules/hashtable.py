@@ -270,6 +270,12 @@ def _scatter_sum(grad_rows, index, unique_size, plan=None):
     return out.view((unique_size,) + tuple(grad_rows.shape[1:]))
 
 
+def pools_readonly(table):
+    """Whether ``HashtableImpl.lookup_pool_readonly`` takes the rows of a table: floats, at most 8192 of them (wider rows go
+    through a plan and the general pooling)."""
+    return table._dtype in (torch.float32, torch.bfloat16, torch.float16) and table._embedding_shape[0] <= 8192
+
+
 # ------------------------------------------------------------------- module
 class HashTable(torch.nn.Module):
     """Dynamic embedding table (recis/nn/modules/hashtable.py:98-423).
@@ -358,8 +364,7 @@ class HashTable(torch.nn.Module):
             if hooked:
                 self._filter_hook_impl(emb_idx)
             return embedding.view(shape + tuple(embedding.shape[1:])) if len(shape) != 1 else embedding
-        if not self.training and len(self._embedding_shape) == 1 and self._dtype in (torch.float32, torch.bfloat16,
-                                                                                    torch.float16):
+        if not self.training and len(self._embedding_shape) == 1 and pools_readonly(self):
             # nothing is inserted and nothing flows back: ids straight to rows, no dedup
             embedding = self._hashtable_impl.lookup_pool_readonly([ids], [None], [None], None, False)[0]
             return embedding.view(shape + tuple(embedding.shape[1:])) if len(shape) != 1 else embedding

@@ -5,8 +5,8 @@ import pytest
 import torch
 
 from recis_amd import _lib, ops
-from recis_amd.nn import EmbeddingEngine, EmbeddingOption, HashTable
-from recis_amd.nn.modules.hashtable import HashtableRegister
+from recis_amd.nn import DynamicEmbedding, EmbeddingEngine, EmbeddingOption, HashTable
+from recis_amd.nn.modules.hashtable import HashtableRegister, filter_out_sparse_param
 from recis_amd.ragged import RaggedTensor
 
 pytestmark = pytest.mark.gpu
@@ -167,4 +167,32 @@ def test_training_raises_what_evaluation_reported():
     ht.train()
     with pytest.raises(RuntimeError, match="offsets not monotone"):
         ht(ids).sum().backward()
+    assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("D,dtype", [(8192, torch.float32), (8196, torch.float32), (9000, torch.bfloat16)])
+def test_evaluation_of_wide_rows(rng, D, dtype):
+    ids = torch.arange(6, device="cuda")
+    rows = torch.from_numpy(rng.standard_normal((6, D)).astype(np.float32)).cuda().to(dtype)
+    tol = dict(rtol=2.0 ** -7 if dtype == torch.bfloat16 else 1e-6, atol=1e-6)
+    HashtableRegister().clear()
+    table = HashTable([D], block_size=8, dtype=dtype, name="wide")
+    table.insert(ids, rows)
+    table.eval()
+    at = torch.tensor([[3, 1], [5, 77]], device="cuda")
+    got = table(at)
+    assert torch.equal(got[0, 0], rows[3]) and torch.equal(got[1, 0], rows[5]) and not got[1, 1].any()
+    HashtableRegister().clear()
+    for module in (DynamicEmbedding(EmbeddingOption(embedding_dim=D, block_size=8, dtype=dtype, shared_name="wide_e")),
+                   EmbeddingEngine({"a": EmbeddingOption(embedding_dim=D, block_size=8, dtype=dtype, shared_name="wide_g",
+                                                         combiner="mean")})):
+        (impl,) = filter_out_sparse_param(module).values()
+        impl.insert(ids, rows)
+        module.eval()
+        x = RaggedTensor(torch.arange(6, device="cuda"), _offsets([2, 0, 4]))
+        got = module({"a": x})["a"] if isinstance(module, EmbeddingEngine) else module(x)
+        parts = [rows[:2].float().sum(0), torch.zeros(D, device="cuda"), rows[2:].float().sum(0)]
+        if isinstance(module, EmbeddingEngine):
+            parts = [parts[0] / 2, parts[1], parts[2] / 4]
+        torch.testing.assert_close(got, torch.stack(parts).to(dtype), **tol)
     assert _lib.poll_device_errors() == 0
