@@ -201,8 +201,8 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
       segments[k] = offsets[k]->numel() - 1;
       unit = false;
     } else {
-      widths[k] = v.dim() <= 1 ? 1 : v.size(-1);
-      segments[k] = widths[k] > 0 ? n_ids[k] / widths[k] : 0;
+      widths[k] = DenseWidth(v);
+      segments[k] = n_ids[k] / widths[k];
       unit = unit && widths[k] == 1;
     }
     any_weight = any_weight || (weights[k].has_value() && weights[k]->defined());

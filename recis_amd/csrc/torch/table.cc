@@ -879,8 +879,8 @@ std::vector<at::Tensor> Hashtable::LookupPoolReadonly(const std::vector<at::Tens
     } else {
       j.offsets = nullptr;
       j.off_is64 = 0;
-      j.width = values[k].dim() <= 1 ? 1 : values[k].size(-1);
-      j.n_seg = j.width > 0 ? j.n_ids / j.width : 0;
+      j.width = DenseWidth(values[k]);
+      j.n_seg = j.n_ids / j.width;
     }
     j.weight = nullptr;
     j.weight_dtype = 0;

@@ -378,6 +378,12 @@ class Hashtable : public torch::CustomClassHolder {
 
  private:
   void MakeRoom(int64_t incoming);
+  // Ids per segment of a dense id tensor ([B]: one).
+  static int64_t DenseWidth(const at::Tensor& ids) {
+    TORCH_CHECK(ids.dim() >= 1 && (ids.dim() == 1 || ids.size(-1) > 0), "dense ids of shape ", ids.sizes(),
+                ": at least one id per segment is wanted");
+    return ids.dim() == 1 ? 1 : ids.size(-1);
+  }
   at::Tensor GroupOffsets(const std::vector<c10::optional<at::Tensor>>& offsets, const std::vector<int64_t>& segments,
                           const std::vector<int64_t>& widths, const std::vector<int64_t>& n_ids) const;
   at::Tensor OnDevice(const at::Tensor& ids) const;

@@ -289,7 +289,7 @@ class DynamicEmbedding(torch.nn.Module):
         allow it. ``width`` ids per segment when the ids were a dense tensor."""
         opt, table = self._emb_opt, self._hashtable
         if table._dtype in (torch.float32, torch.bfloat16, torch.float16) and opt.combiner in ("sum", "mean"):
-            ids, offs = (val, offsets) if width is None or weight is not None else (val.view(-1, width), None)
+            ids, offs = (val, offsets) if not width or weight is not None else (val.view(-1, width), None)
             if not table.training and pools_readonly(table):
                 return table._hashtable_impl.lookup_pool_readonly([ids], [offs], [weight], None, opt.combiner == "mean")[0]
             if table.training and opt.trainable and opt.admit_hook is None and opt.grad_reduce_by != "id":

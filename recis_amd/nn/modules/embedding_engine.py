@@ -135,8 +135,8 @@ class EmbeddingEngine(torch.nn.Module):
         vals, offs, weights, prefixes = [], [], [], []
         for name in names:
             data = inputs[name]
-            if type(data) is torch.Tensor:
-                vals.append(data)
+            if isinstance(data, torch.Tensor):
+                vals.append(data if type(data) is torch.Tensor else data.as_subclass(torch.Tensor))
                 offs.append(None)
                 weights.append(None)
                 prefixes.append(None if data.dim() <= 2 else data.shape[:-1])

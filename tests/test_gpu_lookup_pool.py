@@ -196,3 +196,32 @@ def test_evaluation_of_wide_rows(rng, D, dtype):
             parts = [parts[0] / 2, parts[1], parts[2] / 4]
         torch.testing.assert_close(got, torch.stack(parts).to(dtype), **tol)
     assert _lib.poll_device_errors() == 0
+
+
+class _Ids(torch.Tensor):
+    pass
+
+
+@pytest.mark.parametrize("training", [False, True])
+def test_dense_ids_of_every_kind(rng, training):
+    HashtableRegister().clear()
+    opt = dict(embedding_dim=8, block_size=64, combiner="sum")
+    one = DynamicEmbedding(EmbeddingOption(shared_name="one", **opt)).train(training)
+    out = one(torch.empty(7, 0, dtype=torch.int64, device="cuda"))  # no id in any segment
+    assert out.shape == (7, 8) and not out.detach().any()
+    eng = EmbeddingEngine({"a": EmbeddingOption(shared_name="a", **opt), "b": EmbeddingOption(shared_name="b", **opt)}).train(training)
+    (table,) = eng.hashtables().values()
+    plain = torch.from_numpy(rng.integers(0, 9, (6, 2))).cuda()
+    eng({"a": plain, "b": plain[:, :1]})
+    for block in table._hashtable_impl.emb_blocks()[0]:
+        block.normal_()
+    want = eng({"a": plain, "b": plain[:, :1]})
+    for kind in (lambda t: t.as_subclass(_Ids), lambda t: torch.nn.Parameter(t, requires_grad=False), lambda t: t.int(),
+                 lambda t: t.cpu()):
+        got = eng({"a": kind(plain), "b": kind(plain[:, :1])})
+        assert all(torch.equal(got[k], want[k]) for k in want)
+    with pytest.raises(Exception):
+        eng({"a": torch.empty(7, 0, dtype=torch.int64, device="cuda"), "b": plain[:, :1]})
+    with pytest.raises(Exception):
+        eng({"a": torch.tensor(3, device="cuda"), "b": plain[:, :1]})
+    assert _lib.poll_device_errors() == 0
