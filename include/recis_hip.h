@@ -449,12 +449,16 @@ int recis_block_apply_adagrad(const int64_t* index, const void* grad, int grad_d
  * recis_merge_offsets  merge_offsets, csrc/ops/embedding_segment_reduce_kernel.cu:357-391:
  *                    tensor t contributes its first size_t - 1 entries (all of them
  *                    for the last tensor) plus sum_{u<t} max_values[u]
+ * recis_group_offsets  the same for features of which some are dense: feature t has segments[t] + 1 int32 offsets over
+ *                    n_ids[t] ids, or none (NULL) and widths[t] ids in every segment
  */
 int recis_ids_encode(const int64_t* const* ids_ptrs, const int64_t* sizes,
                      const int64_t* table_ids, int64_t n_tensors, int64_t* out, void* stream);
 int recis_merge_offsets(const void* const* offsets_ptrs, const int64_t* sizes,
                         const int64_t* max_values, int64_t n_tensors, int is64, void* out,
                         void* stream);
+int recis_group_offsets(const int32_t* const* offsets_ptrs, const int64_t* segments, const int64_t* widths,
+                        const int64_t* n_ids, int64_t n_features, int32_t* out, void* stream);
 
 /*
  * Dedup: unique ids (in order of first occurrence), inverse (int32 or int64) with

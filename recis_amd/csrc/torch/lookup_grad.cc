@@ -157,22 +157,19 @@ c10::optional<std::vector<at::Tensor>> Hashtable::DenseLookupTrain(const std::ve
 at::Tensor Hashtable::GroupOffsets(const std::vector<TensorOrNone>& offsets, const std::vector<int64_t>& segments,
                                    const std::vector<int64_t>& widths, const std::vector<int64_t>& n_ids) const {
   auto i32 = at::TensorOptions().device(device_).dtype(at::kInt);
-  std::vector<at::Tensor> offs;
-  for (size_t k = 0; k < offsets.size(); ++k) {
-    if (offsets[k].has_value() && offsets[k]->defined()) {
-      offs.push_back(offsets[k]->to(i32).contiguous());
-    } else {
-      offs.push_back(at::arange(segments[k] + 1, i32).mul_(widths[k]));
-    }
-  }
-  if (offs.size() == 1) return offs[0];
-  auto ptrs = recis::hipabi::host_ptrs<void>(offs);
-  auto sizes = recis::hipabi::numels(offs);
+  std::vector<at::Tensor> keep;  // alive until the launch is queued
+  std::vector<const int32_t*> ptrs(offsets.size(), nullptr);
   int64_t total = 1;
-  for (int64_t s : segments) total += s;
+  for (size_t k = 0; k < offsets.size(); ++k) {
+    total += segments[k];
+    if (!offsets[k].has_value() || !offsets[k]->defined()) continue;
+    keep.push_back(offsets[k]->to(i32).contiguous());
+    ptrs[k] = keep.back().data_ptr<int32_t>();
+  }
+  if (offsets.size() == 1 && !keep.empty()) return keep[0];
   at::Tensor out = at::empty({total}, i32);
-  check(recis_merge_offsets(ptrs.data(), sizes.data(), n_ids.data(), static_cast<int64_t>(offs.size()), 0, out.data_ptr(),
-                            stream_of(device_)));
+  check(recis_group_offsets(ptrs.data(), segments.data(), widths.data(), n_ids.data(), static_cast<int64_t>(offsets.size()),
+                            out.data_ptr<int32_t>(), stream_of(device_)));
   return out;
 }
 

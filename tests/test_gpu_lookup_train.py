@@ -399,3 +399,36 @@ def test_no_gradient_for_an_output_counts_as_zeros(rng, kind):
         rows.append(torch.cat(impl.slot_group().slot_by_name("embedding").kernel_blocks()[0]).clone())
         assert not torch.equal(rows[-1], moved)
     assert torch.equal(rows[0], rows[1])
+
+
+@pytest.mark.parametrize("kinds", ["r", "d", "dd", "rd", "dr", "drdrr", "d" * 50 + "r", "r" * 47 + "dd", "rdz"])
+def test_offsets_of_a_group_in_one_launch(rng, kinds):
+    """Ragged (r), dense (d) and empty (z) features as one list of offsets."""
+    offs, segs, widths, n_ids, want, first = [], [], [], [], [], 0
+    for k in kinds:
+        s = 0 if k == "z" else int(rng.integers(1, 700))
+        if k == "r":
+            o = np.concatenate([[0], np.cumsum(rng.integers(0, 5, s))])
+            offs.append(torch.from_numpy(o.astype(np.int32)).cuda())
+            w = 0
+        else:
+            w = int(rng.integers(1, 6))
+            o = np.arange(s + 1) * w
+            offs.append(None)
+        want.append(first + o[:-1])
+        first += o[-1]
+        segs.append(s)
+        widths.append(w)
+        n_ids.append(int(o[-1]))
+    want.append([first])
+    want = np.concatenate(want)
+    out = torch.full((len(want) + 1,), -7, dtype=torch.int32, device="cuda")
+    n = len(kinds)
+    arr = lambda v: (ctypes.c_int64 * n)(*v)
+    ptrs = (ctypes.c_void_p * n)(*[None if o is None else o.data_ptr() for o in offs])
+    call = lambda w: _lib.lib().recis_group_offsets(ptrs, arr(segs), arr(w), arr(n_ids), ctypes.c_int64(n), _lib.ptr(out),
+                                                    _lib.stream_ptr())
+    assert call(widths) == 0
+    assert out[:-1].tolist() == want.tolist() and int(out[-1]) == -7
+    if "d" in kinds:
+        assert call([w + 1 for w in widths]) != 0  # ids that are not segments of that width
