@@ -306,7 +306,23 @@ struct FillArgs {
   int64_t rbase[kFillFeatures];
   int64_t coarse_stride;  // every coarse_stride-th offset goes into the workgroup's LDS table
   int n_coarse;
+  const int32_t* not_unit;  // [kUnitBlocks] or NULL, see offsets_not_unit_kernel
 };
+
+// As many segments as occurrences: is there one in each (offsets 0, 1, 2, ..., what dense columns have)? Then an occurrence
+// is its own segment and the search, the dearest with as many offsets as entries, is not made. Every workgroup leaves a word; the
+// fill kernel's workgroups read them all. 2.1 M entries: 11 us, both kernels, instead of the search's 159.
+constexpr int kUnitBlocks = kBlock;
+__global__ void __launch_bounds__(kBlock)
+offsets_not_unit_kernel(const void* offsets, int off64, int64_t S, int32_t* __restrict__ not_unit) {
+  bool bad = false;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x; i <= S;
+       i += static_cast<int64_t>(gridDim.x) * kBlock)
+    bad |= load_index(offsets, off64, i) != i;
+  bad = __syncthreads_or(bad);
+  if (threadIdx.x == 0) not_unit[blockIdx.x] = bad;
+}
+
 // The bisection runs in two stages: over every coarse_stride-th offset, in LDS (a workgroup loads
 // that table once for the kFillPer entries of each of its threads), then over the few offsets in
 // between, in memory. A bisection of the whole array out of the caches is a dozen dependent loads
@@ -316,6 +332,17 @@ constexpr int kFillPer = 4;
 __global__ void __launch_bounds__(kBlock)
 fill_lists_kernel(FillArgs a) {
   __shared__ int32_t s_coarse[kFillCoarse];
+  const bool unit = a.not_unit != nullptr && !__syncthreads_or(a.not_unit[threadIdx.x]);
+  if (unit) {
+    for (int x = 0; x < kFillPer; ++x) {
+      const int64_t k = (static_cast<int64_t>(blockIdx.x) * kFillPer + x) * kBlock + threadIdx.x;
+      if (k >= a.n) return;
+      const int32_t i = a.list[k];
+      a.src_pool[k] = i;
+      if (a.coef) a.coef[k] = a.weight ? load_coef(a.weight, a.wdt, i) : 1.0f;
+    }
+    return;
+  }
   for (int c = threadIdx.x; c < a.n_coarse; c += kBlock) {
     const int64_t v = load_index(a.offsets, a.off64, c * a.coarse_stride);
     s_coarse[c] = static_cast<int32_t>(min(v, static_cast<int64_t>(INT32_MAX)));  // places are below 2^30
@@ -412,6 +439,13 @@ int recis_csr_fill_lists(const int32_t* list, int64_t n, const void* offsets, in
   const dim3 grid(static_cast<unsigned>((n + kFillPer * kBlock - 1) / (kFillPer * kBlock)));
   if (!src_tile_out) {
     a.first_group = 1;
+    if (S == n) {
+      void* ws = nullptr;
+      if (int rc = get_workspace(stream, sizeof(int32_t) * kUnitBlocks, &ws)) return rc;
+      offsets_not_unit_kernel<<<dim3(kUnitBlocks), dim3(kBlock), 0, stream>>>(offsets, off_is64, S, static_cast<int32_t*>(ws));
+      RECIS_LAUNCH_CHECK();
+      a.not_unit = static_cast<const int32_t*>(ws);
+    }
     fill_lists_kernel<<<grid, dim3(kBlock), 0, stream>>>(a);
     RECIS_LAUNCH_CHECK();
     return RECIS_OK;

@@ -103,9 +103,8 @@ struct LookupBackward : public torch::autograd::Node {
 //   0.79 M            8.5    1.3   -1.7   -2.8                  11.6    4.5    1.4   -0.8
 //   1.05 M           11.2    2.6   -4.3   -5.4                  15.6    8.1    1.9   -0.9
 //   2.10 M           23.8    8.9  -13.2  -19.8                  36.3   21.4    2.7   -7.6
-// One id per segment, unweighted: the lists are the answer themselves.
 bool NotesOccurrences(int64_t n, int64_t segments, bool weighted) {
-  if (n == 0 || segments == 0 || (segments == n && !weighted)) return false;
+  if (n == 0 || segments == 0) return false;
   return n <= (int64_t(1) << 19) || n <= (weighted ? 128 : 32) * segments;
 }
 

@@ -202,9 +202,6 @@ std::tuple<at::Tensor, c10::optional<at::Tensor>> BatchPlan::SrcCoefForPool(cons
                                                                              const c10::optional<at::Tensor>& weight,
                                                                              bool mean) {
   const bool has_w = weight.has_value() && weight->defined();
-  if (offsets.numel() - 1 == n_ && !has_w) {
-    return std::make_tuple(occ_, c10::optional<at::Tensor>());  // one id per segment: an occurrence is its own segment
-  }
   const void* wp = has_w ? weight->data_ptr() : nullptr;
   if (fill_valid_ && fill_offsets_ == offsets.data_ptr() && fill_weight_ == wp && fill_mean_ == mean) {
     return std::make_tuple(fill_src_, fill_coef_.defined() ? c10::optional<at::Tensor>(fill_coef_) : c10::nullopt);
@@ -227,7 +224,6 @@ void BatchPlan::KeepPoolLists(const at::Tensor& offsets, const at::Tensor& weigh
 }
 
 void BatchPlan::NotePool(const at::Tensor& offsets, const at::Tensor& weight, bool mean) {
-  if (offsets.numel() - 1 == n_ && !weight.defined()) return;  // SrcCoefForPool has nothing to fill
   note_offsets_ = offsets;
   note_weight_ = weight;
   note_mean_ = mean;

@@ -144,7 +144,7 @@ class LookupPoolFunction(torch.autograd.Function):
         else:
             chunks, chunk_rows = impl.emb_blocks()
             out = ops.segment_reduce_forward_blocks(chunks, chunk_rows, index, weight, plan.inverse, offsets, combiner)
-        ctx.impl, ctx.plan, ctx.combiner = impl, plan, combiner
+        ctx.impl, ctx.plan, ctx.combiner, ctx.unit_segments = impl, plan, combiner, unit_segments
         ctx.split, ctx.out_shape, ctx.out_dtype = split, tuple(out.shape), out.dtype
         ctx.save_for_backward(index, weight, offsets)
         ctx.set_materialize_grads(False)
@@ -160,7 +160,10 @@ class LookupPoolFunction(torch.autograd.Function):
         grad = grads[0] if ctx.split is None else _joined(grads, ctx.split, ctx.out_shape)
         # sum / mean: the gradient of a unique row is a gather-reduce over its occurrence list; it is handed
         # over unsummed, so that the optimizer step can sum and update the row in one launch
-        src, coef = ctx.plan.src_coef_for_pool(offsets.contiguous(), weight, ctx.combiner == "mean")
+        if ctx.unit_segments and weight is None:
+            src, coef = ctx.plan.occ, None  # an occurrence is its own segment
+        else:
+            src, coef = ctx.plan.src_coef_for_pool(offsets.contiguous(), weight, ctx.combiner == "mean")
         accept_planned_grad(ctx.impl, index, ctx.plan, grad.contiguous(), src, coef, may_miss=True)
         return (None,) * 8
 

@@ -432,3 +432,30 @@ def test_offsets_of_a_group_in_one_launch(rng, kinds):
     assert out[:-1].tolist() == want.tolist() and int(out[-1]) == -7
     if "d" in kinds:
         assert call([w + 1 for w in widths]) != 0  # ids that are not segments of that width
+
+
+@pytest.mark.parametrize("shape", ["ragged", "mixed"])
+def test_as_many_segments_as_ids(rng, shape):
+    """As many ids as segments, but not one in each: every gradient goes to the rows of its own segment."""
+    HashtableRegister().clear()
+    D = 4
+    lens = {"a": np.array([0, 2, 1, 0, 3, 0])} if shape == "ragged" else {"a": np.array([0, 3]), "b": np.array([2, 1, 0, 0])}
+    assert sum(l.sum() for l in lens.values()) == sum(len(l) for l in lens.values())
+    eng = EmbeddingEngine({n: EmbeddingOption(embedding_dim=D, block_size=64, shared_name="s", combiner="sum", use_weight=False)
+                           for n in lens})
+    eng.train()
+    opt = SparseAdagrad(filter_out_sparse_param(eng), lr=0.1)
+    (table,) = eng.hashtables().values()
+    x, grad, ups, first = {}, np.zeros((6, D)), {}, 0
+    for k, l in lens.items():
+        ids = np.arange(first, first + l.sum())
+        first += l.sum()
+        x[k] = RaggedTensor(torch.from_numpy(ids).cuda(), _offsets(l))
+        ups[k] = rng.random((len(l), D)).astype(np.float32) + 0.5
+        grad[ids] = ups[k][np.repeat(np.arange(len(l)), l)]
+    out = eng(x)
+    torch.autograd.backward([out[k] for k in x], [torch.from_numpy(ups[k]).cuda() for k in x])
+    opt.step()
+    keys, where = table._hashtable_impl.ids_map()
+    accum = torch.cat(table._hashtable_impl.get_slot("sparse_adagrad_accum").kernel_blocks()[0])[where].cpu().numpy()
+    np.testing.assert_allclose(accum, grad[keys.cpu().numpy()] ** 2, rtol=1e-6)

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from recis_amd import _lib
+from recis_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -111,3 +111,31 @@ def test_occurrences_of_bad_segments_have_no_notes(rng, offsets, weighted, mean,
         assert (src.cpu().numpy() == want_src[at]).all(), junk
         np.testing.assert_allclose(coef.cpu().numpy(), want_coef[at], rtol=2.0 ** -23)  # one division in float32
     _lib.poll_device_errors()
+
+
+@pytest.mark.parametrize("n", [1, 2, 256, 1023, 70001])
+@pytest.mark.parametrize("kind", ["one in each", "first", "last", "random", "off by one"])
+@pytest.mark.parametrize("weighted,mean", [(False, False), (False, True), (True, True)])
+def test_lists_of_as_many_segments_as_ids(rng, n, kind, weighted, mean):
+    off = np.arange(n + 1)
+    if kind == "first":
+        off[1:-1] += 1 if n > 1 else 0
+    elif kind == "last":
+        off[-2:] = n if n > 1 else off[-2:]
+    elif kind == "random":
+        off[1:-1] = np.sort(rng.integers(0, n + 1, n - 1))
+    elif kind == "off by one":  # id 0 in no segment
+        off[:-1] += 1
+    ids = rng.integers(0, max(1, n // 3), n)
+    plan = ops.ids_unique_plan(torch.from_numpy(ids).cuda())
+    w = (rng.random(n) + 0.5).astype(np.float32)
+    src, coef = plan.src_coef_for_pool(torch.from_numpy(off.astype(np.int32)).cuda(),
+                                       torch.from_numpy(w).cuda() if weighted else None, mean)
+    at = plan.occ.cpu().numpy()
+    want = np.searchsorted(off, np.arange(n), side="right") - 1
+    inside = (np.arange(n) >= off[0]) & (np.arange(n) < off[-1])
+    c = (w if weighted else np.ones(n, np.float32)) / (np.maximum(np.diff(off)[want], 1) if mean else 1)
+    assert (src.cpu().numpy() == np.where(inside, want, -1)[at]).all()
+    if weighted or mean:
+        np.testing.assert_allclose(coef.cpu().numpy(), np.where(inside, c, 0)[at], rtol=2.0 ** -23)
+    assert _lib.poll_device_errors() == 0
