@@ -172,7 +172,7 @@ at::Tensor Hashtable::GroupOffsets(const std::vector<TensorOrNone>& offsets, con
   return out;
 }
 
-c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::Tensor>> Hashtable::LookupTrain(
+c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, TensorOrNone, at::Tensor>> Hashtable::LookupTrain(
     const std::vector<at::Tensor>& values, const std::vector<TensorOrNone>& offsets,
     const std::vector<TensorOrNone>& weights, const c10::optional<std::vector<int64_t>>& tags,
     const std::string& combiner, const std::vector<int64_t>& tile_len, bool lean,
@@ -294,7 +294,8 @@ c10::optional<std::tuple<std::vector<at::Tensor>, BatchPlanPtr, at::Tensor, at::
       node->seq = tile_len;
     }
   }
-  return std::make_tuple(outputs_of(out, shapes, split, node), plan, merged, index);
+  return std::make_tuple(outputs_of(out, shapes, split, node), plan,
+                         merged.defined() ? TensorOrNone(merged) : TensorOrNone(c10::nullopt), index);
 }
 
 void Hashtable::AcceptTileGrad(const at::Tensor& index, const BatchPlanPtr& plan, const at::Tensor& offsets,

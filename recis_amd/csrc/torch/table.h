@@ -317,10 +317,10 @@ class Hashtable : public torch::CustomClassHolder {
   // the table; "tile": padded, tile_len[k] rows per sample): plan + find-or-insert + pooling, one
   // output per feature. offsets[k] undefined = the rows of a dense tensor. A plan that another group of the
   // same inputs made is taken over (shared_plan, shared_offsets); `lean`: no other group can come to
-  // share this one's plan. Returns (outputs, plan, merged offsets | undefined, rows of the plan's unique ids:
+  // share this one's plan. Returns (outputs, plan, merged offsets | None, rows of the plan's unique ids:
   // the first U of a longer buffer), or None when "mean" has few ids per segment (then it divides by the sum
   // of the weights: another path).
-  c10::optional<std::tuple<std::vector<at::Tensor>, recis::BatchPlanPtr, at::Tensor, at::Tensor>> LookupTrain(
+  c10::optional<std::tuple<std::vector<at::Tensor>, recis::BatchPlanPtr, c10::optional<at::Tensor>, at::Tensor>> LookupTrain(
       const std::vector<at::Tensor>& values, const std::vector<c10::optional<at::Tensor>>& offsets,
       const std::vector<c10::optional<at::Tensor>>& weights, const c10::optional<std::vector<int64_t>>& tags,
       const std::string& combiner, const std::vector<int64_t>& tile_len, bool lean,

@@ -459,3 +459,38 @@ def test_as_many_segments_as_ids(rng, shape):
     keys, where = table._hashtable_impl.ids_map()
     accum = torch.cat(table._hashtable_impl.get_slot("sparse_adagrad_accum").kernel_blocks()[0])[where].cpu().numpy()
     np.testing.assert_allclose(accum, grad[keys.cpu().numpy()] ** 2, rtol=1e-6)
+
+
+@pytest.mark.parametrize("combiner", ["sum", "tile"])
+@pytest.mark.parametrize("kind", ["int64", "int32", "host", "strided", "cube"])
+def test_columns_of_one_id_in_every_form(rng, kind, combiner):
+    """One id per segment in tensors that the shortest path does not take (other types, places, strides, shapes): rows and
+    gradients as for a plain column."""
+    HashtableRegister().clear()
+    D = 8
+    kw = {"combiner_kwargs": {"tile_len": 2}} if combiner == "tile" else {}
+    eng = EmbeddingEngine({n: EmbeddingOption(embedding_dim=D, block_size=64, shared_name=n, combiner=combiner, **kw) for n in "ab"})
+    eng.train()
+    opt = SparseAdagrad(filter_out_sparse_param(eng), lr=0.1)
+    ids = rng.integers(0, 9, (20, 1))
+    plain = torch.from_numpy(ids).cuda()
+    x = {"int64": plain, "int32": plain.int(), "host": plain.cpu(), "strided": torch.cat([plain, plain], 1)[:, :1],
+         "cube": plain.view(10, 2, 1)}[kind]
+    (table,) = eng.hashtables().values()
+    impl = table._hashtable_impl
+    keys = torch.cat([torch.arange(9, device="cuda") | (k << 52) for k in range(2)])
+    rows = torch.from_numpy(rng.standard_normal((18, D)).astype(np.float32)).cuda()
+    impl.insert(keys, rows)
+    out = eng({"a": x, "b": x})
+    up = torch.rand(20, D, device="cuda") + 0.5
+    for k, n in enumerate("ab"):
+        got = out[n].reshape(20, -1)
+        assert out[n].shape[:-1] == (x.shape[:-1] if kind == "cube" else (20,))
+        assert torch.equal(got[:, :D], rows[9 * k + plain.view(-1)]) and not got[:, D:].any()
+        got.backward(torch.cat([up, torch.ones_like(got[:, D:])], 1), retain_graph=True)
+    opt.step()
+    held, where = impl.ids_map()
+    accum = torch.cat(impl.get_slot("sparse_adagrad_accum").kernel_blocks()[0])[where][torch.argsort(held)]
+    one = torch.zeros(9, D, dtype=torch.float64, device="cuda").index_add_(0, plain.view(-1), up.double())
+    torch.testing.assert_close(accum.double(), torch.cat([one, one]) ** 2, rtol=1e-5, atol=0)  # sums of up to 20 terms
+    assert _lib.poll_device_errors() == 0
