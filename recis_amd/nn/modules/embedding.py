@@ -293,7 +293,7 @@ class DynamicEmbedding(torch.nn.Module):
         opt, table = self._emb_opt, self._hashtable
         if table._dtype in (torch.float32, torch.bfloat16, torch.float16) and opt.combiner in ("sum", "mean"):
             ids, offs = (val, offsets) if not width or weight is not None else (val.view(-1, width), None)
-            if not table.training and pools_readonly(table):
+            if not table.training and val.dtype == torch.int64 and pools_readonly(table):
                 return table._hashtable_impl.lookup_pool_readonly([ids], [offs], [weight], None, opt.combiner == "mean")[0]
             if table.training and opt.trainable and opt.admit_hook is None and opt.grad_reduce_by != "id":
                 res = table._hashtable_impl.lookup_train([ids], [offs], [weight], None, opt.combiner, [], True, None, None)

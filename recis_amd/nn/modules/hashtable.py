@@ -364,7 +364,7 @@ class HashTable(torch.nn.Module):
             if hooked:
                 self._filter_hook_impl(emb_idx)
             return embedding.view(shape + tuple(embedding.shape[1:])) if len(shape) != 1 else embedding
-        if not self.training and len(self._embedding_shape) == 1 and pools_readonly(self):
+        if not self.training and ids.dtype == torch.int64 and len(self._embedding_shape) == 1 and pools_readonly(self):
             # nothing is inserted and nothing flows back: ids straight to rows, no dedup
             embedding = self._hashtable_impl.lookup_pool_readonly([ids], [None], [None], None, False)[0]
             return embedding.view(shape + tuple(embedding.shape[1:])) if len(shape) != 1 else embedding

@@ -225,3 +225,17 @@ def test_dense_ids_of_every_kind(rng, training):
     with pytest.raises(Exception):
         eng({"a": torch.tensor(3, device="cuda"), "b": plain[:, :1]})
     assert _lib.poll_device_errors() == 0
+
+
+def test_ids_of_other_types_are_refused_where_they_were():
+    """In evaluation HashTable and DynamicEmbedding take int64 ids and do not convert others (a float id has no key)."""
+    HashtableRegister().clear()
+    table = HashTable([8], block_size=64, name="typed")
+    table(torch.arange(4, device="cuda"))
+    table.eval()
+    one = DynamicEmbedding(EmbeddingOption(embedding_dim=8, block_size=64, shared_name="typed_e"))
+    for kind in (torch.int32, torch.float32):
+        with pytest.raises((TypeError, RuntimeError)):
+            table(torch.arange(4, device="cuda").to(kind))
+        with pytest.raises((TypeError, RuntimeError)):
+            one.eval()(torch.arange(4, device="cuda").to(kind).view(2, 2))
