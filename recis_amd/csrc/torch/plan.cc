@@ -254,16 +254,9 @@ at::Tensor BatchPlan::SrcForTile(const std::vector<int64_t>& batch, const std::v
 std::tuple<at::Tensor, c10::optional<at::Tensor>, at::Tensor> BatchPlan::SrcForPoolAndTile(
     const at::Tensor& offsets, const c10::optional<at::Tensor>& weight, bool mean, const std::vector<int64_t>& batch,
     const std::vector<int64_t>& seq) {
-  const bool has_w = weight.has_value() && weight->defined();
-  auto filled = FillLists(offsets, has_w ? *weight : at::Tensor(), mean, true, &batch, &seq);
-  fill_offsets_ = offsets.data_ptr();
-  fill_weight_ = has_w ? weight->data_ptr() : nullptr;
-  fill_keep_offsets_ = offsets;
-  fill_keep_weight_ = has_w ? *weight : at::Tensor();
-  fill_mean_ = mean;
-  fill_valid_ = true;
-  fill_src_ = std::get<0>(filled);
-  fill_coef_ = std::get<1>(filled);
+  const at::Tensor w = weight.has_value() ? *weight : at::Tensor();
+  auto filled = FillLists(offsets, w, mean, true, &batch, &seq);
+  KeepPoolLists(offsets, w, mean, std::get<0>(filled), std::get<1>(filled));
   return std::make_tuple(fill_src_, fill_coef_.defined() ? c10::optional<at::Tensor>(fill_coef_) : c10::nullopt,
                          std::get<2>(filled));
 }

@@ -24,7 +24,7 @@ def _offsets(lens):
 
 @pytest.mark.parametrize("count", [2, 16, 17, 40])
 def test_counts_of_plans_under_way_together(rng, count):
-    """More plans than the ring of staging words holds: the oldest ones read their own device word."""
+    """Every plan's count has a place of its own until it is read, whatever the order."""
     batches = [rng.integers(0, 50 + 37 * k, size=3000) for k in range(count)]
     plans = [ops.ids_unique_plan(torch.from_numpy(b).cuda(), wait=False) for b in batches]
     for k in rng.permutation(count):

@@ -65,3 +65,45 @@ def test_gradients_of_both_outputs(rng, combiner, weighted, outputs):
     torch.testing.assert_close(accum[:KEYS], want, rtol=1e-4, atol=1e-6)
     assert not accum[KEYS:].any()
     assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("weighted", [False, True])
+@pytest.mark.parametrize("first", ["together", "pool"])
+def test_gradients_of_both_outputs_of_long_segments(rng, weighted, first):
+    """More than half a million ids in long segments: the pooling leaves no notes, and both backwards take their lists from
+    one search of the offsets (or, when the pooled output's comes first, from one each)."""
+    segments, keys = 300, 30000
+    lens = rng.integers(1500, 2600, segments)
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)).cuda()
+    n = int(off[-1])
+    assert n > 1 << 19
+    ids = torch.from_numpy(rng.integers(0, keys, n)).cuda()
+    weight = torch.rand(n, device="cuda") + 0.5 if weighted else None
+    HashtableRegister().clear()
+    common = dict(embedding_dim=4, block_size=4096, shared_name="q")
+    engine = EmbeddingEngine({"p": EmbeddingOption(combiner="mean", use_weight=weighted, **common),
+                              "t": EmbeddingOption(combiner="tile", combiner_kwargs={"tile_len": SEQ}, use_weight=False, **common)})
+    engine.train()
+    opt = SparseAdagrad(filter_out_sparse_param(engine), lr=0.1)
+    up_p, up_t = torch.rand(segments, 4, device="cuda") + 0.5, torch.rand(segments, SEQ * 4, device="cuda") + 0.5
+    seg = torch.repeat_interleave(torch.arange(segments, device="cuda"), (off[1:] - off[:-1]).long())
+    place = torch.arange(n, device="cuda") - off[:-1].long()[seg]
+    coef = (weight.double() if weighted else torch.ones(n, dtype=torch.float64, device="cuda")) / (off[1:] - off[:-1]).double()[seg]
+    grad = torch.zeros(keys, 4, dtype=torch.float64, device="cuda").index_add_(0, ids, up_p.double()[seg] * coef[:, None])
+    kept = place < SEQ
+    grad.index_add_(0, ids[kept], up_t.double().view(segments, SEQ, 4)[seg[kept], place[kept]])
+    rt = RaggedTensor(ids, off, weight)
+    out = engine({"p": rt, "t": rt})
+    if first == "together":
+        torch.autograd.backward([out["p"], out["t"]], [up_p, up_t])
+    else:
+        out["p"].backward(up_p)
+        out["t"].backward(up_t)
+    opt.step()
+    (table,) = engine.hashtables().values()
+    held, rows = table._hashtable_impl.ids_map()
+    slot = table._hashtable_impl.slot_group().slot_by_name("sparse_adagrad_accum")
+    accum = torch.cat(slot.kernel_blocks()[0])[rows].double()
+    # sums of about 50 terms in float32, squared
+    torch.testing.assert_close(accum, grad[held] ** 2, rtol=1e-5, atol=1e-12)
+    assert _lib.poll_device_errors() == 0

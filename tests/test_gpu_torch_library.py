@@ -461,11 +461,12 @@ def test_initialiser_rows_on_device():
 
 def test_config4_shaped_step_through_the_library_boundary():
     """A config-4-shaped step (26 id columns + 13 bucketized float columns on one coalesced table, dim 16,
-    sum pooling of one id per sample, SparseAdam) three ways against the CPU restatement of the reference's
+    sum pooling of one id per sample, SparseAdam) in three ways against the CPU restatement of the reference's
     step: (a) the reference's own call sequence operator by operator (fused_bucketized -> fused_uint64_mod ->
     ids_encode -> ids_partition -> embedding_lookup -> segment_reduce_forward -> segment_reduce_backward ->
-    accept_grad -> step), (b) the fused calls behind the same classes (dense_lookup_expand ->
-    accept_split_grad -> step: one plan, gradient summed where the rows are updated). Each side orders new
+    accept_grad -> step), (b) the fused operators one by one (dense_lookup_expand -> accept_split_grad -> step: one
+    plan, gradient summed where the rows are updated), (c) what the modules call (dense_lookup_train, whose node
+    does the same in autograd's backward). Each side orders new
     keys its own way (the CPU path by np.unique, ids_partition by shard, the plan by hash bucket), so rows start
     from one constant and are compared by key; pooled outputs sample by sample; fp32 within rtol 1e-5 /
     atol 1e-6."""
@@ -473,7 +474,7 @@ def test_config4_shaped_step_through_the_library_boundary():
 
     batch, dim, bs, lr = 2048, 16, 1024, 1e-3
     n_feat = 39
-    # every row starts at the same value: the three sides hand new keys their rows in different orders
+    # every row starts at the same value: the sides hand new keys their rows in different orders
     cpu = cpu_path.CpuTable(dim, bs, lambda b: np.full((bs, dim), 0.05, np.float32), "adam", lr, 1e-8)
 
     def table():
@@ -481,7 +482,7 @@ def test_config4_shaped_step_through_the_library_boundary():
         ht = _make_table(bs, dim, gen, ["f%d" % i for i in range(n_feat)], True)
         return ht, C.SparseAdam.make({"ctr": ht}, lr, 0.9, 0.999, 1e-8, 0.0, False)
 
-    (ht_a, opt_a), (ht_b, opt_b) = table(), table()
+    (ht_a, opt_a), (ht_b, opt_b), (ht_c, opt_c) = table(), table(), table()
     tags = list(range(n_feat))
     offsets = torch.arange(batch * n_feat + 1, dtype=torch.int32, device="cuda")
     rng = np.random.default_rng(44)
@@ -520,11 +521,18 @@ def test_config4_shaped_step_through_the_library_boundary():
         opt_b.step()
         opt_b.zero_grad()
         assert ht_b.pending_grads() == [0, 0]
+        # (c) the modules' call
+        parts = ht_c.dense_lookup_train(cols, tags, None, None)
+        np.testing.assert_allclose(torch.cat([p.detach() for p in parts]).cpu().numpy(), pooled_c, rtol=1e-5, atol=1e-6)
+        torch.autograd.backward(parts, list(g.split(batch)))
+        assert ht_c.pending_grads() == [1, 0]
+        opt_c.step()
+        opt_c.zero_grad()
     keys_c, rows_c = cpu.idmap.snapshot()
     order = np.argsort(keys_c)
     keys_c, rows_c = keys_c[order], rows_c[order]
     want = [np.concatenate(blocks)[rows_c] for blocks in (cpu.emb, cpu.s0, cpu.s1)]
-    for ht in (ht_a, ht_b):
+    for ht in (ht_a, ht_b, ht_c):
         keys, rows = ht.ids_map()
         keys, at = torch.sort(keys)
         np.testing.assert_array_equal(keys.cpu().numpy(), keys_c)
