@@ -494,3 +494,27 @@ def test_columns_of_one_id_in_every_form(rng, kind, combiner):
     one = torch.zeros(9, D, dtype=torch.float64, device="cuda").index_add_(0, plain.view(-1), up.double())
     torch.testing.assert_close(accum.double(), torch.cat([one, one]) ** 2, rtol=1e-5, atol=0)  # sums of up to 20 terms
     assert _lib.poll_device_errors() == 0
+
+
+def test_counts_of_threads():
+    """Threads that plan batches side by side, each on a stream of its own (calls that share a stream share its scratch memory and
+    are queued by one thread at a time): every plan gets its own count."""
+    wrong = []
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for turn in range(12):
+                batches = [rng.integers(0, 20 + int(rng.integers(1, 900)), size=1500) for _ in range(6)]
+                plans = [ops.ids_unique_plan(torch.from_numpy(b).cuda(), wait=False) for b in batches]
+                for k in rng.permutation(6)[: 6 if turn % 2 else 4]:  # some plans go without being asked
+                    if plans[k].U != len(np.unique(batches[k])):
+                        wrong.append((seed, turn, int(k)))
+
+    threads = [threading.Thread(target=work, args=(s,)) for s in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong
+    assert _lib.poll_device_errors() == 0
