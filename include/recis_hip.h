@@ -296,7 +296,7 @@ int recis_idmap_stats(recis_idmap* m, int64_t* live, int64_t* id_num, int64_t* f
  * Synchronises; *count = number of live pairs (only min(count, max_out) written). */
 int recis_idmap_snapshot(recis_idmap* m, int64_t* ids_out, int64_t* index_out, int64_t max_out,
                          int64_t* count, void* stream);
-/* The eviction sweep of a step filter in one pass over the table. Replaces the sequence
+/* The eviction sweep of a step filter, one pass over the table. Replaces the sequence
  * IdMap::SnapShot + block_filter + masked_select + DeleteIds of
  * recis/nn/modules/hashtable_hook_impl.py:487-551 (do_filter / filter) and hashtable.cc:263-278:
  * every live key whose row has stamp < threshold (stamp slot: int32 or int64, one value per row,
@@ -308,6 +308,12 @@ int recis_idmap_evict_older(recis_idmap* m, const void* const* stamp_blocks_dev,
                             int64_t block_rows, int stamp_is64, int64_t threshold,
                             int64_t* ids_out, int64_t* index_out, int64_t max_out, int64_t* count,
                             void* stream);
+/* The same with the threshold worked out on the device: *step_dev (NULL: 0) minus keep_steps, read when the sweep runs. */
+int recis_idmap_evict_unseen(recis_idmap* m, const void* const* stamp_blocks_dev, int64_t n_blocks, int64_t block_rows,
+                             int stamp_is64, const int64_t* step_dev, int64_t keep_steps, int64_t* ids_out,
+                             int64_t* index_out, int64_t max_out, int64_t* count, void* stream);
+/* An upper bound of the live keys without waiting: the last published number and the ids of the calls after it. */
+int recis_idmap_live_bound(recis_idmap* m, int64_t* live_ub);
 /* GpuIdMap::Clear (gpu_id_map.cu:98-103). */
 int recis_idmap_clear(recis_idmap* m, void* stream);
 /* IdMap::Reserve (not implemented for the reference GPU map, gpu_id_map.cu:105-108). */
@@ -398,6 +404,17 @@ int recis_block_gather(const int64_t* ids, void* const* blocks_dev, int64_t n_bl
 int recis_block_insert(const int64_t* ids, const void* emb, int broadcast, const uint8_t* mask,
                        void* const* blocks_dev, int64_t n_blocks, int64_t block_size,
                        int64_t row_pitch_bytes, int64_t n, int64_t row_bytes, void* stream);
+/* Rows ids[0 .. n) of several slots of a table set to one element, a slot each: the rows an eviction frees, whose slots have
+ * constant initialisers (Hashtable::Delete, csrc/embedding/hashtable.cc:263-278). A row outside a slot's blocks sets
+ * the index-range bit. */
+#define RECIS_FILL_ROWS_MAX_SLOTS 8
+typedef struct recis_fill_slot {
+  void* const* blocks_dev;
+  int64_t n_blocks, block_size, row_pitch_bytes, row_bytes;
+  int elem_bytes;             /* 1, 2, 4 or 8 */
+  unsigned char element[8];   /* the first elem_bytes of it */
+} recis_fill_slot;
+int recis_block_fill_rows(const int64_t* ids, int64_t n, const recis_fill_slot* slots, int64_t n_slots, void* stream);
 int recis_block_filter(const int64_t* ids, void* const* blocks_dev, int64_t n_blocks,
                        int64_t block_size, int64_t threshold, int slot_is64, uint8_t* mask_out,
                        int64_t n, void* stream);

@@ -102,6 +102,56 @@ block_insert_kernel(BlockArgs a, const char* __restrict__ emb, int broadcast,
     *reinterpret_cast<Bytes<VB>*>(dst + c) = *reinterpret_cast<const Bytes<VB>*>(src + c);
 }
 
+// Rows of several slots set to one element each: what a constant initialiser gives the rows that an eviction frees. The
+// element travels as an argument (16 bytes of it, repeated), so nothing is materialised or read but the row numbers, and one launch does
+// all slots (grid.y). Bound: one random write request per 128 bytes of row. (A tensor of initial values filled and scattered per slot, six
+// launches for three slots of 32 floats: 70 us for 178 k rows, now 27.)
+struct FillSlot {
+  char* const* blocks;
+  int64_t n_blocks, block_size, pitch_bytes;
+  int row_bytes, vb, lpr_log2;
+  uint32_t element[4];
+};
+struct FillRowsArgs {
+  const int64_t* ids;
+  int64_t n;
+  int* err;
+  FillSlot slot[RECIS_FILL_ROWS_MAX_SLOTS];
+};
+template <int VB>
+__device__ __forceinline__ void fill_row(char* dst, int row_bytes, int cl, int lpr_log2, const uint32_t* element) {
+  Bytes<VB> v;
+  __builtin_memcpy(&v, element, VB);
+  for (int c = cl * VB; c < row_bytes; c += VB << lpr_log2) *reinterpret_cast<Bytes<VB>*>(dst + c) = v;
+}
+__global__ void __launch_bounds__(kBlock)
+block_fill_rows_kernel(FillRowsArgs f) {
+  const FillSlot& s = f.slot[blockIdx.y];  // uniform
+  BlockArgs a;
+  a.blocks = s.blocks;
+  a.n_blocks = s.n_blocks;
+  a.block_size = s.block_size;
+  a.pitch_bytes = s.pitch_bytes;
+  const int rows_per_block = kBlock >> s.lpr_log2;
+  const int cl = threadIdx.x & ((1 << s.lpr_log2) - 1);
+  const uint32_t element[4] = {s.element[0], s.element[1], s.element[2], s.element[3]};
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * rows_per_block + (threadIdx.x >> s.lpr_log2); i < f.n;
+       i += static_cast<int64_t>(gridDim.x) * rows_per_block) {
+    char* dst = row_address(a, f.ids[i]);
+    if (!dst) {
+      raise_device_error(f.err, RECIS_DEVERR_INDEX_RANGE);
+      continue;
+    }
+    switch (s.vb) {  // uniform
+      case 16: fill_row<16>(dst, s.row_bytes, cl, s.lpr_log2, element); break;
+      case 8: fill_row<8>(dst, s.row_bytes, cl, s.lpr_log2, element); break;
+      case 4: fill_row<4>(dst, s.row_bytes, cl, s.lpr_log2, element); break;
+      case 2: fill_row<2>(dst, s.row_bytes, cl, s.lpr_log2, element); break;
+      default: fill_row<1>(dst, s.row_bytes, cl, s.lpr_log2, element); break;
+    }
+  }
+}
+
 // flat table gather: out[i] = emb[ids[i]]
 template <int VB>
 __global__ void __launch_bounds__(kBlock)
@@ -248,6 +298,42 @@ int recis_block_insert(const int64_t* ids, const void* emb, int broadcast, const
     RECIS_LAUNCH_CHECK();
     return RECIS_OK;
   });
+}
+
+int recis_block_fill_rows(const int64_t* ids, int64_t n, const recis_fill_slot* slots, int64_t n_slots, void* stream_) {
+  hipStream_t stream = static_cast<hipStream_t>(stream_);
+  RECIS_REQUIRE(n >= 0 && n_slots >= 0 && n_slots <= RECIS_FILL_ROWS_MAX_SLOTS, "bad sizes");
+  if (n == 0 || n_slots == 0) return RECIS_OK;
+  RECIS_REQUIRE(slots != nullptr, "slots must not be NULL");
+  FillRowsArgs f{};
+  f.ids = ids;
+  f.n = n;
+  f.err = device_error_word(current_device());
+  int64_t grid = 1;
+  for (int64_t k = 0; k < n_slots; ++k) {
+    const recis_fill_slot& in = slots[k];
+    RECIS_REQUIRE((in.elem_bytes == 1 || in.elem_bytes == 2 || in.elem_bytes == 4 || in.elem_bytes == 8) &&
+                      in.row_bytes % in.elem_bytes == 0 && in.row_pitch_bytes % in.elem_bytes == 0,
+                  "slot %lld: rows of %lld bytes of elements of %d", (long long)k, (long long)in.row_bytes, in.elem_bytes);
+    const int vb = pick_vec_bytes(in.row_bytes, static_cast<uintptr_t>(in.row_pitch_bytes));
+    BlockArgs a;
+    if (int rc = fill_args(a, ids, in.blocks_dev, in.n_blocks, in.block_size, in.row_pitch_bytes, n, in.row_bytes, vb)) return rc;
+    FillSlot& out = f.slot[k];
+    out.blocks = a.blocks;
+    out.n_blocks = a.n_blocks;
+    out.block_size = a.block_size;
+    out.pitch_bytes = a.pitch_bytes;
+    out.row_bytes = a.row_bytes;
+    out.vb = vb;
+    out.lpr_log2 = a.lpr_log2;
+    for (int b = 0; b < 16; b += in.elem_bytes) __builtin_memcpy(reinterpret_cast<char*>(out.element) + b, in.element, in.elem_bytes);
+    const int64_t rows_per_block = kBlock >> a.lpr_log2;
+    grid = std::max(grid, std::min<int64_t>((n + rows_per_block - 1) / rows_per_block, 256 * 32));
+  }
+  RECIS_TIME_KERNEL("block_fill_rows_kernel", stream)
+  block_fill_rows_kernel<<<dim3(static_cast<unsigned>(grid), static_cast<unsigned>(n_slots)), dim3(kBlock), 0, stream>>>(f);
+  RECIS_LAUNCH_CHECK();
+  return RECIS_OK;
 }
 
 int recis_block_filter(const int64_t* ids, void* const* blocks_dev, int64_t n_blocks,

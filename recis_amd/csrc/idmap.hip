@@ -256,89 +256,131 @@ erase_kernel(Slot* __restrict__ table, uint64_t mask, const int64_t* __restrict_
               static_cast<unsigned long long>(total));
 }
 
-// Eviction sweep in one pass over the table: every live slot reads the stamp of its row and,
-// when the stamp is older than the threshold, leaves the table (tombstone), hands its row to the
-// free list and reports (key, row) so that the caller can re-initialise the row.
-// The places in the output come from ONE counter, and atomics on one word are served one after the
-// other (some 12 - 25 ns each on this part): with an atomic per 256 slots a sweep over a table of
-// 2^29 slots spent 25 ms on two million of them and a tenth of that on the table. So a workgroup
-// takes kEvictPer * 256 slots per round and one atomic per round: a thread first only notes which
-// of its slots leave (a bit each), the counts are scanned over the workgroup, and the slots that
-// leave are read again (the lines were fetched a moment ago) when their places are known.
-constexpr int kEvictPer = 32;
-__global__ void __launch_bounds__(kBlock)
-evict_older_kernel(Slot* __restrict__ table, int64_t capacity, const void* const* __restrict__ stamp_blocks,
-                   int64_t n_blocks, int64_t block_rows, int stamp64, int64_t threshold,
-                   int64_t* __restrict__ ids_out, int64_t* __restrict__ index_out, int64_t max_out,
-                   int64_t* __restrict__ free_list, int64_t* __restrict__ state, int* err) {
-  __shared__ int wave_counts[kBlock / kWave];
-  __shared__ int64_t s_base;
+// Eviction sweep: every live slot reads the stamp of its row; keys whose stamp is older than the threshold leave the
+// table (tombstone), hand their rows to the free list and are reported as (key, row) so that the caller can re-initialise
+// the rows. Two launches: this one notes which slots leave, a bit each, and how many per workgroup; evict_leave_kernel, which
+// touches nothing else, knows the places in the output from those counts. (With places from one counter a workgroup waits for
+// an atomic that all others want too, 12 - 25 ns apiece, while nothing streams: 70 of 194 us.)
+// Bound: the stream of the slots, 16 bytes each; the stamps are one random request per live key beside it. They overlap
+// only with no branch around a load: a slot without a key reads `state` in place of a stamp. 2^25 slots, 2.3 M keys, 180 k of
+// them leaving: 203 - 240 us with the stamps one at a time and an atomic per 8192 slots, now 117 (4.6 TB/s) + 20.
+constexpr int kEvictBlock = 512;
+constexpr int kEvictPer = 4;         // slots of a thread in flight
+constexpr int kEvictMost = 64;       // slots of a thread: a bit each
+constexpr int64_t kEvictGrid = 1024; // workgroups a small table is spread over
+template <typename TStamp>
+__global__ void __launch_bounds__(kEvictBlock, 8)
+evict_note_kernel(const Slot* __restrict__ table, int64_t capacity, int batches, const void* const* __restrict__ stamp_blocks,
+                  int64_t n_blocks, int64_t block_rows, const int64_t* __restrict__ step, int64_t threshold,
+                  const int64_t* __restrict__ state, uint64_t* __restrict__ leaves_out, int32_t* __restrict__ counts, int* err) {
+  __shared__ int wave_counts[kEvictBlock / kWave];
+  if (step) threshold += *step;
+  const TStamp* nothing = reinterpret_cast<const TStamp*>(state);
+  const TStamp* only = n_blocks > 0 ? static_cast<const TStamp*>(stamp_blocks[0]) : nothing;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kEvictBlock * kEvictPer * batches;
+  uint64_t leaves = 0;
+  bool beyond = false;
+  for (int t = 0; t < batches; ++t) {
+    longlong2 kv[kEvictPer];
+#pragma unroll
+    for (int x = 0; x < kEvictPer; ++x) {
+      const int64_t i = r0 + static_cast<int64_t>(t * kEvictPer + x) * kEvictBlock + threadIdx.x;
+      kv[x] = i < capacity ? *reinterpret_cast<const longlong2*>(&table[i]) : make_longlong2(kEmpty, 0);
+    }
+    const TStamp* at[kEvictPer];
+    uint32_t live = 0;
+#pragma unroll
+    for (int x = 0; x < kEvictPer; ++x) {
+      const int64_t k = kv[x].x, v = kv[x].y;
+      bool has = k != kEmpty && k != kTomb && v >= 0;
+      at[x] = nothing;
+      if (n_blocks == 1) {  // (uniform)
+        beyond = beyond | (has & (v >= block_rows));
+        has = has & (v < block_rows);
+        at[x] = has ? only + v : nothing;
+      } else if (has) {
+        const bool narrow = ((static_cast<uint64_t>(v) | static_cast<uint64_t>(block_rows)) >> 32) == 0;
+        const int64_t b = narrow ? static_cast<uint32_t>(v) / static_cast<uint32_t>(block_rows) : v / block_rows;
+        has = b < n_blocks;
+        beyond = beyond | !has;
+        if (has) at[x] = static_cast<const TStamp*>(stamp_blocks[b]) + (v - b * block_rows);
+      }
+      live |= has ? 1u << x : 0u;
+    }
+    TStamp stamp[kEvictPer];
+#pragma unroll
+    for (int x = 0; x < kEvictPer; ++x) stamp[x] = *at[x];
+    uint32_t old = 0;
+#pragma unroll
+    for (int x = 0; x < kEvictPer; ++x) old |= static_cast<int64_t>(stamp[x]) < threshold ? 1u << x : 0u;
+    leaves |= static_cast<uint64_t>(old & live) << (t * kEvictPer);
+  }
+  if (beyond) raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
+  leaves_out[static_cast<int64_t>(blockIdx.x) * kEvictBlock + threadIdx.x] = leaves;
+  int mine = __popcll(leaves);
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) mine += __shfl_xor(mine, o, kWave);
+  if ((threadIdx.x & (kWave - 1)) == 0) wave_counts[threadIdx.x / kWave] = mine;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int total = 0;
+#pragma unroll
+    for (int w = 0; w < kEvictBlock / kWave; ++w) total += wave_counts[w];
+    counts[blockIdx.x] = total;
+  }
+}
+
+// The slots that evict_note_kernel noted (the same grid) leave; ST_TMP = their number (the last workgroup writes it).
+__global__ void __launch_bounds__(kEvictBlock)
+evict_leave_kernel(Slot* __restrict__ table, int batches, const uint64_t* __restrict__ leaves_in,
+                   const int32_t* __restrict__ counts, int64_t* __restrict__ ids_out, int64_t* __restrict__ index_out,
+                   int64_t max_out, int64_t* __restrict__ free_list, int64_t* __restrict__ state) {
+  __shared__ int64_t wave_before[kEvictBlock / kWave];
+  __shared__ int wave_counts[kEvictBlock / kWave];
+  const bool last = blockIdx.x == gridDim.x - 1;
+  const int here = counts[blockIdx.x];
+  if (here == 0 && !last) return;  // uniform
   const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int64_t per_round = static_cast<int64_t>(kBlock) * kEvictPer;
+  uint64_t leaves = leaves_in[static_cast<int64_t>(blockIdx.x) * kEvictBlock + threadIdx.x];
+  const int mine = __popcll(leaves);
+  int incl = mine;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int y = __shfl_up(incl, o, kWave);
+    if (lane >= o) incl += y;
+  }
+  int64_t earlier = 0;  // noted by the workgroups before
+  for (unsigned g = threadIdx.x; g < blockIdx.x; g += kEvictBlock) earlier += counts[g];
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) earlier += __shfl_xor(earlier, o, kWave);
+  if (lane == kWave - 1) {
+    wave_counts[wave] = incl;
+    wave_before[wave] = earlier;
+  }
+  __syncthreads();
+  int64_t base = 0;
+  int before = incl - mine;
+#pragma unroll
+  for (int w = 0; w < kEvictBlock / kWave; ++w) {
+    base += wave_before[w];
+    if (w < wave) before += wave_counts[w];
+  }
+  if (last && threadIdx.x == 0) state[ST_TMP] = base + here;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * kEvictBlock * kEvictPer * batches;
   const int64_t free_at = state[ST_FREE];  // advanced by the commit kernel, after this one
-  for (int64_t r0 = static_cast<int64_t>(blockIdx.x) * per_round; r0 < capacity;
-       r0 += static_cast<int64_t>(gridDim.x) * per_round) {  // uniform in the workgroup (barriers inside)
-    uint32_t leaves = 0;
-    for (int x0 = 0; x0 < kEvictPer; x0 += 8) {  // eight slots in flight, then their stamps
-      longlong2 kv[8];
-#pragma unroll
-      for (int x = 0; x < 8; ++x) {
-        const int64_t i = r0 + static_cast<int64_t>(x0 + x) * kBlock + threadIdx.x;
-        kv[x] = i < capacity ? *reinterpret_cast<const longlong2*>(&table[i]) : make_longlong2(kEmpty, 0);
-      }
-#pragma unroll
-      for (int x = 0; x < 8; ++x) {
-        const int64_t k = kv[x].x, v = kv[x].y;
-        if (k != kEmpty && k != kTomb && v >= 0) {
-          const int64_t b = v / block_rows, r = v - b * block_rows;
-          if (b < n_blocks) {
-            const int64_t stamp = stamp64 ? static_cast<const int64_t*>(stamp_blocks[b])[r]
-                                          : static_cast<int64_t>(static_cast<const int32_t*>(stamp_blocks[b])[r]);
-            if (stamp < threshold) leaves |= 1u << (x0 + x);
-          } else {
-            raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
-          }
-        }
-      }
+  int64_t pos = base + before;
+  while (leaves) {
+    const int x = __ffsll(static_cast<unsigned long long>(leaves)) - 1;
+    leaves &= leaves - 1;
+    if (pos < max_out) {  // beyond the caller's buffers the key stays (counted, reported by the host)
+      const int64_t i = r0 + static_cast<int64_t>(x) * kEvictBlock + threadIdx.x;
+      const longlong2 kv = *reinterpret_cast<const longlong2*>(&table[i]);
+      ids_out[pos] = kv.x;
+      index_out[pos] = kv.y;
+      free_list[free_at + pos] = kv.y;
+      *reinterpret_cast<longlong2*>(&table[i]) = make_longlong2(kTomb, kValUnset);
     }
-    // exclusive scan of the threads' counts over the workgroup
-    const int mine = __popc(leaves);
-    int incl = mine;
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) {
-      const int y = __shfl_up(incl, o, kWave);
-      if (lane >= o) incl += y;
-    }
-    if (lane == kWave - 1) wave_counts[wave] = incl;
-    __syncthreads();
-    int before = incl - mine, total = 0;
-#pragma unroll
-    for (int w = 0; w < kBlock / kWave; ++w) {
-      if (w < wave) before += wave_counts[w];
-      total += wave_counts[w];
-    }
-    if (threadIdx.x == 0 && total)
-      s_base = static_cast<int64_t>(atomicAdd(reinterpret_cast<unsigned long long*>(&state[ST_TMP]),
-                                              static_cast<unsigned long long>(total)));
-    __syncthreads();
-    if (total) {
-      int64_t pos = s_base + before;
-      while (leaves) {
-        const int x = __ffs(leaves) - 1;
-        leaves &= leaves - 1;
-        const int64_t i = r0 + static_cast<int64_t>(x) * kBlock + threadIdx.x;
-        if (pos < max_out) {  // beyond the caller's buffers the key stays (counted, reported by the host)
-          const longlong2 kv = *reinterpret_cast<const longlong2*>(&table[i]);
-          ids_out[pos] = kv.x;
-          index_out[pos] = kv.y;
-          free_list[free_at + pos] = kv.y;
-          table[i].key = kTomb;
-          table[i].val = kValUnset;
-        }
-        ++pos;
-      }
-    }
-    __syncthreads();  // wave_counts and s_base are reused by the next round
+    ++pos;
   }
 }
 
@@ -492,13 +534,14 @@ int sync_stats(recis_idmap* m, hipStream_t stream, int64_t* words) {
 
 // Upper bounds of occupied slots and of the allocator's high-water mark from the mirror, without
 // waiting: what the last landed publication says plus every id of the calls issued after it.
-void mirror_bounds(recis_idmap* m, int64_t* occ_ub, int64_t* cur_ub) {
-  int64_t seq, occ, cur;
+void mirror_bounds(recis_idmap* m, int64_t* occ_ub, int64_t* cur_ub, int64_t* live_ub = nullptr) {
+  int64_t seq, occ, cur, live;
   do {
     seq = m->mirror[MR_SEQ];
     __atomic_thread_fence(__ATOMIC_ACQUIRE);
     occ = m->mirror[MR_OCC];
     cur = m->mirror[MR_CUR];
+    live = m->mirror[MR_LIVE];
     __atomic_thread_fence(__ATOMIC_ACQUIRE);
   } while (seq != m->mirror[MR_SEQ]);
   while (!m->in_flight.empty() && m->in_flight.front().first <= seq) m->in_flight.pop_front();
@@ -506,6 +549,7 @@ void mirror_bounds(recis_idmap* m, int64_t* occ_ub, int64_t* cur_ub) {
   for (const auto& c : m->in_flight) pending += c.second;
   if (occ_ub) *occ_ub = occ + pending;
   if (cur_ub) *cur_ub = cur + pending;
+  if (live_ub) *live_ub = live + pending;
 }
 
 // After the stream has been drained and `words` read back: the mirror is exact.
@@ -699,6 +743,12 @@ int recis_idmap_settle_call(recis_idmap* m, int64_t seq, int64_t n_true) {
   return RECIS_OK;  // a call whose publication has landed is not in the list any more: nothing to settle
 }
 
+int recis_idmap_live_bound(recis_idmap* m, int64_t* live_ub) {
+  RECIS_REQUIRE(m != nullptr && live_ub != nullptr, "bad arguments");
+  mirror_bounds(m, nullptr, nullptr, live_ub);
+  return RECIS_OK;
+}
+
 int recis_idmap_bounds(recis_idmap* m, int64_t* id_num_ub, int64_t* occupied_ub) {
   RECIS_REQUIRE(m != nullptr, "id map is NULL");
   mirror_bounds(m, occupied_ub, id_num_ub);
@@ -767,6 +817,13 @@ int recis_idmap_snapshot(recis_idmap* m, int64_t* ids_out, int64_t* index_out, i
 int recis_idmap_evict_older(recis_idmap* m, const void* const* stamp_blocks_dev, int64_t n_blocks,
                             int64_t block_rows, int stamp_is64, int64_t threshold, int64_t* ids_out,
                             int64_t* index_out, int64_t max_out, int64_t* count, void* stream_) {
+  return recis_idmap_evict_unseen(m, stamp_blocks_dev, n_blocks, block_rows, stamp_is64, nullptr, -threshold, ids_out,
+                                  index_out, max_out, count, stream_);
+}
+
+int recis_idmap_evict_unseen(recis_idmap* m, const void* const* stamp_blocks_dev, int64_t n_blocks, int64_t block_rows,
+                             int stamp_is64, const int64_t* step_dev, int64_t keep_steps, int64_t* ids_out,
+                             int64_t* index_out, int64_t max_out, int64_t* count, void* stream_) {
   hipStream_t stream = static_cast<hipStream_t>(stream_);
   RECIS_REQUIRE(m != nullptr && count != nullptr, "id map / count is NULL");
   RECIS_REQUIRE(stamp_blocks_dev != nullptr && n_blocks >= 0 && block_rows > 0, "bad stamp blocks");
@@ -776,10 +833,26 @@ int recis_idmap_evict_older(recis_idmap* m, const void* const* stamp_blocks_dev,
   int* err = device_error_word(current_device());
   RECIS_REQUIRE(err != nullptr, "could not reach the device error word");
   if (int rc = ensure_free_room(m, max_out, stream)) return rc;
-  const int64_t rounds = (m->capacity + static_cast<int64_t>(kBlock) * kEvictPer - 1) / (static_cast<int64_t>(kBlock) * kEvictPer);
-  evict_older_kernel<<<dim3(static_cast<unsigned>(std::min<int64_t>(rounds, 256 * 16))), dim3(kBlock), 0, stream>>>(
-      m->table, m->capacity, stamp_blocks_dev, n_blocks, block_rows, stamp_is64, threshold, ids_out, index_out,
-      max_out, m->free_list, m->state, err);
+  const int64_t per_batch = static_cast<int64_t>(kEvictBlock) * kEvictPer;
+  const int64_t batches = std::max<int64_t>(1, std::min<int64_t>(kEvictMost / kEvictPer, m->capacity / (per_batch * kEvictGrid)));
+  const int64_t rounds = (m->capacity + per_batch * batches - 1) / (per_batch * batches);
+  RECIS_REQUIRE(rounds <= INT32_MAX, "a table of %lld slots", (long long)m->capacity);
+  void* ws = nullptr;
+  if (int rc = get_workspace(stream, (sizeof(uint64_t) * kEvictBlock + sizeof(int32_t)) * static_cast<size_t>(rounds), &ws)) return rc;
+  uint64_t* leaves = static_cast<uint64_t*>(ws);
+  int32_t* counts = reinterpret_cast<int32_t*>(leaves + rounds * kEvictBlock);
+  const dim3 grid(static_cast<unsigned>(rounds)), block(kEvictBlock);
+  auto note = [&](auto kernel) {
+    kernel<<<grid, block, 0, stream>>>(m->table, m->capacity, static_cast<int>(batches), stamp_blocks_dev, n_blocks, block_rows,
+                                       step_dev, -keep_steps, m->state, leaves, counts, err);
+  };
+  if (stamp_is64)
+    note(evict_note_kernel<int64_t>);
+  else
+    note(evict_note_kernel<int32_t>);
+  RECIS_LAUNCH_CHECK();
+  evict_leave_kernel<<<grid, block, 0, stream>>>(m->table, static_cast<int>(batches), leaves, counts, ids_out, index_out,
+                                                 max_out, m->free_list, m->state);
   RECIS_LAUNCH_CHECK();
   evict_commit_kernel<<<1, 1, 0, stream>>>(m->state, max_out);
   RECIS_LAUNCH_CHECK();

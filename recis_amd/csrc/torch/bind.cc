@@ -206,6 +206,7 @@ TORCH_LIBRARY(recis, m) {
       .def("accept_grad_ex", &Hashtable::AcceptGradEx)
       .def("accept_planned_grad", &Hashtable::AcceptPlannedGrad)
       .def("evict_older", &Hashtable::EvictOlder)
+      .def("evict_unseen", &Hashtable::EvictUnseen)
       .def("id_map_stats", &Hashtable::IdMapStats)
       .def("pending_grads", &Hashtable::PendingGrads)
       .def("id_map_handle", [](const HashTablePtr& self) { return reinterpret_cast<int64_t>(self->id_map()); });

@@ -4,6 +4,7 @@
 
 #include <cmath>
 #include <cstdlib>
+#include <cstring>
 #include <set>
 
 #include "abi_util.h"
@@ -121,6 +122,20 @@ void Generator::Fill(at::Tensor& t, const std::vector<int64_t>& fan_shape) {
       return;
     }
   }
+}
+
+int Generator::ConstantElement(at::ScalarType dtype, unsigned char* bytes) const {
+  if (kind_ != Kind::kConstant || options_.dtype() != dtype || c10::isComplexType(dtype)) return 0;
+  at::Tensor one = at::empty({1}, at::TensorOptions().dtype(dtype));
+  if (at::isIntegralType(dtype, true)) {
+    one.fill_(static_cast<int64_t>(p0_));
+  } else {
+    one.fill_(p0_);
+  }
+  const int size = static_cast<int>(one.element_size());
+  if (size > 8) return 0;
+  std::memcpy(bytes, one.data_ptr(), size);
+  return size;
 }
 
 GeneratorPtr MakeConstantGenerator(const std::vector<int64_t>& shape, at::ScalarType dtype, double init_val) {
@@ -698,39 +713,69 @@ void Hashtable::Delete(const at::Tensor& ids, const at::Tensor& index, const std
   at::Tensor i = OnDevice(ids).view({-1}), x = OnDevice(index).view({-1});
   TORCH_CHECK(i.numel() == x.numel(), "ids and index differ in length");
   check(recis_idmap_erase(map_->map, i.data_ptr<int64_t>(), x.data_ptr<int64_t>(), i.numel(), stream_of(device_)));
-  const int64_t keep = preserve_slot.empty() ? -1 : slot_group_->GetSlotIndex(preserve_slot);
+  ReinitRows(x, preserve_slot.empty() ? -1 : slot_group_->GetSlotIndex(preserve_slot));
+}
+
+// Constant slots (the optimizers' state, and rows that start at zero) in one launch; the others draw a tensor of new rows each,
+// in the order of the slots, which is the order in which they take from their random number generators.
+void Hashtable::ReinitRows(const at::Tensor& index, int64_t keep) {
+  const int64_t n = index.numel();
   auto slots = slot_group_->Slots();
+  std::vector<recis_fill_slot> fills;
+  std::vector<at::Tensor> tables;  // alive until the launch is queued
+  auto flush = [&]() {
+    check(recis_block_fill_rows(index.data_ptr<int64_t>(), n, fills.data(), static_cast<int64_t>(fills.size()), stream_of(device_)));
+    fills.clear();
+  };
   for (int64_t s = 0; s < static_cast<int64_t>(slots.size()); ++s) {
-    if (s != keep) slots[s]->IndexInsert(x, slots[s]->GenVal(i.numel()));
+    if (s == keep) continue;
+    const auto& chunks = slots[s]->Chunks();
+    recis_fill_slot f{};
+    f.elem_bytes = chunks.empty() ? 0 : slots[s]->ConstantElement(f.element);
+    if (f.elem_bytes == 0) {
+      slots[s]->IndexInsert(index, slots[s]->GenVal(n));
+      continue;
+    }
+    tables.push_back(block_ptr_table(chunks));
+    f.blocks_dev = reinterpret_cast<void* const*>(tables.back().data_ptr());
+    f.n_blocks = static_cast<int64_t>(chunks.size());
+    f.block_size = slots[s]->ChunkRows();
+    f.row_pitch_bytes = recis::hipabi::row_pitch_bytes(chunks[0]);
+    f.row_bytes = slots[s]->FlatSize() * static_cast<int64_t>(chunks[0].element_size());
+    fills.push_back(f);
+    if (fills.size() == RECIS_FILL_ROWS_MAX_SLOTS) flush();
   }
+  flush();
 }
 
 std::tuple<at::Tensor, at::Tensor> Hashtable::EvictOlder(const std::string& stamp_slot, int64_t threshold) {
+  return EvictUnseen(stamp_slot, c10::nullopt, -threshold);
+}
+
+std::tuple<at::Tensor, at::Tensor> Hashtable::EvictUnseen(const std::string& stamp_slot, const c10::optional<at::Tensor>& step,
+                                                          int64_t keep_steps) {
   c10::DeviceGuard guard(device_);
   auto stamps = slot_group_->GetSlotByName(stamp_slot);
   TORCH_CHECK((stamps->Dtype() == at::kLong || stamps->Dtype() == at::kInt) && stamps->FlatSize() == 1,
               "the stamp slot must be int32/int64 of width 1");
+  const bool on_device = step.has_value() && step->defined();
+  TORCH_CHECK(!on_device || (step->device() == device_ && step->scalar_type() == at::kLong && step->numel() == 1),
+              "the step must be one int64 on the table's device");
   void* stream = stream_of(device_);
   int64_t live = 0, count = 0;
-  check(recis_idmap_stats(map_->map, &live, nullptr, nullptr, nullptr, stream));
+  check(recis_idmap_live_bound(map_->map, &live));
   auto opt = at::TensorOptions().device(device_).dtype(at::kLong);
   at::Tensor ids = at::empty({live}, opt), index = at::empty({live}, opt);
   if (!stamps->Chunks().empty()) {
     at::Tensor tab = block_ptr_table(stamps->Chunks());
-    check(recis_idmap_evict_older(map_->map, reinterpret_cast<const void* const*>(tab.data_ptr()),
-                                  static_cast<int64_t>(stamps->Chunks().size()), stamps->ChunkRows(),
-                                  stamps->Dtype() == at::kLong ? 1 : 0, threshold, ids.data_ptr<int64_t>(),
-                                  index.data_ptr<int64_t>(), live, &count, stream));
+    check(recis_idmap_evict_unseen(map_->map, reinterpret_cast<const void* const*>(tab.data_ptr()),
+                                   static_cast<int64_t>(stamps->Chunks().size()), stamps->ChunkRows(),
+                                   stamps->Dtype() == at::kLong ? 1 : 0, on_device ? step->data_ptr<int64_t>() : nullptr,
+                                   keep_steps, ids.data_ptr<int64_t>(), index.data_ptr<int64_t>(), live, &count, stream));
   }
   ids = ids.narrow(0, 0, count);
   index = index.narrow(0, 0, count);
-  if (count) {
-    const int64_t keep = slot_group_->GetSlotIndex(stamp_slot);
-    auto slots = slot_group_->Slots();
-    for (int64_t s = 0; s < static_cast<int64_t>(slots.size()); ++s) {
-      if (s != keep) slots[s]->IndexInsert(index, slots[s]->GenVal(count));
-    }
-  }
+  if (count) ReinitRows(index, slot_group_->GetSlotIndex(stamp_slot));
   return std::make_tuple(ids, index);
 }
 

@@ -37,6 +37,8 @@ class Generator : public torch::CustomClassHolder {
   const std::vector<int64_t>& Shape() const { return shape_; }
   at::TensorOptions TensorOption() const { return options_; }
   static at::Tensor DoGenerator(c10::intrusive_ptr<Generator> g) { return g->Generate(); }
+  // The one element of a constant initialiser as it lies in memory (`bytes`, at most 8); 0: not constant.
+  int ConstantElement(at::ScalarType dtype, unsigned char* bytes) const;
   // kFromTensor: the rows are handed out from `source`, in order, starting over at its end.
   void SetSource(at::Tensor source) { source_ = std::move(source); }
 
@@ -124,6 +126,7 @@ class Slot : public torch::CustomClassHolder {
   void IndexInsert(const at::Tensor& index, at::Tensor value);
   void IndexInsert(const at::Tensor& index, at::Tensor value, const at::Tensor& accept_indicator);
   at::Tensor GenVal(int64_t rows);
+  int ConstantElement(unsigned char* bytes) const { return generator_->ConstantElement(dtype_, bytes); }
   // what the row kernels take as (blocks, block_size)
   const std::vector<at::Tensor>& Chunks() const { return chunks_; }
   int64_t ChunkRows() const { return chunk_rows_; }
@@ -372,6 +375,11 @@ class Hashtable : public torch::CustomClassHolder {
   // Eviction sweep in one pass over the map: erase every key whose row has stamp_slot < threshold,
   // free the rows, re-initialise every other slot there; returns the evicted (ids, index).
   std::tuple<at::Tensor, at::Tensor> EvictOlder(const std::string& stamp_slot, int64_t threshold);
+  // The same with threshold = *step - keep_steps, the step read on the device when the sweep runs.
+  std::tuple<at::Tensor, at::Tensor> EvictUnseen(const std::string& stamp_slot, const c10::optional<at::Tensor>& step,
+                                                 int64_t keep_steps);
+  // Initial values again in every slot but `keep` (-1: in all) at rows whose keys have left.
+  void ReinitRows(const at::Tensor& index, int64_t keep);
   // (live keys, allocator high-water mark, free-list length, slot capacity); waits for the stream
   std::vector<int64_t> IdMapStats();
   recis_idmap* id_map() const { return map_->map; }

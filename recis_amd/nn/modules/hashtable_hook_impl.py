@@ -113,12 +113,15 @@ class GlobalStepFilterHookImpl(BaseFilterHookImpl):
 
     def _threshold(self) -> int:
         # the counter lives on the device (it is part of the checkpoint and may be loaded or reset
-        # behind this object's back); it is read back only here, when a sweep runs
+        # behind this object's back); it is read back only here
         return int(self._global_step.item()) - self._filter_step
 
     def do_filter(self) -> None:
-        # one pass over the id map instead of snapshot + filter + delete
-        self._ht.evict_older(self._name, self._threshold())
+        # one pass over the id map instead of snapshot + filter + delete; the sweep reads the step on the device
+        if self._global_step.is_cuda and self._global_step.dtype == torch.int64:
+            self._ht.evict_unseen(self._name, self._global_step, self._filter_step)
+        else:
+            self._ht.evict_older(self._name, self._threshold())
 
     def filter(self, ids, index):
         slot = self._ht.get_slot(self._name)

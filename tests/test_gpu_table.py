@@ -270,6 +270,60 @@ def test_evict_older_equals_snapshot_filter_erase(rng, dt):
     assert _lib.poll_device_errors() == 0
 
 
+@pytest.mark.parametrize("reserve,n_blocks,dt", [(300_000, 1, torch.int64), (300_000, 3, torch.int32),
+                                                 (2_000_000, 1, torch.int32), (2_000_000, 3, torch.int64)])
+def test_evict_older_of_small_and_large_tables(rng, reserve, n_blocks, dt):
+    """A thread of the sweep takes four slots of a table of 2^20 and eight of 2^22; a row beyond the blocks keeps its key and
+    is reported."""
+    n = 9000
+    m = ops.IdMap(reserve=reserve)
+    assert m.stats()[3] == (1 << 20 if reserve == 300_000 else 1 << 22)
+    keys = np.unique(rng.integers(-10**15, 10**15, size=n))
+    rows = m.lookup(_dev(keys)).cpu().numpy()
+    bs = -(-(keys.size - 100) // n_blocks)  # the last rows lie beyond
+    held = bs * n_blocks
+    stamps = rng.integers(0, 100, size=held)
+    blocks = [torch.from_numpy(stamps[i * bs:(i + 1) * bs].reshape(bs, 1)).cuda().to(dt) for i in range(n_blocks)]
+    gone_ids, gone_rows = m.evict_older(blocks, bs, 37)
+    expect = np.zeros(keys.size, bool)
+    expect[rows < held] = stamps[rows[rows < held]] < 37
+    order = np.argsort(gone_ids.cpu().numpy())
+    np.testing.assert_array_equal(gone_ids.cpu().numpy()[order], keys[expect])
+    np.testing.assert_array_equal(gone_rows.cpu().numpy()[order], rows[expect])
+    np.testing.assert_array_equal(m.lookup_readonly(_dev(keys)).cpu().numpy(), np.where(expect, -1, rows))
+    assert _lib.poll_device_errors() == 1  # RECIS_DEVERR_INDEX_RANGE
+
+
+@pytest.mark.parametrize("dim,dtype", [(1, torch.float32), (3, torch.bfloat16), (10, torch.float32), (300, torch.float32)])
+def test_rows_of_deleted_keys_start_over(dim, dtype):
+    """Slots with a constant initialiser are set in one launch, the others get new rows; the preserved slot keeps its own."""
+    from recis_amd.nn import HashTable
+    from recis_amd.nn.initializers import ConstantInitializer
+    from recis_amd.nn.modules.hashtable import HashtableRegister
+
+    HashtableRegister().clear()
+    t = HashTable([dim], block_size=512, dtype=dtype, name="startover", children=["startover"],
+                  initializer=ConstantInitializer(init_val=0.3))._hashtable_impl
+    group = t.slot_group()
+    t.append_step_filter_slot("seen", 7)
+    keys = torch.arange(1500, device="cuda") * 3 + 1
+    t.insert(keys, torch.randn(1500, dim, device="cuda").to(dtype))
+    ids, index = t.ids_map()
+    for slot in group.slots():
+        if slot.name() == "seen":
+            t.update_slot("seen", index, torch.full((1500, 1), 9, dtype=torch.int64, device="cuda"))
+    before = {s.name(): [b.clone() for b in s.kernel_blocks()[0]] for s in group.slots()}
+    out = ids % 2 == 0
+    t.delete(ids[out], index[out], "seen")
+    for slot in group.slots():
+        for was, now in zip(before[slot.name()], slot.kernel_blocks()[0]):
+            want = was.clone()
+            if slot.name() != "seen":
+                want[index[out]] = torch.full((1,), 0.3).to(want.dtype).cuda()
+            assert torch.equal(now, want)
+    assert _lib.poll_device_errors() == 0
+
+
 # ------------------------------------------------------------------ optimizers
 def _np_blocks(w, bs):
     nb = (w.shape[0] + bs - 1) // bs
