@@ -118,11 +118,38 @@ struct RowPlaces {
   T* s0;
   T* s1;
 };
+// The first block of every slot: of a table with one block per slot, the usual case, all there is to ask for. Loaded at the top
+// of a kernel (scalar registers), so that the addresses of a row do not wait for a second load behind its row number. (FIRST
+// false: not used. The kernels with one input that work their long lists through shuffles spill with it; the others know the places
+// early anyway.)
+template <typename T>
+struct FirstBlocks {
+  T *w = nullptr, *s0 = nullptr, *s1 = nullptr;
+};
 template <typename T, int EPI>
-__device__ __forceinline__ RowPlaces<T> row_places(const FuseArgs& f, int* err, int64_t idx) {
+__device__ __forceinline__ FirstBlocks<T> first_blocks(const FuseArgs& f) {
+  FirstBlocks<T> b;
+  b.w = static_cast<T*>(f.emb[0]);
+  b.s0 = static_cast<T*>(f.s0[0]);
+  if constexpr (epi_is_adam(EPI)) b.s1 = static_cast<T*>(f.s1[0]);
+  return b;
+}
+template <typename T, int EPI, bool FIRST>
+__device__ __forceinline__ RowPlaces<T> row_places(const FuseArgs& f, const FirstBlocks<T>& first, int* err, int64_t idx) {
   RowPlaces<T> p{nullptr, nullptr, nullptr};
   int64_t b, off;
   if (idx < 0) return p;
+  if (FIRST && f.rb.n_blocks == 1) {  // uniform
+    if (idx >= f.rb.block_size) {
+      raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
+      return p;
+    }
+    const int64_t at = idx * f.rb.pitch;
+    p.w = first.w + at;
+    p.s0 = first.s0 + at;
+    if constexpr (epi_is_adam(EPI)) p.s1 = first.s1 + at;
+    return p;
+  }
   if (!block_row(f.rb, idx, b, off)) {
     raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
     return p;
@@ -145,14 +172,42 @@ __device__ __forceinline__ void fused_row_update_at(const FuseArgs& f, const Row
   }
 }
 
+// The same in two steps, for a caller that has registers to ask for the table's packs before the gradient is summed.
+template <typename T, int VEC>
+struct TablePacks {
+  Pack<T, VEC> w, s0, s1;
+};
+template <typename T, int VEC, int EPI>
+__device__ __forceinline__ TablePacks<T, VEC> load_table_packs(const RowPlaces<T>& p, int c0, bool have, const T* zero_row) {
+  constexpr bool kStream = EPI == kEpiAdam;
+  TablePacks<T, VEC> t;
+  t.w = load_row_pack_of_table<T, VEC, kStream>(have ? p.w + c0 : zero_row);
+  t.s0 = load_row_pack_of_table<T, VEC, kStream>(have ? p.s0 + c0 : zero_row);
+  if constexpr (epi_is_adam(EPI)) t.s1 = load_row_pack_of_table<T, VEC, kStream>(have ? p.s1 + c0 : zero_row);
+  return t;
+}
+template <typename T, int VEC, int EPI>
+__device__ __forceinline__ void update_table_packs(const FuseArgs& f, const RowPlaces<T>& p, int c0, TablePacks<T, VEC>& t,
+                                                   const float (&acc)[VEC], double alpha) {
+  constexpr bool kStream = EPI == kEpiAdam;
+  if constexpr (epi_is_adam(EPI)) {
+    adam_compute_pack<T, VEC>(t.w, t.s0, t.s1, acc, alpha, f.adam);
+    store_row_pack_of_table<T, VEC, kStream>(p.s1 + c0, t.s1);
+  } else {
+    adagrad_compute_pack<T, VEC>(t.w, t.s0, acc, f.lr, f.eps);
+  }
+  store_row_pack_of_table<T, VEC, kStream>(p.w + c0, t.w);
+  store_row_pack_of_table<T, VEC, kStream>(p.s0 + c0, t.s0);
+}
+
 // The epilogue of one pack of one finished row; T = the table's row type for the optimizer kinds.
 // idx = row_index[u] of the finished row (callers load it early: it heads a chain of dependent
 // accesses); alpha: of this step (Adam only).
-template <typename T, int VEC, int EPI>
-__device__ __forceinline__ void fused_row_update(const FuseArgs& f, int* err, int64_t idx, int c0,
-                                                 const float (&acc)[VEC], double alpha) {
+template <typename T, int VEC, int EPI, bool FIRST>
+__device__ __forceinline__ void fused_row_update(const FuseArgs& f, const FirstBlocks<T>& first, int* err, int64_t idx,
+                                                 int c0, const float (&acc)[VEC], double alpha) {
   // (a key the table does not hold, idx < 0, takes no gradient)
-  fused_row_update_at<T, VEC, EPI>(f, row_places<T, EPI>(f, err, idx), c0, acc, alpha);
+  fused_row_update_at<T, VEC, EPI>(f, row_places<T, EPI, FIRST>(f, first, err, idx), c0, acc, alpha);
 }
 
 
@@ -203,86 +258,135 @@ __device__ __forceinline__ void cover_range(const CsrArgs& a, int64_t& lo, int64
   }
 }
 
-// A whole wave works the list entries [e_begin, e_end) (uniform arguments, every lane calls):
-// `src` and `coef` of 64 entries come from one coalesced load, a lane each, and reach the lanes
-// that gather the rows through shuffles; lane group g of `groups` takes entries g, g + groups,
-// ... with several row loads in flight. acc: this group's partial sum for columns
-// c0 .. c0 + VEC (the caller folds the groups).
-template <typename TIn, int VEC, bool PARTS, bool NT>
-__device__ __forceinline__ void wave_gather_range_nt(const SrcView<TIn>& s, const CsrArgs& a, int32_t e_begin,
-                                                     int32_t e_end, int c0, bool col_ok, int g, int groups,
-                                                     float (&acc)[VEC]) {
-  constexpr int kFly = 4;  // row loads in flight per lane, all of them at once (no branches below)
-  const int lane = threadIdx.x & (kWave - 1);
-  const TIn* zero_row = reinterpret_cast<const TIn*>(g_csr_zero_row);
-  const int64_t zero_at = PARTS ? 0 : zero_row - s.rows;  // the row of zeros as an offset from the input
-  bool beyond = false;
-  for (int32_t cb = e_begin; cb < e_end; cb += kWave) {
-    const int n_here = min(kWave, e_end - cb);
-    // the row this lane's entry reads (none: -1 / NULL). With parts, where it lies is worked out once
-    // per entry, here, not by every lane that gathers it, and the address travels to those lanes.
-    int32_t s_mine = -1;
-    const TIn* p_mine = nullptr;
-    float w_mine = 0.f;
-    if (lane < n_here) {
-      const int32_t sv = s.src[cb + lane];
-      if (sv >= s.lo && sv < s.hi) {
-        s_mine = sv;
-        if constexpr (PARTS) p_mine = src_row<TIn, true>(s.rows, a, sv);
-        w_mine = s.coef ? load_coef(s.coef, s.coef_dt, cb + lane) : 1.0f;
-      } else {
-        beyond = beyond | (static_cast<int64_t>(sv) >= s.n_rows);
-      }
-    }
-    for (int q0 = 0; q0 < n_here; q0 += kFly * groups) {  // same trip count for the whole wave (shuffles inside)
-      float v[kFly][VEC];
-      float w[kFly];
-#pragma unroll
-      for (int k = 0; k < kFly; ++k) {  // no branches in here: see g_csr_zero_row
-        const int first = q0 + k * groups;  // this round's entries: first + 0 .. first + groups - 1, one per group
-        const int e = first + g;
-        const int from = min(e, kWave - 1);
-        const bool in_round = (e < n_here) & col_ok;
-        const float w_got = s.coef ? __shfl(w_mine, from, kWave) : 1.0f;  // every lane takes part in the shuffle
-        const TIn* row;
-        if constexpr (PARTS) {
-          const uintptr_t bits = reinterpret_cast<uintptr_t>(p_mine);
-          const uint32_t p_lo = __shfl(static_cast<uint32_t>(bits), from, kWave);
-          const uint32_t p_hi = __shfl(static_cast<uint32_t>(bits >> 32), from, kWave);
-          const uintptr_t got = (static_cast<uintptr_t>(p_hi) << 32) | p_lo;
-          const bool have = in_round & (got != 0);
-          row = have ? reinterpret_cast<const TIn*>(got) + c0 : zero_row;
-          w[k] = have ? w_got : 0.f;
-        } else {
-          const int32_t id = __shfl(s_mine, from, kWave);
-          const bool have = in_round & (id >= 0);
-          row = s.rows + (have ? static_cast<int64_t>(id) * a.D + c0 : zero_at);
-          w[k] = have ? w_got : 0.f;
-        }
-        if constexpr (NT) {
-          load_pack_stream<TIn, VEC>(row, v[k]);
-        } else {
-          load_pack<TIn, VEC>(row, v[k]);
-        }
-      }
-#pragma unroll
-      for (int k = 0; k < kFly; ++k) {
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) acc[j] = fmaf(v[k][j], w[k], acc[j]);
-      }
-    }
+// A pack of a gathered row as it was loaded: converted when it is added, so that rows in flight cost the registers of their own
+// type (eight rows of eight bfloat16 as floats: 146 registers instead of 117).
+template <typename T, int VEC, bool NT>
+__device__ __forceinline__ Pack<T, VEC> load_raw_pack(const T* p) {
+  if constexpr (NT && sizeof(T) * VEC == 16) {
+    typedef uint32_t u4 __attribute__((ext_vector_type(4)));
+    const u4 raw = __builtin_nontemporal_load(reinterpret_cast<const u4*>(p));
+    Pack<T, VEC> pk;
+    __builtin_memcpy(&pk, &raw, 16);
+    return pk;
+  } else {
+    return *reinterpret_cast<const Pack<T, VEC>*>(p);
   }
+}
+template <typename T, int VEC>
+__device__ __forceinline__ void add_pack(const Pack<T, VEC>& v, float w, float (&acc)[VEC]) {
+#pragma unroll
+  for (int j = 0; j < VEC; ++j) acc[j] = fmaf(to_float(v.v[j]), w, acc[j]);
+}
+
+// One list entry as a lane holds it: where its row lies (a row of zeros where there is nothing to add) and its factor. The lane that
+// holds the entry works the address out, so that the lanes that gather the row only add their column (these kernels spend more
+// of their time on instructions than on waiting: 2 x 1.5 M rows of 128 bfloat16: 70 M vector instructions and 178 us
+// with the row number handed round and tested in every lane, now 59 M and 164 us).
+template <typename T>
+struct ListEntry {
+  const T* p;
+  float w;
+};
+template <typename T, bool PARTS>
+__device__ __forceinline__ ListEntry<T> load_entry(const SrcView<T>& in, const CsrArgs& a, int32_t k, bool have, bool& beyond) {
+  int32_t sv = 0;
+  float w = 1.0f;
+  if (have) {
+    sv = in.src[k];
+    if (in.coef) w = load_coef(in.coef, in.coef_dt, k);
+  }
+  const bool inside = have & (sv >= in.lo) & (sv < in.hi);
+  beyond = beyond | (have & !inside & (static_cast<int64_t>(sv) >= in.n_rows));
+  ListEntry<T> e;
+  const T* at = src_row<T, PARTS>(in.rows, a, inside ? sv : 0);
+  e.p = inside ? at : reinterpret_cast<const T*>(g_csr_zero_row);
+  e.w = inside ? w : 0.f;
+  return e;
+}
+__device__ __forceinline__ uint32_t from_lane(uint32_t v, int lane_x4) {
+  return static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(lane_x4, static_cast<int>(v)));
+}
+// The pack at column c0 of the row of lane `lane_x4` / 4's entry, and its factor (1 for inputs without factors: a row of
+// zeros adds nothing). Every lane of the wave calls.
+template <typename T, int VEC, bool NT>
+__device__ __forceinline__ Pack<T, VEC> load_row_of(const SrcView<T>& in, const ListEntry<T>& mine, int lane_x4, int c0, float& w) {
+  const uintptr_t bits = reinterpret_cast<uintptr_t>(mine.p);
+  const uint32_t lo = from_lane(static_cast<uint32_t>(bits), lane_x4), hi = from_lane(static_cast<uint32_t>(bits >> 32), lane_x4);
+  w = in.coef ? __uint_as_float(from_lane(__float_as_uint(mine.w), lane_x4)) : 1.0f;  // uniform
+  return load_raw_pack<T, VEC, NT>(reinterpret_cast<const T*>((static_cast<uintptr_t>(hi) << 32) | lo) + c0);
+}
+
+// A whole wave sums the rows of up to 64 list entries, a lane each (`mine`): lane group g of `groups` takes entries g, g +
+// groups, ... with FLY row loads in flight at once. acc: this group's partial sum for columns c0 .. c0 + VEC (the caller
+// folds the groups; c0 is a column of the row in every lane, also in those that have none to sum).
+template <typename T, int VEC, bool NT, int FLY>
+__device__ __forceinline__ void wave_gather_entries(const SrcView<T>& s, const ListEntry<T>& mine, int n_here, int c0, int g,
+                                                    int groups, float (&acc)[VEC]) {
+  static_assert(FLY == 4 || FLY == 8, "a turn of FLY entries for each of up to eight groups divides the 64 of a wave");
+  for (int q0 = 0; q0 < n_here; q0 += FLY * groups) {  // same trip count for the whole wave (shuffles inside)
+    Pack<T, VEC> v[FLY];
+    float w[FLY];
+#pragma unroll
+    for (int k = 0; k < FLY; ++k)  // no branches in here: see g_csr_zero_row
+      v[k] = load_row_of<T, VEC, NT>(s, mine, (q0 + k * groups + g) * 4, c0, w[k]);
+    __builtin_amdgcn_sched_barrier(0);  // all loads first
+#pragma unroll
+    for (int k = 0; k < FLY; ++k) add_pack<T, VEC>(v[k], w[k], acc);
+  }
+}
+// The same over the list entries [e_begin, e_end) (uniform arguments, every lane calls), 64 at a time. AHEAD: the next 64 are
+// asked for before the rows of these.
+template <typename T, int VEC, bool PARTS, int FLY, bool AHEAD>
+__device__ __forceinline__ void wave_gather_range(const SrcView<T>& s, const CsrArgs& a, int32_t e_begin, int32_t e_end, int c0,
+                                                  int g, int groups, float (&acc)[VEC]) {
+  const int lane = threadIdx.x & (kWave - 1);
+  bool beyond = false;
+  auto run = [&](auto nt_tag) {
+    ListEntry<T> mine{};
+    if constexpr (AHEAD) mine = load_entry<T, PARTS>(s, a, e_begin + lane, e_begin + lane < e_end, beyond);
+    for (int32_t cb = e_begin; cb < e_end; cb += kWave) {
+      const int32_t k = cb + lane + (AHEAD ? kWave : 0);
+      const ListEntry<T> next = load_entry<T, PARTS>(s, a, k, k < e_end, beyond);
+      if constexpr (!AHEAD) mine = next;
+      wave_gather_entries<T, VEC, decltype(nt_tag)::value, FLY>(s, mine, min(kWave, e_end - cb), c0, g, groups, acc);
+      if constexpr (AHEAD) mine = next;
+    }
+  };
+  if (s.nt)  // uniform; picked here, outside the loops
+    run(std::true_type{});
+  else
+    run(std::false_type{});
   if (beyond) raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
 }
-template <typename TIn, int VEC, bool PARTS>
-__device__ __forceinline__ void wave_gather_range(const SrcView<TIn>& s, const CsrArgs& a, int32_t e_begin,
-                                                  int32_t e_end, int c0, bool col_ok, int g, int groups,
-                                                  float (&acc)[VEC]) {
-  if (s.nt) {  // uniform; picked here, outside the loops
-    wave_gather_range_nt<TIn, VEC, PARTS, true>(s, a, e_begin, e_end, c0, col_ok, g, groups, acc);
-  } else {
-    wave_gather_range_nt<TIn, VEC, PARTS, false>(s, a, e_begin, e_end, c0, col_ok, g, groups, acc);
-  }
+// Up to 64 entries [first, last), a row of either input each: both inputs' entries are asked for together.
+template <typename T1, typename T2, int VEC, bool PARTS, int FLY>
+__device__ __forceinline__ void wave_gather_two(const SrcView<T1>& in1, const SrcView<T2>& in2, const CsrArgs& a, int32_t first,
+                                                int32_t last, int c0, int g, int groups, float (&acc)[VEC]) {
+  const int32_t k = first + static_cast<int32_t>(threadIdx.x & (kWave - 1));
+  bool beyond = false;
+  const auto e1 = load_entry<T1, false>(in1, a, k, k < last, beyond);
+  const auto e2 = load_entry<T2, PARTS>(in2, a, k, k < last, beyond);
+  if (beyond) raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
+  wave_gather_entries<T1, VEC, false, FLY>(in1, e1, last - first, c0, g, groups, acc);
+  if (in2.nt)
+    wave_gather_entries<T2, VEC, true, FLY>(in2, e2, last - first, c0, g, groups, acc);
+  else
+    wave_gather_entries<T2, VEC, false, FLY>(in2, e2, last - first, c0, g, groups, acc);
+}
+
+// Short lists (at most as many entries as a lane group has lanes), a lane group each: every lane of the group has one
+// entry, so a list costs one load of src and one of coef whatever its length, and N rows of it go out together (entries j0 .. j0 + N
+// of every list: past a list's end lie lanes without an entry).
+template <typename T, int VEC, bool NT, int N>
+__device__ __forceinline__ void load_list_rows(const SrcView<T>& in, const ListEntry<T>& mine, int first_lane, int j0, int c0,
+                                               Pack<T, VEC> (&v)[N], float (&w)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) v[k] = load_row_of<T, VEC, NT>(in, mine, (first_lane + j0 + k) * 4, c0, w[k]);
+}
+template <typename T, int VEC, int N>
+__device__ __forceinline__ void add_rows(const Pack<T, VEC> (&v)[N], const float (&w)[N], float (&acc)[VEC]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) add_pack<T, VEC>(v[k], w[k], acc);
 }
 
 // Workgroups of kBlock threads that a row kernel which strides over its rows launches on the current
@@ -325,6 +429,9 @@ __global__ void __launch_bounds__(kBlock, (!SHUFFLE && EPI != kEpiStore && (std:
 csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a, FuseArgs f) {
   constexpr bool TWO = !std::is_void<TIn2>::value;
   using TSecond = typename std::conditional<TWO, TIn2, TIn>::type;
+  using TRow = typename std::conditional<EPI != kEpiStore, TOut, float>::type;
+  FirstBlocks<TRow> first{};
+  if constexpr (TWO && EPI != kEpiStore) first = first_blocks<TRow, EPI>(f);
   extern __shared__ float s_part[];  // [waves][D], hot part only
   const int D = a.D;
   const int cl = threadIdx.x & ((1 << a.lpr_log2) - 1);
@@ -337,10 +444,25 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   // bound: 12 - 15 us of the update kernel were theirs).
   // Likewise a workgroup of the hot part that no work item is left for (block 0 stays: it leaves
   // alpha behind for the finish kernel).
+  // What a cold workgroup needs of its rows (bounds, table row) goes out beside that count, not behind it.
+  const int64_t hot_blocks = static_cast<int64_t>(gridDim.x) - a.cold_blocks;
+  const int rows_per_block = kBlock >> a.lpr_log2;
+  const int64_t u = (static_cast<int64_t>(blockIdx.x) - hot_blocks) * rows_per_block + (threadIdx.x >> a.lpr_log2);
+  // (The kernels with one input and shuffles have no registers left for that.)
+  constexpr bool kEarlyBounds = TWO || !SHUFFLE;
+  int32_t start = 0, end = 0;
+  int64_t idx_mine = -1;
+  auto ask_bounds = [&](bool there) {
+    if (there) {
+      start = a.row_start[u];
+      end = a.row_start[u + 1];
+      if constexpr (EPI != kEpiStore) idx_mine = f.row_index[u];
+    }
+  };
+  if constexpr (kEarlyBounds) ask_bounds(u >= 0 && u < a.U);  // (negative: the hot part)
   {
-    const int64_t first_cold = static_cast<int64_t>(gridDim.x) - a.cold_blocks;
     const int64_t b = static_cast<int64_t>(blockIdx.x);
-    if (b >= first_cold ? (b - first_cold) * (kBlock >> a.lpr_log2) >= min(a.U, a.counts[0])
+    if (b >= hot_blocks ? (b - hot_blocks) * rows_per_block >= min(a.U, a.counts[0])
                         : (b > 0 && b >= min(a.counts[1], a.hot_cap)))
       return;
   }
@@ -411,13 +533,23 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
     gather_one(in1, std::integral_constant<bool, PARTS && !TWO>{}, first, last, step, c0, acc);
     if constexpr (TWO) gather_one(in2, std::integral_constant<bool, PARTS>{}, first, last, step, c0, acc);
   };
+  constexpr int kFly = 4;  // rows in flight per lane of a list that a wave shares (two inputs with eight: 184 -> 204 us, 4 waves)
   // the wave's sum over the list entries [first, last) for columns c0.., the same in every group
   auto wave_sum = [&](int32_t first, int32_t last, int c0, bool col_ok, float (&acc)[VEC]) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) acc[j] = 0.f;
     if constexpr (SHUFFLE) {
-      wave_gather_range<TIn, VEC, PARTS && !TWO>(in1, a, first, last, c0, col_ok, g, groups, acc);
-      if constexpr (TWO) wave_gather_range<TSecond, VEC, PARTS>(in2, a, first, last, c0, col_ok, g, groups, acc);
+      const int c = col_ok ? c0 : 0;
+      if constexpr (TWO) {
+        if (last - first <= kWave) {
+          wave_gather_two<TIn, TSecond, VEC, PARTS, kFly>(in1, in2, a, first, last, c, g, groups, acc);
+        } else {
+          wave_gather_range<TIn, VEC, false, kFly, true>(in1, a, first, last, c, g, groups, acc);
+          wave_gather_range<TSecond, VEC, PARTS, kFly, true>(in2, a, first, last, c, g, groups, acc);
+        }
+      } else {
+        wave_gather_range<TIn, VEC, PARTS, kFly, false>(in1, a, first, last, c, g, groups, acc);
+      }
     } else {
       if (col_ok) gather_sum(first + g, last, groups, c0, acc);
     }
@@ -427,7 +559,6 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
     }
   };
 
-  const int64_t hot_blocks = static_cast<int64_t>(gridDim.x) - a.cold_blocks;
   if (static_cast<int64_t>(blockIdx.x) < hot_blocks) {
     // ---- hot work items (the first workgroups: the longest-running ones start first)
     int64_t n_items = a.counts[1];
@@ -463,13 +594,14 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   }
 
   // ---- cold rows
-  const int rows_per_block = kBlock >> a.lpr_log2;
-  const int64_t u = (static_cast<int64_t>(blockIdx.x) - hot_blocks) * rows_per_block + (threadIdx.x >> a.lpr_log2);
   // a.U may be an upper bound (a caller that has not read the plan's count back passes the number of
   // ids): rows at and past the count the plan left on the device have no list
   const bool valid = u < a.U && u < a.counts[0];
-  const int32_t start = valid ? a.row_start[u] : 0;
-  int32_t end = valid ? a.row_start[u + 1] : 0;
+  if constexpr (!kEarlyBounds) ask_bounds(valid);
+  if (!valid) {
+    start = end = 0;
+    idx_mine = -1;
+  }
   const bool hot = end - start > a.hot_len;  // left to the work items and the finish kernel
   if (hot) end = start;
   // The table row of this group's unique id is asked for before the gathers; the kernel with
@@ -477,12 +609,9 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   // that the block-table reads run under the gathers instead of heading the row update (config 4:
   // 146 -> 136 us; the other kernels spill with six registers more and lose 10 %).
   constexpr bool kEarlyPlaces = EPI != kEpiStore && !SHUFFLE && !TWO;
-  using TRow = typename std::conditional<EPI != kEpiStore, TOut, float>::type;
   RowPlaces<TRow> places{nullptr, nullptr, nullptr};
-  int64_t idx_mine = -1;
   if constexpr (EPI != kEpiStore) {
-    if (valid) idx_mine = f.row_index[u];  // (under the same test as the list bounds: the three loads go out together)
-    if constexpr (kEarlyPlaces) places = row_places<TRow, EPI>(f, a.err, idx_mine);
+    if constexpr (kEarlyPlaces) places = row_places<TRow, EPI, false>(f, first, a.err, idx_mine);
   }
   // the finished sum of this lane group's own row u
   auto finish = [&](int64_t row, int c0, float (&acc)[VEC]) {
@@ -490,7 +619,7 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
       if constexpr (kEarlyPlaces)
         fused_row_update_at<TRow, VEC, EPI>(f, places, c0, acc, epi_is_adam(EPI) ? s_alpha : 0.0);
       else
-        fused_row_update<TOut, VEC, EPI>(f, a.err, idx_mine, c0, acc, epi_is_adam(EPI) ? s_alpha : 0.0);
+        fused_row_update<TOut, VEC, EPI, TWO>(f, first, a.err, idx_mine, c0, acc, epi_is_adam(EPI) ? s_alpha : 0.0);
     } else {
       TOut* dst = out + (a.out_rows ? static_cast<int64_t>(a.out_rows[row]) : row) * D + c0;
       if (a.accumulate) {
@@ -504,10 +633,80 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   };
   // short rows: every lane group works its own row
   const bool is_long = a.lpr_log2 < 6 && end - start > kCoopLen;  // with one group per wave there is nobody to share with
-  if (valid && !is_long && !hot) {
-    // (Asking for the row's parameter and state packs before the gradient is gathered, to run their
-    // latency under that of the gathers, was measured and lost: 150 -> 205 us in config 4. The packs
-    // cost registers, hence resident waves, and the gathers then queue behind the table reads.)
+  const bool is_short = valid && !is_long && !hot;
+  // (Asking for the row's parameter and state packs before the gradient is gathered, to run their
+  // latency under that of the gathers, was measured and lost: 150 -> 205 us in config 4. The packs
+  // cost registers, hence resident waves, and the gathers then queue behind the table reads.)
+  if constexpr (SHUFFLE && TWO) {
+    // All lists of the wave side by side, as many rows of each in flight as the longest of them has (up to four: the longest
+    // decides for all, and most hold one or two), of both inputs together where they fit: the chain is bounds, entries, rows,
+    // table row. With each list's entries taken as they come, src and row of one after the other and the second input
+    // behind the first, a list of four was up to sixteen round trips (two inputs of 128 bfloat16, 1.5 M entries, three quarters of them in hot rows: 239 us, 188 in this form).
+    // (One input in this form: 128 -> 136 us with 2 M entries of 32 floats, whose kernel has registers for 64 only.)
+    const int len = is_short ? end - start : 0;
+    const int first_lane = lane & ~((1 << a.lpr_log2) - 1);
+    bool beyond = false;
+    const bool have = cl < len;
+    const auto e1 = load_entry<TIn, false>(in1, a, start + cl, have, beyond);
+    const auto e2 = load_entry<TSecond, PARTS>(in2, a, start + cl, have, beyond);
+    if (beyond) raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
+    const bool over1 = __ballot(len > 1) != 0, over2 = __ballot(len > 2) != 0;
+    RowPlaces<TRow> mine{nullptr, nullptr, nullptr};
+    if constexpr (EPI != kEpiStore) mine = row_places<TRow, EPI, true>(f, first, a.err, is_short ? idx_mine : -1);
+    for (int cbase = 0; cbase < D; cbase += VEC << a.lpr_log2) {  // uniform: shuffles inside
+      const int c0 = cbase + cl * VEC;
+      const bool col_ok = c0 < D;
+      TablePacks<TRow, VEC> packs;
+      bool touched = false;
+      if constexpr (EPI != kEpiStore) {
+        touched = is_short & col_ok & (mine.w != nullptr);
+        packs = load_table_packs<TRow, VEC, EPI>(mine, c0, touched, reinterpret_cast<const TRow*>(g_csr_zero_row));
+      }
+      float acc[VEC];
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) acc[j] = 0.f;
+      const int c = col_ok ? c0 : 0;
+      auto up_to = [&](auto n_tag, auto nt_tag) {  // every list of the wave has at most N entries
+        constexpr int N = decltype(n_tag)::value;
+        Pack<TIn, VEC> v[N];
+        Pack<TSecond, VEC> v_2[N];
+        float w[N], w_2[N];
+        load_list_rows<TIn, VEC, false, N>(in1, e1, first_lane, 0, c, v, w);
+        load_list_rows<TSecond, VEC, decltype(nt_tag)::value, N>(in2, e2, first_lane, 0, c, v_2, w_2);
+        __builtin_amdgcn_sched_barrier(0);  // all loads first
+        add_rows<TIn, VEC, N>(v, w, acc);
+        add_rows<TSecond, VEC, N>(v_2, w_2, acc);
+      };
+      auto with_hint = [&](auto nt_tag) {  // (of the two inputs the first, pooled gradients, is the small one)
+        if (!over1) {
+          up_to(std::integral_constant<int, 1>{}, nt_tag);
+        } else if (!over2) {
+          up_to(std::integral_constant<int, 2>{}, nt_tag);
+        } else {
+          float w[kFly];
+          for (int j0 = 0; __ballot(j0 < len) != 0; j0 += kFly) {
+            Pack<TIn, VEC> v[kFly];
+            load_list_rows<TIn, VEC, false, kFly>(in1, e1, first_lane, j0, c, v, w);
+            add_rows<TIn, VEC, kFly>(v, w, acc);
+          }
+          for (int j0 = 0; __ballot(j0 < len) != 0; j0 += kFly) {
+            Pack<TSecond, VEC> v[kFly];
+            load_list_rows<TSecond, VEC, decltype(nt_tag)::value, kFly>(in2, e2, first_lane, j0, c, v, w);
+            add_rows<TSecond, VEC, kFly>(v, w, acc);
+          }
+        }
+      };
+      if (in2.nt)
+        with_hint(std::true_type{});
+      else
+        with_hint(std::false_type{});
+      if constexpr (EPI != kEpiStore) {
+        if (touched) update_table_packs<TRow, VEC, EPI>(f, mine, c0, packs, acc, epi_is_adam(EPI) ? s_alpha : 0.0);
+      } else {
+        if (is_short && col_ok) finish(u, c0, acc);
+      }
+    }
+  } else if (is_short) {
     for (int c0 = cl * VEC; c0 < D; c0 += VEC << a.lpr_log2) {
       float acc[VEC];
 #pragma unroll
@@ -599,7 +798,7 @@ csr_hot_finish_kernel(TOut* __restrict__ out, CsrArgs a, FuseArgs f) {
       }
       if (g != 0 || !col_ok) continue;
       if constexpr (EPI != kEpiStore) {
-        fused_row_update<TOut, VEC, EPI>(f, a.err, f.row_index[u], c0, acc, alpha);
+        fused_row_update<TOut, VEC, EPI, false>(f, {}, a.err, f.row_index[u], c0, acc, alpha);
       } else {
         TOut* dst = out + static_cast<int64_t>(a.out_rows ? a.out_rows[u] : u) * D + c0;
         if (a.accumulate) {
