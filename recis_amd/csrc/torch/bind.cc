@@ -282,6 +282,7 @@ TORCH_LIBRARY(recis, m) {
   m.def("block_apply_adamw", recis::functional::block_apply_adamw);
   m.def("block_apply_adagrad", recis::functional::block_apply_adagrad);  // an addition
   m.def("fused_bucketized_mod", recis::functional::fused_bucketized_mod);  // an addition
+  m.def("feature_chains", recis::functional::feature_chains);  // an addition
 
   m.def("generate_ids", recis::functional::generate_ids_op);
   m.def("free_ids", recis::functional::free_ids_op);

@@ -4,8 +4,10 @@
 // every op; these are the device branches only).
 #include "ops.h"
 
+#include <ATen/hip/HIPEvent.h>
 #include <c10/hip/HIPStream.h>
 
+#include <algorithm>
 #include <cstring>
 #include <map>
 #include <mutex>
@@ -1027,6 +1029,235 @@ std::tuple<TensorList, TensorList, TensorList> fused_ragged_cutoff_3D(TensorList
   if (values.empty()) return std::make_tuple(TensorList(), TensorList(), TensorList());
   CutoffResult r = ragged_cutoff(values, outer_offsets, &inner_offsets, keep_lengths, drop_sides, pad_sides);
   return std::make_tuple(r.values, r.outer, r.offsets);
+}
+
+// ------------------------------------------------------------------------------------ chains of feature operators
+namespace {
+// A tensor of its own over elements [first, first + n) of a buffer (not a view in autograd's sense: no shared version).
+Tensor part_of(const Tensor& whole, int64_t first, at::IntArrayRef shape) {
+  auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(whole.storage()), whole.key_set(), whole.dtype());
+  impl->set_storage_offset(first);
+  impl->set_sizes_contiguous(shape);
+  return Tensor(std::move(impl));
+}
+bool plain(const TensorList& ts, at::Device device, std::initializer_list<at::ScalarType> types) {
+  for (const auto& t : ts) {
+    if (t.device() != device || t.layout() != at::kStrided) return false;
+    if (std::find(types.begin(), types.end(), t.scalar_type()) == types.end()) return false;
+  }
+  return true;
+}
+}  // namespace
+
+// The waiting part of the truncations, the lengths of what is kept, needs the offsets only: it is queued first, and has
+// long arrived when the operators behind it are queued (operator by operator, the host stood waiting for all of them).
+TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::vector<int64_t> hash_kinds,
+                          TensorList mod_values, std::vector<int64_t> mods, TensorList bucket_values, TensorList boundaries,
+                          std::vector<int64_t> bucket_mods, TensorList multi_values, std::vector<int64_t> multi_counts,
+                          std::vector<int64_t> muls, std::vector<int64_t> primes, std::vector<int64_t> buckets,
+                          TensorList cut_values, std::vector<int64_t> cut_from, TensorList cut_offsets,
+                          std::vector<int64_t> keep, std::vector<int64_t> drop_left) {
+  const int64_t n_hash = hash_values.size(), n_mod = mod_values.size(), n_bucket = bucket_values.size(),
+                n_multi = multi_values.size(), n_cut = cut_offsets.size();
+  const Tensor* any = n_hash ? &hash_values[0] : n_mod ? &mod_values[0] : n_bucket ? &bucket_values[0]
+                      : n_multi ? &multi_values[0] : n_cut && !cut_values.empty() ? &cut_values[0] : nullptr;
+  if (any == nullptr || !any->is_cuda()) return {};
+  const at::Device device = any->device();
+  if (device.index() != c10::hip::current_device()) return {};
+  TORCH_CHECK(static_cast<int64_t>(hash_offsets.size()) == n_hash && static_cast<int64_t>(hash_kinds.size()) == n_hash &&
+                  static_cast<int64_t>(mods.size()) == n_mod && static_cast<int64_t>(boundaries.size()) == n_bucket &&
+                  static_cast<int64_t>(bucket_mods.size()) == n_bucket && static_cast<int64_t>(multi_counts.size()) == n_multi &&
+                  static_cast<int64_t>(cut_from.size()) == n_cut && static_cast<int64_t>(keep.size()) == n_cut &&
+                  static_cast<int64_t>(drop_left.size()) == n_cut && muls.size() == primes.size() && muls.size() == buckets.size(),
+              "feature_chains: lists of different lengths");
+  // ---- what the operators one by one would convert or refuse is left to them
+  if (!plain(hash_values, device, {at::kChar, at::kByte}) || !plain(hash_offsets, device, {at::kInt, at::kLong}) ||
+      !plain(mod_values, device, {at::kLong}) || !plain(bucket_values, device, {at::kFloat}) ||
+      !plain(boundaries, device, {at::kFloat}) || !plain(multi_values, device, {at::kLong}) ||
+      !plain(cut_values, device, {at::kLong}) || !plain(cut_offsets, device, {at::kInt, at::kLong}))
+    return {};
+  for (int64_t k = 0; k < n_hash; ++k)
+    if (hash_offsets[k].scalar_type() != hash_offsets[0].scalar_type() || hash_offsets[k].numel() < 1 || hash_kinds[k] < 0 ||
+        hash_kinds[k] > 1)
+      return {};
+  for (int64_t m : mods)
+    if (m == 0) return {};
+  for (int64_t m : bucket_mods)
+    if (m <= 0) return {};
+  int64_t n_jobs = 0;
+  for (int64_t c : multi_counts) n_jobs += c;
+  TORCH_CHECK(n_jobs == static_cast<int64_t>(muls.size()), "feature_chains: lists of different lengths");
+  for (int64_t k = 0; k < n_jobs; ++k)
+    if (primes[k] == 0 || buckets[k] == 0) return {};
+  const int64_t n_direct = cut_values.size();
+  for (int64_t k = 0; k < n_cut; ++k) {
+    TORCH_CHECK(cut_from[k] >= -n_direct && cut_from[k] < n_hash + n_mod, "feature_chains: bad cut_from");
+    if (cut_offsets[k].scalar_type() != cut_offsets[0].scalar_type() || cut_offsets[k].numel() < 1 || keep[k] < 0) return {};
+  }
+  void* stream = stream_of(device);
+  auto lopt = at::TensorOptions().device(device).dtype(at::kLong);
+
+  // ---- outputs of the operators in front of the truncations, one buffer per kind
+  TensorList outs, hash_in, hash_off, mod_in, bucket_in, bucket_bd, multi_in;
+  std::vector<int64_t> n_strings(n_hash);
+  for (int64_t k = 0; k < n_hash; ++k) {
+    hash_in.push_back(hash_values[k].contiguous());
+    hash_off.push_back(hash_offsets[k].contiguous());
+    n_strings[k] = hash_off[k].numel() - 1;
+    outs.push_back(at::empty({n_strings[k]}, lopt));
+  }
+  auto ids_like = [&](const TensorList& values, TensorList& in, bool flat) {  // int64 outputs, shaped as the inputs or flat
+    int64_t total = 0;
+    for (const auto& v : values) {
+      in.push_back(v.contiguous());
+      total += v.numel();
+    }
+    if (values.empty()) return;
+    Tensor buf = at::empty({total}, lopt);
+    int64_t first = 0;
+    for (const auto& v : values) {
+      outs.push_back(flat ? part_of(buf, first, {v.numel()}) : part_of(buf, first, v.sizes()));
+      first += v.numel();
+    }
+  };
+  ids_like(mod_values, mod_in, n_mod > 1);  // (fused_uint64_mod of several is flat, a modulus alone keeps the shape)
+  ids_like(bucket_values, bucket_in, false);
+  for (const auto& b : boundaries) bucket_bd.push_back(b.contiguous());
+  const int64_t multi_first = outs.size();
+  for (int64_t k = 0; k < n_multi; ++k) {
+    multi_in.push_back(multi_values[k].contiguous());
+    const int64_t size = multi_in[k].numel();
+    Tensor buf = at::empty({size * multi_counts[k]}, lopt);
+    for (int64_t j = 0; j < multi_counts[k]; ++j) outs.push_back(part_of(buf, j * size, {size}));  // (flat, as the operator returns them)
+  }
+
+  // ---- lengths of the truncations
+  TensorList cut_off, cut_in;
+  std::vector<int64_t> rows(n_cut), n_values(n_cut);
+  Tensor off_buf, src_buf, cnt_buf, totals;
+  std::vector<void*> off_p(n_cut), drop_p(n_cut), pad_p(n_cut);
+  std::vector<const void*> outer_p(n_cut);
+  std::vector<int64_t*> src_p(n_cut);
+  std::vector<int64_t> off_at(n_cut), cnt_at(n_cut);
+  int64_t sum_rows = 0;
+  int is64 = 0;
+  at::cuda::CUDAEvent arrived;
+  if (n_cut) {
+    is64 = index_kind(cut_offsets[0], "offsets");
+    for (int64_t k = 0; k < n_cut; ++k) {
+      cut_off.push_back(cut_offsets[k].contiguous());
+      cut_in.push_back(cut_from[k] >= 0 ? outs[cut_from[k]] : cut_values[-cut_from[k] - 1].contiguous());
+      rows[k] = cut_off[k].numel() - 1;
+      n_values[k] = cut_in[k].numel();
+      off_at[k] = sum_rows + k;
+      cnt_at[k] = sum_rows;
+      sum_rows += rows[k];
+    }
+    auto iopt = cut_off[0].options();
+    off_buf = at::empty({sum_rows + n_cut}, iopt);
+    src_buf = at::empty({std::max<int64_t>(sum_rows, 1)}, lopt);
+    cnt_buf = at::empty({std::max<int64_t>(2 * sum_rows, 1)}, iopt);
+    totals = at::empty({n_cut}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));  // written by the kernel itself
+    const int64_t isize = off_buf.element_size();
+    std::vector<uint8_t> drop8(n_cut), pad8(n_cut, 0);
+    for (int64_t k = 0; k < n_cut; ++k) {
+      outer_p[k] = cut_off[k].data_ptr();
+      off_p[k] = static_cast<char*>(off_buf.data_ptr()) + off_at[k] * isize;
+      drop_p[k] = static_cast<char*>(cnt_buf.data_ptr()) + cnt_at[k] * isize;
+      pad_p[k] = static_cast<char*>(cnt_buf.data_ptr()) + (sum_rows + cnt_at[k]) * isize;
+      src_p[k] = src_buf.data_ptr<int64_t>() + cnt_at[k];
+      if (rows[k] == 0) {  // never used: any valid address
+        drop_p[k] = pad_p[k] = cnt_buf.data_ptr();
+        src_p[k] = src_buf.data_ptr<int64_t>();
+      }
+      drop8[k] = drop_left[k] ? 1 : 0;
+    }
+    check(recis_ragged_cutoff_rows(outer_p.data(), nullptr, is64, rows.data(), nullptr, n_values.data(), keep.data(),
+                                   drop8.data(), pad8.data(), n_cut, off_p.data(), nullptr, drop_p.data(), pad_p.data(),
+                                   src_p.data(), totals.data_ptr<int64_t>(), stream));
+    arrived.record();
+  }
+
+  // ---- the operators in front, a launch per kind
+  for (int64_t kind = 0; kind < 2; ++kind) {
+    std::vector<const int8_t*> vp;
+    std::vector<const void*> fp;
+    std::vector<int64_t> sizes, strings;
+    std::vector<int64_t*> op;
+    for (int64_t k = 0; k < n_hash; ++k) {
+      if (hash_kinds[k] != kind) continue;
+      vp.push_back(static_cast<const int8_t*>(hash_in[k].data_ptr()));
+      fp.push_back(hash_off[k].data_ptr());
+      sizes.push_back(hash_in[k].numel());
+      strings.push_back(n_strings[k]);
+      op.push_back(outs[k].data_ptr<int64_t>());
+    }
+    if (!vp.empty())
+      check(recis_fused_hash(vp.data(), sizes.data(), fp.data(), index_kind(hash_off[0], "offsets"), strings.data(), op.data(),
+                             static_cast<int64_t>(vp.size()), static_cast<int>(kind), stream));
+  }
+  auto out_ptrs = [&](int64_t first, int64_t n) {
+    std::vector<int64_t*> p(n);
+    for (int64_t k = 0; k < n; ++k) p[k] = outs[first + k].data_ptr<int64_t>();
+    return p;
+  };
+  if (n_mod) {
+    auto ip = host_ptrs<int64_t>(mod_in);
+    auto op = out_ptrs(n_hash, n_mod);
+    auto sizes = numels(mod_in);
+    check(recis_fused_uint64_mod(ip.data(), sizes.data(), mods.data(), op.data(), n_mod, stream));
+  }
+  if (n_bucket) {
+    auto ip = host_ptrs<float>(bucket_in), bp = host_ptrs<float>(bucket_bd);
+    auto op = out_ptrs(n_hash + n_mod, n_bucket);
+    auto sizes = numels(bucket_in), lens = numels(bucket_bd);
+    check(recis_fused_bucketized_mod(ip.data(), sizes.data(), bp.data(), lens.data(), bucket_mods.data(), op.data(), n_bucket,
+                                     stream));
+  }
+  if (n_jobs) {
+    std::vector<const int64_t*> ip;
+    std::vector<int64_t> sizes;
+    for (int64_t k = 0; k < n_multi; ++k) {
+      ip.insert(ip.end(), multi_counts[k], multi_in[k].data_ptr<int64_t>());
+      sizes.insert(sizes.end(), multi_counts[k], multi_in[k].numel());
+    }
+    auto op = out_ptrs(multi_first, n_jobs);
+    check(recis_fused_multi_hash(ip.data(), sizes.data(), muls.data(), primes.data(), buckets.data(), op.data(), n_jobs, stream));
+  }
+
+  // ---- the truncated values
+  if (n_cut) {
+    arrived.synchronize();
+    const int64_t* total = totals.data_ptr<int64_t>();
+    int64_t sum_total = 0;
+    for (int64_t k = 0; k < n_cut; ++k) sum_total += total[k];
+    Tensor val_buf = at::empty({sum_total}, lopt);
+    Tensor sides = at::empty({2 * n_cut}, at::TensorOptions().dtype(at::kBool));
+    bool* side = sides.data_ptr<bool>();
+    std::vector<void*> val_p(n_cut);
+    std::vector<const void*> in_p(n_cut), off_cp(off_p.begin(), off_p.end());
+    std::vector<const int64_t*> src_cp(src_p.begin(), src_p.end());
+    TensorList vals, offs, drops, pads, drop_sides, pad_sides;
+    int64_t first = 0;
+    for (int64_t k = 0; k < n_cut; ++k) {
+      in_p[k] = n_values[k] ? cut_in[k].data_ptr() : src_buf.data_ptr();
+      val_p[k] = total[k] ? static_cast<void*>(val_buf.data_ptr<int64_t>() + first) : src_buf.data_ptr();
+      vals.push_back(part_of(val_buf, first, {total[k]}));
+      offs.push_back(part_of(off_buf, off_at[k], {rows[k] + 1}));
+      drops.push_back(part_of(cnt_buf, cnt_at[k], {rows[k]}));
+      pads.push_back(part_of(cnt_buf, sum_rows + cnt_at[k], {rows[k]}));
+      side[2 * k] = drop_left[k] != 0;
+      side[2 * k + 1] = false;
+      drop_sides.push_back(part_of(sides, 2 * k, {}));
+      pad_sides.push_back(part_of(sides, 2 * k + 1, {}));
+      first += total[k];
+    }
+    check(recis_ragged_cutoff_copy(in_p.data(), static_cast<int>(sizeof(int64_t)), off_cp.data(), is64, rows.data(), src_cp.data(),
+                                   total, val_p.data(), n_cut, stream));
+    for (TensorList* list : {&vals, &offs, &drops, &pads, &drop_sides, &pad_sides})
+      outs.insert(outs.end(), list->begin(), list->end());
+  }
+  return outs;
 }
 
 // ------------------------------------------------------------------------------------ feature cross

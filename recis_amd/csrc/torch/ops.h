@@ -61,6 +61,17 @@ TensorList fused_bucketized(TensorList inputs, TensorList boundaries);
 // pass: an addition (the reference runs the two operators one after the other).
 TensorList fused_bucketized_mod(TensorList inputs, TensorList boundaries, std::vector<int64_t> mods);
 TensorList fused_hash(TensorList inputs, TensorList input_offsets, const std::string& hash_type);
+// An addition: the chains of a feature engine's step in one call (recis/features/feature_engine.py:107-284 runs them operator by
+// operator). Hashes (kinds: 0 farm, 1 murmur), moduli, buckets with a modulus, multi hashes (multi_counts[k] jobs of input k), then the
+// truncations: cut k takes output cut_from[k] of the hashes and moduli, or cut_values[-cut_from[k] - 1], and keeps keep[k] of
+// every row, the last ones where drop_left. Returns hashes, moduli, buckets, multi hashes, then per kind for all cuts: values,
+// offsets, dropped, padded, drop side, pad side. Empty when an input needs what only the single operators do (another type or device) or refuse.
+TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::vector<int64_t> hash_kinds,
+                          TensorList mod_values, std::vector<int64_t> mods, TensorList bucket_values, TensorList boundaries,
+                          std::vector<int64_t> bucket_mods, TensorList multi_values, std::vector<int64_t> multi_counts,
+                          std::vector<int64_t> muls, std::vector<int64_t> primes, std::vector<int64_t> buckets,
+                          TensorList cut_values, std::vector<int64_t> cut_from, TensorList cut_offsets,
+                          std::vector<int64_t> keep, std::vector<int64_t> drop_left);
 TensorList fused_multi_hash(TensorList inputs, TensorList muls, TensorList primes, TensorList bucket_num);
 // csrc/ops/ragged_tile.h:9-18
 TensorList ragged_tile(const std::vector<int64_t>& batch, const std::vector<int64_t>& seq, Tensor value,
