@@ -11,8 +11,8 @@
 //
 // Bound: random requests to memory (one 16-byte slot and one row per distinct id) for large
 // batches, the chain id -> slot -> row -> store (three round trips) for a request of a few hundred samples.
-// Measured with 26 id columns and 4 ragged features (0..20 ids) of rows of 16 floats: batch 256 in 7.0 us where the plan,
-// the look-up of its unique ids and the pooling took 63 us; batch 16384 (1.1 M ids) in 38 us instead of 145; one row
+// Measured with 26 id columns and 4 ragged features (0..20 ids) of rows of 16 floats: batch 256 in 6.7 us where the plan,
+// the look-up of its unique ids and the pooling took 63 us; batch 16384 (1.1 M ids) in 32 us instead of 145; one row
 // per lookup of 0.5 M Zipf ids over rows of 32 floats (half a million rows of 128 bytes written) 27 us instead of 107.
 #include <hip/hip_runtime.h>
 
@@ -109,12 +109,14 @@ __device__ __forceinline__ float weight_at(const void* w, int dt, int64_t i) {
 }
 
 // A workgroup takes a tile of consecutive segments of one feature: its threads look up the ids of
-// the tile, one id each at a time, and leave the addresses of the rows in LDS; then teams of lanes
+// the tile, up to four each at a time, and leave the addresses of the rows in LDS; then teams of lanes
 // (2^lpr lanes per row, 2^rg row groups per segment) sum the rows of their segments, several row
 // loads in flight per lane, and store each pooled row once. Looking an id up by one lane instead of
 // by the whole lane group that reads its row keeps 256 probes of the map in flight per workgroup.
+// (Six waves a SIMD: four rows and four probes in flight are 80 registers; held to 64 they spill, 36.6 us instead of 32.2 for
+// 1.1 M ids of rows of 64 bytes.)
 template <typename T, int VEC>
-__global__ void __launch_bounds__(kBlock, 8)
+__global__ void __launch_bounds__(kBlock, 6)
 lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
   __shared__ uint64_t s_row[kPoolRows];
   __shared__ float s_w[kPoolRows];
@@ -171,17 +173,43 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
   }
 
   // rows of the ids [from, to) of the feature into LDS
-  auto look_up = [&](int32_t from, int32_t to) {
-    for (int32_t q = from + tid; q < to; q += kBlock) {
-      const int64_t key = (ids[q] & a.id_mask) | tag;
-      int64_t row = -1;
-      if (key != kEmpty && key != kTomb) {
-        const uint64_t home = home_slot(key, a.mask);
-        row = find_row(a.table, a.mask, key, home, *reinterpret_cast<const longlong2*>(&a.table[home]));
+  auto look_up_by = [&](auto probes, int32_t from, int32_t to) {
+    constexpr int kProbes = decltype(probes)::value;  // of a thread in flight
+    for (int32_t q0 = from + tid; q0 < to; q0 += kProbes * kBlock) {
+      int64_t key[kProbes];
+      longlong2 hint[kProbes];
+#pragma unroll
+      for (int x = 0; x < kProbes; ++x) key[x] = q0 + x * kBlock < to ? (ids[q0 + x * kBlock] & a.id_mask) | tag : kEmpty;
+#pragma unroll
+      for (int x = 0; x < kProbes; ++x)  // (a reserved key has a home slot too: no branch around the load)
+        hint[x] = *reinterpret_cast<const longlong2*>(&a.table[home_slot(key[x], a.mask)]);
+      uint32_t further = 0;  // probes that the home slot does not end
+#pragma unroll
+      for (int x = 0; x < kProbes; ++x) {
+        const bool reserved = key[x] == kEmpty || key[x] == kTomb, found = hint[x].x == key[x] && !reserved;
+        further |= !found && !reserved && hint[x].x != kEmpty ? 1u << x : 0u;
+        if (q0 + x * kBlock < to) s_row[q0 + x * kBlock - from] = static_cast<uint64_t>(found ? hint[x].y : -1);
       }
-      s_row[q - from] = address_of_row<T>(a, row);
-      if (weight) s_w[q - from] = weight_at<T>(weight, wdt, q);
+#pragma unroll 1
+      for (int x = 0; x < kProbes; ++x) {  // (one body: four of them spill)
+        const int32_t q = q0 + x * kBlock;
+        if (q >= to) break;
+        int64_t row = static_cast<int64_t>(s_row[q - from]);
+        if ((further >> x) & 1u) {
+          const int64_t k = (ids[q] & a.id_mask) | tag;
+          const uint64_t home = home_slot(k, a.mask);
+          row = find_row(a.table, a.mask, k, home, *reinterpret_cast<const longlong2*>(&a.table[home]));
+        }
+        s_row[q - from] = address_of_row<T>(a, row);
+        if (weight) s_w[q - from] = weight_at<T>(weight, wdt, q);
+      }
     }
+  };
+  auto look_up = [&](int32_t from, int32_t to) {
+    if (to - from <= kBlock)  // uniform
+      look_up_by(std::integral_constant<int, 1>{}, from, to);
+    else
+      look_up_by(std::integral_constant<int, 4>{}, from, to);
   };
   const int lane_t = tid & ((1 << team_log2) - 1);
   const int team = tid >> team_log2;
@@ -196,24 +224,18 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
   // acc += the rows first, first + step, ... < last of the LDS list, columns c0 ..
   auto add_rows = [&](int first, int last, int c0, float (&acc)[VEC]) {
     constexpr int kFly = 4;
-    int q = first;
-    for (; q + (kFly - 1) * step < last; q += kFly * step) {
-      float v[kFly][VEC];
+    for (int q = first; q < last; q += kFly * step) {  // past the end: the row of zeros, so that a short list is one round trip too
+      Pack<T, VEC> v[kFly];  // (converted as they are added: in flight they cost the registers of their own type)
 #pragma unroll
-      for (int k = 0; k < kFly; ++k) load_pack<T, VEC>(row_of(q + k * step) + c0, v[k]);
+      for (int k = 0; k < kFly; ++k)
+        v[k] = *reinterpret_cast<const Pack<T, VEC>*>((q + k * step < last ? row_of(q + k * step) : zero_row) + c0);
+      __builtin_amdgcn_sched_barrier(0);  // all loads first
 #pragma unroll
       for (int k = 0; k < kFly; ++k) {
-        const float w = weight ? s_w[q + k * step] : 1.0f;
+        const float w = weight ? (q + k * step < last ? s_w[q + k * step] : 0.f) : 1.0f;
 #pragma unroll
-        for (int x = 0; x < VEC; ++x) acc[x] = fmaf(v[k][x], w, acc[x]);
+        for (int x = 0; x < VEC; ++x) acc[x] = fmaf(to_float(v[k].v[x]), w, acc[x]);
       }
-    }
-    for (; q < last; q += step) {
-      float v[VEC];
-      load_pack<T, VEC>(row_of(q) + c0, v);
-      const float w = weight ? s_w[q] : 1.0f;
-#pragma unroll
-      for (int x = 0; x < VEC; ++x) acc[x] = fmaf(v[x], w, acc[x]);
     }
   };
   auto weight_sum = [&](int first, int last) {
@@ -389,7 +411,7 @@ extern "C" int recis_lookup_pool_readonly(recis_idmap* map, const recis_lookup_j
   }
   PoolJobs J;
   J.n_jobs = 0;
-  int64_t tiles = 0, out_row = 0;
+  int64_t tiles = 0;
   auto launch = [&]() -> int {
     if (tiles == 0) return RECIS_OK;
     RECIS_TIME_KERNEL("lookup_pool_kernel", stream) {
@@ -412,9 +434,12 @@ extern "C" int recis_lookup_pool_readonly(recis_idmap* map, const recis_lookup_j
     tiles = 0;
     return RECIS_OK;
   };
-  for (int64_t k = 0; k < n_jobs; ++k) {
-    const recis_lookup_job& q = jobs[k];
-    if (q.n_seg == 0) continue;
+  // Features of several ids per segment first: workgroups start in the order of their index, and what starts last should be
+  // short.
+  for (int64_t turn = 0, row0 = 0; turn < 2 * n_jobs; row0 += jobs[turn++ % n_jobs].n_seg) {
+    if (turn == n_jobs) row0 = 0;
+    const recis_lookup_job& q = jobs[turn % n_jobs];
+    if (q.n_seg == 0 || (q.n_ids > q.n_seg) != (turn < n_jobs)) continue;
     const int rg = groups_of(q);
     const int teams = kBlock >> (g.lpr_log2 + rg);
     const int64_t avg = (q.n_ids + q.n_seg - 1) / q.n_seg;
@@ -429,13 +454,12 @@ extern "C" int recis_lookup_pool_readonly(recis_idmap* map, const recis_lookup_j
     p.n_ids = static_cast<int32_t>(q.n_ids);
     p.n_seg = static_cast<int32_t>(q.n_seg);
     p.first_tile = static_cast<int32_t>(tiles);
-    p.out_row0 = static_cast<int32_t>(out_row);
+    p.out_row0 = static_cast<int32_t>(row0);
     p.width = static_cast<int32_t>(q.width);
     p.flags = (tagged ? static_cast<uint32_t>(q.table_id) : 0u) | (q.off_is64 ? 1u << 12 : 0u) |
               (q.weight ? static_cast<uint32_t>(q.weight_dtype) << 13 : 0u) | (static_cast<uint32_t>(rg) << 16) |
               (static_cast<uint32_t>(spt) << 20);
     tiles += (q.n_seg + (teams << spt) - 1) / (teams << spt);
-    out_row += q.n_seg;
     if (J.n_jobs == kPoolJobs) {
       if (int rc = launch()) return rc;
     }

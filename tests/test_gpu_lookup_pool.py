@@ -51,6 +51,7 @@ def _feature(rng, kind, n_seg, pool):
     (100, torch.float16, False, True, ["wide", "long"]),
     (600, torch.float32, False, False, ["huge"]),
     (8, torch.float32, False, True, ["column"] * 70),  # more features than one launch takes
+    (8, torch.float32, False, True, ["column", "long"] * 35),  # the ragged ones go first, over both launches
 ])
 @pytest.mark.parametrize("n_seg", [1, 65, 3000])
 def test_lookup_pool_matches_float64(rng, D, dtype, weighted, tagged, kinds, n_seg, mean):
