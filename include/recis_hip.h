@@ -699,6 +699,12 @@ int recis_csr_gather_reduce_parts(const void* const* part_rows, const int64_t* p
                                   const int32_t* row_start, const int32_t* hot_items,
                                   int64_t hot_cap, const int64_t* counts_dev, void* out, int64_t U,
                                   int64_t D, int accumulate, void* stream);
+/* The same sums over the rows of n_columns columns that lie side by side in a wider array (what a model that concatenates its features
+ * hands back): src names row src % rows_each of column src / rows_each, at rows + column * column_step + row * row_stride
+ * (elements). */
+int recis_csr_gather_reduce_grid(const void* rows, int rows_dtype, int64_t n_columns, int64_t rows_each, int64_t column_step,
+                                 int64_t row_stride, const int32_t* src, const int32_t* row_start, const int32_t* hot_items,
+                                 int64_t hot_cap, const int64_t* counts_dev, void* out, int64_t U, int64_t D, void* stream);
 
 /*
  * recis_csr_gather_reduce whose result never reaches memory: the finished sum of row u IS the

@@ -544,6 +544,26 @@ int recis_csr_gather_reduce_parts(const void* const* part_rows, const int64_t* p
   return csr_gather_reduce_run<false>(r);
 }
 
+int recis_csr_gather_reduce_grid(const void* rows, int rows_dtype, int64_t n_columns, int64_t rows_each, int64_t column_step,
+                                 int64_t row_stride, const int32_t* src, const int32_t* row_start, const int32_t* hot_items,
+                                 int64_t hot_cap, const int64_t* counts_dev, void* out, int64_t U, int64_t D, void* stream_) {
+  RECIS_REQUIRE(n_columns >= 1 && rows_each >= 1 && n_columns <= INT32_MAX / rows_each, "bad grid of %lld columns of %lld rows",
+                (long long)n_columns, (long long)rows_each);
+  RECIS_REQUIRE(rows != nullptr && column_step >= 0 && row_stride >= 0, "bad grid");
+  const int64_t count = n_columns * rows_each;
+  CsrRequest r = one_input_request(nullptr, rows_dtype, count, src, nullptr, 0, row_start, hot_items, hot_cap, counts_dev, U, D,
+                                   nullptr, 0, 0, stream_);
+  r.part_rows = &rows;
+  r.part_counts = &count;
+  r.n_parts = 1;
+  r.grid_rows = rows_each;
+  r.grid_step = column_step;
+  r.grid_stride = row_stride;
+  r.out = out;
+  r.out_dtype = RECIS_F32;
+  return csr_gather_reduce_run<false>(r);
+}
+
 int recis_csr_gather_reduce_adamw(const void* rows, int rows_dtype, int64_t n_rows, const int32_t* src,
                                   const void* coef, int coef_dtype, const int32_t* row_start,
                                   const int32_t* hot_items, int64_t hot_cap, const int64_t* counts_dev, int64_t U,

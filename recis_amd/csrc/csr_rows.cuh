@@ -62,6 +62,13 @@ struct CsrArgs {
   int n_parts;
   const void* part_rows[kMaxParts];
   int32_t part_lo32[kMaxParts];
+  // grid_rows > 0: the one part is a grid, columns side by side in a wider array: input row s is row s % grid_rows of column s / grid_rows,
+  // at part_rows[0] + column * grid_step + row * grid_stride (elements). s / grid_rows = s * grid_magic >> grid_shift for all s < 2^31:
+  // the shift is 31 + l with 2^l the power of two at or above grid_rows, the factor 2^shift / grid_rows rounded up, below 2^32.
+  int32_t grid_rows;
+  uint32_t grid_magic;
+  int grid_shift;
+  int64_t grid_step, grid_stride;
 };
 
 // What a gather-reduce launch does with the finished sum of row u (template parameter EPI):
@@ -237,6 +244,11 @@ __device__ __forceinline__ const TIn* src_row(const TIn* rows, const CsrArgs& a,
     return rows + s * a.D;
   } else {
     const TIn* base = static_cast<const TIn*>(a.part_rows[0]);
+    if (a.grid_rows > 0) {  // uniform
+      const uint32_t u = static_cast<uint32_t>(s);
+      const uint32_t column = static_cast<uint32_t>((static_cast<uint64_t>(u) * a.grid_magic) >> a.grid_shift);
+      return base + static_cast<int64_t>(column) * a.grid_step + static_cast<int64_t>(u - column * a.grid_rows) * a.grid_stride;
+    }
     int32_t lo = 0;
     const int32_t s32 = static_cast<int32_t>(s);  // src entries are 32-bit, and so are the parts' first rows
 #pragma unroll
@@ -322,7 +334,7 @@ __device__ __forceinline__ Pack<T, VEC> load_row_of(const SrcView<T>& in, const 
 template <typename T, int VEC, bool NT, int FLY>
 __device__ __forceinline__ void wave_gather_entries(const SrcView<T>& s, const ListEntry<T>& mine, int n_here, int c0, int g,
                                                     int groups, float (&acc)[VEC]) {
-  static_assert(FLY == 4 || FLY == 8, "a turn of FLY entries for each of up to eight groups divides the 64 of a wave");
+  static_assert(FLY == 4, "a turn of four entries for each of up to sixteen groups divides the 64 of a wave");
   for (int q0 = 0; q0 < n_here; q0 += FLY * groups) {  // same trip count for the whole wave (shuffles inside)
     Pack<T, VEC> v[FLY];
     float w[FLY];
@@ -412,8 +424,9 @@ constexpr int kCoopLen = 8;  // longer lists are shared among the lane groups of
 // walk the hot work items (row, chunk of kHotChunk occurrences): four waves share the chunk,
 // fold their sums through LDS and store ONE partial row per item; csr_hot_finish_kernel adds up
 // the partial rows of every hot row in chunk order. No atomics anywhere.
-// SHUFFLE: long lists go through wave_gather_range (pays off when a wave has at most eight lane
-// groups, i.e. rows of 128 bytes and more); otherwise every group loads its own entries.
+// SHUFFLE: long lists go through wave_gather_range, for up to sixteen lane groups a wave, i.e. rows of 64 bytes and more (rows of
+// 64 bytes, their entries loaded by every group for itself / through shuffles: 160 k entries 24.2 / 22.3 us, 43 k 14.5 / 10.8);
+// otherwise every group loads its own entries.
 // TIn2 != void: every list entry adds a row of a second input as well (see CsrArgs); PARTS then
 // says that the second input comes in parts.
 template <typename TIn, typename TOut, int VEC, bool SHUFFLE, bool PARTS = false, int EPI = kEpiStore,
@@ -448,8 +461,8 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   const int64_t hot_blocks = static_cast<int64_t>(gridDim.x) - a.cold_blocks;
   const int rows_per_block = kBlock >> a.lpr_log2;
   const int64_t u = (static_cast<int64_t>(blockIdx.x) - hot_blocks) * rows_per_block + (threadIdx.x >> a.lpr_log2);
-  // (The kernels with one input and shuffles have no registers left for that.)
-  constexpr bool kEarlyBounds = TWO || !SHUFFLE;
+  // (The kernels with one input and shuffles that update rows have no registers left for that.)
+  constexpr bool kEarlyBounds = TWO || !SHUFFLE || EPI == kEpiStore;
   int32_t start = 0, end = 0;
   int64_t idx_mine = -1;
   auto ask_bounds = [&](bool there) {
@@ -850,6 +863,7 @@ struct CsrRequest {
   const void* const* part_rows = nullptr;       // in1 as n_parts arrays laid end to end (in1.rows is NULL then)
   const int64_t* part_counts = nullptr;
   int n_parts = 0;
+  int64_t grid_rows = 0, grid_step = 0, grid_stride = 0;  // the one part as a grid (see CsrArgs)
   const int32_t* row_start = nullptr;
   const int32_t* hot_items = nullptr;
   int64_t hot_cap = 0;
@@ -889,6 +903,10 @@ int csr_gather_reduce_run(const CsrRequest& r) {
   RECIS_REQUIRE(r.in1.coef == nullptr || dtype_size(r.in1.coef_dtype), "invalid coef dtype");
   uintptr_t align_of = reinterpret_cast<uintptr_t>(r.in1.rows);
   for (int f = 0; f < n_parts; ++f) align_of |= reinterpret_cast<uintptr_t>(r.part_rows[f]);  // the coarsest alignment
+  if (r.grid_rows > 0) {
+    RECIS_REQUIRE(!TWO && n_parts == 1 && r.grid_rows <= INT32_MAX && r.grid_step >= 0 && r.grid_stride >= 0, "bad grid");
+    align_of |= static_cast<uintptr_t>(r.grid_step * in_sz) | static_cast<uintptr_t>(r.grid_stride * in_sz);
+  }
   // with two inputs an fp32 one may go in 32-byte packs, so that a half-precision partner (or
   // table row) still gets its 16 bytes per lane
   const int vb_in = (TWO && in_sz == 4) ? pick_vec_bytes_max(D * in_sz, align_of, 32) : pick_vec_bytes(D * in_sz, align_of);
@@ -964,6 +982,13 @@ int csr_gather_reduce_run(const CsrRequest& r) {
     a.part_lo32[f] = f < a.n_parts ? static_cast<int32_t>(part_first) : INT32_MAX;
     if (f < a.n_parts) part_first += counts_of[f];
   }
+  if (r.grid_rows > 0) {
+    a.grid_rows = static_cast<int32_t>(r.grid_rows);
+    a.grid_shift = 31 + ilog2_ceil(r.grid_rows);
+    a.grid_magic = static_cast<uint32_t>(((uint64_t(1) << a.grid_shift) + r.grid_rows - 1) / r.grid_rows);
+    a.grid_step = r.grid_step;
+    a.grid_stride = r.grid_stride;
+  }
   RECIS_REQUIRE(part_first <= INT32_MAX, "the parts hold %lld rows, more than 32-bit src entries name",
                 (long long)part_first);
   int64_t hot_blocks = 0;
@@ -990,7 +1015,10 @@ int csr_gather_reduce_run(const CsrRequest& r) {
       } else {
         const TIn* rin = static_cast<const TIn*>(r.in1.rows);
         TOut* o = static_cast<TOut*>(r.out);
-        const bool shuffle = a.lpr_log2 >= 3;  // at most eight lane groups per wave
+        // At most sixteen lane groups per wave: a turn of four entries each is 64. With two inputs at most eight: a lane group holds the
+        // entries of a short list, a lane each, and short is up to kCoopLen.
+        static_assert(kCoopLen <= 8, "short lists fit a lane group");
+        const bool shuffle = a.lpr_log2 >= (TWO ? 3 : 2);
         const dim3 grid(a.cold_blocks + hot_blocks), block(kBlock);
         const int64_t fin = std::min<int64_t>((hot_cap + kBlock / kWave - 1) / (kBlock / kWave), 2048);  // a wave per item
         auto launch = [&](auto epi_tag) {

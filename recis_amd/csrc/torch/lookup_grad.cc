@@ -51,6 +51,7 @@ struct LookupBackward : public torch::autograd::Node {
   bool mean = false;
   std::vector<int64_t> batch, seq;   // padded outputs (tile): samples and rows per sample of each
   bool tile = false;
+  bool columns = false;              // one id per sample, of a plan that no other lookup shares
 
   torch::autograd::variable_list apply(torch::autograd::variable_list&& grads) override {
     std::lock_guard<std::mutex> lock(mutex_);
@@ -65,6 +66,7 @@ struct LookupBackward : public torch::autograd::Node {
       table->AcceptTileGrad(index, plan, offsets, batch, seq, grads);
       return {};
     }
+    if (columns && table->AcceptColumnSlices(index, plan, grads, split)) return {};
     std::vector<TensorOrNone> parts;
     parts.reserve(grads.size());
     for (auto& g : grads) parts.push_back(g.defined() ? TensorOrNone(std::move(g)) : c10::nullopt);
@@ -147,6 +149,7 @@ c10::optional<std::vector<at::Tensor>> Hashtable::DenseLookupTrain(const std::ve
     node->saved_index = SavedVariable(std::get<1>(*found), false);
     node->split = split;
     node->first_shape = shapes[0];
+    node->columns = true;
   }
   return outputs_of(out, shapes, split, node);
 }

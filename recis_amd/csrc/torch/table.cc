@@ -954,6 +954,44 @@ std::vector<at::Tensor> Hashtable::LookupPoolReadonly(const std::vector<at::Tens
   return at::split_with_sizes(out, split, 0);
 }
 
+// Gradients of the columns of one lookup, one id per sample, that are column slices of one wide gradient, side by side
+// (what a concatenation of the outputs hands back): summed from where they lie. False: they are something else, or small.
+// Copied into one array first (collect.hip), with the sum left to the optimizer's launch, every row is read and written once more.
+// Summed here, the optimizer's launch is one more and reads the sums. us a step, copied / summed, 39 columns, Adam: 65536 rows of
+// 16 floats 528 / 503, of 16 bfloat16 607 / 523, of 4 floats 496 / 434; 32768 of 16 floats 319 / 309, of 32 413 / 390; 16384 of 16
+// floats, where the host and its launches count, 248 / 278. So the number of rows decides, from a million on. (The sums are taken
+// at once: the slices may be a buffer of the caller's, which is theirs again when the backward returns.)
+constexpr int64_t kColumnSliceRows = int64_t(1) << 20;
+bool Hashtable::AcceptColumnSlices(const at::Tensor& index_in, const BatchPlanPtr& plan, const std::vector<at::Tensor>& grads,
+                                   const std::vector<int64_t>& split) {
+  const int64_t D = slot_group_->EmbSlot()->FlatSize(), n = static_cast<int64_t>(grads.size());
+  const at::Tensor& g0 = grads[0];
+  if (n < 2 || !g0.defined() || g0.device() != device_ || g0.dim() != 2 || g0.stride(1) != 1 || split[0] < 2) return false;
+  const auto type = g0.scalar_type();
+  if (type != at::kFloat && type != at::kBFloat16 && type != at::kHalf) return false;
+  const int64_t bytes = static_cast<int64_t>(g0.element_size());
+  if (n * split[0] < kColumnSliceRows || plan->n() != n * split[0] || g0.stride(0) < n * D) return false;
+  for (int64_t f = 0; f < n; ++f) {
+    const at::Tensor& g = grads[f];
+    if (!g.defined() || g.scalar_type() != type || g.device() != device_ || g.dim() != 2 || g.size(0) != split[f] ||
+        split[f] != split[0] || g.size(1) != D || g.stride(1) != 1 || g.stride(0) != g0.stride(0) || g.is_neg() ||
+        static_cast<const char*>(g.data_ptr()) != static_cast<const char*>(g0.data_ptr()) + f * D * bytes)
+      return false;
+  }
+  const at::Tensor index = SettledRows(index_in, plan);
+  const int64_t U = plan->U();
+  PlannedGrad g;
+  g.index = index;
+  g.key = plan->serial();
+  at::Tensor summed = at::empty({U, D}, g0.options().dtype(at::kFloat));
+  check(recis_csr_gather_reduce_grid(g0.data_ptr(), dtype_code(type), n, split[0], D, g0.stride(0), plan->occ().data_ptr<int32_t>(),
+                                     plan->row_start().data_ptr<int32_t>(), plan->hot_items().data_ptr<int32_t>(), plan->hot_cap(),
+                                     plan->counts().data_ptr<int64_t>(), summed.data_ptr(), U, D, stream_of(device_)));
+  SumPlanned();
+  AcceptSummed(g, summed);
+  return true;
+}
+
 void Hashtable::AcceptSplitGrad(const at::Tensor& index_in, const BatchPlanPtr& plan,
                                 const std::vector<c10::optional<at::Tensor>>& grads, const std::vector<int64_t>& split,
                                 const c10::optional<at::Tensor>& src, const c10::optional<at::Tensor>& coef, int64_t key,

@@ -344,6 +344,9 @@ class Hashtable : public torch::CustomClassHolder {
                                              const std::vector<c10::optional<at::Tensor>>& offsets,
                                              const std::vector<c10::optional<at::Tensor>>& weights,
                                              const c10::optional<std::vector<int64_t>>& tags, bool mean);
+  // Sums gradients that are column slices of one wide array where they lie (see table.cc); false: not such, nothing done.
+  bool AcceptColumnSlices(const at::Tensor& index, const recis::BatchPlanPtr& plan, const std::vector<at::Tensor>& grads,
+                          const std::vector<int64_t>& split);
   // The backward of an output that was handed out in parts (`split` rows each): `grads` are the parts'
   // gradients as autograd delivers them (None = zeros). Consecutive slices of one buffer are used in
   // place, anything else is concatenated; then the count of `plan` is settled (`settle`) and the

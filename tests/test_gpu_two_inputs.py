@@ -12,7 +12,7 @@ LENGTHS = {"ones": [1], "twos": [1, 2], "threes": [1, 3, 2], "short": [1, 2, 4, 
 
 
 @pytest.mark.parametrize("blocks", [1, 3])
-@pytest.mark.parametrize("dim,dtype", [(128, torch.bfloat16), (72, torch.bfloat16), (64, torch.float32), (36, torch.float32),
+@pytest.mark.parametrize("dim,dtype", [(128, torch.bfloat16), (72, torch.bfloat16), (32, torch.bfloat16), (16, torch.float32), (64, torch.float32), (36, torch.float32),
                                        (1030, torch.float32)])
 @pytest.mark.parametrize("lengths", sorted(LENGTHS))
 def test_short_lists_of_two_inputs(rng, lengths, dim, dtype, blocks):
