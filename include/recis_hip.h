@@ -864,6 +864,20 @@ int recis_fused_bucketized_mod(const float* const* in_ptrs, const int64_t* sizes
 int recis_fused_multi_hash(const int64_t* const* in_ptrs, const int64_t* sizes,
                            const int64_t* muls, const int64_t* primes, const int64_t* buckets,
                            int64_t* const* out_ptrs, int64_t n_jobs, void* stream);
+/* Several of the operators above in as few launches as their tables fit (48 jobs each). FARM / MURMUR: in = bytes, aux = offsets [size + 1]
+ * (off_is64), p0 = number of bytes; MOD: p0 = modulus; BUCKET: in = float32, aux = boundaries, p0 = their number (at most
+ * RECIS_FEATURE_MAX_BOUNDARIES), p1 = a positive modulus; MULTI_HASH: p0 = factor, p1 = prime, p2 = buckets. out: int64 [size]. */
+enum { RECIS_FEATURE_FARM = 0, RECIS_FEATURE_MURMUR = 1, RECIS_FEATURE_MOD = 2, RECIS_FEATURE_BUCKET = 3,
+       RECIS_FEATURE_MULTI_HASH = 4 };
+#define RECIS_FEATURE_MAX_BOUNDARIES 2048
+typedef struct recis_feature_job {
+  int kind, off_is64;
+  const void* in;
+  const void* aux;
+  int64_t* out;
+  int64_t size, p0, p1, p2;
+} recis_feature_job;
+int recis_feature_jobs(const recis_feature_job* jobs, int64_t n_jobs, void* stream);
 
 /* ------------------------------------------------------------------------- *
  * Sequence truncation of lists of ragged tensors

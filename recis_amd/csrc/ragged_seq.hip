@@ -56,6 +56,82 @@ __device__ __forceinline__ int64_t block_sum(int64_t v, int64_t* lds) {
   return total;
 }
 
+// Row r of a 2-D truncation: what is kept of it and where that starts; its counts are written (fused_ragged_cutoff_kernel.cu:55-69, 706-727).
+__device__ __forceinline__ int64_t cut_row(const CutJobs& j, int t, int is64, int64_t r, int64_t keep, int64_t beg, int64_t end,
+                                           int64_t& src, int* err) {
+  const int64_t src_len = end > beg ? end - beg : 0;
+  const bool dropped = src_len >= keep;
+  int64_t len = dropped ? keep : src_len;
+  const int64_t drop = dropped ? src_len - keep : 0;
+  if (j.drop_nums[t]) store_index(j.drop_nums[t], is64, r, drop);
+  if (j.pad_nums[t]) store_index(j.pad_nums[t], is64, r, dropped ? 0 : keep - src_len);
+  src = beg + (j.drop_left[t] ? drop : 0);
+  if (len > 0 && (src < 0 || src + len > j.n_values[t])) {
+    raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
+    len = 0;
+  }
+  return len;
+}
+
+// All steps of 2-D truncations of at most kOneThreads * ITEMS rows in one launch, a workgroup per tensor: a wave takes ITEMS times 64
+// consecutive rows, scans them as it goes and keeps their places in registers until the waves know each other's sums. (8 tensors
+// of 8192 rows: 23 us in the three launches below, 16 in this one; with consecutive rows in a thread, every load and store spread
+// over 64 lines, 21. A tensor of more rows would keep one compute unit busy and leave the others idle.)
+constexpr int kOneThreads = 1024;
+constexpr int kOneItems = 16;  // at most
+template <int ITEMS>
+__global__ void __launch_bounds__(kOneThreads) cutoff_one_kernel(CutJobs j, int is64, int64_t* totals, int64_t totals_base,
+                                                                 int* err) {
+  __shared__ int64_t waves[kOneThreads / kWave];
+  const int t = blockIdx.x;
+  const int64_t rows = j.rows[t], keep = j.keep[t];
+  const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
+  const int64_t r0 = static_cast<int64_t>(wave) * ITEMS * kWave + lane;
+  int64_t beg[ITEMS], end[ITEMS];
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int64_t r = r0 + i * kWave;
+    beg[i] = r < rows ? load_index(j.outer[t], is64, r) : 0;
+    end[i] = r < rows ? load_index(j.outer[t], is64, r + 1) : 0;
+  }
+  int64_t sum = 0;  // of the wave so far
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int64_t r = r0 + i * kWave;
+    int64_t len = 0;
+    if (r < rows) {
+      int64_t src;
+      len = cut_row(j, t, is64, r, keep, beg[i], end[i], src, err);
+      j.src[t][r] = src;
+    }
+    int64_t incl = len;
+#pragma unroll
+    for (int o = 1; o < kWave; o <<= 1) {
+      const int64_t up = __shfl_up(incl, o, kWave);
+      if (lane >= o) incl += up;
+    }
+    beg[i] = sum + incl - len;  // the row's place in the wave
+    sum += __shfl(incl, kWave - 1, kWave);
+  }
+  if (lane == 0) waves[wave] = sum;
+  __syncthreads();
+  int64_t before = 0, total = 0;
+#pragma unroll
+  for (int w = 0; w < kOneThreads / kWave; ++w) {
+    if (w < wave) before += waves[w];
+    total += waves[w];
+  }
+#pragma unroll
+  for (int i = 0; i < ITEMS; ++i) {
+    const int64_t r = r0 + i * kWave;
+    if (r < rows) store_index(j.out_off[t], is64, r, before + beg[i]);
+  }
+  if (threadIdx.x == 0) {
+    totals[totals_base + t] = total;
+    store_index(j.out_off[t], is64, rows, total);
+  }
+}
+
 // Step 1. Lengths go into out_off[r] (rescanned in place by step 2c).
 template <bool THREE_D>
 __global__ void __launch_bounds__(kBlock) cutoff_rows_kernel(CutJobs j, int is64, int64_t* block_sums, int* err) {
@@ -72,15 +148,7 @@ __global__ void __launch_bounds__(kBlock) cutoff_rows_kernel(CutJobs j, int is64
     if (r >= out_rows) continue;
     int64_t len, src;
     if (!THREE_D) {
-      // fused_ragged_cutoff_kernel.cu:55-69, 706-727
-      const int64_t beg = load_index(j.outer[t], is64, r), end = load_index(j.outer[t], is64, r + 1);
-      const int64_t src_len = end > beg ? end - beg : 0;
-      const bool dropped = src_len >= keep;
-      len = dropped ? keep : src_len;
-      const int64_t drop = dropped ? src_len - keep : 0;
-      if (j.drop_nums[t]) store_index(j.drop_nums[t], is64, r, drop);
-      if (j.pad_nums[t]) store_index(j.pad_nums[t], is64, r, dropped ? 0 : keep - src_len);
-      src = beg + (j.drop_left[t] ? drop : 0);
+      len = cut_row(j, t, is64, r, keep, load_index(j.outer[t], is64, r), load_index(j.outer[t], is64, r + 1), src, err);
     } else {
       // fused_ragged_cutoff_kernel.cu:300-337
       const int64_t seq = r / keep, col = r % keep;
@@ -117,7 +185,7 @@ __global__ void __launch_bounds__(kBlock) cutoff_rows_kernel(CutJobs j, int is64
         }
       }
     }
-    if (len > 0 && (src < 0 || src + len > j.n_values[t])) {
+    if (THREE_D && len > 0 && (src < 0 || src + len > j.n_values[t])) {
       raise_device_error(err, RECIS_DEVERR_INDEX_RANGE);
       len = 0;
     }
@@ -649,6 +717,16 @@ extern "C" int recis_ragged_cutoff_rows(const void* const* outer_ptrs, const voi
       n_sums += (j.out_rows[k] + kRowsPerBlock - 1) / kRowsPerBlock;
       // the outer offsets of a 3-D output (rows + 1 entries) are written by the same grid
       max_rows = std::max(max_rows, std::max(j.out_rows[k], three_d ? j.rows[k] + 1 : 0));
+    }
+    if (!three_d && max_rows <= kOneThreads * kOneItems) {
+      RECIS_TIME_KERNEL("cutoff_one_kernel", stream) {
+        if (max_rows <= kOneThreads * kOneItems / 2)
+          cutoff_one_kernel<kOneItems / 2><<<dim3(cnt), dim3(kOneThreads), 0, stream>>>(j, off_is64, totals_dev, first, err);
+        else
+          cutoff_one_kernel<kOneItems><<<dim3(cnt), dim3(kOneThreads), 0, stream>>>(j, off_is64, totals_dev, first, err);
+      }
+      RECIS_LAUNCH_CHECK();
+      continue;
     }
     void* ws = nullptr;
     int rc = get_workspace(stream, static_cast<size_t>(std::max<int64_t>(n_sums, 1)) * sizeof(int64_t), &ws);

@@ -1090,6 +1090,9 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
   for (int64_t k = 0; k < n_jobs; ++k)
     if (primes[k] == 0 || buckets[k] == 0) return {};
   const int64_t n_direct = cut_values.size();
+  for (const TensorList* list : {&hash_offsets, &mod_values, &bucket_values, &multi_values})
+    for (const auto& t : *list)
+      if (t.numel() >= INT32_MAX - 4096) return {};  // (columns past the one launch's indices)
   for (int64_t k = 0; k < n_cut; ++k) {
     TORCH_CHECK(cut_from[k] >= -n_direct && cut_from[k] < n_hash + n_mod, "feature_chains: bad cut_from");
     if (cut_offsets[k].scalar_type() != cut_offsets[0].scalar_type() || cut_offsets[k].numel() < 1 || keep[k] < 0) return {};
@@ -1178,52 +1181,53 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
     arrived.record();
   }
 
-  // ---- the operators in front, a launch per kind
-  for (int64_t kind = 0; kind < 2; ++kind) {
-    std::vector<const int8_t*> vp;
-    std::vector<const void*> fp;
-    std::vector<int64_t> sizes, strings;
-    std::vector<int64_t*> op;
-    for (int64_t k = 0; k < n_hash; ++k) {
-      if (hash_kinds[k] != kind) continue;
-      vp.push_back(static_cast<const int8_t*>(hash_in[k].data_ptr()));
-      fp.push_back(hash_off[k].data_ptr());
-      sizes.push_back(hash_in[k].numel());
-      strings.push_back(n_strings[k]);
-      op.push_back(outs[k].data_ptr<int64_t>());
-    }
-    if (!vp.empty())
-      check(recis_fused_hash(vp.data(), sizes.data(), fp.data(), index_kind(hash_off[0], "offsets"), strings.data(), op.data(),
-                             static_cast<int64_t>(vp.size()), static_cast<int>(kind), stream));
-  }
-  auto out_ptrs = [&](int64_t first, int64_t n) {
-    std::vector<int64_t*> p(n);
-    for (int64_t k = 0; k < n; ++k) p[k] = outs[first + k].data_ptr<int64_t>();
-    return p;
+  // ---- the operators in front, all in one launch (but buckets of more boundaries than that takes, and columns past its indices)
+  std::vector<recis_feature_job> jobs;
+  std::vector<const float*> long_in, long_bounds;
+  std::vector<int64_t> long_sizes, long_lens, long_mods;
+  std::vector<int64_t*> long_out;
+  auto add_job = [&](int kind, const void* in, const void* aux, int64_t* out, int64_t size, int64_t p0, int64_t p1, int64_t p2) {
+    recis_feature_job j{};
+    j.kind = kind;
+    j.off_is64 = n_hash ? index_kind(hash_off[0], "offsets") : 0;
+    j.in = in;
+    j.aux = aux;
+    j.out = out;
+    j.size = size;
+    j.p0 = p0;
+    j.p1 = p1;
+    j.p2 = p2;
+    jobs.push_back(j);
   };
-  if (n_mod) {
-    auto ip = host_ptrs<int64_t>(mod_in);
-    auto op = out_ptrs(n_hash, n_mod);
-    auto sizes = numels(mod_in);
-    check(recis_fused_uint64_mod(ip.data(), sizes.data(), mods.data(), op.data(), n_mod, stream));
-  }
-  if (n_bucket) {
-    auto ip = host_ptrs<float>(bucket_in), bp = host_ptrs<float>(bucket_bd);
-    auto op = out_ptrs(n_hash + n_mod, n_bucket);
-    auto sizes = numels(bucket_in), lens = numels(bucket_bd);
-    check(recis_fused_bucketized_mod(ip.data(), sizes.data(), bp.data(), lens.data(), bucket_mods.data(), op.data(), n_bucket,
-                                     stream));
-  }
-  if (n_jobs) {
-    std::vector<const int64_t*> ip;
-    std::vector<int64_t> sizes;
-    for (int64_t k = 0; k < n_multi; ++k) {
-      ip.insert(ip.end(), multi_counts[k], multi_in[k].data_ptr<int64_t>());
-      sizes.insert(sizes.end(), multi_counts[k], multi_in[k].numel());
+  jobs.reserve(outs.size());
+  for (int64_t k = 0; k < n_hash; ++k)
+    add_job(hash_kinds[k] == 0 ? RECIS_FEATURE_FARM : RECIS_FEATURE_MURMUR, hash_in[k].data_ptr(), hash_off[k].data_ptr(),
+            outs[k].data_ptr<int64_t>(), n_strings[k], hash_in[k].numel(), 0, 0);
+  for (int64_t k = 0; k < n_mod; ++k)
+    add_job(RECIS_FEATURE_MOD, mod_in[k].data_ptr(), nullptr, outs[n_hash + k].data_ptr<int64_t>(), mod_in[k].numel(), mods[k], 0, 0);
+  for (int64_t k = 0; k < n_bucket; ++k) {
+    int64_t* out = outs[n_hash + n_mod + k].data_ptr<int64_t>();
+    if (bucket_bd[k].numel() <= RECIS_FEATURE_MAX_BOUNDARIES) {
+      add_job(RECIS_FEATURE_BUCKET, bucket_in[k].data_ptr(), bucket_bd[k].data_ptr(), out, bucket_in[k].numel(),
+              bucket_bd[k].numel(), bucket_mods[k], 0);
+    } else {
+      long_in.push_back(bucket_in[k].data_ptr<float>());
+      long_bounds.push_back(bucket_bd[k].data_ptr<float>());
+      long_sizes.push_back(bucket_in[k].numel());
+      long_lens.push_back(bucket_bd[k].numel());
+      long_mods.push_back(bucket_mods[k]);
+      long_out.push_back(out);
     }
-    auto op = out_ptrs(multi_first, n_jobs);
-    check(recis_fused_multi_hash(ip.data(), sizes.data(), muls.data(), primes.data(), buckets.data(), op.data(), n_jobs, stream));
   }
+  for (int64_t k = 0, job = 0; k < n_multi; ++k) {
+    for (int64_t c = 0; c < multi_counts[k]; ++c, ++job)
+      add_job(RECIS_FEATURE_MULTI_HASH, multi_in[k].data_ptr(), nullptr, outs[multi_first + job].data_ptr<int64_t>(),
+              multi_in[k].numel(), muls[job], primes[job], buckets[job]);
+  }
+  check(recis_feature_jobs(jobs.data(), static_cast<int64_t>(jobs.size()), stream));
+  if (!long_in.empty())
+    check(recis_fused_bucketized_mod(long_in.data(), long_sizes.data(), long_bounds.data(), long_lens.data(), long_mods.data(),
+                                     long_out.data(), static_cast<int64_t>(long_in.size()), stream));
 
   // ---- the truncated values
   if (n_cut) {

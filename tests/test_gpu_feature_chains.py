@@ -113,3 +113,55 @@ def test_what_the_call_does_not_take_runs_operator_by_operator(rng):
         FeatureEngine(checked())(data)
     other = [Feature("b").add_op(SelectField("real")).add_op(Bucketize([0.0]))]
     assert FeatureEngine(other)._chains is None
+
+
+def test_more_columns_than_a_launch_takes_and_long_boundaries(rng):
+    data = {"c%d" % k: torch.from_numpy(rng.integers(-(2**62), 2**62, size=int(n))).cuda()
+            for k, n in enumerate(rng.integers(0, 4000, size=60))}
+    data.update({"r%d" % k: torch.randn(3001).cuda() for k in range(4)})
+    mods = [1, 2, 2**31 - 1, 2**31, 2**32 - 1, 2**32, 2**40 + 3, -5]
+
+    def features():
+        out = [Feature("c%d" % k).add_op(SelectField("c%d" % k)).add_op(Mod(mods[k % len(mods)])) for k in range(60)]
+        for k, n in enumerate((0, 2048, 2049, 9000)):
+            bounds = torch.sort(torch.randn(n, generator=torch.Generator().manual_seed(k))).values
+            out.append(Feature("r%d" % k).add_op(SelectField("r%d" % k)).add_op(Bucketize(bounds)).add_op(Mod(700)))
+        return out
+
+    _both(features, data)
+    assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("rows", [0, 1, 1023, 1025, 8192, 8193, 16384, 16385])
+@pytest.mark.parametrize("off_dtype", [torch.int32, torch.int64])
+def test_truncations_around_the_rows_of_one_launch(rng, rows, off_dtype):
+    """Up to 16384 rows a tensor are truncated by one workgroup, more in three launches."""
+    from recis_amd import ops
+
+    seqs = [(_offsets(rng, r, 12, off_dtype), k, side) for r, k, side in
+            ((rows, 5, True), (max(0, rows - 1), 0, False), (rows // 2, 100, False))]
+    values = [torch.from_numpy(rng.integers(0, 10**9, size=int(o[-1]))) for o, _, _ in seqs]
+    vals, offs, drops, pads, _, _ = ops.fused_ragged_cutoff([v.cuda() for v in values], [o.cuda() for o, _, _ in seqs],
+                                                            [k for _, k, _ in seqs], [s for _, _, s in seqs], [False] * 3)
+    for t, (off, keep, left) in enumerate(seqs):
+        lens = (off[1:] - off[:-1]).long()
+        kept = lens.clamp(max=keep)
+        want = torch.cat([torch.zeros(1, dtype=torch.int64), torch.cumsum(kept, 0)])
+        assert torch.equal(offs[t].cpu().long(), want) and offs[t].dtype == off_dtype
+        assert torch.equal(drops[t].cpu().long(), lens - kept) and torch.equal(pads[t].cpu().long(), keep - kept)
+        start = off[:-1].long() + (lens - kept if left else 0)
+        at = torch.arange(int(want[-1])) - torch.repeat_interleave(want[:-1], kept) + torch.repeat_interleave(start, kept)
+        assert torch.equal(vals[t].cpu(), values[t][at])
+    assert _lib.poll_device_errors() == 0
+
+
+def test_offsets_out_of_range_are_reported_by_the_one_launch():
+    from recis_amd import ops
+
+    values = torch.arange(10).cuda()
+    for bad in ([0, 4, 11], [-2, 3, 10], [0, 7, 3]):  # past the values, before them, decreasing (an empty row)
+        off = torch.tensor(bad).cuda()
+        vals, offs, *_ = ops.fused_ragged_cutoff([values], [off], [20], [False], [False])
+        lens = [e - b if 0 <= b <= e <= 10 else 0 for b, e in zip(bad[:-1], bad[1:])]
+        assert offs[0].cpu().tolist() == [0, lens[0], sum(lens)]
+        assert _lib.poll_device_errors() == (0 if bad == [0, 7, 3] else 1)
