@@ -310,6 +310,17 @@ def _check_plan(ids):
     return p
 
 
+@pytest.mark.parametrize("n", [5, 2047, 4100, 40_000, 81_921, 174_000, 178_500])
+def test_plan_around_the_sizes_whose_columns_the_scatter_sums_itself(rng, n):
+    """Up to 16384 words of histogram (174 k ids: 84 tiles of 192 columns) without a column scan; a heavy id, repeats, the
+    reserved values and ids that occur once."""
+    ids = np.where(rng.random(n) < 0.4, 77, np.where(rng.random(n) < 0.5, rng.integers(-2, 500, size=n), rng.integers(-2**60, 2**60, size=n)))
+    _check_plan(ids)
+    _check_plan(rng.integers(0, 2**50, size=n))
+    _check_plan(np.full(n, -1))
+
+
+
 @pytest.mark.parametrize("n,hi", [(0, 10), (1, 10), (1000, 50), (1025, 10**6), (300000, 40), (200000, 3000),
                                   (1000000, 10**7), (3000000, 10**12), (8000000, 10**12),
                                   (2047, 10**6), (2049, 10**6), (4097, 20), (256 * 10240 - 1, 300),
