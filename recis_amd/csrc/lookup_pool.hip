@@ -436,10 +436,7 @@ extern "C" int recis_lookup_pool_readonly(recis_idmap* map, const recis_lookup_j
   };
   // Features of several ids per segment first: workgroups start in the order of their index, and what starts last should be
   // short.
-  for (int64_t turn = 0, row0 = 0; turn < 2 * n_jobs; row0 += jobs[turn++ % n_jobs].n_seg) {
-    if (turn == n_jobs) row0 = 0;
-    const recis_lookup_job& q = jobs[turn % n_jobs];
-    if (q.n_seg == 0 || (q.n_ids > q.n_seg) != (turn < n_jobs)) continue;
+  auto add = [&](const recis_lookup_job& q, int64_t row0) -> int {
     const int rg = groups_of(q);
     const int teams = kBlock >> (g.lpr_log2 + rg);
     const int64_t avg = (q.n_ids + q.n_seg - 1) / q.n_seg;
@@ -462,6 +459,14 @@ extern "C" int recis_lookup_pool_readonly(recis_idmap* map, const recis_lookup_j
     tiles += (q.n_seg + (teams << spt) - 1) / (teams << spt);
     if (J.n_jobs == kPoolJobs) {
       if (int rc = launch()) return rc;
+    }
+    return RECIS_OK;
+  };
+  for (const bool several : {true, false}) {
+    int64_t row0 = 0;
+    for (int64_t k = 0; k < n_jobs; row0 += jobs[k++].n_seg) {
+      if (jobs[k].n_seg == 0 || (jobs[k].n_ids > jobs[k].n_seg) != several) continue;
+      if (int rc = add(jobs[k], row0)) return rc;
     }
   }
   return launch();
