@@ -760,6 +760,63 @@ seg_pool_bwd_fast_kernel(const TG* __restrict__ grad_out, TOut* __restrict__ gra
   }
 }
 
+// The same onto rows in order (and the maximum's, see seg_max_bwd_rows_kernel), kBwdWaves waves per segment instead of one. What binds
+// these kernels is the stream of their stores, and that runs the faster the less memory the resident workgroups are spread over: a
+// fill by workgroups of 8 KB in runs on one XCD reaches 6.9 TB/s, of 16 KB 6.6, of 32 KB 6.3 (four segments of 30 rows of 256 bytes).
+// 4 GB of such segments: sum 753, mean 708, max 769 us with a wave per segment, now 704, 681 and 736. (Four waves: 870, 650 and 890: each waits for its gradient to store a
+// microsecond; the gradient asked for beside the bounds: 843, 680 and 910 with two.)
+constexpr int kBwdWaves = 2;
+template <typename TG, typename TOut, int VEC, bool MAX>
+__global__ void __launch_bounds__(kBlock)
+seg_bwd_wide_kernel(const TG* __restrict__ grad_out, const int32_t* __restrict__ argmax, TOut* __restrict__ grad_unique, SegArgs a) {
+  constexpr int kPerBlock = kBlock / kWave / kBwdWaves;
+  const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
+  const int64_t s = static_cast<int64_t>(block_in_runs()) * kPerBlock + wave / kBwdWaves;
+  if (s >= a.S) return;  // whole waves leave together
+  int64_t start = load_index(a.offs, a.off64, s);
+  int64_t end = load_index(a.offs, a.off64, s + 1);
+  if (start < 0 || end > a.B || end < start) {
+    raise_device_error(a.err, RECIS_DEVERR_OFFSETS);
+    start = end = 0;
+  }
+  const int groups = kWave >> a.lpr_log2;
+  const int first = (wave % kBwdWaves) * groups + (lane >> a.lpr_log2), step = kBwdWaves * groups;
+  const int cl = lane & ((1 << a.lpr_log2) - 1);
+  const int D = a.D;
+  const float scale = (!MAX && a.mean && end > start) ? 1.0f / static_cast<float>(end - start) : 1.0f;
+  if (end > a.U) {  // (rows in order: occurrence r is row r)
+    raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
+    end = a.U;
+  }
+  for (int c0 = cl * VEC; c0 < D; c0 += VEC << a.lpr_log2) {
+    float g[VEC];
+    int32_t win[VEC];
+    load_pack<TG, VEC>(grad_out + s * D + c0, g);
+    if constexpr (MAX) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) win[j] = argmax[s * D + c0 + j];
+    } else {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) g[j] *= scale;
+    }
+    for (int64_t r = start + first; r < end; r += step) {
+      TOut* dst = grad_unique + r * D + c0;
+      if constexpr (MAX) {
+        float v[VEC];
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) v[j] = win[j] == static_cast<int32_t>(r) ? g[j] : 0.f;
+        if (a.nt_out) {
+          store_pack_stream<TOut, VEC>(dst, v);
+        } else {
+          store_pack<TOut, VEC>(dst, v);
+        }
+      } else {
+        store_pack_stream<TOut, VEC>(dst, g);
+      }
+    }
+  }
+}
+
 template <typename TG, typename TOut, int VEC, bool ATOMIC>
 __global__ void __launch_bounds__(kBlock)
 seg_pool_bwd_kernel(const TG* __restrict__ grad_out, TOut* __restrict__ grad_unique, SegArgs a) {
@@ -1300,6 +1357,9 @@ extern "C" int recis_segment_reduce_backward(
   a.team_log2 = pick_team_log2(B, S, lpr_log2);
   a.mean = (mode == RECIS_MEAN);
   a.in_runs = B * D * out_sz * (kBlock >> a.team_log2) >= kRunWriteBytes * S;
+  // rows in order, a wave per segment and enough of them: several waves per segment (see seg_bwd_wide_kernel)
+  const bool wide = a.rev == nullptr && a.in_runs && (1 << a.team_log2) == kWave;
+  const int64_t wide_grid = (S * kBwdWaves + kBlock / kWave - 1) / (kBlock / kWave);
   // 1 GiB is far past what L2 and the 256 MB memory-side cache keep for the next kernel
   a.nt_out = U * D * out_sz >= (int64_t(1) << 30);
   a.nt_in = 0;
@@ -1338,7 +1398,9 @@ extern "C" int recis_segment_reduce_backward(
             const TG* gsrc = static_cast<const TG*>(grad_out);
             TOut* gdst = static_cast<TOut*>(grad_unique);
             RECIS_TIME_KERNEL("seg_max_bwd_kernel", stream)
-            if (a.rev == nullptr)
+            if (wide)
+              seg_bwd_wide_kernel<TG, TOut, VEC, true><<<dim3(wide_grid), dim3(kBlock), 0, stream>>>(gsrc, argmax, gdst, a);
+            else if (a.rev == nullptr)
               seg_max_bwd_rows_kernel<TG, TOut, VEC, kFastPlain><<<dim3(grid), dim3(kBlock), 0, stream>>>(gsrc, argmax, gdst, a);
             else if (!a.rev64)
               seg_max_bwd_rows_kernel<TG, TOut, VEC, kFastRev32><<<dim3(grid), dim3(kBlock), 0, stream>>>(gsrc, argmax, gdst, a);
@@ -1378,7 +1440,9 @@ extern "C" int recis_segment_reduce_backward(
           const bool fast = unique && a.weight == nullptr && U < (int64_t(1) << 31) && a.team_log2 > a.lpr_log2;
           if (fast) {
             RECIS_TIME_KERNEL("seg_pool_bwd_kernel", stream)
-            if (a.rev == nullptr)
+            if (wide)
+              seg_bwd_wide_kernel<TG, TOut, VEC, false><<<dim3(wide_grid), dim3(kBlock), 0, stream>>>(gsrc, argmax, gdst, a);
+            else if (a.rev == nullptr)
               seg_pool_bwd_fast_kernel<TG, TOut, VEC, kFastPlain><<<dim3(grid), dim3(kBlock), 0, stream>>>(gsrc, gdst, a);
             else if (!a.rev64)
               seg_pool_bwd_fast_kernel<TG, TOut, VEC, kFastRev32><<<dim3(grid), dim3(kBlock), 0, stream>>>(gsrc, gdst, a);

@@ -518,3 +518,32 @@ def test_long_segments_out_of_the_table_blocks(dtype, D):
         copied = ops.segment_reduce_forward(rows, None, rev, off, mode, out_dtype=torch.float32)
         assert torch.equal(direct, copied)                   # the same rows summed in the same order
     assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("dim,dtype", [(64, torch.float32), (40, torch.float32), (128, torch.bfloat16), (100, torch.float16)])
+@pytest.mark.parametrize("combiner", ["sum", "mean", "max"])
+def test_backward_of_long_segments_in_order(rng, dim, dtype, combiner):
+    """Two waves per segment: segments of no row, of fewer rows than the waves take at a time, of hundreds; each value is one
+    product, so it is exact."""
+    from recis_amd.nn.functional.embedding_ops import ragged_embedding_segment_reduce
+
+    lens = np.concatenate([[0, 1, 2, 7, 8, 9, 300, 0], rng.integers(60, 140, size=301), [0]])
+    off = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)).cuda()
+    values = torch.randn(int(lens.sum()), dim, device="cuda").to(dtype).requires_grad_(True)
+    out = ragged_embedding_segment_reduce(values, None, None, off, combiner)
+    up = torch.randn(len(lens), dim, device="cuda").to(out.dtype)
+    (got,) = torch.autograd.grad(out, values, up)
+    seg = torch.repeat_interleave(torch.arange(len(lens), device="cuda"), torch.from_numpy(lens).cuda())
+    want = up[seg].float()
+    if combiner == "mean":
+        want = want * (1.0 / torch.from_numpy(lens).cuda().clamp(min=1).float())[seg][:, None]
+    elif combiner == "max":
+        best = torch.full((len(lens), dim), -float("inf"), device="cuda").scatter_reduce(
+            0, seg[:, None].expand(-1, dim), values.detach().float(), "amax")
+        hit = values.detach().float() == best[seg]
+        row = torch.arange(len(seg), device="cuda")[:, None].expand(-1, dim)
+        first = torch.full((len(lens), dim), len(seg), device="cuda").scatter_reduce(
+            0, seg[:, None].expand(-1, dim), torch.where(hit, row, len(seg)), "amin")
+        want = torch.where(first[seg] == row, want, torch.zeros_like(want))
+    assert torch.equal(got, want.to(got.dtype))
+    assert _lib.poll_device_errors() == 0
