@@ -424,9 +424,8 @@ constexpr int kCoopLen = 8;  // longer lists are shared among the lane groups of
 // walk the hot work items (row, chunk of kHotChunk occurrences): four waves share the chunk,
 // fold their sums through LDS and store ONE partial row per item; csr_hot_finish_kernel adds up
 // the partial rows of every hot row in chunk order. No atomics anywhere.
-// SHUFFLE: long lists go through wave_gather_range, for up to sixteen lane groups a wave, i.e. rows of 64 bytes and more (rows of
-// 64 bytes, their entries loaded by every group for itself / through shuffles: 160 k entries 24.2 / 22.3 us, 43 k 14.5 / 10.8);
-// otherwise every group loads its own entries.
+// SHUFFLE: long lists go through wave_gather_range, for up to sixteen lane groups a wave (rows of 64 bytes and more, see the rule at
+// the launch); otherwise every group loads its own entries.
 // TIn2 != void: every list entry adds a row of a second input as well (see CsrArgs); PARTS then
 // says that the second input comes in parts.
 template <typename TIn, typename TOut, int VEC, bool SHUFFLE, bool PARTS = false, int EPI = kEpiStore,
@@ -1016,9 +1015,13 @@ int csr_gather_reduce_run(const CsrRequest& r) {
         const TIn* rin = static_cast<const TIn*>(r.in1.rows);
         TOut* o = static_cast<TOut*>(r.out);
         // At most sixteen lane groups per wave: a turn of four entries each is 64. With two inputs at most eight: a lane group holds the
-        // entries of a short list, a lane each, and short is up to kCoopLen.
+        // entries of a short list, a lane each, and short is up to kCoopLen. Sixteen groups and a row update: only while the
+        // long lists count, up to kShuffleUnique unique rows; with more, most lists hold an entry or two and the kernel
+        // without shuffles, which knows its rows' places early, is the faster (update of rows of 64 bytes, without / with: 13 k
+        // unique 14.5 / 10.8 us, 46 k 24.2 / 22.3, 850 k 132 / 141).
         static_assert(kCoopLen <= 8, "short lists fit a lane group");
-        const bool shuffle = a.lpr_log2 >= (TWO ? 3 : 2);
+        constexpr int64_t kShuffleUnique = int64_t(1) << 17;
+        const bool shuffle = a.lpr_log2 >= 3 || (!TWO && a.lpr_log2 == 2 && (epi == kEpiStore || U <= kShuffleUnique));
         const dim3 grid(a.cold_blocks + hot_blocks), block(kBlock);
         const int64_t fin = std::min<int64_t>((hot_cap + kBlock / kWave - 1) / (kBlock / kWave), 2048);  // a wave per item
         auto launch = [&](auto epi_tag) {
