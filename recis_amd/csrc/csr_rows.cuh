@@ -1019,9 +1019,13 @@ int csr_gather_reduce_run(const CsrRequest& r) {
         // long lists count, up to kShuffleUnique unique rows; with more, most lists hold an entry or two and the kernel
         // without shuffles, which knows its rows' places early, is the faster (update of rows of 64 bytes, without / with: 13 k
         // unique 14.5 / 10.8 us, 46 k 24.2 / 22.3, 850 k 132 / 141).
-        static_assert(kCoopLen <= 8, "short lists fit a lane group");
+        // A lane group that is the whole wave shares its lists with nobody, so there every list is short, and without work items
+        // (hot_cap == 0) of any length: those go to the kernels that take the entries as they come.
+        static_assert(kCoopLen <= 8 && kHotLen <= kWave, "short lists fit a lane group");
         constexpr int64_t kShuffleUnique = int64_t(1) << 17;
-        const bool shuffle = a.lpr_log2 >= 3 || (!TWO && a.lpr_log2 == 2 && (epi == kEpiStore || U <= kShuffleUnique));
+        const bool lists_fit = !TWO || a.lpr_log2 < 6 || hot_cap > 0;
+        const bool shuffle = (a.lpr_log2 >= 3 && lists_fit) ||
+                             (!TWO && a.lpr_log2 == 2 && (epi == kEpiStore || U <= kShuffleUnique));
         const dim3 grid(a.cold_blocks + hot_blocks), block(kBlock);
         const int64_t fin = std::min<int64_t>((hot_cap + kBlock / kWave - 1) / (kBlock / kWave), 2048);  // a wave per item
         auto launch = [&](auto epi_tag) {

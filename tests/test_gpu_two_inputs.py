@@ -1,5 +1,7 @@
 """The gather-reduce with two inputs on short lists: the lists of a wave are worked side by side, one, two or four rows of
 each at a time as the longest of them asks, and a key's table row is asked for before its gradient is summed."""
+import types
+
 import numpy as np
 import pytest
 import torch
@@ -73,4 +75,48 @@ def test_short_lists_of_two_inputs(rng, lengths, dim, dtype, blocks):
                                  size_of_block)
     for a, b in zip(w + s0 + s1, w2 + m0 + m1):
         assert torch.equal(torch.nan_to_num(a.float()), torch.nan_to_num(b.float()))
+    assert _lib.poll_device_errors() == 0
+
+
+@pytest.mark.parametrize("blocks", [1, 3])
+@pytest.mark.parametrize("dim,dtype", [(128, torch.float32), (132, torch.float32), (256, torch.float32), (1030, torch.float32),
+                                       (33, torch.float32), (264, torch.bfloat16)])
+def test_lists_of_any_length_without_work_items(rng, dim, dtype, blocks):
+    """hot_cap == 0: no list is too long for the row kernel, also where a row takes all lanes of a wave."""
+    lens = [64, 65, 200, 1, 66, 100, 130, 8, 9]
+    uniques = len(lens)
+    ids = rng.permutation(np.repeat(rng.choice(10**9, uniques, replace=False), lens))
+    n = len(ids)
+    made = ops.ids_unique_plan(torch.from_numpy(ids).cuda())
+    plan = types.SimpleNamespace(U=uniques, row_start=made.row_start, hot_items=None, hot_cap=0, counts=made.counts)
+    occ = made.occ[:n].cpu().numpy()
+    # small whole numbers: every sum is exact in float
+    rows1, rows2 = (torch.randint(-8, 9, (n, dim)).to(dtype) for _ in range(2))
+    src1 = rng.permutation(n).astype(np.int32)
+    coef = rng.integers(-3, 4, size=n).astype(np.float32)
+    first = (rows1.cuda(), torch.from_numpy(src1).cuda(), torch.from_numpy(coef).cuda())
+    second = (rows2.cuda(), torch.from_numpy(occ).cuda(), None)
+    of = np.repeat(np.arange(uniques), np.diff(made.row_start.cpu().numpy()[: uniques + 1]))
+    want = np.zeros((uniques, dim))
+    np.add.at(want, of, coef[:, None] * rows1.double().numpy()[src1] + rows2.double().numpy()[occ])
+    np.testing.assert_array_equal(ops.csr_gather_reduce2(plan, first, second).cpu().numpy(), want)
+
+    size_of_block = uniques
+    index = torch.from_numpy(rng.permutation(blocks * size_of_block)[:uniques]).cuda()
+    total = torch.from_numpy(want).float().cuda()
+    def slot():
+        t = (torch.rand(blocks * size_of_block, dim, generator=torch.Generator().manual_seed(3)) + 0.1).to(dtype)
+        return [b.cuda() for b in torch.split(t, size_of_block)]
+    w, acc, w2, acc2 = slot(), slot(), slot(), slot()
+    ops.block_apply_adagrad(index, total, w, acc, 1e-2, 1e-8, size_of_block)
+    ops.csr_gather_reduce2_adagrad(plan, first, second, index, w2, acc2, 1e-2, 1e-8, size_of_block)
+    for a, b in zip(w + acc, w2 + acc2):
+        assert torch.equal(a, b)
+    s0, s1, m0, m1 = slot(), slot(), slot(), slot()
+    powers = [torch.full((1,), v, dtype=torch.float64, device="cuda") for v in (0.9, 0.999, 0.9, 0.999)]
+    ops.block_apply_adamw(index, total, w, powers[0], powers[1], None, s0, s1, 1e-2, 0.9, 0.999, 0.99, 1e-8, size_of_block)
+    ops.csr_gather_reduce2_adamw(plan, first, second, index, w2, powers[2], powers[3], m0, m1, 1e-2, 0.9, 0.999, 0.99, 1e-8,
+                                 size_of_block)
+    for a, b in zip(w + s0 + s1, w2 + m0 + m1):
+        assert torch.equal(a, b)
     assert _lib.poll_device_errors() == 0
