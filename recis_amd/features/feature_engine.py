@@ -73,6 +73,13 @@ _FUSED = {Mod: _fused_mod, Bucketize: _fused_bucketize, Hash: _fused_hash, IDMul
           SequenceTruncate: sequence_truncate, _CHAIN: _fused_bucketize_mod}
 
 
+def _int64s(values):
+    """Python numbers as the operators hand them to the kernels, modulo 2^64: a modulus may be any uint64."""
+    if not values or (max(values) < 2**63 and min(values) >= -2**63):
+        return values
+    return [(v + 2**63) % 2**64 - 2**63 for v in values]
+
+
 class _Chains:
     """The features of an engine whose operators are all of the forms that ``feature_chains`` runs in one call: a selected
     field, then one of Hash, Mod, Bucketize + Mod, IDMultiHash or nothing, the ids possibly truncated. (31 features, batch 8192:
@@ -138,13 +145,13 @@ class _Chains:
         outs = ops.recis_ops().feature_chains(
             [vals[p] for p, _ in self.hash], [xs[p]._offsets[-1] for p, _ in self.hash],
             [1 if op.hash_type == "murmur" else 0 for _, op in self.hash],
-            [vals[p] for p, _ in self.mod], [op.mod_value for _, op in self.mod],
+            [vals[p] for p, _ in self.mod], _int64s([op.mod_value for _, op in self.mod]),
             [vals[p] for p, _, _ in self.bucket], [b.boundary_on(vals[p].device) for p, b, _ in self.bucket],
             [m.mod_value for _, _, m in self.bucket],
             [vals[p] for p, _ in self.multi], [len(op.muls) for _, op in self.multi],
-            [v for _, op in self.multi for v in op.muls], [v for _, op in self.multi for v in op.primes],
-            [v for _, op in self.multi for v in op.num_buckets],
-            direct, cut_from, cut_offsets, [op.seq_len for _, op in self.cut],
+            _int64s([v for _, op in self.multi for v in op.muls]), _int64s([v for _, op in self.multi for v in op.primes]),
+            _int64s([v for _, op in self.multi for v in op.num_buckets]),
+            direct, cut_from, cut_offsets, _int64s([op.seq_len for _, op in self.cut]),
             [op.truncate_side == "left" for _, op in self.cut])
         if not outs:
             return None

@@ -132,6 +132,18 @@ def test_more_columns_than_a_launch_takes_and_long_boundaries(rng):
     assert _lib.poll_device_errors() == 0
 
 
+@pytest.mark.parametrize("mods", [[2**63 + 5], [2**64 - 59], [2**63, 2**63 - 1, 2**64 - 1, 2**64 + 7, 2**63 + 1]])
+def test_moduli_are_any_uint64(rng, mods):
+    data = {"c%d" % k: torch.from_numpy(rng.integers(-(2**63), 2**63 - 1, size=300)).cuda() for k in range(len(mods))}
+    features = lambda: [Feature("c%d" % k).add_op(SelectField("c%d" % k)).add_op(Mod(m)) for k, m in enumerate(mods)]
+    got = _both(features, data)(data)
+    for k, m in enumerate(mods):
+        want = [(x % 2**64) % (m % 2**64) for x in data["c%d" % k].tolist()]
+        assert [x % 2**64 for x in got["c%d" % k].tolist()] == want
+    with pytest.raises(RuntimeError):  # 0 modulo 2^64
+        FeatureEngine([Feature("c0").add_op(SelectField("c0")).add_op(Mod(2**64))])(data)
+
+
 @pytest.mark.parametrize("rows", [0, 1, 1023, 1025, 8192, 8193, 16384, 16385])
 @pytest.mark.parametrize("off_dtype", [torch.int32, torch.int64])
 def test_truncations_around_the_rows_of_one_launch(rng, rows, off_dtype):
