@@ -758,9 +758,11 @@ std::tuple<at::Tensor, at::Tensor> Hashtable::EvictUnseen(const std::string& sta
   auto stamps = slot_group_->GetSlotByName(stamp_slot);
   TORCH_CHECK((stamps->Dtype() == at::kLong || stamps->Dtype() == at::kInt) && stamps->FlatSize() == 1,
               "the stamp slot must be int32/int64 of width 1");
-  const bool on_device = step.has_value() && step->defined();
-  TORCH_CHECK(!on_device || (step->device() == device_ && step->scalar_type() == at::kLong && step->numel() == 1),
-              "the step must be one int64 on the table's device");
+  at::Tensor counter;  // the step where the sweep reads it (one counter may serve the tables of several devices)
+  if (step.has_value() && step->defined()) {
+    TORCH_CHECK(step->scalar_type() == at::kLong && step->numel() == 1, "the step must be one int64");
+    counter = step->to(device_);
+  }
   void* stream = stream_of(device_);
   int64_t live = 0, count = 0;
   check(recis_idmap_live_bound(map_->map, &live));
@@ -770,7 +772,7 @@ std::tuple<at::Tensor, at::Tensor> Hashtable::EvictUnseen(const std::string& sta
     at::Tensor tab = block_ptr_table(stamps->Chunks());
     check(recis_idmap_evict_unseen(map_->map, reinterpret_cast<const void* const*>(tab.data_ptr()),
                                    static_cast<int64_t>(stamps->Chunks().size()), stamps->ChunkRows(),
-                                   stamps->Dtype() == at::kLong ? 1 : 0, on_device ? step->data_ptr<int64_t>() : nullptr,
+                                   stamps->Dtype() == at::kLong ? 1 : 0, counter.defined() ? counter.data_ptr<int64_t>() : nullptr,
                                    keep_steps, ids.data_ptr<int64_t>(), index.data_ptr<int64_t>(), live, &count, stream));
   }
   ids = ids.narrow(0, 0, count);

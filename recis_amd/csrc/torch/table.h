@@ -378,7 +378,8 @@ class Hashtable : public torch::CustomClassHolder {
   // Eviction sweep in one pass over the map: erase every key whose row has stamp_slot < threshold,
   // free the rows, re-initialise every other slot there; returns the evicted (ids, index).
   std::tuple<at::Tensor, at::Tensor> EvictOlder(const std::string& stamp_slot, int64_t threshold);
-  // The same with threshold = *step - keep_steps, the step read on the device when the sweep runs.
+  // The same with threshold = *step - keep_steps, the step read on the device when the sweep runs (copied there when it
+  // lives elsewhere).
   std::tuple<at::Tensor, at::Tensor> EvictUnseen(const std::string& stamp_slot, const c10::optional<at::Tensor>& step,
                                                  int64_t keep_steps);
   // Initial values again in every slot but `keep` (-1: in all) at rows whose keys have left.

@@ -294,6 +294,33 @@ def test_evict_older_of_small_and_large_tables(rng, reserve, n_blocks, dt):
     assert _lib.poll_device_errors() == 1  # RECIS_DEVERR_INDEX_RANGE
 
 
+@pytest.mark.parametrize("where", ["cuda", "cpu"])
+@pytest.mark.parametrize("step,keep", [(50, 10), (0, 5), (-3, -40), (2**62, 1)])
+def test_eviction_by_step_equals_eviction_by_threshold(rng, where, step, keep):
+    """``evict_unseen`` reads the step when the sweep runs; it may live on another device than the table."""
+    from recis_amd.nn import HashTable
+    from recis_amd.nn.modules.hashtable import HashtableRegister
+
+    HashtableRegister().clear()
+    keys = torch.arange(3000, device="cuda") * 5 + 2
+    stamps = torch.from_numpy(rng.integers(-60, 60, size=(3000, 1))).cuda()
+    tables = []
+    for name in ("by_step", "by_threshold"):
+        t = HashTable([4], block_size=512, name=name, children=[name])._hashtable_impl
+        t.append_step_filter_slot("seen", 7)
+        t.insert(keys, torch.randn(3000, 4, device="cuda"))
+        ids, index = t.ids_map()
+        t.update_slot("seen", index, stamps[torch.searchsorted(keys, ids)])
+        tables.append(t)
+    counter = torch.tensor([step], dtype=torch.int64, device=where)
+    gone = tables[0].evict_unseen("seen", counter, keep)
+    want = tables[1].evict_older("seen", step - keep)
+    assert torch.equal(torch.sort(gone[0]).values, torch.sort(want[0]).values)
+    assert gone[0].numel() == int((stamps < step - keep).sum()) == gone[1].numel()
+    assert torch.equal(torch.sort(tables[0].ids_map()[0]).values, torch.sort(tables[1].ids_map()[0]).values)
+    assert _lib.poll_device_errors() == 0
+
+
 @pytest.mark.parametrize("dim,dtype", [(1, torch.float32), (3, torch.bfloat16), (10, torch.float32), (300, torch.float32)])
 def test_rows_of_deleted_keys_start_over(dim, dtype):
     """Slots with a constant initialiser are set in one launch, the others get new rows; the preserved slot keeps its own."""
