@@ -1130,8 +1130,8 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
   for (int64_t k = 0; k < n_multi; ++k) {
     multi_in.push_back(multi_values[k].contiguous());
     const int64_t size = multi_in[k].numel();
-    Tensor buf = at::empty({size * multi_counts[k]}, lopt);
-    for (int64_t j = 0; j < multi_counts[k]; ++j) outs.push_back(part_of(buf, j * size, {size}));  // (flat, as the operator returns them)
+    // (flat and each of a storage of its own, as the operator returns them)
+    for (int64_t j = 0; j < multi_counts[k]; ++j) outs.push_back(at::empty({size}, lopt));
   }
 
   // ---- lengths of the truncations

@@ -93,6 +93,13 @@ def test_outputs_do_not_share_a_version(rng):
     assert (out["wide"]._version, out["farm_cut"].values()._version, out["m_1"]._version) == before
 
 
+def test_multi_hashes_have_storages_of_their_own(rng):
+    out = FeatureEngine(_features())(_data(rng, 50, torch.int64))
+    hashes = [out["m_%d" % j] for j in range(2)] + [out["ms_%d" % j].values() for j in range(4)]
+    assert all(h.untyped_storage().nbytes() == 8 * h.numel() for h in hashes)
+    assert len({h.untyped_storage().data_ptr() for h in hashes}) == 6
+
+
 def test_what_the_call_does_not_take_runs_operator_by_operator(rng):
     data = _data(rng, 40, torch.int64)
     on_host = {k: (v.cpu() if k in ("wide", "real") else v) for k, v in data.items()}
