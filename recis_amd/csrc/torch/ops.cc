@@ -1047,6 +1047,15 @@ bool plain(const TensorList& ts, at::Device device, std::initializer_list<at::Sc
   }
   return true;
 }
+// What a queued kernel writes to pinned host memory has to have arrived before that memory goes back to its cache, which knows
+// nothing of the kernel: an exception between the launch and the wait would otherwise hand the block out too early.
+struct WaitOnExit {
+  void* stream;
+  bool waited = false;
+  ~WaitOnExit() {
+    if (!waited) (void)hipStreamSynchronize(static_cast<hipStream_t>(stream));
+  }
+};
 }  // namespace
 
 // The waiting part of the truncations, the lengths of what is kept, needs the offsets only: it is queued first, and has
@@ -1145,6 +1154,7 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
   int64_t sum_rows = 0;
   int is64 = 0;
   at::cuda::CUDAEvent arrived;
+  WaitOnExit in_flight{stream, n_cut == 0};  // (declared after the buffers the truncations write: it waits before they go)
   if (n_cut) {
     is64 = index_kind(cut_offsets[0], "offsets");
     for (int64_t k = 0; k < n_cut; ++k) {
@@ -1181,7 +1191,7 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
     arrived.record();
   }
 
-  // ---- the operators in front, all in one launch (but buckets of more boundaries than that takes, and columns past its indices)
+  // ---- the operators in front, all in one launch (but buckets of more boundaries than that takes)
   std::vector<recis_feature_job> jobs;
   std::vector<const float*> long_in, long_bounds;
   std::vector<int64_t> long_sizes, long_lens, long_mods;
@@ -1232,6 +1242,7 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
   // ---- the truncated values
   if (n_cut) {
     arrived.synchronize();
+    in_flight.waited = true;
     const int64_t* total = totals.data_ptr<int64_t>();
     int64_t sum_total = 0;
     for (int64_t k = 0; k < n_cut; ++k) sum_total += total[k];
