@@ -172,14 +172,16 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
     }
   }
 
-  // rows of the ids [from, to) of the feature into LDS
-  auto look_up_by = [&](auto probes, int32_t from, int32_t to) {
+  // rows of the n ids from id `from` of the feature on into LDS (at most kPoolRows: places in LDS cannot overflow, as numbers of
+  // ids up to 2^31 may)
+  auto look_up_by = [&](auto probes, int32_t from, int n) {
     constexpr int kProbes = decltype(probes)::value;  // of a thread in flight
-    for (int32_t q0 = from + tid; q0 < to; q0 += kProbes * kBlock) {
+    const int64_t* __restrict__ id = ids + from;
+    for (int q0 = tid; q0 < n; q0 += kProbes * kBlock) {
       int64_t key[kProbes];
       longlong2 hint[kProbes];
 #pragma unroll
-      for (int x = 0; x < kProbes; ++x) key[x] = q0 + x * kBlock < to ? (ids[q0 + x * kBlock] & a.id_mask) | tag : kEmpty;
+      for (int x = 0; x < kProbes; ++x) key[x] = q0 + x * kBlock < n ? (id[q0 + x * kBlock] & a.id_mask) | tag : kEmpty;
 #pragma unroll
       for (int x = 0; x < kProbes; ++x)  // (a reserved key has a home slot too: no branch around the load)
         hint[x] = *reinterpret_cast<const longlong2*>(&a.table[home_slot(key[x], a.mask)]);
@@ -188,28 +190,28 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
       for (int x = 0; x < kProbes; ++x) {
         const bool reserved = key[x] == kEmpty || key[x] == kTomb, found = hint[x].x == key[x] && !reserved;
         further |= !found && !reserved && hint[x].x != kEmpty ? 1u << x : 0u;
-        if (q0 + x * kBlock < to) s_row[q0 + x * kBlock - from] = static_cast<uint64_t>(found ? hint[x].y : -1);
+        if (q0 + x * kBlock < n) s_row[q0 + x * kBlock] = static_cast<uint64_t>(found ? hint[x].y : -1);
       }
 #pragma unroll 1
       for (int x = 0; x < kProbes; ++x) {  // (one body: four of them spill)
-        const int32_t q = q0 + x * kBlock;
-        if (q >= to) break;
-        int64_t row = static_cast<int64_t>(s_row[q - from]);
+        const int q = q0 + x * kBlock;
+        if (q >= n) break;
+        int64_t row = static_cast<int64_t>(s_row[q]);
         if ((further >> x) & 1u) {
-          const int64_t k = (ids[q] & a.id_mask) | tag;
+          const int64_t k = (id[q] & a.id_mask) | tag;
           const uint64_t home = home_slot(k, a.mask);
           row = find_row(a.table, a.mask, k, home, *reinterpret_cast<const longlong2*>(&a.table[home]));
         }
-        s_row[q - from] = address_of_row<T>(a, row);
-        if (weight) s_w[q - from] = weight_at<T>(weight, wdt, q);
+        s_row[q] = address_of_row<T>(a, row);
+        if (weight) s_w[q] = weight_at<T>(weight, wdt, static_cast<int64_t>(from) + q);
       }
     }
   };
-  auto look_up = [&](int32_t from, int32_t to) {
-    if (to - from <= kBlock)  // uniform
-      look_up_by(std::integral_constant<int, 1>{}, from, to);
+  auto look_up = [&](int32_t from, int n) {
+    if (n <= kBlock)  // uniform
+      look_up_by(std::integral_constant<int, 1>{}, from, n);
     else
-      look_up_by(std::integral_constant<int, 4>{}, from, to);
+      look_up_by(std::integral_constant<int, 4>{}, from, n);
   };
   const int lane_t = tid & ((1 << team_log2) - 1);
   const int team = tid >> team_log2;
@@ -262,7 +264,7 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
 
   const int32_t lo = s_off[0], hi = s_off[n_here];
   if (hi - lo <= kPoolRows) {  // the usual tile: one look-up for all of it
-    look_up(lo, hi);
+    look_up(lo, hi - lo);
     __syncthreads();
     if (offs == nullptr && width == 1 && !weight) {  // a dense column: its rows, four in flight per lane
       for (int c0 = cl * VEC; c0 < D; c0 += VEC << a.lpr_log2) {
@@ -307,18 +309,18 @@ lookup_pool_kernel(PoolJobs J, PoolArgs a, T* __restrict__ out) {
       float acc[VEC], w_sum = 0.f;
 #pragma unroll
       for (int x = 0; x < VEC; ++x) acc[x] = 0.f;
-      for (int32_t base = b_lo; base < b_hi; base += kPoolRows) {
-        const int32_t end = min(b_hi, base + kPoolRows);
+      for (int32_t base = b_lo; base < b_hi; base = b_hi - base > kPoolRows ? base + kPoolRows : b_hi) {
+        const int n = min(b_hi - base, kPoolRows);
         __syncthreads();  // the previous round has been read
-        look_up(base, end);
+        look_up(base, n);
         __syncthreads();
-        // the row group's next row at or after `base`
-        const int32_t behind = base > first ? (base - first + step - 1 - rg) / step : 0;
-        const int32_t from = first + rg + max(behind, 0) * step;
-        const int32_t to = min(last, end);
+        // the row group's rows of this round, counted from `base`
+        const uint32_t behind = base > first ? (static_cast<uint32_t>(base - first) + step - 1 - rg) >> rg_log2 : 0;
+        const int from = static_cast<int>(static_cast<uint32_t>(first - base) + rg + (behind << rg_log2));
+        const int to = min(last - base, n);
         if (mine && from < to) {
-          if (c0 < D) add_rows(from - base, to - base, c0, acc);
-          if (a.mode == RECIS_LOOKUP_WEIGHT_MEAN) w_sum += weight_sum(from - base, to - base);
+          if (c0 < D) add_rows(from, to, c0, acc);
+          if (a.mode == RECIS_LOOKUP_WEIGHT_MEAN) w_sum += weight_sum(from, to);
         }
       }
 #pragma unroll

@@ -240,3 +240,30 @@ def test_ids_of_other_types_are_refused_where_they_were():
             table(torch.arange(4, device="cuda").to(kind))
         with pytest.raises((TypeError, RuntimeError)):
             one.eval()(torch.arange(4, device="cuda").to(kind).view(2, 2))
+
+
+@pytest.mark.parametrize("lens", [[3, 700, 0, 200, 20], [900, 2500, 1100, 0, 5], [0, 1, 0, 40, 2] * 20])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_the_last_ids_of_a_feature_of_two_thousand_million(lens, weighted):
+    """Ids are numbered up to 2^31 - 2: offsets that name the last ones of such a list."""
+    n = 2**31 - 2
+    if torch.cuda.mem_get_info()[0] < 16 * n:
+        pytest.skip("needs %d GB of device memory" % (16 * n >> 30))
+    keys = torch.arange(1, 5000, device="cuda")
+    HashtableRegister().clear()
+    ht = HashTable([4], block_size=512, name="pool_table")
+    rows = torch.randint(-8, 9, (keys.numel(), 4), device="cuda").float()
+    ht.insert(keys, rows)
+    tail = sum(lens)
+    ids = torch.empty(n, dtype=torch.int64, device="cuda")  # only the last ones are ever read
+    ids[-tail:] = keys[torch.randint(0, keys.numel(), (tail,), device="cuda")]
+    weight = None
+    if weighted:
+        weight = torch.empty(n, device="cuda")
+        weight[-tail:] = torch.randint(-3, 4, (tail,), device="cuda").float()
+    off = torch.tensor([n - tail] + lens).cumsum(0).int().cuda()
+    got = ht._hashtable_impl.lookup_pool_readonly([ids], [off], [weight], None, False)[0].cpu()
+    terms = rows[ids[-tail:] - 1] * (weight[-tail:, None] if weighted else 1)
+    want = torch.stack([t.sum(0) if len(t) else torch.zeros(4) for t in torch.split(terms.cpu(), lens)])
+    assert torch.equal(got, want)
+    assert _lib.poll_device_errors() == 0
