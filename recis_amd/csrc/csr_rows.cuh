@@ -456,22 +456,10 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   // bound: 12 - 15 us of the update kernel were theirs).
   // Likewise a workgroup of the hot part that no work item is left for (block 0 stays: it leaves
   // alpha behind for the finish kernel).
-  // What a cold workgroup needs of its rows (bounds, table row) goes out beside that count, not behind it.
+  // (Bounds and table row of a workgroup's rows asked for beside that count instead of behind it: 179.2 / 179.2 us with two inputs of
+  // 128 bfloat16, 170.3 / 169.8 with one of 16 floats, 14.5 / 14.5 with 10 k ids. And a.U may be more than row_index holds.)
   const int64_t hot_blocks = static_cast<int64_t>(gridDim.x) - a.cold_blocks;
   const int rows_per_block = kBlock >> a.lpr_log2;
-  const int64_t u = (static_cast<int64_t>(blockIdx.x) - hot_blocks) * rows_per_block + (threadIdx.x >> a.lpr_log2);
-  // (The kernels with one input and shuffles that update rows have no registers left for that.)
-  constexpr bool kEarlyBounds = TWO || !SHUFFLE || EPI == kEpiStore;
-  int32_t start = 0, end = 0;
-  int64_t idx_mine = -1;
-  auto ask_bounds = [&](bool there) {
-    if (there) {
-      start = a.row_start[u];
-      end = a.row_start[u + 1];
-      if constexpr (EPI != kEpiStore) idx_mine = f.row_index[u];
-    }
-  };
-  if constexpr (kEarlyBounds) ask_bounds(u >= 0 && u < a.U);  // (negative: the hot part)
   {
     const int64_t b = static_cast<int64_t>(blockIdx.x);
     if (b >= hot_blocks ? (b - hot_blocks) * rows_per_block >= min(a.U, a.counts[0])
@@ -606,14 +594,12 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   }
 
   // ---- cold rows
+  const int64_t u = (static_cast<int64_t>(blockIdx.x) - hot_blocks) * rows_per_block + (threadIdx.x >> a.lpr_log2);
   // a.U may be an upper bound (a caller that has not read the plan's count back passes the number of
   // ids): rows at and past the count the plan left on the device have no list
   const bool valid = u < a.U && u < a.counts[0];
-  if constexpr (!kEarlyBounds) ask_bounds(valid);
-  if (!valid) {
-    start = end = 0;
-    idx_mine = -1;
-  }
+  const int32_t start = valid ? a.row_start[u] : 0;
+  int32_t end = valid ? a.row_start[u + 1] : 0;
   const bool hot = end - start > a.hot_len;  // left to the work items and the finish kernel
   if (hot) end = start;
   // The table row of this group's unique id is asked for before the gathers; the kernel with
@@ -622,7 +608,9 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   // 146 -> 136 us; the other kernels spill with six registers more and lose 10 %).
   constexpr bool kEarlyPlaces = EPI != kEpiStore && !SHUFFLE && !TWO;
   RowPlaces<TRow> places{nullptr, nullptr, nullptr};
+  int64_t idx_mine = -1;
   if constexpr (EPI != kEpiStore) {
+    if (valid) idx_mine = f.row_index[u];  // (under the same test as the list bounds: the three loads go out together)
     if constexpr (kEarlyPlaces) places = row_places<TRow, EPI, false>(f, first, a.err, idx_mine);
   }
   // the finished sum of this lane group's own row u

@@ -1,5 +1,6 @@
 """The gather-reduce with two inputs on short lists: the lists of a wave are worked side by side, one, two or four rows of
 each at a time as the longest of them asks, and a key's table row is asked for before its gradient is summed."""
+import ctypes
 import types
 
 import numpy as np
@@ -119,4 +120,26 @@ def test_lists_of_any_length_without_work_items(rng, dim, dtype, blocks):
                                  size_of_block)
     for a, b in zip(w + s0 + s1, w2 + m0 + m1):
         assert torch.equal(a, b)
+    assert _lib.poll_device_errors() == 0
+
+
+def test_rows_past_the_count_are_not_asked_for(rng):
+    """U may be a bound (the number of ids): row_index need not hold more rows than there are unique ids."""
+    from recis_amd._lib import check, dtype_code, i64, lib, ptr, stream_ptr
+
+    dim, uniques = 64, 300
+    ids = torch.from_numpy(rng.permutation(np.repeat(rng.choice(10**9, uniques, replace=False), 9))).cuda()
+    n = ids.numel()
+    plan = ops.ids_unique_plan(ids)
+    first = (torch.randn(n, dim, device="cuda"), plan.occ[:n], None)
+    second = (torch.randn(n, dim, device="cuda"), plan.occ[:n].flip(0), None)
+    index = torch.randperm(uniques, device="cuda")
+    slot = lambda: [torch.rand(uniques, dim, generator=torch.Generator().manual_seed(3)).cuda()]
+    w, acc, w2, acc2 = slot(), slot(), slot(), slot()
+    ops.csr_gather_reduce2_adagrad(plan, first, second, index, w, acc, 1e-2, 1e-8, uniques)
+    head, _, dev, keep = ops._two_inputs(plan, first, second)
+    check(lib().recis_csr_gather_reduce2_adagrad(
+        *head, i64(n), i64(dim), ptr(index), ptr(ops.block_ptr_table(w2)), ptr(ops.block_ptr_table(acc2)), i64(1), i64(uniques),
+        i64(0), dtype_code(torch.float32), ctypes.c_double(1e-2), ctypes.c_double(1e-8), stream_ptr(dev)))
+    assert torch.equal(w[0], w2[0]) and torch.equal(acc[0], acc2[0])
     assert _lib.poll_device_errors() == 0
