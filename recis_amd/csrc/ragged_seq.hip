@@ -73,30 +73,32 @@ __device__ __forceinline__ int64_t cut_row(const CutJobs& j, int t, int is64, in
   return len;
 }
 
-// All steps of 2-D truncations of at most kOneThreads * ITEMS rows in one launch, a workgroup per tensor: a wave takes ITEMS times 64
-// consecutive rows, scans them as it goes and keeps their places in registers until the waves know each other's sums. (8 tensors
-// of 8192 rows: 23 us in the three launches below, 16 in this one; with consecutive rows in a thread, every load and store spread
-// over 64 lines, 21. A tensor of more rows would keep one compute unit busy and leave the others idle.)
+// All steps of 2-D truncations of at most kOneRows rows in one launch, a workgroup per tensor: a wave takes kOneItems times 64
+// consecutive rows, scans them as it goes and keeps their places in registers until the waves know each other's sums (with consecutive
+// rows in a thread every load and store spreads over 64 lines). A tensor keeps one compute unit busy and leaves the others idle, so
+// the line lies where that takes as long as the three launches below. us, three launches / this one, int32 offsets, one
+// tensor (eight, sixteen: within 1.5 us of it): 256 rows 10.2 / 8.3, 2048 15.7 / 10.6, 8192 16.2 / 11.9; 16384 with twice the rows a thread
+// 17.0 / 21.1.
 constexpr int kOneThreads = 1024;
-constexpr int kOneItems = 16;  // at most
-template <int ITEMS>
+constexpr int kOneItems = 8;
+constexpr int kOneRows = kOneThreads * kOneItems;
 __global__ void __launch_bounds__(kOneThreads) cutoff_one_kernel(CutJobs j, int is64, int64_t* totals, int64_t totals_base,
                                                                  int* err) {
   __shared__ int64_t waves[kOneThreads / kWave];
   const int t = blockIdx.x;
   const int64_t rows = j.rows[t], keep = j.keep[t];
   const int lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
-  const int64_t r0 = static_cast<int64_t>(wave) * ITEMS * kWave + lane;
-  int64_t beg[ITEMS], end[ITEMS];
+  const int64_t r0 = static_cast<int64_t>(wave) * kOneItems * kWave + lane;
+  int64_t beg[kOneItems], end[kOneItems];
 #pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
+  for (int i = 0; i < kOneItems; ++i) {
     const int64_t r = r0 + i * kWave;
     beg[i] = r < rows ? load_index(j.outer[t], is64, r) : 0;
     end[i] = r < rows ? load_index(j.outer[t], is64, r + 1) : 0;
   }
   int64_t sum = 0;  // of the wave so far
 #pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
+  for (int i = 0; i < kOneItems; ++i) {
     const int64_t r = r0 + i * kWave;
     int64_t len = 0;
     if (r < rows) {
@@ -122,7 +124,7 @@ __global__ void __launch_bounds__(kOneThreads) cutoff_one_kernel(CutJobs j, int 
     total += waves[w];
   }
 #pragma unroll
-  for (int i = 0; i < ITEMS; ++i) {
+  for (int i = 0; i < kOneItems; ++i) {
     const int64_t r = r0 + i * kWave;
     if (r < rows) store_index(j.out_off[t], is64, r, before + beg[i]);
   }
@@ -718,13 +720,9 @@ extern "C" int recis_ragged_cutoff_rows(const void* const* outer_ptrs, const voi
       // the outer offsets of a 3-D output (rows + 1 entries) are written by the same grid
       max_rows = std::max(max_rows, std::max(j.out_rows[k], three_d ? j.rows[k] + 1 : 0));
     }
-    if (!three_d && max_rows <= kOneThreads * kOneItems) {
-      RECIS_TIME_KERNEL("cutoff_one_kernel", stream) {
-        if (max_rows <= kOneThreads * kOneItems / 2)
-          cutoff_one_kernel<kOneItems / 2><<<dim3(cnt), dim3(kOneThreads), 0, stream>>>(j, off_is64, totals_dev, first, err);
-        else
-          cutoff_one_kernel<kOneItems><<<dim3(cnt), dim3(kOneThreads), 0, stream>>>(j, off_is64, totals_dev, first, err);
-      }
+    if (!three_d && max_rows <= kOneRows) {
+      RECIS_TIME_KERNEL("cutoff_one_kernel", stream)
+      cutoff_one_kernel<<<dim3(cnt), dim3(kOneThreads), 0, stream>>>(j, off_is64, totals_dev, first, err);
       RECIS_LAUNCH_CHECK();
       continue;
     }

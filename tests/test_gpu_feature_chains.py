@@ -154,7 +154,7 @@ def test_moduli_are_any_uint64(rng, mods):
 @pytest.mark.parametrize("rows", [0, 1, 1023, 1025, 8192, 8193, 16384, 16385])
 @pytest.mark.parametrize("off_dtype", [torch.int32, torch.int64])
 def test_truncations_around_the_rows_of_one_launch(rng, rows, off_dtype):
-    """Up to 16384 rows a tensor are truncated by one workgroup, more in three launches."""
+    """Up to 8192 rows a tensor are truncated by one workgroup, more in three launches."""
     from recis_amd import ops
 
     seqs = [(_offsets(rng, r, 12, off_dtype), k, side) for r, k, side in
