@@ -760,11 +760,11 @@ seg_pool_bwd_fast_kernel(const TG* __restrict__ grad_out, TOut* __restrict__ gra
   }
 }
 
-// The same onto rows in order (and the maximum's, see seg_max_bwd_rows_kernel), kBwdWaves waves per segment instead of one. What binds
-// these kernels is the stream of their stores, and that runs the faster the less memory the resident workgroups are spread over: a
-// fill by workgroups of 8 KB in runs on one XCD reaches 6.9 TB/s, of 16 KB 6.6, of 32 KB 6.3 (four segments of 30 rows of 256 bytes).
-// 4 GB of such segments: sum 753, mean 708, max 769 us with a wave per segment, now 704, 681 and 736. (Four waves: 870, 650 and 890: each waits for its gradient to store a
-// microsecond; the gradient asked for beside the bounds: 843, 680 and 910 with two.)
+// The same onto rows in order (occurrence r is row r; and the maximum's, see seg_max_bwd_rows_kernel), kBwdWaves waves per segment instead of
+// one. What binds these kernels is the stream of their stores, and that runs the faster the less memory the resident workgroups are
+// spread over: a fill by workgroups of 8 KB in runs on one XCD reaches 6.9 TB/s, of 16 KB 6.6, of 32 KB 6.3 (four segments of 30
+// rows of 256 bytes). 4 GB of such segments, one / two waves: sum 681 / 685, mean 685 / 672, max 693 / 655 us. (Four waves: 870, 650 and
+// 890: each waits for its gradient to store a microsecond; the gradient asked for beside the bounds: 843, 680 and 910 with two.)
 constexpr int kBwdWaves = 2;
 template <typename TG, typename TOut, int VEC, bool MAX>
 __global__ void __launch_bounds__(kBlock)
@@ -784,10 +784,6 @@ seg_bwd_wide_kernel(const TG* __restrict__ grad_out, const int32_t* __restrict__
   const int cl = lane & ((1 << a.lpr_log2) - 1);
   const int D = a.D;
   const float scale = (!MAX && a.mean && end > start) ? 1.0f / static_cast<float>(end - start) : 1.0f;
-  if (end > a.U) {  // (rows in order: occurrence r is row r)
-    raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
-    end = a.U;
-  }
   for (int c0 = cl * VEC; c0 < D; c0 += VEC << a.lpr_log2) {
     float g[VEC];
     int32_t win[VEC];
@@ -1357,8 +1353,17 @@ extern "C" int recis_segment_reduce_backward(
   a.team_log2 = pick_team_log2(B, S, lpr_log2);
   a.mean = (mode == RECIS_MEAN);
   a.in_runs = B * D * out_sz * (kBlock >> a.team_log2) >= kRunWriteBytes * S;
-  // rows in order, a wave per segment and enough of them: several waves per segment (see seg_bwd_wide_kernel)
-  const bool wide = a.rev == nullptr && a.in_runs && (1 << a.team_log2) == kWave;
+  // Rows in order, a wave per segment and enough of them: two waves per segment (see seg_bwd_wide_kernel). Sum and mean: 23 shapes of
+  // 17 to 500 rows a segment, float and bfloat16, 1000 segments to half a million: 0.90 - 1.01 of the time of one wave. The maximum, whose
+  // workgroups read the winners too, is the slower where its plain stores go past the memory-side cache (30 rows of 64 floats, one / two
+  // waves, us, at 60 MB 14.9 / 13.9, 150 26.1 / 25.3, 350 73 / 80, 768 150 / 175), as are streams of rows of 512 bytes and of
+  // bfloat16 (17 rows of 128 floats, 2.6 GB: 501 / 527); not so rows of all lanes (17 of 256 floats, 60 MB to 2.6 GB: 0.91 -
+  // 1.01) and streams of float rows of up to 256 bytes (64 floats: 17 rows, 1.2 GB 203 / 187, 2.6 GB 651
+  // / 607 and, another card, 582 / 619; 30 rows, 4 GB 692 / 664).
+  constexpr int64_t kWideMaxBytes = 192 << 20;  // the memory-side cache and what else wants to be in it
+  const bool wide_rows = a.rev == nullptr && a.in_runs && (1 << a.team_log2) == kWave;
+  const bool wide = wide_rows && (mode != RECIS_MAX || lpr_log2 == 6 || U * D * out_sz <= kWideMaxBytes ||
+                                  (U * D * out_sz >= (int64_t(1) << 30) && out_sz == 4 && lpr_log2 <= 4));
   const int64_t wide_grid = (S * kBwdWaves + kBlock / kWave - 1) / (kBlock / kWave);
   // 1 GiB is far past what L2 and the 256 MB memory-side cache keep for the next kernel
   a.nt_out = U * D * out_sz >= (int64_t(1) << 30);
