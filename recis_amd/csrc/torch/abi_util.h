@@ -52,6 +52,15 @@ inline int index_kind(const at::Tensor& t, const char* name) {
   return 0;
 }
 
+// Elements first, first + 1, ... of a contiguous buffer as a tensor of its own over the same storage: no view in autograd's sense, so
+// parts share no version and each may be an output of a node.
+inline at::Tensor part_of(const at::Tensor& whole, int64_t first, at::IntArrayRef shape) {
+  auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(whole.storage()), whole.key_set(), whole.dtype());
+  impl->set_storage_offset(whole.storage_offset() + first);
+  impl->set_sizes_contiguous(shape);
+  return at::Tensor(std::move(impl));
+}
+
 inline at::Tensor flat_i64(const at::Tensor& t, const char* name) {
   require_gpu(t, name);
   TORCH_CHECK(t.scalar_type() == at::kLong, name, " must be int64, got ", t.scalar_type());

@@ -21,19 +21,11 @@ using recis::hipabi::block_ptr_table;
 using recis::hipabi::check;
 using recis::hipabi::dtype_code;
 using recis::hipabi::index_kind;
+using recis::hipabi::part_of;
 using recis::hipabi::stream_of;
 using recis::hipabi::TensorOrNone;
 
 namespace {
-
-// Rows [first, first + rows) of a contiguous [n, D] buffer as a tensor of its own (not a view in
-// autograd's sense: the parts do not overlap and each is an output of the node).
-at::Tensor rows_of(const at::Tensor& whole, int64_t first, at::IntArrayRef shape) {
-  auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(whole.storage()), whole.key_set(), whole.dtype());
-  impl->set_storage_offset(whole.storage_offset() + first * whole.size(1));
-  impl->set_sizes_contiguous(shape);
-  return at::Tensor(std::move(impl));
-}
 
 using torch::autograd::SavedVariable;
 
@@ -117,7 +109,7 @@ std::vector<at::Tensor> outputs_of(const at::Tensor& whole, const std::vector<st
   out.reserve(split.size());
   int64_t first = 0;
   for (size_t k = 0; k < split.size(); ++k) {
-    out.push_back(rows_of(whole, first, shapes[k]));
+    out.push_back(part_of(whole, first * whole.size(1), shapes[k]));
     first += split[k];
   }
   if (node) {

@@ -1033,13 +1033,6 @@ std::tuple<TensorList, TensorList, TensorList> fused_ragged_cutoff_3D(TensorList
 
 // ------------------------------------------------------------------------------------ chains of feature operators
 namespace {
-// A tensor of its own over elements [first, first + n) of a buffer (not a view in autograd's sense: no shared version).
-Tensor part_of(const Tensor& whole, int64_t first, at::IntArrayRef shape) {
-  auto impl = c10::make_intrusive<c10::TensorImpl>(c10::Storage(whole.storage()), whole.key_set(), whole.dtype());
-  impl->set_storage_offset(first);
-  impl->set_sizes_contiguous(shape);
-  return Tensor(std::move(impl));
-}
 bool plain(const TensorList& ts, at::Device device, std::initializer_list<at::ScalarType> types) {
   for (const auto& t : ts) {
     if (t.device() != device || t.layout() != at::kStrided) return false;

@@ -271,13 +271,14 @@ def test_evict_older_equals_snapshot_filter_erase(rng, dt):
 
 
 @pytest.mark.parametrize("reserve,n_blocks,dt", [(300_000, 1, torch.int64), (300_000, 3, torch.int32),
-                                                 (2_000_000, 1, torch.int32), (2_000_000, 3, torch.int64)])
+                                                 (2_000_000, 1, torch.int32), (2_000_000, 3, torch.int64),
+                                                 (16_000_000, 1, torch.int64), (16_000_000, 3, torch.int32)])
 def test_evict_older_of_small_and_large_tables(rng, reserve, n_blocks, dt):
-    """A thread of the sweep takes four slots of a table of 2^20 and eight of 2^22; a row beyond the blocks keeps its key and
-    is reported."""
+    """A thread of the sweep takes four slots of a table of 2^20, eight of 2^22 and from 2^25 on 64, all bits of its mask; a
+    row beyond the blocks keeps its key and is reported."""
     n = 9000
     m = ops.IdMap(reserve=reserve)
-    assert m.stats()[3] == (1 << 20 if reserve == 300_000 else 1 << 22)
+    assert m.stats()[3] == {300_000: 1 << 20, 2_000_000: 1 << 22, 16_000_000: 1 << 25}[reserve]
     keys = np.unique(rng.integers(-10**15, 10**15, size=n))
     rows = m.lookup(_dev(keys)).cpu().numpy()
     bs = -(-(keys.size - 100) // n_blocks)  # the last rows lie beyond
