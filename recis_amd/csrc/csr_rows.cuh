@@ -24,7 +24,7 @@ __device__ __forceinline__ float load_coef(const void* w, int wdt, int64_t i) {
   return to_float(static_cast<const f16_t*>(w)[i]);
 }
 
-constexpr int kMaxParts = 8;  // input arrays of one gather-reduce launch (PARTS kernels)
+constexpr int kMaxParts = 8;  // input arrays of one gather-reduce launch (kParts kernels)
 
 struct CsrArgs {
   const int32_t* row_start;  // [U + 1]
@@ -54,15 +54,16 @@ struct CsrArgs {
   const int32_t* hot_items;  // [2 * hot_cap]
   const int64_t* counts;     // counts[1] = number of items
   int64_t hot_cap;
+  int hot_by_shuffles;       // kernels with one array and without SHUFFLE: the work items go through wave_gather_range all the same
   float* hot_part;           // [hot_cap, D]
   int64_t cold_blocks;       // the last cold_blocks workgroups work per row, the ones before per hot item
-  // PARTS kernels: the input rows as n_parts arrays laid end to end in src's numbering; part f
+  // kParts kernels: the input rows as n_parts arrays laid end to end in src's numbering; part f
   // holds rows from part_lo32[f] on (INT32_MAX for an unused part). Of the one input; in kernels
   // with two inputs, of the SECOND.
   int n_parts;
   const void* part_rows[kMaxParts];
   int32_t part_lo32[kMaxParts];
-  // grid_rows > 0: the one part is a grid, columns side by side in a wider array: input row s is row s % grid_rows of column s / grid_rows,
+  // kGrid kernels: the one part is a grid, columns side by side in a wider array: input row s is row s % grid_rows of column s / grid_rows,
   // at part_rows[0] + column * grid_step + row * grid_stride (elements). s / grid_rows = s * grid_magic >> grid_shift for all s < 2^31:
   // the shift is 31 + l with 2^l the power of two at or above grid_rows, the factor 2^shift / grid_rows rounded up, below 2^32.
   int32_t grid_rows;
@@ -236,19 +237,21 @@ struct SrcView {
   int64_t n_rows, lo, hi;
 };
 
-// Row s of the input: of the one array (PARTS == false), or of the part that holds it. No
-// branches: the callers keep several of these loads in flight.
-template <typename TIn, bool PARTS>
+// Row s of the input: of the one array (PARTS == 0), of the part that holds it, or of a grid of columns. No
+// branches: the callers keep several of these loads in flight. (The grid in kernels of its own: beside the part table it took the
+// scalar registers of a wave, 106 and some spilled, and parts of 10 entries a row 50 us instead of 41.)
+constexpr int kParts = 1, kGrid = 2;
+template <typename TIn, int PARTS>
 __device__ __forceinline__ const TIn* src_row(const TIn* rows, const CsrArgs& a, int64_t s) {
-  if constexpr (!PARTS) {
+  if constexpr (PARTS == 0) {
     return rows + s * a.D;
+  } else if constexpr (PARTS == kGrid) {
+    const uint32_t u = static_cast<uint32_t>(s);
+    const uint32_t column = static_cast<uint32_t>((static_cast<uint64_t>(u) * a.grid_magic) >> a.grid_shift);
+    return static_cast<const TIn*>(a.part_rows[0]) + static_cast<int64_t>(column) * a.grid_step +
+           static_cast<int64_t>(u - column * a.grid_rows) * a.grid_stride;
   } else {
     const TIn* base = static_cast<const TIn*>(a.part_rows[0]);
-    if (a.grid_rows > 0) {  // uniform
-      const uint32_t u = static_cast<uint32_t>(s);
-      const uint32_t column = static_cast<uint32_t>((static_cast<uint64_t>(u) * a.grid_magic) >> a.grid_shift);
-      return base + static_cast<int64_t>(column) * a.grid_step + static_cast<int64_t>(u - column * a.grid_rows) * a.grid_stride;
-    }
     int32_t lo = 0;
     const int32_t s32 = static_cast<int32_t>(s);  // src entries are 32-bit, and so are the parts' first rows
 #pragma unroll
@@ -292,14 +295,14 @@ __device__ __forceinline__ void add_pack(const Pack<T, VEC>& v, float w, float (
 
 // One list entry as a lane holds it: where its row lies (a row of zeros where there is nothing to add) and its factor. The lane that
 // holds the entry works the address out, so that the lanes that gather the row only add their column (these kernels spend more
-// of their time on instructions than on waiting: 2 x 1.5 M rows of 128 bfloat16: 70 M vector instructions and 178 us
-// with the row number handed round and tested in every lane, now 59 M and 164 us).
+// of their time on instructions than on waiting: 2 x 1.5 M rows of 128 bfloat16, 70 M vector instructions with the row number handed
+// round and tested in every lane, 59 M so, and 8 % of the time less).
 template <typename T>
 struct ListEntry {
   const T* p;
   float w;
 };
-template <typename T, bool PARTS>
+template <typename T, int PARTS>
 __device__ __forceinline__ ListEntry<T> load_entry(const SrcView<T>& in, const CsrArgs& a, int32_t k, bool have, bool& beyond) {
   int32_t sv = 0;
   float w = 1.0f;
@@ -328,27 +331,30 @@ __device__ __forceinline__ Pack<T, VEC> load_row_of(const SrcView<T>& in, const 
   return load_raw_pack<T, VEC, NT>(reinterpret_cast<const T*>((static_cast<uintptr_t>(hi) << 32) | lo) + c0);
 }
 
+// Rows in flight per lane of a list that a wave shares (two inputs with eight: 11 % slower, four waves a SIMD instead of five). A turn of
+// four entries for each of up to sixteen lane groups divides the 64 of a wave.
+constexpr int kFly = 4;
+
 // A whole wave sums the rows of up to 64 list entries, a lane each (`mine`): lane group g of `groups` takes entries g, g +
-// groups, ... with FLY row loads in flight at once. acc: this group's partial sum for columns c0 .. c0 + VEC (the caller
+// groups, ... with kFly row loads in flight at once. acc: this group's partial sum for columns c0 .. c0 + VEC (the caller
 // folds the groups; c0 is a column of the row in every lane, also in those that have none to sum).
-template <typename T, int VEC, bool NT, int FLY>
+template <typename T, int VEC, bool NT>
 __device__ __forceinline__ void wave_gather_entries(const SrcView<T>& s, const ListEntry<T>& mine, int n_here, int c0, int g,
                                                     int groups, float (&acc)[VEC]) {
-  static_assert(FLY == 4, "a turn of four entries for each of up to sixteen groups divides the 64 of a wave");
-  for (int q0 = 0; q0 < n_here; q0 += FLY * groups) {  // same trip count for the whole wave (shuffles inside)
-    Pack<T, VEC> v[FLY];
-    float w[FLY];
+  for (int q0 = 0; q0 < n_here; q0 += kFly * groups) {  // same trip count for the whole wave (shuffles inside)
+    Pack<T, VEC> v[kFly];
+    float w[kFly];
 #pragma unroll
-    for (int k = 0; k < FLY; ++k)  // no branches in here: see g_csr_zero_row
+    for (int k = 0; k < kFly; ++k)  // no branches in here: see g_csr_zero_row
       v[k] = load_row_of<T, VEC, NT>(s, mine, (q0 + k * groups + g) * 4, c0, w[k]);
     __builtin_amdgcn_sched_barrier(0);  // all loads first
 #pragma unroll
-    for (int k = 0; k < FLY; ++k) add_pack<T, VEC>(v[k], w[k], acc);
+    for (int k = 0; k < kFly; ++k) add_pack<T, VEC>(v[k], w[k], acc);
   }
 }
 // The same over the list entries [e_begin, e_end) (uniform arguments, every lane calls), 64 at a time. AHEAD: the next 64 are
 // asked for before the rows of these.
-template <typename T, int VEC, bool PARTS, int FLY, bool AHEAD>
+template <typename T, int VEC, int PARTS, bool AHEAD>
 __device__ __forceinline__ void wave_gather_range(const SrcView<T>& s, const CsrArgs& a, int32_t e_begin, int32_t e_end, int c0,
                                                   int g, int groups, float (&acc)[VEC]) {
   const int lane = threadIdx.x & (kWave - 1);
@@ -360,7 +366,7 @@ __device__ __forceinline__ void wave_gather_range(const SrcView<T>& s, const Csr
       const int32_t k = cb + lane + (AHEAD ? kWave : 0);
       const ListEntry<T> next = load_entry<T, PARTS>(s, a, k, k < e_end, beyond);
       if constexpr (!AHEAD) mine = next;
-      wave_gather_entries<T, VEC, decltype(nt_tag)::value, FLY>(s, mine, min(kWave, e_end - cb), c0, g, groups, acc);
+      wave_gather_entries<T, VEC, decltype(nt_tag)::value>(s, mine, min(kWave, e_end - cb), c0, g, groups, acc);
       if constexpr (AHEAD) mine = next;
     }
   };
@@ -371,19 +377,19 @@ __device__ __forceinline__ void wave_gather_range(const SrcView<T>& s, const Csr
   if (beyond) raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
 }
 // Up to 64 entries [first, last), a row of either input each: both inputs' entries are asked for together.
-template <typename T1, typename T2, int VEC, bool PARTS, int FLY>
+template <typename T1, typename T2, int VEC, int PARTS>
 __device__ __forceinline__ void wave_gather_two(const SrcView<T1>& in1, const SrcView<T2>& in2, const CsrArgs& a, int32_t first,
                                                 int32_t last, int c0, int g, int groups, float (&acc)[VEC]) {
   const int32_t k = first + static_cast<int32_t>(threadIdx.x & (kWave - 1));
   bool beyond = false;
-  const auto e1 = load_entry<T1, false>(in1, a, k, k < last, beyond);
+  const auto e1 = load_entry<T1, 0>(in1, a, k, k < last, beyond);
   const auto e2 = load_entry<T2, PARTS>(in2, a, k, k < last, beyond);
   if (beyond) raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
-  wave_gather_entries<T1, VEC, false, FLY>(in1, e1, last - first, c0, g, groups, acc);
+  wave_gather_entries<T1, VEC, false>(in1, e1, last - first, c0, g, groups, acc);
   if (in2.nt)
-    wave_gather_entries<T2, VEC, true, FLY>(in2, e2, last - first, c0, g, groups, acc);
+    wave_gather_entries<T2, VEC, true>(in2, e2, last - first, c0, g, groups, acc);
   else
-    wave_gather_entries<T2, VEC, false, FLY>(in2, e2, last - first, c0, g, groups, acc);
+    wave_gather_entries<T2, VEC, false>(in2, e2, last - first, c0, g, groups, acc);
 }
 
 // Short lists (at most as many entries as a lane group has lanes), a lane group each: every lane of the group has one
@@ -424,11 +430,12 @@ constexpr int kCoopLen = 8;  // longer lists are shared among the lane groups of
 // walk the hot work items (row, chunk of kHotChunk occurrences): four waves share the chunk,
 // fold their sums through LDS and store ONE partial row per item; csr_hot_finish_kernel adds up
 // the partial rows of every hot row in chunk order. No atomics anywhere.
-// SHUFFLE: long lists go through wave_gather_range, for up to sixteen lane groups a wave (rows of 64 bytes and more, see the rule at
-// the launch); otherwise every group loads its own entries.
+// SHUFFLE: long lists go through wave_gather_range (see the rule at the launch); otherwise every group loads its own entries, of hot rows too
+// unless hot_by_shuffles says so.
+// PARTS: how the rows lie (kParts, kGrid, 0: one array).
 // TIn2 != void: every list entry adds a row of a second input as well (see CsrArgs); PARTS then
 // says that the second input comes in parts.
-template <typename TIn, typename TOut, int VEC, bool SHUFFLE, bool PARTS = false, int EPI = kEpiStore,
+template <typename TIn, typename TOut, int VEC, bool SHUFFLE, int PARTS = 0, int EPI = kEpiStore,
           typename TIn2 = void>
 // Register budgets of the variants that end in a row update, found by measurement: 64 registers (8
 // waves per SIMD) for the one-input kernels, also for those that hand list entries round by
@@ -436,8 +443,11 @@ template <typename TIn, typename TOut, int VEC, bool SHUFFLE, bool PARTS = false
 // branch-free gathers in flight the kernel needs 65, and 64 with 44 bytes spilled reads 161 us
 // against 168 at 72); no bound for those with two inputs (a bound of 80 registers spills 24-60
 // bytes and costs 20 us in config 5).
-__global__ void __launch_bounds__(kBlock, (!SHUFFLE && EPI != kEpiStore && (std::is_void<TIn2>::value || sizeof(TOut) == 4))
-                                              ? 8 : (SHUFFLE && EPI != kEpiStore && std::is_void<TIn2>::value) ? 8 : 1)
+// A sum in packs of up to four elements needs 57, but more than 80 scalar registers, which leave seven waves unless it is told (1.2 M
+// entries of 16 floats: 48 us with seven, 37 with eight).
+__global__ void __launch_bounds__(kBlock, (std::is_void<TIn2>::value && (EPI != kEpiStore || (!SHUFFLE && PARTS == 0 && VEC <= 4))) ||
+                                                  (!SHUFFLE && EPI != kEpiStore && sizeof(TOut) == 4)
+                                              ? 8 : 1)
 csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a, FuseArgs f) {
   constexpr bool TWO = !std::is_void<TIn2>::value;
   using TSecond = typename std::conditional<TWO, TIn2, TIn>::type;
@@ -530,26 +540,27 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
   };
   // the first input's entries, then the second's: one fixed order of summation
   auto gather_sum = [&](int32_t first, int32_t last, int32_t step, int c0, float (&acc)[VEC]) {
-    gather_one(in1, std::integral_constant<bool, PARTS && !TWO>{}, first, last, step, c0, acc);
-    if constexpr (TWO) gather_one(in2, std::integral_constant<bool, PARTS>{}, first, last, step, c0, acc);
+    gather_one(in1, std::integral_constant<int, TWO ? 0 : PARTS>{}, first, last, step, c0, acc);
+    if constexpr (TWO) gather_one(in2, std::integral_constant<int, PARTS>{}, first, last, step, c0, acc);
   };
-  constexpr int kFly = 4;  // rows in flight per lane of a list that a wave shares (two inputs with eight: 184 -> 204 us, 4 waves)
   // the wave's sum over the list entries [first, last) for columns c0.., the same in every group
-  auto wave_sum = [&](int32_t first, int32_t last, int c0, bool col_ok, float (&acc)[VEC]) {
+  auto wave_sum = [&](int32_t first, int32_t last, int c0, bool col_ok, auto by_shuffles, float (&acc)[VEC]) {
 #pragma unroll
     for (int j = 0; j < VEC; ++j) acc[j] = 0.f;
     if constexpr (SHUFFLE) {
       const int c = col_ok ? c0 : 0;
       if constexpr (TWO) {
         if (last - first <= kWave) {
-          wave_gather_two<TIn, TSecond, VEC, PARTS, kFly>(in1, in2, a, first, last, c, g, groups, acc);
+          wave_gather_two<TIn, TSecond, VEC, PARTS>(in1, in2, a, first, last, c, g, groups, acc);
         } else {
-          wave_gather_range<TIn, VEC, false, kFly, true>(in1, a, first, last, c, g, groups, acc);
-          wave_gather_range<TSecond, VEC, PARTS, kFly, true>(in2, a, first, last, c, g, groups, acc);
+          wave_gather_range<TIn, VEC, 0, true>(in1, a, first, last, c, g, groups, acc);
+          wave_gather_range<TSecond, VEC, PARTS, true>(in2, a, first, last, c, g, groups, acc);
         }
       } else {
-        wave_gather_range<TIn, VEC, PARTS, kFly, false>(in1, a, first, last, c, g, groups, acc);
+        wave_gather_range<TIn, VEC, PARTS, false>(in1, a, first, last, c, g, groups, acc);
       }
+    } else if (!TWO && PARTS == 0 && by_shuffles) {  // uniform; hot rows only
+      wave_gather_range<TIn, VEC, 0, false>(in1, a, first, last, col_ok ? c0 : 0, g, groups, acc);
     } else {
       if (col_ok) gather_sum(first + g, last, groups, c0, acc);
     }
@@ -576,7 +587,7 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
         const int c0 = cbase + cl * VEC;
         const bool col_ok = c0 < D;
         float acc[VEC];
-        wave_sum(w_begin, w_end, c0, col_ok, acc);
+        wave_sum(w_begin, w_end, c0, col_ok, a.hot_by_shuffles != 0, acc);
         if (g == 0 && col_ok) {
 #pragma unroll
           for (int j = 0; j < VEC; ++j) s_part[wave * D + c0 + j] = acc[j];
@@ -641,13 +652,14 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
     // All lists of the wave side by side, as many rows of each in flight as the longest of them has (up to four: the longest
     // decides for all, and most hold one or two), of both inputs together where they fit: the chain is bounds, entries, rows,
     // table row. With each list's entries taken as they come, src and row of one after the other and the second input
-    // behind the first, a list of four was up to sixteen round trips (two inputs of 128 bfloat16, 1.5 M entries, three quarters of them in hot rows: 239 us, 188 in this form).
+    // behind the first, a list of four was up to sixteen round trips (two inputs of 128 bfloat16, 1.5 M entries, three quarters of them in hot rows: 239 us, now
+    // 164; 51 of the difference by this form, 10 by the table rows asked for before the gathers, 14 by load_entry).
     // (One input in this form: 128 -> 136 us with 2 M entries of 32 floats, whose kernel has registers for 64 only.)
     const int len = is_short ? end - start : 0;
     const int first_lane = lane & ~((1 << a.lpr_log2) - 1);
     bool beyond = false;
     const bool have = cl < len;
-    const auto e1 = load_entry<TIn, false>(in1, a, start + cl, have, beyond);
+    const auto e1 = load_entry<TIn, 0>(in1, a, start + cl, have, beyond);
     const auto e2 = load_entry<TSecond, PARTS>(in2, a, start + cl, have, beyond);
     if (beyond) raise_device_error(a.err, RECIS_DEVERR_INDEX_RANGE);
     const bool over1 = __ballot(len > 1) != 0, over2 = __ballot(len > 2) != 0;
@@ -733,7 +745,7 @@ csr_rows_kernel(const TIn* __restrict__ rows, TOut* __restrict__ out, CsrArgs a,
     const int r = owner >> a.lpr_log2;
     const int32_t r_start = __shfl(start, owner, kWave), r_end = __shfl(end, owner, kWave);
     float acc[VEC];
-    wave_sum(r_start, r_end, c0, col_ok, acc);
+    wave_sum(r_start, r_end, c0, col_ok, std::false_type{}, acc);
     if (g == r) {
 #pragma unroll
       for (int j = 0; j < VEC; ++j) keep[j] = acc[j];
@@ -957,6 +969,12 @@ int csr_gather_reduce_run(const CsrRequest& r) {
   a.hot_items = r.hot_items;
   a.counts = r.counts_dev;
   a.hot_cap = hot_cap;
+  // Hot rows of up to sixteen lane groups a wave by shuffles whatever the kernel does with the others, while there are few entries: the
+  // work items are then few as well, and each is a chain of loads that shuffles shorten. With more they fill the chip, and what counts
+  // is instructions. The room for work items tells the number of entries. Power-law ids, rows of 16 floats, us as they come / by shuffles: 0.1 M
+  // entries 24.5 / 19.8 (sum 13.2 / 10.9), 0.3 M 30.3 / 29.7 (23.6 / 18.5), 1 M 40.8 / 42.9 (30.2 / 31.9), 3 M 132.2 / 133.3 (74.0 / 76.1).
+  constexpr int64_t kShuffleEntries = int64_t(1) << 19;
+  a.hot_by_shuffles = a.lpr_log2 >= 2 && hot_cap <= kShuffleEntries / kHotLen + kShuffleEntries / kHotChunk + 2;
   a.hot_part = nullptr;
   // the part table: of the one input, or of the second of two; the kernels find a row's part by
   // comparing with the parts' first rows, so an unused part starts past every row
@@ -1002,18 +1020,16 @@ int csr_gather_reduce_run(const CsrRequest& r) {
       } else {
         const TIn* rin = static_cast<const TIn*>(r.in1.rows);
         TOut* o = static_cast<TOut*>(r.out);
-        // At most sixteen lane groups per wave: a turn of four entries each is 64. With two inputs at most eight: a lane group holds the
-        // entries of a short list, a lane each, and short is up to kCoopLen. Sixteen groups and a row update: only while the
-        // long lists count, up to kShuffleUnique unique rows; with more, most lists hold an entry or two and the kernel
-        // without shuffles, which knows its rows' places early, is the faster (update of rows of 64 bytes, without / with: 13 k
-        // unique 14.5 / 10.8 us, 46 k 24.2 / 22.3, 850 k 132 / 141).
+        // Lists through shuffles: at most eight lane groups a wave (with two inputs a lane group holds the entries of a short list, a
+        // lane each, and short is up to kCoopLen). Rows of sixteen groups, 64 bytes, only where they are columns of a wider array
+        // (39 columns of 16 floats, 32768 rows: 38.8 us against 40.8); in other lists of nine and more a group of sixteen has less
+        // than an entry, and the kernel without shuffles knows its rows' places early (uniform ids, ten a row, without / with: 70 k
+        // unique rows 29.9 / 34.4, update 35.9 / 42.0, 400 k 114 / 136, update 163 / 182).
         // A lane group that is the whole wave shares its lists with nobody, so there every list is short, and without work items
         // (hot_cap == 0) of any length: those go to the kernels that take the entries as they come.
         static_assert(kCoopLen <= 8 && kHotLen <= kWave, "short lists fit a lane group");
-        constexpr int64_t kShuffleUnique = int64_t(1) << 17;
         const bool lists_fit = !TWO || a.lpr_log2 < 6 || hot_cap > 0;
-        const bool shuffle = (a.lpr_log2 >= 3 && lists_fit) ||
-                             (!TWO && a.lpr_log2 == 2 && (epi == kEpiStore || U <= kShuffleUnique));
+        const bool shuffle = (a.lpr_log2 >= 3 && lists_fit) || (a.lpr_log2 == 2 && r.grid_rows > 0);
         const dim3 grid(a.cold_blocks + hot_blocks), block(kBlock);
         const int64_t fin = std::min<int64_t>((hot_cap + kBlock / kWave - 1) / (kBlock / kWave), 2048);  // a wave per item
         auto launch = [&](auto epi_tag) {
@@ -1024,19 +1040,26 @@ int csr_gather_reduce_run(const CsrRequest& r) {
             if (a.n_parts > 0) {
               if constexpr (TWO) {  // the second input in parts
                 if (shuffle)
-                  csr_rows_kernel<TIn, TOut, VEC, true, true, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
+                  csr_rows_kernel<TIn, TOut, VEC, true, kParts, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
                 else
-                  csr_rows_kernel<TIn, TOut, VEC, false, true, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
+                  csr_rows_kernel<TIn, TOut, VEC, false, kParts, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
               } else if constexpr (sizeof(TOut) == 4 && EPI == kEpiStore) {  // parts go to fp32 rows only
-                if (shuffle)
-                  csr_rows_kernel<TIn, TOut, VEC, true, true><<<grid, block, lds, stream>>>(rin, o, a, f);
+                auto from = [&](auto parts_tag) {
+                  constexpr int P = decltype(parts_tag)::value;
+                  if (shuffle)
+                    csr_rows_kernel<TIn, TOut, VEC, true, P><<<grid, block, lds, stream>>>(rin, o, a, f);
+                  else
+                    csr_rows_kernel<TIn, TOut, VEC, false, P><<<grid, block, lds, stream>>>(rin, o, a, f);
+                };
+                if (r.grid_rows > 0)
+                  from(std::integral_constant<int, kGrid>{});
                 else
-                  csr_rows_kernel<TIn, TOut, VEC, false, true><<<grid, block, lds, stream>>>(rin, o, a, f);
+                  from(std::integral_constant<int, kParts>{});
               }
             } else if (shuffle) {
-              csr_rows_kernel<TIn, TOut, VEC, true, false, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
+              csr_rows_kernel<TIn, TOut, VEC, true, 0, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
             } else {
-              csr_rows_kernel<TIn, TOut, VEC, false, false, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
+              csr_rows_kernel<TIn, TOut, VEC, false, 0, EPI, TIn2><<<grid, block, lds, stream>>>(rin, o, a, f);
             }
             RECIS_LAUNCH_CHECK();
           }
