@@ -74,7 +74,7 @@ _FUSED = {Mod: _fused_mod, Bucketize: _fused_bucketize, Hash: _fused_hash, IDMul
 
 
 def _int64s(values):
-    """Python numbers as the operators hand them to the kernels, modulo 2^64: a modulus may be any uint64."""
+    """Moduli as the operators hand them to the kernels, modulo 2^64: they may be any uint64."""
     if not values or (max(values) < 2**63 and min(values) >= -2**63):
         return values
     return [(v + 2**63) % 2**64 - 2**63 for v in values]
@@ -89,10 +89,11 @@ class _Chains:
 
     @classmethod
     def of(cls, features):
-        """None when some feature has another form."""
+        """None when some feature has another form, or none has an operator."""
         self = cls()
         self.names, self.selects, self.hooks = [], [], []
         self.hash, self.mod, self.bucket, self.multi, self.cut = [], [], [], [], []  # (place of the feature, its op(s))
+        self.first = None  # the first feature with an operator
         for place, f in enumerate(features):
             ops_of = f.ops
             kinds = tuple(type(op) for op in ops_of)
@@ -113,17 +114,24 @@ class _Chains:
                 getattr(self, kind).append((place, ops_of[1]))
             if cut:
                 self.cut.append((place, ops_of[-1]))
-        return self
+            if len(kinds) > 1 and self.first is None:
+                self.first = place
+        return None if self.first is None else self
 
     def run(self, data):
         """The results of the features in order, or None: something asks for the operators one by one."""
         if any(self.hooks):
             return None
+        for _, op in self.cut:
+            if op.check_length or not op.truncate or op.n_dims != 2:
+                return None
         xs = [data[op._name] if op._from_dict else data for op in self.selects]
         vals = [x._values if type(x) is RaggedTensor else x for x in xs]
         for v in vals:
             if type(v) is not torch.Tensor:
                 return None
+        if not vals[self.first].is_cuda:
+            return None
         for place, _ in self.hash:
             x = xs[place]
             if type(x) is not RaggedTensor or len(x._offsets) < 2 or not all(o.is_cuda for o in x._offsets):
@@ -134,7 +142,7 @@ class _Chains:
         direct, cut_from, cut_offsets = [], [], []
         for place, op in self.cut:
             x = xs[place]
-            if type(x) is not RaggedTensor or op.check_length or not op.truncate or op.n_dims != 2:
+            if type(x) is not RaggedTensor:
                 return None
             at = hash_at.get(place, mod_at.get(place))
             if at is None:
@@ -149,9 +157,9 @@ class _Chains:
             [vals[p] for p, _, _ in self.bucket], [b.boundary_on(vals[p].device) for p, b, _ in self.bucket],
             [m.mod_value for _, _, m in self.bucket],
             [vals[p] for p, _ in self.multi], [len(op.muls) for _, op in self.multi],
-            _int64s([v for _, op in self.multi for v in op.muls]), _int64s([v for _, op in self.multi for v in op.primes]),
-            _int64s([v for _, op in self.multi for v in op.num_buckets]),
-            direct, cut_from, cut_offsets, _int64s([op.seq_len for _, op in self.cut]),
+            [v for _, op in self.multi for v in op.muls], [v for _, op in self.multi for v in op.primes],
+            [v for _, op in self.multi for v in op.num_buckets],
+            direct, cut_from, cut_offsets, [op.seq_len for _, op in self.cut],
             [op.truncate_side == "left" for _, op in self.cut])
         if not outs:
             return None

@@ -120,6 +120,8 @@ def test_what_the_call_does_not_take_runs_operator_by_operator(rng):
         FeatureEngine(checked())(data)
     other = [Feature("b").add_op(SelectField("real")).add_op(Bucketize([0.0]))]
     assert FeatureEngine(other)._chains is None
+    plain = FeatureEngine([Feature("as_is").add_op(SelectField("wide"))])  # nothing for the call to do
+    assert plain._chains is None and plain(data)["as_is"] is data["wide"]
 
 
 def test_more_columns_than_a_launch_takes_and_long_boundaries(rng):
