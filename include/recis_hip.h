@@ -296,7 +296,7 @@ int recis_idmap_stats(recis_idmap* m, int64_t* live, int64_t* id_num, int64_t* f
  * Synchronises; *count = number of live pairs (only min(count, max_out) written). */
 int recis_idmap_snapshot(recis_idmap* m, int64_t* ids_out, int64_t* index_out, int64_t max_out,
                          int64_t* count, void* stream);
-/* The eviction sweep of a step filter, one pass over the table. Replaces the sequence
+/* The eviction sweep of a step filter. Replaces the sequence
  * IdMap::SnapShot + block_filter + masked_select + DeleteIds of
  * recis/nn/modules/hashtable_hook_impl.py:487-551 (do_filter / filter) and hashtable.cc:263-278:
  * every live key whose row has stamp < threshold (stamp slot: int32 or int64, one value per row,
@@ -660,8 +660,9 @@ int recis_csr_fill_lists(const int32_t* list, int64_t n, const void* offsets, in
  * for the backward of the TILE mode where src is the occurrence itself).
  * U may be an upper bound of the number of unique ids (a caller that has not read the plan's
  * count back yet passes n): rows at and past counts_dev[0], the count the plan left on the device,
- * are skipped (out must then hold U rows, of which the first counts_dev[0] are written). The same
- * holds for every recis_csr_gather_reduce* entry point below.
+ * are skipped (out must then hold U rows, of which the first counts_dev[0] are written; row_start and
+ * row_index are read up to that count only). The same holds for every recis_csr_gather_reduce* entry
+ * point below.
  */
 int recis_csr_gather_reduce(const void* rows, int rows_dtype, int64_t n_rows, const int32_t* src,
                             const void* coef, int coef_dtype, const int32_t* row_start,

@@ -681,7 +681,9 @@ plan_scatter_kernel(const int64_t* __restrict__ ids, IdJobs jobs, PlanGeom g, He
 // waited for the stores of the round before, 11 us of a 25 us workgroup).
 // A histogram of at most kOwnScan words is summed by every workgroup for itself, where a launch of the column scan would take the
 // host and the device as long as the rest of this kernel (batch of 10 k ids: 4.2 + 13.5 us for column scan and scatter, 14.4
-// for the scatter alone; at kOwnScan words a thread reads sixteen).
+// for the scatter alone; at kOwnScan words a thread reads sixteen). Whole plan with the column scan / without, us: 1 k ids 25.9 / 23.8,
+// 10 k 32.9 / 30.9, 43 k 46.3 / 44.9, 160 k 59.0 / 57.6 (all distinct 88.6 / 84.3); with a line at 65536 words 400 k ids 63.2 / 66.2,
+// 39 columns of 8192 52.1 / 53.9.
 constexpr int64_t kOwnScan = 16384;
 constexpr size_t scatter_runs_lds(int nc) {
   return sizeof(int32_t) * (2 * (nc + 1) + kPartBlock) + 8 + (sizeof(int64_t) + 2 * sizeof(uint16_t)) * kTile;

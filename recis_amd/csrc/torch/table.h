@@ -375,7 +375,7 @@ class Hashtable : public torch::CustomClassHolder {
   std::vector<int64_t> PendingGrads() const {
     return {static_cast<int64_t>(planned_.size()), static_cast<int64_t>(grad_.size())};
   }
-  // Eviction sweep in one pass over the map: erase every key whose row has stamp_slot < threshold,
+  // Eviction sweep over the map: erase every key whose row has stamp_slot < threshold,
   // free the rows, re-initialise every other slot there; returns the evicted (ids, index).
   std::tuple<at::Tensor, at::Tensor> EvictOlder(const std::string& stamp_slot, int64_t threshold);
   // The same with threshold = *step - keep_steps, the step read on the device when the sweep runs (copied there when it

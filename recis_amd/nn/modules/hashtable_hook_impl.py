@@ -117,7 +117,7 @@ class GlobalStepFilterHookImpl(BaseFilterHookImpl):
         return int(self._global_step.item()) - self._filter_step
 
     def do_filter(self) -> None:
-        # one pass over the id map instead of snapshot + filter + delete; the sweep reads the step on the device
+        # one sweep over the id map instead of snapshot + filter + delete; it reads the step on the device
         if self._global_step.is_cuda and self._global_step.dtype == torch.int64:
             self._ht.evict_unseen(self._name, self._global_step, self._filter_step)
         else:
