@@ -4,6 +4,7 @@
 // every op; these are the device branches only).
 #include "ops.h"
 
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/HIPEvent.h>
 #include <c10/hip/HIPStream.h>
 
@@ -1040,6 +1041,8 @@ bool plain(const TensorList& ts, at::Device device, std::initializer_list<at::Sc
   }
   return true;
 }
+// An empty tensor on the current device without the dispatcher, which a call of some twenty outputs would pay for each.
+Tensor fresh(at::IntArrayRef shape, const at::TensorOptions& options) { return Tensor(at::detail::empty_cuda(shape, options)); }
 // What a queued kernel writes to pinned host memory has to have arrived before that memory goes back to its cache, which knows
 // nothing of the kernel: an exception between the launch and the wait would otherwise hand the block out too early.
 struct WaitOnExit {
@@ -1109,7 +1112,7 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
     hash_in.push_back(hash_values[k].contiguous());
     hash_off.push_back(hash_offsets[k].contiguous());
     n_strings[k] = hash_off[k].numel() - 1;
-    outs.push_back(at::empty({n_strings[k]}, lopt));
+    outs.push_back(fresh({n_strings[k]}, lopt));
   }
   auto ids_like = [&](const TensorList& values, TensorList& in, bool flat) {  // int64 outputs, shaped as the inputs or flat
     int64_t total = 0;
@@ -1118,7 +1121,7 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
       total += v.numel();
     }
     if (values.empty()) return;
-    Tensor buf = at::empty({total}, lopt);
+    Tensor buf = fresh({total}, lopt);
     int64_t first = 0;
     for (const auto& v : values) {
       outs.push_back(flat ? part_of(buf, first, {v.numel()}) : part_of(buf, first, v.sizes()));
@@ -1133,7 +1136,7 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
     multi_in.push_back(multi_values[k].contiguous());
     const int64_t size = multi_in[k].numel();
     // (flat and each of a storage of its own, as the operator returns them)
-    for (int64_t j = 0; j < multi_counts[k]; ++j) outs.push_back(at::empty({size}, lopt));
+    for (int64_t j = 0; j < multi_counts[k]; ++j) outs.push_back(fresh({size}, lopt));
   }
 
   // ---- lengths of the truncations
@@ -1160,9 +1163,9 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
       sum_rows += rows[k];
     }
     auto iopt = cut_off[0].options();
-    off_buf = at::empty({sum_rows + n_cut}, iopt);
-    src_buf = at::empty({std::max<int64_t>(sum_rows, 1)}, lopt);
-    cnt_buf = at::empty({std::max<int64_t>(2 * sum_rows, 1)}, iopt);
+    off_buf = fresh({sum_rows + n_cut}, iopt);
+    src_buf = fresh({std::max<int64_t>(sum_rows, 1)}, lopt);
+    cnt_buf = fresh({std::max<int64_t>(2 * sum_rows, 1)}, iopt);
     totals = at::empty({n_cut}, at::TensorOptions().dtype(at::kLong).pinned_memory(true));  // written by the kernel itself
     const int64_t isize = off_buf.element_size();
     std::vector<uint8_t> drop8(n_cut), pad8(n_cut, 0);
@@ -1239,7 +1242,7 @@ TensorList feature_chains(TensorList hash_values, TensorList hash_offsets, std::
     const int64_t* total = totals.data_ptr<int64_t>();
     int64_t sum_total = 0;
     for (int64_t k = 0; k < n_cut; ++k) sum_total += total[k];
-    Tensor val_buf = at::empty({sum_total}, lopt);
+    Tensor val_buf = fresh({sum_total}, lopt);
     Tensor sides = at::empty({2 * n_cut}, at::TensorOptions().dtype(at::kBool));
     bool* side = sides.data_ptr<bool>();
     std::vector<void*> val_p(n_cut);
